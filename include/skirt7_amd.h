@@ -153,8 +153,8 @@ int sg_sim_destroy(sg_sim* s);
  *   [4] peel-offs detected [5] stuck-path escapes [6] npp [7] walks [8] re-walk crossings
  *   [9] FP64 wall recomputes [10] device microseconds (emission and transport kernels)
  *   [11] transport workgroups per launch [12] transport microseconds (device span of the transport
- *   passes) [13] transport (walk-kernel) launches [14] walk-kernel microseconds: the sum over those
- *   launches of each launch's own duration (HIP events on its stream; launches on two streams overlap) */
+ *   passes) [13] transport (walk-kernel) launches that had walks [14] walk-kernel microseconds: the sum over
+ *   those launches of each launch's own duration (on the device's clock; launches on two streams overlap) */
 int sg_sim_run(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64_t npp, int precision,
                uint64_t* counters);
 /* sg_sim_run that allocates no device memory. No counterpart in the reference: it is for callers that
@@ -242,7 +242,8 @@ int sg_ga_population(sg_ga* ga, double* genes, double* scores);
 
 /* Transport organisation used by sg_sim_run (both give the same per-packet histories):
  * 1 (default) alternating kernels -- an event kernel over in-flight packet slots that runs the
- *   packet state machine and queues walks, and a persistent walk kernel over that queue;
+ *   packet state machine and queues peel-offs and own paths, and a persistent walk kernel over that queue,
+ *   which takes each packet on to its interaction point;
  * 0 one persistent kernel whose lanes run the state machine and the walks in turn. */
 int sg_set_pipeline(int mode);
 /* Launch tuning used by sg_sim_run (0 = keep current, negative = back to the default): block size
@@ -277,7 +278,7 @@ int sg_set_batch_alone(uint64_t min_packets);
  * FP64 walks always use the tree's own method. */
 int sg_set_mixed_topdown(int descend);
 /* Order in which the walk kernel of the event/walk pipeline takes a pass's walks: 1 sorted by a
- * coherence key (peel-offs by instrument and pixel, other walks by start point), 2 sorted and cut into
+ * coherence key (peel-offs by instrument and pixel, own paths by start point), 2 sorted and cut into
  * eight contiguous segments, each workgroup taking walks from its XCD's segment first (so that walks near
  * each other in the order share that XCD's L2), 0 (default) as appended. The order changes no packet
  * history, only the order of the tally additions. No counterpart in the reference, whose threads walk

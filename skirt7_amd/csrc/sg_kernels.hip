@@ -1106,20 +1106,11 @@ int sg_sim_destroy(sg_sim* s)
 }
 } // extern "C"
 
-// Device time of a series of transport launches: an event pair around each launch on the default
-// stream, summed once the stream has drained.
 // Device time of a run's transport: the span of its passes (start/stop on stream 0, or a span
-// measured elsewhere) and, per launch of the walk kernel, that launch's own duration between HIP
-// events recorded on its stream just before and after it. The per-launch events come from a
-// process-wide pool that is reused from call to call (one host thread drives the library).
+// measured elsewhere) and the walk kernel's own duration, summed over its launches (the start/stop spans
+// hold one kernel each; the event/walk passes take the duration on the device, PassCtl).
 struct LaunchTimer {
     std::vector<std::pair<hipEvent_t, hipEvent_t>> ev;
-    static std::vector<std::pair<hipEvent_t, hipEvent_t>>& kpool()
-    {
-        static std::vector<std::pair<hipEvent_t, hipEvent_t>> p;
-        return p;
-    }
-    size_t kused = 0;
     void start()
     {
         hipEvent_t a, b;
@@ -1129,22 +1120,14 @@ struct LaunchTimer {
         SG_HIP(hipEventRecord(a, 0));
     }
     void stop() { SG_HIP(hipEventRecord(ev.back().second, 0)); }
-    // a span measured elsewhere that covered `launches` launches
-    void add(double ms, int launches) { extra_ms += ms; extra_launches += launches; }
-    // brackets one walk-kernel launch on stream s
-    void kbefore(hipStream_t s)
+    // a span measured elsewhere that covered `launches` launches of kernel_ms in all
+    void add(double ms, int launches, double kernel_ms)
     {
-        auto& p = kpool();
-        if (kused == p.size()) {
-            hipEvent_t a, b;
-            SG_HIP(hipEventCreate(&a));
-            SG_HIP(hipEventCreate(&b));
-            p.push_back({a, b});
-        }
-        SG_HIP(hipEventRecord(p[kused].first, s));
+        extra_ms += ms;
+        extra_launches += launches;
+        extra_kernel_ms += kernel_ms;
     }
-    void kafter(hipStream_t s) { SG_HIP(hipEventRecord(kpool()[kused++].second, s)); }
-    double extra_ms = 0;
+    double extra_ms = 0, extra_kernel_ms = 0;
     int extra_launches = 0;
     int launches() const { return (int)ev.size() + extra_launches; }
     double total_ms()
@@ -1158,19 +1141,7 @@ struct LaunchTimer {
         }
         return t;
     }
-    // summed per-launch durations: the bracketed launches and the start/stop spans (one kernel each)
-    double kernel_ms()
-    {
-        double t = total_ms() - extra_ms;
-        auto& p = kpool();
-        for (size_t i = 0; i < kused; i++) {
-            float ms = 0;
-            SG_HIP(hipEventSynchronize(p[i].second));
-            SG_HIP(hipEventElapsedTime(&ms, p[i].first, p[i].second));
-            t += ms;
-        }
-        return t;
-    }
+    double kernel_ms() { return total_ms() - extra_ms + extra_kernel_ms; }
     ~LaunchTimer()
     {
         for (auto& p : ev) { (void)hipEventDestroy(p.first); (void)hipEventDestroy(p.second); }
@@ -1338,11 +1309,17 @@ __global__ void k_revive(uint32_t* state, int64_t n)
 
 static const int64_t kSplitSlots = (int64_t)1 << 22;
 static const uint64_t kSplitEmit = (uint64_t)1 << 25;   // packets emitted at once
-static const int kSplitCheck = 4;                       // passes between progress checks
+// Passes enqueued ahead of the last one whose progress the host has seen: the device never waits for the host,
+// and a run ends with at most this many empty passes (about 10 us each).
+static const int kSplitAhead = 3;
+static const int kProgressRing = 8;                     // progress words per group (more than are in flight)
 
-// Two non-blocking streams of default priority, one per slot group, and a pinned progress buffer.
+// Two non-blocking streams of default priority, one per slot group, and their progress words, which the walk
+// kernels write into coherent host memory.
 static hipStream_t g_split_stream[2] = {nullptr, nullptr};
 static unsigned long long* g_split_host = nullptr;
+static unsigned long long* g_split_host_dev = nullptr;
+static double g_clock_khz = 100000.0;                   // of the device's wall clock
 // Work buffers of the split pipeline and of the emission, shared by every simulation of the process
 // (runs are synchronous and driven by one host thread): slot groups, walk queues, progress counters,
 // launch states. Allocated on first use, grown as needed, kept until the process ends.
@@ -1361,13 +1338,108 @@ static void split_resources()
 {
     if (g_split_stream[0]) return;
     for (int g = 0; g < 2; g++) SG_HIP(hipStreamCreateWithFlags(&g_split_stream[g], hipStreamNonBlocking));
-    SG_HIP(hipHostMalloc(reinterpret_cast<void**>(&g_split_host), 8 * sizeof(unsigned long long), hipHostMallocDefault));
+    SG_HIP(hipHostMalloc(reinterpret_cast<void**>(&g_split_host), 2 * kProgressRing * sizeof(unsigned long long),
+                         hipHostMallocMapped | hipHostMallocCoherent));
+    SG_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&g_split_host_dev), g_split_host, 0));
+    int khz = 0;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, g_device) == hipSuccess && khz > 0) g_clock_khz = khz;
+}
+
+// Waits until a walk kernel on stream st has written its progress word. The stream's state is looked at now and
+// then, so that a stream that failed, or drained without writing, ends the wait.
+static unsigned long long wait_progress(const unsigned long long* word, hipStream_t st)
+{
+    for (uint64_t spin = 1;; spin++) {
+        unsigned long long v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+        if (v >> 63) return v;
+        if ((spin & 0xffff) == 0) {
+            const hipError_t e = hipStreamQuery(st);
+            if (e == hipErrorNotReady) continue;
+            SG_HIP(e);
+            v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+            if (v >> 63) return v;
+            set_error("a transport pass ended without reporting its progress");
+            throw Fail{-2};
+        }
+        __builtin_ia32_pause();
+    }
+}
+
+// The slot groups of a run of the event/walk pipeline, and the launch shapes of its kernels.
+template <typename R> struct PassGroups {
+    int n;
+    Slots<R> sl[2];
+    WalkQueue<R> q[2];
+    GroupCtl* ctl[2];
+    int pass[2];                // passes enqueued so far (the place in the progress rings)
+    int blocks, bs, ebs, nlds, order;
+    size_t shm, eshm;
+};
+
+// Event and walk passes of every group until all packets of ab have been claimed and the groups' walk queues stay
+// empty. Each group keeps kSplitAhead passes enqueued beyond the one whose progress is awaited. Returns the
+// walk launches that had requests.
+template <class W, bool ABS>
+static int run_passes(const typename W::View& v, const McArgs& ab, PassGroups<typename W::Real>& pg)
+{
+    using R = typename W::Real;
+    const hipStream_t* st = g_split_stream;
+    int seen[2] = {pg.pass[0], pg.pass[1]};
+    bool done[2] = {false, pg.n < 2};
+    int launches = 0;
+    auto enqueue = [&](int g) {
+        const int p = pg.pass[g]++;
+        const int w = g * kProgressRing + p % kProgressRing;
+        __atomic_store_n(g_split_host + w, 0ull, __ATOMIC_RELEASE);
+        PassCtl* pc = &pg.ctl[g]->pass[p % kPassRing];
+        WalkQueue<R> q = pg.q[g];
+        q.tail = &pc->tail;
+        const int64_t P = pg.sl[g].n;
+        hipLaunchKernelGGL(k_events<R>, dim3((P + pg.ebs - 1) / pg.ebs), dim3(pg.ebs), pg.eshm, st[g], ab, pg.sl[g], q,
+                           pg.ctl[g], p);
+        SG_HIP(hipGetLastError());
+        if (q.sorted) {
+            hipLaunchKernelGGL(k_key_scan, dim3(1), dim3(1024), 0, st[g], q.hist, q.off);
+            hipLaunchKernelGGL(k_key_scatter<R>, dim3(g_cus * 8), dim3(256), 0, st[g], q, ab.error);
+            SG_HIP(hipGetLastError());
+        }
+        hipLaunchKernelGGL((k_walks<W, ABS>), dim3(pg.blocks), dim3(pg.bs), pg.shm, st[g], v, ab, q, pg.sl[g], pc,
+                           g_split_host_dev + w, pg.nlds, pg.order == 2 ? kXcdSegs : 0);
+        SG_HIP(hipGetLastError());
+    };
+    while (!done[0] || !done[1]) {
+        for (int i = 0; i < kSplitAhead; i++)
+            for (int g = 0; g < pg.n; g++)
+                if (!done[g] && pg.pass[g] < seen[g] + kSplitAhead) enqueue(g);
+        for (int g = 0; g < pg.n; g++) {
+            if (done[g]) continue;
+            const unsigned long long w = wait_progress(g_split_host + g * kProgressRing + seen[g] % kProgressRing, st[g]);
+            seen[g]++;
+            const unsigned long long nq = w & ((1ull << 62) - 1);
+            SG_REQUIRE(nq <= (unsigned long long)pg.q[g].cap, "walk queue overflow");
+            launches += nq > 0;
+            // every packet claimed and no walk queued: the slots stay as they are in the passes enqueued beyond
+            done[g] = nq == 0 && ((w >> 62) & 1);
+        }
+    }
+    return launches;
+}
+
+// Duration of the groups' walk kernels (the passes have ended).
+static double walk_ms(GroupCtl* const* ctl, int n)
+{
+    double ms = 0;
+    for (int g = 0; g < n; g++) {
+        unsigned long long t = 0;
+        SG_HIP(hipMemcpy(&t, &ctl[g]->ticks, sizeof t, hipMemcpyDeviceToHost));
+        ms += (double)t / g_clock_khz;
+    }
+    return ms;
 }
 
 // Packets [first, first+count) through event and walk passes over two slot groups that alternate on two
 // streams, so that one group's event pass and the drain of its walk pass overlap the other group's
-// walks. Up to 2^25 packets are emitted at once; the host reads the progress every few passes and
-// stops when every packet has been claimed and neither group queued a walk in its last pass.
+// walks. Up to 2^25 packets are emitted at once.
 template <class W, bool ABS>
 static void run_split(sg_sim* s, const typename W::View& v, const McArgs& a, uint64_t first, uint64_t count, int nlds,
                       LaunchTimer& lt, int& blocks)
@@ -1377,11 +1449,9 @@ static void run_split(sg_sim* s, const typename W::View& v, const McArgs& a, uin
     hipStream_t* st = g_split_stream;
     const int64_t slots = g_tune_slots > 0 ? g_tune_slots : kSplitSlots;
     const int64_t P = (int64_t)std::max<uint64_t>(1, std::min<uint64_t>(count, (uint64_t)slots));
-    const int G = (P >= 2 && g_slot_groups == 2) ? 2 : 1;
+    PassGroups<R> pg{};
+    const int G = pg.n = (P >= 2 && g_slot_groups == 2) ? 2 : 1;
     const int64_t Pg[2] = {G == 2 ? (P + 1) / 2 : P, G == 2 ? P / 2 : 0};
-    Slots<R> sl[2];
-    WalkQueue<R> q[2];
-    unsigned long long* pc[2];   // per group: [1] queue tail, [3] requests claimed
     for (int g = 0; g < G; g++) {
         const int64_t cap = Pg[g] * (a.ni + 1);
         SplitPool& pl = pool();
@@ -1392,40 +1462,41 @@ static void run_split(sg_sim* s, const typename W::View& v, const McArgs& a, uin
             pl.bins[g].alloc(2 * (size_t)kKeyBins * sizeof(uint32_t));
             SG_HIP(hipMemsetAsync(pl.bins[g].p, 0, kKeyBins * sizeof(uint32_t), st[g]));
         }
-        // [1] queue tail, [3] requests claimed, [4..11] requests claimed per XCD segment
-        if (pl.prog[g].bytes < 12 * sizeof(unsigned long long)) pl.prog[g].alloc(12 * sizeof(unsigned long long));
-        pc[g] = pl.prog[g].as<unsigned long long>();
-        sl[g] = Slots<R>{pl.slots[g].as<R>(),
-                         reinterpret_cast<uint32_t*>(pl.slots[g].as<unsigned char>() + (size_t)Pg[g] * SR_NR * sizeof(R)),
-                         Pg[g]};
+        if (pl.prog[g].bytes < sizeof(GroupCtl)) pl.prog[g].alloc(sizeof(GroupCtl));
+        pg.ctl[g] = pl.prog[g].as<GroupCtl>();
+        Slots<R>& sl = pg.sl[g];
+        sl = Slots<R>{pl.slots[g].as<R>(),
+                      reinterpret_cast<uint32_t*>(pl.slots[g].as<unsigned char>() + (size_t)Pg[g] * SR_NR * sizeof(R)), Pg[g]};
         // requests, then (sorted order) the sorted requests, keys, ranks, bin counts and offsets
         unsigned char* qb = pl.queue[g].as<unsigned char>();
-        q[g] = WalkQueue<R>{};
-        q[g].req = reinterpret_cast<WalkReq<R>*>(qb);
-        q[g].cap = cap;
-        q[g].tail = pc[g] + 1;
+        WalkQueue<R>& q = pg.q[g];
+        q.req = reinterpret_cast<WalkReq<R>*>(qb);
+        q.cap = cap;
         if (sorted) {
             unsigned char* p = qb + (size_t)cap * sizeof(WalkReq<R>);
-            q[g].sorted = reinterpret_cast<WalkReq<R>*>(p);
+            q.sorted = reinterpret_cast<WalkReq<R>*>(p);
             p += (size_t)cap * sizeof(WalkReq<R>);
-            q[g].key = reinterpret_cast<uint32_t*>(p);
-            q[g].rank = q[g].key + cap;
-            q[g].hist = pl.bins[g].as<uint32_t>();
-            q[g].off = q[g].hist + kKeyBins;
+            q.key = reinterpret_cast<uint32_t*>(p);
+            q.rank = q.key + cap;
+            q.hist = pl.bins[g].as<uint32_t>();
+            q.off = q.hist + kKeyBins;
         }
-        // slot states PS_FRESH and slot counts zero (adjacent arrays)
-        SG_HIP(hipMemsetAsync(sl[g].u + (size_t)SU_STATE * Pg[g], 0, (size_t)Pg[g] * (SU_NU - SU_STATE) * sizeof(uint32_t),
+        // progress records; slot states PS_FRESH and slot counts zero (adjacent arrays)
+        SG_HIP(hipMemsetAsync(pg.ctl[g], 0, sizeof(GroupCtl), st[g]));
+        SG_HIP(hipMemsetAsync(sl.u + (size_t)SU_STATE * Pg[g], 0, (size_t)Pg[g] * (SU_NU - SU_STATE) * sizeof(uint32_t),
                               st[g]));
     }
-    const int bs = g_tune_block;
-    const size_t shm = (size_t)nlds * sizeof(int32_t);
+    const int bs = pg.bs = g_tune_block;
+    pg.nlds = nlds;
+    pg.order = g_walk_order;
+    pg.shm = (size_t)nlds * sizeof(int32_t);
     int per = 0;
-    SG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_walks<W, ABS>, bs, shm));
-    blocks = std::max(1, per) * g_cus;
+    SG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_walks<W, ABS>, bs, pg.shm));
+    pg.blocks = blocks = std::max(1, per) * g_cus;
     // event workgroups stage up to blockDim * (ni + 1) requests in LDS
-    int ebs = 256;
-    while (ebs > 64 && staged_bytes<R>(ebs, a.ni) > 64 * 1024) ebs /= 2;
-    const size_t eshm = staged_bytes<R>(ebs, a.ni);
+    pg.ebs = 256;
+    while (pg.ebs > 64 && staged_bytes<R>(pg.ebs, a.ni) > 64 * 1024) pg.ebs /= 2;
+    pg.eshm = staged_bytes<R>(pg.ebs, a.ni);
     const uint64_t batch = std::min<uint64_t>(count, g_emit_batch ? g_emit_batch : kSplitEmit);
     const size_t rsz = sizeof(R);
     DevBuf& emitted = pool().emitted;
@@ -1455,61 +1526,28 @@ static void run_split(sg_sim* s, const typename W::View& v, const McArgs& a, uin
         hipLaunchKernelGGL(k_emit<R>, dim3(emb), dim3(256), 0, st[0], ab, emitted.as<R>(), emitdraw.as<uint32_t>());
         SG_HIP(hipGetLastError());
         for (int g = 0; g < G && b > 0; g++)
-            hipLaunchKernelGGL(k_revive, dim3((Pg[g] + 255) / 256), dim3(256), 0, st[0], sl[g].u + (size_t)SU_STATE * Pg[g],
-                               Pg[g]);
+            hipLaunchKernelGGL(k_revive, dim3((Pg[g] + 255) / 256), dim3(256), 0, st[0],
+                               pg.sl[g].u + (size_t)SU_STATE * Pg[g], Pg[g]);
         if (b == 0) SG_HIP(hipEventRecord(ev_start, st[0]));
         if (G == 2) {
             SG_HIP(hipEventRecord(ev_join, st[0]));
             SG_HIP(hipStreamWaitEvent(st[1], ev_join, 0));
         }
-        for (;;) {
-            for (int p = 0; p < kSplitCheck; p++)
-                for (int g = 0; g < G; g++) {
-                    SG_HIP(hipMemsetAsync(pc[g] + 1, 0, sizeof(unsigned long long), st[g]));
-                    hipLaunchKernelGGL(k_events<R>, dim3((Pg[g] + ebs - 1) / ebs), dim3(ebs), eshm, st[g], ab, sl[g], q[g]);
-                    SG_HIP(hipGetLastError());
-                    if (q[g].sorted) {
-                        hipLaunchKernelGGL(k_key_scan, dim3(1), dim3(1024), 0, st[g], q[g].hist, q[g].off);
-                        hipLaunchKernelGGL(k_key_scatter<R>, dim3(g_cus * 8), dim3(256), 0, st[g], q[g], ab.error);
-                        SG_HIP(hipGetLastError());
-                    }
-                    SG_HIP(hipMemsetAsync(pc[g] + 3, 0, (1 + kXcdSegs) * sizeof(unsigned long long), st[g]));
-                    lt.kbefore(st[g]);
-                    hipLaunchKernelGGL((k_walks<W, ABS>), dim3(blocks), dim3(bs), shm, st[g], v, ab, q[g], sl[g], pc[g] + 3,
-                                       nlds, g_walk_order == 2 ? kXcdSegs : 0);
-                    SG_HIP(hipGetLastError());
-                    lt.kafter(st[g]);
-                    walk_launches++;
-                }
-            // progress after the last pass of each group: packets claimed, walks each group queued
-            if (G == 2) {
-                SG_HIP(hipEventRecord(ev_join, st[1]));
-                SG_HIP(hipStreamWaitEvent(st[0], ev_join, 0));
-            }
-            SG_HIP(hipMemcpyAsync(g_split_host, claims, sizeof(unsigned long long), hipMemcpyDeviceToHost, st[0]));
-            for (int g = 0; g < G; g++)
-                SG_HIP(hipMemcpyAsync(g_split_host + 1 + g, pc[g] + 1, sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                                      st[0]));
-            SG_HIP(hipStreamSynchronize(st[0]));
-            bool queued = false;
-            for (int g = 0; g < G; g++) {
-                SG_REQUIRE(g_split_host[1 + g] <= (unsigned long long)(Pg[g] * (a.ni + 1)), "walk queue overflow");
-                queued = queued || g_split_host[1 + g] > 0;
-            }
-            if (g_split_host[0] >= ab.count && !queued) break;
-        }
+        walk_launches += run_passes<W, ABS>(v, ab, pg);
     }
-    for (int g = 0; g < G; g++)
-        hipLaunchKernelGGL(k_slot_counts, dim3(std::min<int64_t>((Pg[g] + 255) / 256, 1024)), dim3(256), 0, st[0], sl[g].u,
-                           Pg[g], a.counters);
-    SG_HIP(hipGetLastError());
-    for (int g = 0; g < G; g++) SG_HIP(hipEventRecord(ev_end[g], st[g]));
+    // each group's counts on its own stream, behind its last passes
+    for (int g = 0; g < G; g++) {
+        hipLaunchKernelGGL(k_slot_counts, dim3(std::min<int64_t>((Pg[g] + 255) / 256, 1024)), dim3(256), 0, st[g],
+                           pg.sl[g].u, Pg[g], a.counters);
+        SG_HIP(hipGetLastError());
+        SG_HIP(hipEventRecord(ev_end[g], st[g]));
+    }
     SG_HIP(hipStreamSynchronize(st[0]));
     if (G == 2) SG_HIP(hipStreamSynchronize(st[1]));
     float ms = 0, ms1 = 0;
     SG_HIP(hipEventElapsedTime(&ms, ev_start, ev_end[0]));
     if (G == 2) SG_HIP(hipEventElapsedTime(&ms1, ev_start, ev_end[1]));
-    lt.add(std::max(ms, ms1), walk_launches);
+    lt.add(std::max(ms, ms1), walk_launches, walk_ms(pg.ctl, G));
     (void)hipEventDestroy(ev_start);
     (void)hipEventDestroy(ev_join);
     for (int g = 0; g < 2; g++) (void)hipEventDestroy(ev_end[g]);
@@ -1800,61 +1838,49 @@ static void run_static(sg_sim* s, const typename W::View& v, const McArgs& a0, i
     hipStream_t st = g_split_stream[0];
     const int64_t P = (int64_t)std::max<uint64_t>(1, std::min<uint64_t>(a0.count, (uint64_t)kStaticSlots));
     const int64_t cap = P * (a0.ni + 1);
-    // layout of the static array: slots, walk requests, progress counters, launch states, draw counts
+    // layout of the static array: slots, walk requests, progress records, launch states, draw counts
     const size_t o_q = align256(slot_bytes<R>(P));
     const size_t o_pc = o_q + align256((size_t)cap * sizeof(WalkReq<R>));
-    const size_t o_em = o_pc + 256;
+    const size_t o_em = o_pc + align256(sizeof(GroupCtl));
     const size_t o_ed = o_em + align256(7 * a0.count * sizeof(R));
     const size_t need = o_ed + align256(a0.count * sizeof(uint32_t));
     SG_REQUIRE(need <= kStaticScratchBytes, "sg_sim_run_static: the run needs " + std::to_string(need) +
                                                 " bytes of work memory, more than the static array holds");
     unsigned char* base = static_cast<unsigned char*>(g_scratch[g_device]);
     SG_REQUIRE(base != nullptr, "sg_sim_run_static: the static work array of this device is not set up");
-    Slots<R> sl{reinterpret_cast<R*>(base), reinterpret_cast<uint32_t*>(base + (size_t)P * SR_NR * sizeof(R)), P};
-    unsigned long long* pc = reinterpret_cast<unsigned long long*>(base + o_pc);   // [1] queue tail, [3] claims
-    WalkQueue<R> q{};
-    q.req = reinterpret_cast<WalkReq<R>*>(base + o_q);
-    q.cap = cap;
-    q.tail = pc + 1;
+    PassGroups<R> pg{};
+    pg.n = 1;
+    Slots<R>& sl = pg.sl[0];
+    sl = Slots<R>{reinterpret_cast<R*>(base), reinterpret_cast<uint32_t*>(base + (size_t)P * SR_NR * sizeof(R)), P};
+    pg.ctl[0] = reinterpret_cast<GroupCtl*>(base + o_pc);
+    pg.q[0].req = reinterpret_cast<WalkReq<R>*>(base + o_q);
+    pg.q[0].cap = cap;
     McArgs a = a0;
     a.emitted = base + o_em;
     a.emit_draw = reinterpret_cast<uint32_t*>(base + o_ed);
     a.next_packet = s->next.as<unsigned long long>();
     // cleared by kernels: slot states (PS_FRESH) and counts, progress, the packet claims, counters, error flag
     fill_u32(sl.u + (size_t)SU_STATE * P, P * (SU_NU - SU_STATE), st);
-    fill_u32(pc, 8, st);
+    fill_u32(pg.ctl[0], sizeof(GroupCtl) / sizeof(uint32_t), st);
     fill_u32(s->next.p, 2, st);
     fill_u32(s->counters.p, 2 * SG_NCOUNTERS, st);
     fill_u32(s->err.p, 1, st);
-    const int bs = g_tune_block;
-    const size_t shm = (size_t)nlds * sizeof(int32_t);
+    pg.bs = g_tune_block;
+    pg.nlds = nlds;
+    pg.shm = (size_t)nlds * sizeof(int32_t);
     int per = 0;
-    SG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_walks<W, ABS>, bs, shm));
-    blocks = std::max(1, per) * g_cus;
-    int ebs = 256;
-    while (ebs > 64 && staged_bytes<R>(ebs, a.ni) > 64 * 1024) ebs /= 2;
-    const size_t eshm = staged_bytes<R>(ebs, a.ni);
+    SG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_walks<W, ABS>, pg.bs, pg.shm));
+    pg.blocks = blocks = std::max(1, per) * g_cus;
+    pg.ebs = 256;
+    while (pg.ebs > 64 && staged_bytes<R>(pg.ebs, a.ni) > 64 * 1024) pg.ebs /= 2;
+    pg.eshm = staged_bytes<R>(pg.ebs, a.ni);
     if (a.count > 0) {
         const int emb = (int)std::min<uint64_t>((a.count + 255) / 256, (uint64_t)g_cus * 16);
         hipLaunchKernelGGL(k_emit<R>, dim3(emb), dim3(256), 0, st, a, static_cast<R*>(const_cast<void*>(a.emitted)),
                            const_cast<uint32_t*>(a.emit_draw));
         SG_HIP(hipGetLastError());
     }
-    for (;;) {
-        for (int p = 0; p < kSplitCheck; p++) {
-            fill_u32(pc + 1, 2, st);
-            hipLaunchKernelGGL(k_events<R>, dim3((P + ebs - 1) / ebs), dim3(ebs), eshm, st, a, sl, q);
-            SG_HIP(hipGetLastError());
-            fill_u32(pc + 3, 2, st);
-            hipLaunchKernelGGL((k_walks<W, ABS>), dim3(blocks), dim3(bs), shm, st, v, a, q, sl, pc + 3, nlds, 0);
-            SG_HIP(hipGetLastError());
-        }
-        SG_HIP(hipMemcpyAsync(g_split_host, a.next_packet, sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
-        SG_HIP(hipMemcpyAsync(g_split_host + 1, pc + 1, sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
-        SG_HIP(hipStreamSynchronize(st));
-        SG_REQUIRE(g_split_host[1] <= (unsigned long long)cap, "walk queue overflow");
-        if (g_split_host[0] >= a.count && g_split_host[1] == 0) break;
-    }
+    run_passes<W, ABS>(v, a, pg);
     hipLaunchKernelGGL(k_slot_counts, dim3(std::min<int64_t>((P + 255) / 256, 1024)), dim3(256), 0, st, sl.u, P, a.counters);
     SG_HIP(hipGetLastError());
     SG_HIP(hipStreamSynchronize(st));

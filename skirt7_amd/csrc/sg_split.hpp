@@ -1,14 +1,14 @@
 // sg_split.hpp -- the photon-packet life cycle (MonteCarloSimulation::dostellaremissionchunk,
 // MonteCarloSimulation.cpp:259-297) as two alternating kernels over device-resident queues:
 //
-//   k_events: one thread per in-flight packet slot runs the packet's state machine up to its next
-//             walk -- launch, emission peel-offs, escape/absorption and the stop test, biased
-//             propagation, scattering peel-offs and the new direction -- and appends the walks it
-//             needs (peel-off, own path, propagation re-walk) to the walk queue;
+//   k_events: one thread per in-flight packet slot runs the packet's state machine from the end of
+//             its propagation (or its launch) to its next own path -- launch, peel-offs, the new
+//             direction -- and appends the walks it needs (peel-offs and the own path) to the queue;
 //   k_walks:  persistent lanes take walk requests from the queue and run the cell walks, with the
 //             same ballot-compacted refill as the lane pipeline; a peel-off walk ends with its
-//             detection (FrameInstrument::detect), an own-path or propagation walk with its result
-//             written back to the packet slot.
+//             detection (FrameInstrument::detect); a lane that ends an own path draws the packet's
+//             escape, absorption, stop test and biased path length, and walks on to the interaction
+//             point itself (own_path_end), whose place goes to the packet slot.
 //
 // The walk kernel carries only the walker and the running sums, so it keeps several times more
 // waves in flight than a kernel that also holds the event logic; the event kernel's FP64 and libm
@@ -27,8 +27,10 @@ enum SlotR { SR_RX = 0, SR_RY, SR_RZ, SR_KX, SR_KY, SR_KZ, SR_L, SR_RES, SR_NR }
 // propagation walk left it (-1: unknown), handed to the walks that start there.
 enum SlotU { SU_PLO = 0, SU_PHI, SU_DRAW, SU_W0, SU_W1, SU_W2, SU_W3, SU_NSCATT, SU_HINT,
              SU_STATE, SU_CPK, SU_CSCAT, SU_CPEEL, SU_CWALK, SU_NU };
+// PS_OWN: the packet's own path is in the walk queue; the walk kernel leaves it at its interaction point
+// (PS_PROP) or finished (PS_FRESH: the slot takes a new packet).
 enum PacketState : uint32_t { PS_FRESH = 0, PS_OWN, PS_PROP, PS_DEAD };
-enum WalkKind : uint32_t { WK_PEEL = 0, WK_OWN = 1, WK_PROP = 2 };
+enum WalkKind : uint32_t { WK_PEEL = 0, WK_OWN = 1 };
 
 // Packet slots: structure of arrays, n slots.
 template <typename R> struct Slots {
@@ -44,8 +46,7 @@ template <typename R> __host__ __device__ constexpr size_t slot_bytes(int64_t n)
 }
 
 // Walk requests: origin (3), direction (3, unused for peel-offs: the instrument's direction is
-// taken from its record) and a value (peel-off luminosity, own-path luminosity, or propagation
-// target optical depth) in the run's real type; a tag (kind | instrument << 2), an index (packet
+// taken from its record) and a value (peel-off or own-path luminosity) in the run's real type; a tag (kind | instrument << 2), an index (packet
 // slot, or pixel for a peel-off) and the start leaf hint of the walker. In the LDS staging area
 // they are structure-of-arrays (QR_*, QU_* fields); in the queues one record per request, so that
 // a request moved to its sorted place, or read by a lane, is one contiguous block.
@@ -57,10 +58,24 @@ template <typename R> struct alignas(16) WalkReq {
 };
 static_assert(sizeof(WalkReq<float>) == 48 && sizeof(WalkReq<double>) == 80, "walk request records");
 
+constexpr int kXcdSegs = 8;
+// Progress of one pass of a slot group. A group's passes use a ring of these records; the event kernel of
+// a pass clears the next one, so that no fill runs between the kernels.
+struct PassCtl {
+    unsigned long long tail;            // requests appended by the event kernel
+    unsigned long long claim;           // requests taken by the walk kernel
+    unsigned long long seg[kXcdSegs];   // the same per XCD segment
+    unsigned long long t0inv, t1;       // walk kernel: complement of its first wave's start, last wave's end (clock ticks)
+};
+constexpr int kPassRing = 4;
+struct GroupCtl {
+    PassCtl pass[kPassRing];
+    unsigned long long ticks;           // walk kernels' durations, summed over the finished passes
+};
+
 // Walk order. The walks of a pass are sorted by a coherence key before the walk kernel takes them:
 // peel-offs by instrument and the Morton order of their pixel (rays toward one instrument through
-// neighbouring pixels cross the same cells), own-path and propagation walks by the Morton order of
-// their start point. Lanes and waves that run at the same time then touch a small part of the grid,
+// neighbouring pixels cross the same cells), own paths by the Morton order of their start point. Lanes and waves that run at the same time then touch a small part of the grid,
 // which the L2 cache of their XCD holds. A counting sort: the event kernel counts each request into
 // its key's bin and keeps its rank there, a one-block scan turns the counts into bin offsets (and
 // clears them), and a scatter moves each request to offset + rank. Histories do not depend on the
@@ -100,8 +115,7 @@ __device__ __forceinline__ uint32_t spread3(uint32_t v)   // 5 bits -> every thi
     v = (v | (v << 2)) & 0x1249u;
     return v;
 }
-// The coherence key of a request: 4 bits of class (peel-off instrument 0-7, own path 8, propagation
-// 9) above 12 bits of Morton order (a peel-off's pixel on a 64 x 64 raster of its frame; a start
+// The coherence key of a request: 4 bits of class (peel-off instrument 0-7, own path 8) above 12 bits of Morton order (a peel-off's pixel on a 64 x 64 raster of its frame; a start
 // point on a 16 x 16 x 16 raster of the grid box).
 template <typename R>
 __device__ __forceinline__ uint32_t walk_key(const McArgs& a, const InstrDev* instr, uint32_t tag, uint32_t idx, R ox,
@@ -122,7 +136,7 @@ __device__ __forceinline__ uint32_t walk_key(const McArgs& a, const InstrDev* in
     const uint32_t qx = q((double)ox, a.key_lo[0], a.key_scale[0]);
     const uint32_t qy = q((double)oy, a.key_lo[1], a.key_scale[1]);
     const uint32_t qz = q((double)oz, a.key_lo[2], a.key_scale[2]);
-    return ((kind == WK_OWN ? 8u : 9u) << 12) | spread3(qx) | (spread3(qy) << 1) | (spread3(qz) << 2);
+    return (8u << 12) | spread3(qx) | (spread3(qy) << 1) | (spread3(qz) << 2);
 }
 
 // Appends one request per active lane (one atomic per wave); returns this lane's queue position.
@@ -141,8 +155,8 @@ __device__ __forceinline__ uint64_t wave_append(unsigned long long* tail)
 
 // Walk requests of one workgroup staged in LDS (structure of arrays) in two parts: peel-offs (origin,
 // value, tag, index, hint: a peel-off walks toward its instrument, so it carries no direction) in capp
-// entries, and the own-path and propagation walks (with their direction) in capw entries, each part with
-// its own count. A lane stages at most ni peel-offs and one other walk per pass, so capp = ni and capw = 1
+// entries, and the own paths (with their direction) in capw entries, each part with
+// its own count. A lane stages at most ni peel-offs and one own path per pass, so capp = ni and capw = 1
 // entries per lane suffice, 28 + 40 / ni bytes per request slot in FP32 instead of 40, which leaves room
 // for more workgroups per CU. The workgroup appends them to the walk queue as one block with a single
 // global atomic.
@@ -269,11 +283,12 @@ __device__ __forceinline__ void hg_scatter(PacketRng& rng, R gg, R& kx, R& ky, R
     kx = nkx; ky = nky; kz = nkz;
 }
 
-// Event pass: every slot advances its packet to its next walk (or takes a new packet). Dynamic LDS:
-// the workgroup's staged requests, blockDim.x * a.ni peel-offs and blockDim.x other walks (the most one
-// pass can append: a lane's pass ends with the walk it requests, after at most one set of peel-offs).
+// Event pass: every slot advances its packet to its next own path (or takes a new packet). Dynamic LDS:
+// the workgroup's staged requests, blockDim.x * a.ni peel-offs and blockDim.x own paths (the most one
+// pass can append: a lane's pass ends with the own path it requests, after at most one set of peel-offs).
+// gc/pass: the group's progress ring; this pass's record is q.tail's.
 template <typename R>
-__global__ void __launch_bounds__(256) k_events(const McArgs a, Slots<R> sl, WalkQueue<R> q)
+__global__ void __launch_bounds__(256) k_events(const McArgs a, Slots<R> sl, WalkQueue<R> q, GroupCtl* gc, int pass)
 {
     __shared__ InstrDev s_instr[SG_MAX_INSTR];
     __shared__ unsigned s_cntp, s_cntw;
@@ -286,13 +301,22 @@ __global__ void __launch_bounds__(256) k_events(const McArgs a, Slots<R> sl, Wal
                       reinterpret_cast<uint32_t*>(wbase + (size_t)capw * QR_NR * sizeof(R)), capw, &s_cntw};
     if (threadIdx.x < SG_MAX_INSTR) s_instr[threadIdx.x] = a.scene->instr[threadIdx.x];
     if (threadIdx.x == 0) { s_cntp = 0; s_cntw = 0; }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        // the previous pass's walk kernel has ended: its duration; the next pass's record, last used three
+        // passes ago, is cleared
+        const PassCtl& pv = gc->pass[(pass + kPassRing - 1) % kPassRing];
+        if (pv.t1 > ~pv.t0inv) gc->ticks += pv.t1 - ~pv.t0inv;
+        PassCtl& nx = gc->pass[(pass + 1) % kPassRing];
+        nx.tail = 0; nx.claim = 0; nx.t0inv = 0; nx.t1 = 0;
+        for (int k = 0; k < kXcdSegs; k++) nx.seg[k] = 0;
+    }
     __syncthreads();
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     // every lane stays to the end: the counts below are summed over the whole wave
     uint32_t state = i < sl.n ? sl.fu(SU_STATE, i) : (uint32_t)PS_DEAD;
     uint32_t c_pk = 0, c_scat = 0, c_npeel = 0, c_walks = 0;
     if (state != PS_DEAD) {
-        const R albedo = (R)a.albedo, gg = (R)a.g;
+        const R gg = (R)a.g;
         R rx = sl.fr(SR_RX, i), ry = sl.fr(SR_RY, i), rz = sl.fr(SR_RZ, i);
         R kx = sl.fr(SR_KX, i), ky = sl.fr(SR_KY, i), kz = sl.fr(SR_KZ, i);
         R L = sl.fr(SR_L, i);
@@ -333,38 +357,6 @@ __global__ void __launch_bounds__(256) k_events(const McArgs a, Slots<R> sl, Wal
                 state = PS_OWN;
                 break;
             }
-            if (state == PS_OWN) {
-                // DustSystem::fillOpticalDepth check (DustSystem.cpp:952-955)
-                R taupath = sl.fr(SR_RES, i);
-                if (taupath < (R)0 || isnan(taupath) || isinf(taupath)) {
-                    atomicOr(a.error, 1);
-                    state = PS_FRESH;
-                    continue;
-                }
-                // simulateescapeandabsorption, single component (MonteCarloSimulation.cpp:432-461)
-                R expfactor = -rexpm1<R>(-taupath);
-                L = L * albedo * expfactor;
-                if (L <= (R)0 || (L <= (R)a.Lthreshold && nscatt >= a.minfs)) { state = PS_FRESH; continue; }
-                if (taupath != (R)0) {
-                    // simulatepropagation (MonteCarloSimulation.cpp:513-531): biased free path, then the
-                    // re-walk to the interaction point
-                    R tt;
-                    if (a.xi == 0.0) tt = exponcutoff(rng, taupath);
-                    else {
-                        R X = uni<R>(rng);
-                        tt = (X < (R)a.xi) ? uni<R>(rng) * taupath : exponcutoff(rng, taupath);
-                        R pp = -rexp<R>(-tt) / rexpm1<R>(-taupath);
-                        R qq = ((R)1.0 - (R)a.xi) * pp + (R)a.xi / taupath;
-                        L = L * (pp / qq);
-                    }
-                    sq.push(WK_PROP, 0, (uint32_t)i, rx, ry, rz, kx, ky, kz, tt, hint);
-                    state = PS_PROP;
-                    break;
-                }
-                // zero optical depth along the path: scattering in place
-                state = PS_PROP;
-                sl.fr(SR_RES, i) = (R)0;
-            }
             if (state == PS_PROP) {
                 // PhotonPackage::propagate (PhotonPackage.cpp:93-96) by pathlength(tau)
                 R d = sl.fr(SR_RES, i);
@@ -377,8 +369,8 @@ __global__ void __launch_bounds__(256) k_events(const McArgs a, Slots<R> sl, Wal
                 c_walks += np + 1;
                 sq.push(WK_OWN, 0, (uint32_t)i, rx, ry, rz, kx, ky, kz, L, hint);
                 state = PS_OWN;
-                break;
             }
+            break;   // PS_OWN here: a request that was refused; the slot stays idle
         }
         sl.fr(SR_RX, i) = rx; sl.fr(SR_RY, i) = ry; sl.fr(SR_RZ, i) = rz;
         sl.fr(SR_KX, i) = kx; sl.fr(SR_KY, i) = ky; sl.fr(SR_KZ, i) = kz;
@@ -491,33 +483,43 @@ __global__ void __launch_bounds__(256) k_slot_counts(const uint32_t* u, int64_t 
     }
 }
 
-// Request claims of one wave: chunks of kClaimChunk requests per global atomic, handed out in order to
-// the lanes that ask. Called by the whole wave; cur/end is the wave's current chunk (equal in every
-// lane). Returns whether this lane got request r.
-constexpr uint64_t kClaimChunk = 128;
-__device__ __forceinline__ bool chunk_claim(unsigned long long* ctr, uint64_t nq, bool want, uint64_t& cur,
-                                            uint64_t& end, uint64_t& r)
+// Request claims of one wave: chunks of requests by one global atomic each, handed out in order to the lanes
+// that ask. Called by the whole wave; cur/end is the wave's current chunk and last the place of its latest
+// claim (wave-uniform). The chunk follows what is left of the queue, an eighth of a wave's even share at
+// most kClaimChunk: large while the queue is long (few atomics), small near its end and for short queues, so
+// that the last walks are spread over the waves instead of queueing up in a few. Returns whether this lane
+// got request r; a lane that did not finds the queue exhausted.
+constexpr uint64_t kClaimChunk = 128, kClaimMin = 16;
+__device__ __forceinline__ bool chunk_claim(unsigned long long* ctr, uint64_t nq, uint64_t nwaves, bool want,
+                                            uint64_t& cur, uint64_t& end, uint64_t& last, uint64_t& r)
 {
-    const uint64_t mask = __ballot(want);
-    const uint64_t k = (uint64_t)__popcll(mask);
-    if (k == 0) return false;
+    bool served = false;
     const int lane = __lane_id();
-    const uint64_t rank = (uint64_t)__popcll(mask & (lane ? (~0ull >> (64 - lane)) : 0ull));
-    const uint64_t avail = end - cur;
-    uint64_t nb = 0, ne = 0;
-    if (avail < k) {
-        unsigned long long b = 0;
-        if (lane == 0) b = atomicAdd(ctr, (unsigned long long)kClaimChunk);
-        const uint32_t lo = __shfl((uint32_t)b, 0), hi = __shfl((uint32_t)(b >> 32), 0);
-        nb = ((uint64_t)hi << 32) | lo;
-        ne = nb >= nq ? nb : min(nb + kClaimChunk, nq);
+    for (;;) {
+        const uint64_t mask = __ballot(want && !served);
+        const uint64_t k = (uint64_t)__popcll(mask);
+        if (k == 0) break;
+        if (cur == end) {
+            if (last >= nq) break;
+            const uint64_t chunk = min(max((nq - last) / (2 * nwaves), kClaimMin), kClaimChunk);
+            unsigned long long b = 0;
+            if (lane == 0) b = atomicAdd(ctr, (unsigned long long)chunk);
+            const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b);
+            const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
+            last = ((uint64_t)hi << 32) | lo;
+            cur = min(last, nq);
+            end = min(last + chunk, nq);
+            if (cur == end) break;
+        }
+        const uint64_t take = min(k, end - cur);
+        const uint64_t rank = (uint64_t)__popcll(mask & (lane ? (~0ull >> (64 - lane)) : 0ull));
+        if (want && !served && rank < take) {
+            r = cur + rank;
+            served = true;
+        }
+        cur += take;
     }
-    bool ok;
-    if (rank < avail) { r = cur + rank; ok = true; }
-    else { r = nb + (rank - avail); ok = r < ne; }
-    if (avail >= k) cur += k;
-    else { cur = min(nb + (k - avail), ne); end = ne; }
-    return ok && want;
+    return served;
 }
 
 // Request claims by XCD segment: the requests [0, nq) of a pass, in walk order, are cut into kXcdSegs
@@ -526,7 +528,6 @@ __device__ __forceinline__ bool chunk_claim(unsigned long long* ctr, uint64_t nq
 // is exhausted. Walks that are neighbours in the walk order (start points or pixels close together) thus meet
 // in the same XCD's L2. ctr holds one counter per segment. Lanes the wave's chunk does not serve stay idle
 // until the next claim; exhausted (wave-uniform) becomes true when every segment is exhausted.
-constexpr int kXcdSegs = 8;
 __device__ __forceinline__ bool seg_claim(unsigned long long* ctr, uint64_t nq, bool want, int& seg, int& tried,
                                           uint64_t& cur, uint64_t& end, uint64_t& r, bool& exhausted)
 {
@@ -582,15 +583,104 @@ template <> struct WalkWaves<TreeW64> { static constexpr int value = SG_W64_WAVE
 template <> struct WalkWaves<VoroW<double>> { static constexpr int value = 3; };   // 4 would spill
 template <> struct WalkWaves<VoroW<float>> { static constexpr int value = 3; };
 
-// Walk pass: persistent lanes over the requests [0, *q.tail).
+// The end of an own path (lane's walk of slot idx, request w): DustSystem::fillOpticalDepth's check
+// (DustSystem.cpp:952-955), simulateescapeandabsorption (MonteCarloSimulation.cpp:432-461), the stop test
+// and simulatepropagation (:513-531). Either the packet is finished or scatters where it is, which the slot's
+// state tells the next event pass, or the lane goes on with the walk to the interaction point (ST_PROP).
+// Done here rather than in the event kernel, the re-walk shares this pass with the long walks: as a pass of
+// its own it took a fifth of the walk time for 3% of the crossings, and each scattering took two event
+// passes.
+template <class W>
+__device__ __forceinline__ void own_path_end(Hot<W>& h, const typename W::View& g, const int32_t* lds, int nlds,
+                                             const McArgs& a, const Slots<typename W::Real>& sl, uint32_t idx,
+                                             const WalkReq<typename W::Real>* w)
+{
+    using R = typename W::Real;
+    const R taupath = h.tau;
+    h.stage = ST_NEWPKT;
+    if (taupath < (R)0 || isnan(taupath) || isinf(taupath)) {
+        atomicOr(a.error, 1);
+        sl.fu(SU_STATE, idx) = PS_FRESH;
+        return;
+    }
+    const R expfactor = -rexpm1<R>(-taupath);
+    R L = h.L0 * (R)a.albedo * expfactor;
+    if (L <= (R)0 || (L <= (R)a.Lthreshold && (int)sl.fu(SU_NSCATT, idx) >= a.minfs)) {
+        sl.fu(SU_STATE, idx) = PS_FRESH;
+        return;
+    }
+    sl.fu(SU_STATE, idx) = PS_PROP;
+    if (taupath == (R)0) {
+        // zero optical depth along the path: scattering in place
+        sl.fr(SR_L, idx) = L;
+        sl.fr(SR_RES, idx) = (R)0;
+        return;
+    }
+    PacketRng rng;
+    rng.k0 = a.seed; rng.k1 = a.member; rng.ell = (uint32_t)a.ell;
+    rng.plo = sl.fu(SU_PLO, idx); rng.phi = sl.fu(SU_PHI, idx); rng.draw = sl.fu(SU_DRAW, idx);
+    rng.w0 = sl.fu(SU_W0, idx); rng.w1 = sl.fu(SU_W1, idx); rng.w2 = sl.fu(SU_W2, idx); rng.w3 = sl.fu(SU_W3, idx);
+    R tt;
+    if (a.xi == 0.0) tt = exponcutoff(rng, taupath);
+    else {
+        const R X = uni<R>(rng);
+        tt = (X < (R)a.xi) ? uni<R>(rng) * taupath : exponcutoff(rng, taupath);
+        const R pp = -rexp<R>(-tt) / rexpm1<R>(-taupath);
+        const R qq = ((R)1.0 - (R)a.xi) * pp + (R)a.xi / taupath;
+        L = L * (pp / qq);
+    }
+    sl.fr(SR_L, idx) = L;
+    sl.fu(SU_DRAW, idx) = rng.draw;
+    sl.fu(SU_W0, idx) = rng.w0; sl.fu(SU_W1, idx) = rng.w1; sl.fu(SU_W2, idx) = rng.w2; sl.fu(SU_W3, idx) = rng.w3;
+    if constexpr (W::kHint) h.w.init_hinted(g, lds, nlds, w->o[0], w->o[1], w->o[2], w->d[0], w->d[1], w->d[2], (int)w->hint);
+    else h.w.init(g, lds, nlds, w->o[0], w->o[1], w->o[2], w->d[0], w->d[1], w->d[2]);
+    h.start_walk(ST_PROP, tt);
+}
+
+// A finished walk's result: a peel-off's detection (FrameInstrument::detect, FrameInstrument.cpp:33-47), an own
+// path's end, or the interaction point's distance and leaf for the packet slot. Afterwards the lane is idle, or
+// walks on to the interaction point.
+template <class W>
+__device__ __forceinline__ void walk_end(Hot<W>& h, const typename W::View& g, const int32_t* lds, int nlds,
+                                         const McArgs& a, const Slots<typename W::Real>& sl, const InstrDev* instr,
+                                         uint32_t inst, uint32_t idx, const WalkReq<typename W::Real>* w)
+{
+    if (h.stage == ST_PEELW_DONE) {
+        const InstrDev& in = instr[inst];
+        unsafeAtomicAdd(in.frame + (size_t)a.ell * in.Nx * in.Ny + idx, (double)(h.L0 * rexp<typename W::Real>(-h.tau)));
+        h.stage = ST_NEWPKT;
+    } else if (h.stage == ST_PROP_DONE) {
+        sl.fr(SR_RES, idx) = prop_length(h);
+        // the leaf holding the interaction point: where the packet's next walks start
+        if constexpr (W::kHint) sl.fu(SU_HINT, idx) = (uint32_t)h.w.hint();
+        h.stage = ST_NEWPKT;
+    } else if (h.stage == ST_OWN_DONE) own_path_end(h, g, lds, nlds, a, sl, idx, w);
+}
+
+// Walk kernel bookkeeping of a pass: its first wave's start and, by block 0, the host's progress word (bit 63:
+// written, bit 62: every packet claimed, below: requests of the pass).
+__device__ __forceinline__ void pass_begin(PassCtl* pc, const McArgs& a, uint64_t nq, unsigned long long* progress)
+{
+    if (blockIdx.x != 0 || threadIdx.x != 0) return;
+    const bool claimed = *a.next_packet >= a.count;
+    pc->t0inv = ~(unsigned long long)wall_clock64();
+    __hip_atomic_store(progress, (1ull << 63) | (claimed ? 1ull << 62 : 0ull) | (unsigned long long)nq, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Walk pass: persistent lanes over the requests [0, *q.tail). A queue with fewer requests than the launch
+// has chunks needs only the first workgroups.
 template <class W, bool ABS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WalkWaves<W>::value, 8))) k_walks(const typename W::View g, const McArgs a, WalkQueue<typename W::Real> q,
-                                              Slots<typename W::Real> sl, unsigned long long* claim, int nlds_req,
-                                              int xcd_segments)
+                                              Slots<typename W::Real> sl, PassCtl* pc, unsigned long long* progress,
+                                              int nlds_req, int xcd_segments)
 {
     using R = typename W::Real;
     __shared__ InstrDev s_instr[SG_MAX_INSTR];
     extern __shared__ __align__(16) unsigned char smem[];
+    const uint64_t nq = *q.tail;
+    pass_begin(pc, a, nq, progress);
+    if ((uint64_t)blockIdx.x * (blockDim.x >> 6) * kClaimMin >= nq) return;
     int32_t* s_nodes = reinterpret_cast<int32_t*>(smem);
     int nlds = 0;
     if (nlds_req > 0) {
@@ -599,38 +689,27 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WalkWa
     }
     if (threadIdx.x < SG_MAX_INSTR) s_instr[threadIdx.x] = a.scene->instr[threadIdx.x];
     __syncthreads();
-    const uint64_t nq = *q.tail;
     const WalkReq<R>* reqs = q.sorted ? q.sorted : q.req;
+    const uint64_t nwaves = (uint64_t)gridDim.x * (blockDim.x >> 6);
     Hot<W> h;
     h.stage = ST_NEWPKT;   // idle: needs a request
     h.nseg = 0; h.nent = 0;
     h.w.nrecompute = 0; h.w.nstuck = 0;
-    uint32_t idx = 0, inst = 0;
+    uint32_t idx = 0, inst = 0, req = 0;
     uint32_t n_own = 0, n_peel = 0, n_re = 0;   // the lane's crossings by walk kind
-    uint64_t ccur = 0, cend = 0;                 // the wave's chunk of requests
+    uint64_t ccur = 0, cend = 0, clast = 0;      // the wave's chunk of requests
     int seg = blockIdx.x % kXcdSegs, tried = 0;  // XCD segments: the wave's segment, segments left behind
     bool exhausted = false;
     const int thr = a.compact;
     for (;;) {
-        if (h.stage == ST_PEELW_DONE) {
-            // FrameInstrument::detect (FrameInstrument.cpp:33-47)
-            const InstrDev& in = s_instr[inst];
-            unsafeAtomicAdd(in.frame + (size_t)a.ell * in.Nx * in.Ny + idx, (double)(h.L0 * rexp<R>(-h.tau)));
-        } else if (h.stage == ST_OWN_DONE) {
-            sl.fr(SR_RES, idx) = h.tau;
-        } else if (h.stage == ST_PROP_DONE) {
-            sl.fr(SR_RES, idx) = prop_length(h);
-            // the leaf holding the interaction point: where the packet's next walks start
-            if constexpr (W::kHint) sl.fu(SU_HINT, idx) = (uint32_t)h.w.hint();
-        }
         if (finished_stage(h.stage)) {
             count_walk(h, n_own, n_peel, n_re);
-            h.stage = ST_NEWPKT;
+            walk_end(h, g, s_nodes, nlds, a, sl, s_instr, inst, idx, reqs + req);
         }
         const bool want = h.stage == ST_NEWPKT;
         uint64_t r = 0;
-        const bool got = xcd_segments ? seg_claim(claim + 1, nq, want, seg, tried, ccur, cend, r, exhausted)
-                                      : chunk_claim(claim, nq, want, ccur, cend, r);
+        const bool got = xcd_segments ? seg_claim(pc->seg, nq, want, seg, tried, ccur, cend, r, exhausted)
+                                      : chunk_claim(&pc->claim, nq, nwaves, want, ccur, cend, clast, r);
         if (want && !got && xcd_segments && !exhausted) {
             // not served by this claim: the lane stays idle and claims again
         } else if (want) {
@@ -640,14 +719,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WalkWa
             // a request that names no pixel of an instrument or no packet slot is reported (error bit 2)
             // and dropped, never followed; the lane stays idle and takes the next one
             const uint32_t npix = wi < (uint32_t)a.ni ? (uint32_t)(s_instr[wi].Nx * s_instr[wi].Ny) : 0u;
-            const bool valid = kind == WK_PEEL ? w.idx < npix : kind <= WK_PROP && (int64_t)w.idx < sl.n;
+            const bool valid = kind == WK_PEEL ? w.idx < npix : kind == WK_OWN && (int64_t)w.idx < sl.n;
             if (!got) h.stage = ST_DEAD;
             else if (!valid) atomicOr(a.error, 4);
             else {
                 idx = w.idx;
                 inst = wi;
+                req = (uint32_t)r;
                 const R ox = w.o[0], oy = w.o[1], oz = w.o[2];
-                const R val = w.val;
                 double dx, dy, dz;
                 if (kind == WK_PEEL) {
                     const InstrDev& in = s_instr[inst];
@@ -659,11 +738,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WalkWa
                     h.w.init_hinted(g, s_nodes, nlds, ox, oy, oz, dx, dy, dz, (int)w.hint);
                 else
                     h.w.init(g, s_nodes, nlds, ox, oy, oz, dx, dy, dz);
-                // the value: a peel-off's or own path's luminosity, or the propagation target depth
-                h.L0 = val;
+                h.L0 = w.val;
                 if (kind == WK_PEEL) h.start_walk(ST_PEELW, (R)a.tau_cut);
-                else if (kind == WK_OWN) h.start_walk(ST_OWN, (R)0);
-                else h.start_walk(ST_PROP, val);
+                else h.start_walk(ST_OWN, (R)0);
             }
         }
         const uint64_t alive = __ballot(h.stage != ST_DEAD);
@@ -683,6 +760,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WalkWa
     add_wave(a.counters + 8, n_re);
     add_wave(a.counters + 5, h.w.nstuck);
     add_wave(a.counters + 9, h.w.nrecompute);
+    if (__lane_id() == 0) atomicMax(&pc->t1, (unsigned long long)wall_clock64());
 }
 
 } // namespace sg
