@@ -8,8 +8,8 @@
 //               counts, density or first child, six ropes or split planes).
 //   Voronoi   : one 32-byte record per site (x, y, z, rho); per cell a 32-byte header (its site and
 //               density) followed by its neighbour entries (walls -1..-6), each a 32-byte record
-//               holding the neighbour's site, the cells' blocks in Morton order of their sites; a
-//               uniform bucket grid over the sites with one start site per bucket for cellIndex.
+//               holding the neighbour's site and the place of its list, the cells' blocks on 128-byte
+//               lines in Morton order of their sites; a uniform bucket grid over the sites with one start site per bucket for cellIndex.
 //   Tallies   : FP64, instrument frames [ell][pixel], absorption [ell][m].
 #pragma once
 #include <hip/hip_runtime.h>
@@ -89,8 +89,18 @@ struct TreeView {
 
 struct alignas(16) VoroSite { double x, y, z, rho; };
 // One entry of a cell's neighbour list with the neighbour's site inline (walls: id -1..-6, no site),
-// so that a walk step reads its cell's list as one contiguous stream instead of gathering sites.
-struct alignas(32) VoroNbr { double x, y, z; int32_t id, pad; };
+// so that a walk step reads its cell's list as one contiguous stream instead of gathering sites. `list` is the
+// place of the neighbour's own list, so that a step onto the neighbour does not look it up first: the header's
+// 128-byte line times 128 plus the entry count, or 0 where that does not fit (the list is then looked up).
+struct alignas(32) VoroNbr { double x, y, z; int32_t id; uint32_t list; };
+constexpr int kVoroLine = 4;              // records per 128-byte line; a cell's block starts on a line
+constexpr uint32_t kVoroMaxCount = 127;   // largest entry count and
+constexpr uint32_t kVoroMaxLine = (1u << 25) - 1;   // largest line that `list` holds
+__host__ __device__ inline uint32_t voro_list(int64_t header, int64_t count)
+{
+    const int64_t line = header / kVoroLine;
+    return count <= (int64_t)kVoroMaxCount && line <= (int64_t)kVoroMaxLine ? (uint32_t)(line << 7 | count) : 0u;
+}
 
 struct VoroView {
     const VoroSite* site;
@@ -101,9 +111,29 @@ struct VoroView {
     const int32_t* brep;             // start site per bucket for the greedy location, nbk^3
     int32_t nsites;
     int nbk;
+    int walls_lead;                  // 1: every list has its walls among its first kVoroWalls entries
     double ext[6];
     double eps;
 };
+constexpr int kVoroWalls = 8;
+
+// A list record through a global-memory pointer: the view's pointers are generic where they have passed
+// through registers, and flat loads wait on the LDS counter too.
+__device__ __forceinline__ VoroNbr load_nbr(const VoroNbr* p)
+{
+    typedef double f64x2 __attribute__((ext_vector_type(2)));
+    const auto* q = (const __attribute__((address_space(1))) f64x2*)p;
+    const f64x2 a = q[0], b = q[1];
+    const unsigned long long w = (unsigned long long)__double_as_longlong(b.y);
+    return VoroNbr{a.x, a.y, b.x, (int32_t)(uint32_t)w, (uint32_t)(w >> 32)};
+}
+__device__ __forceinline__ VoroSite load_header(const VoroNbr* p)
+{
+    typedef double f64x2 __attribute__((ext_vector_type(2)));
+    const auto* q = (const __attribute__((address_space(1))) f64x2*)p;
+    const f64x2 a = q[0], b = q[1];
+    return VoroSite{a.x, a.y, b.x, b.y};
+}
 
 // ------------------------------------------------------------------------- scene records
 
@@ -165,6 +195,7 @@ struct McArgs {
     // and the number of random draws the emission consumed
     const void* emitted;
     const uint32_t* emit_draw;
+    const int32_t* emit_hint;        // start cell (walker's hint) per packet, or null
     // coherence keys of walk requests (event/walk pipeline): start points are binned on a raster of
     // the grid box, t = (r - key_lo) * key_scale in [0, 16)
     double key_lo[3], key_scale[3];

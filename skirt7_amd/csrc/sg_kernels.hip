@@ -534,7 +534,7 @@ int sg_grid_create_voronoi(const double ext[6], const double* sites, int64_t n, 
     for (int64_t t = 0; t < nb_offsets[n]; t++)
         SG_REQUIRE(nb_ids[t] >= -6 && nb_ids[t] < n && nb_ids[t] != -99, "neighbour id out of range");
     // Device lists: per cell a header record (its own site and density) followed by its neighbour
-    // entries; the cells' blocks in Morton order of their sites, so that cells a walk crosses one
+    // entries; the cells' blocks on 128-byte lines in Morton order of their sites, so that cells a walk crosses one
     // after another, which are neighbours in space, lie near each other in memory. voff holds each
     // cell's (first record, entry count).
     std::vector<uint64_t> key(n);
@@ -551,20 +551,25 @@ int sg_grid_create_voronoi(const double ext[6], const double* sites, int64_t n, 
     for (int64_t i = 0; i < n; i++) order[i] = (int32_t)i;
     std::sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return key[a] < key[b] || (key[a] == key[b] && a < b); });
     std::vector<int32_t> be(2 * n);
-    g->hvnb.clear();
-    g->hvnb.reserve(n + nb_offsets[n]);
+    int64_t records = 0;
     for (int32_t m : order) {
-        be[2 * m] = (int32_t)g->hvnb.size();
-        be[2 * m + 1] = (int32_t)(nb_offsets[m + 1] - nb_offsets[m]);
-        VoroNbr head{g->hsite[m].x, g->hsite[m].y, g->hsite[m].z, 0, 0};   // density set by set_rho
-        g->hvnb.push_back(head);
+        SG_REQUIRE(records < ((int64_t)1 << 31), "neighbour lists too long");
+        const int64_t count = nb_offsets[m + 1] - nb_offsets[m];
+        be[2 * m] = (int32_t)records;
+        be[2 * m + 1] = (int32_t)count;
+        records = (records + 1 + count + kVoroLine - 1) / kVoroLine * kVoroLine;
+    }
+    SG_REQUIRE(records < ((int64_t)1 << 31), "neighbour lists too long");
+    g->hvnb.assign(records, VoroNbr{});
+    for (int64_t m = 0; m < n; m++) {
+        VoroNbr* r = &g->hvnb[be[2 * m]];
+        *r++ = VoroNbr{g->hsite[m].x, g->hsite[m].y, g->hsite[m].z, 0, 0};   // density set by set_rho
         for (int64_t t = nb_offsets[m]; t < nb_offsets[m + 1]; t++) {
             const int32_t v = nb_ids[t];
-            g->hvnb.push_back(v >= 0 ? VoroNbr{g->hsite[v].x, g->hsite[v].y, g->hsite[v].z, v, 0}
-                                     : VoroNbr{0.0, 0.0, 0.0, v, 0});
+            *r++ = v >= 0 ? VoroNbr{g->hsite[v].x, g->hsite[v].y, g->hsite[v].z, v, voro_list(be[2 * v], be[2 * v + 1])}
+                          : VoroNbr{0.0, 0.0, 0.0, v, 0};
         }
     }
-    SG_REQUIRE(g->hvnb.size() < ((size_t)1 << 31), "neighbour lists too long");
     g->voff.upload(be);
     g->vnb.upload(g->hvnb);
     // bucket grid for the nearest-site search: about 2 sites per bucket
@@ -625,6 +630,10 @@ int sg_grid_create_voronoi(const double ext[6], const double* sites, int64_t n, 
     v.bids = g->bids.as<int32_t>();
     v.brep = g->brep.as<int32_t>();
     v.nsites = (int32_t)n;
+    v.walls_lead = 1;
+    for (int64_t m = 0; m < n && v.walls_lead; m++)
+        for (int64_t t = nb_offsets[m] + kVoroWalls; t < nb_offsets[m + 1]; t++)
+            if (nb_ids[t] < 0) { v.walls_lead = 0; break; }
     v.nbk = nbk;
     for (int i = 0; i < 6; i++) v.ext[i] = ext[i];
     double wx = ext[3] - ext[0], wy = ext[4] - ext[1], wz = ext[5] - ext[2];
@@ -1324,7 +1333,7 @@ static double g_clock_khz = 100000.0;                   // of the device's wall 
 // (runs are synchronous and driven by one host thread): slot groups, walk queues, progress counters,
 // launch states. Allocated on first use, grown as needed, kept until the process ends.
 struct SplitPool {
-    DevBuf slots[2], queue[2], prog[2], emitted, emitdraw;
+    DevBuf slots[2], queue[2], prog[2], emitted, emitdraw, emithint;
     DevBuf bins[2];   // per group: bin counts (zero between passes: cleared once, then by each pass's scan), offsets
 };
 static SplitPool* g_pool = nullptr;
@@ -1425,6 +1434,21 @@ static int run_passes(const typename W::View& v, const McArgs& ab, PassGroups<ty
     return launches;
 }
 
+// Emission of the packets of a for event/walk passes, with their start cells where the walker takes them.
+template <class W>
+static void launch_emit(const typename W::View& v, McArgs& a, void* emitted, uint32_t* draws, int32_t* hint, hipStream_t st)
+{
+    using R = typename W::Real;
+    a.emitted = emitted;
+    a.emit_draw = draws;
+    const int blocks = (int)std::min<uint64_t>((a.count + 255) / 256, (uint64_t)g_cus * 16);
+    if constexpr (W::kHint) {
+        a.emit_hint = hint;
+        hipLaunchKernelGGL(k_emit_located<W>, dim3(blocks), dim3(256), 0, st, v, a, static_cast<R*>(emitted), draws, hint);
+    } else hipLaunchKernelGGL(k_emit<R>, dim3(blocks), dim3(256), 0, st, a, static_cast<R*>(emitted), draws);
+    SG_HIP(hipGetLastError());
+}
+
 // Duration of the groups' walk kernels (the passes have ended).
 static double walk_ms(GroupCtl* const* ctl, int n)
 {
@@ -1503,6 +1527,8 @@ static void run_split(sg_sim* s, const typename W::View& v, const McArgs& a, uin
     DevBuf& emitdraw = pool().emitdraw;
     if (emitted.bytes < 7 * batch * rsz) emitted.alloc(7 * batch * rsz);
     if (emitdraw.bytes < batch * sizeof(uint32_t)) emitdraw.alloc(batch * sizeof(uint32_t));
+    DevBuf& emithint = pool().emithint;
+    if (W::kHint && emithint.bytes < batch * sizeof(int32_t)) emithint.alloc(batch * sizeof(int32_t));
     unsigned long long* claims = s->next.as<unsigned long long>();
     hipEvent_t ev_start, ev_join, ev_end[2];
     SG_HIP(hipEventCreateWithFlags(&ev_join, hipEventDisableTiming));
@@ -1513,8 +1539,6 @@ static void run_split(sg_sim* s, const typename W::View& v, const McArgs& a, uin
         McArgs ab = a;
         ab.first = first + b;
         ab.count = std::min(batch, count - b);
-        ab.emitted = emitted.p;
-        ab.emit_draw = emitdraw.as<uint32_t>();
         ab.next_packet = claims;
         // the previous batch is finished on both streams: emit on stream 0, then both groups start
         if (G == 2) {
@@ -1522,9 +1546,7 @@ static void run_split(sg_sim* s, const typename W::View& v, const McArgs& a, uin
             SG_HIP(hipStreamWaitEvent(st[0], ev_join, 0));
         }
         SG_HIP(hipMemsetAsync(claims, 0, sizeof(unsigned long long), st[0]));
-        int emb = (int)std::min<uint64_t>((ab.count + 255) / 256, (uint64_t)g_cus * 16);
-        hipLaunchKernelGGL(k_emit<R>, dim3(emb), dim3(256), 0, st[0], ab, emitted.as<R>(), emitdraw.as<uint32_t>());
-        SG_HIP(hipGetLastError());
+        launch_emit<W>(v, ab, emitted.p, emitdraw.as<uint32_t>(), emithint.as<int32_t>(), st[0]);
         for (int g = 0; g < G && b > 0; g++)
             hipLaunchKernelGGL(k_revive, dim3((Pg[g] + 255) / 256), dim3(256), 0, st[0],
                                pg.sl[g].u + (size_t)SU_STATE * Pg[g], Pg[g]);
@@ -1574,8 +1596,8 @@ static void dispatch_split(sg_sim* s, const McArgs& a, int precision, uint64_t f
         else if (rope_walk(g)) run_split<TreeW32, ABS>(s, g->tree, a, first, count, SG_LDS_NODES, lt, blocks);
         else run_split<TreeW32TopDown, ABS>(s, g->tree, a, first, count, SG_LDS_NODES, lt, blocks);
     } else {
-        if (mixed) run_split<VoroW<float>, ABS>(s, g->voro, a, first, count, 0, lt, blocks);
-        else run_split<VoroW<double>, ABS>(s, g->voro, a, first, count, 0, lt, blocks);
+        if (mixed) run_split<VoroWalk<float>, ABS>(s, g->voro, a, first, count, 0, lt, blocks);
+        else run_split<VoroWalk<double>, ABS>(s, g->voro, a, first, count, 0, lt, blocks);
     }
 }
 
@@ -1838,12 +1860,13 @@ static void run_static(sg_sim* s, const typename W::View& v, const McArgs& a0, i
     hipStream_t st = g_split_stream[0];
     const int64_t P = (int64_t)std::max<uint64_t>(1, std::min<uint64_t>(a0.count, (uint64_t)kStaticSlots));
     const int64_t cap = P * (a0.ni + 1);
-    // layout of the static array: slots, walk requests, progress records, launch states, draw counts
+    // layout of the static array: slots, walk requests, progress records, launch states, draw counts, start cells
     const size_t o_q = align256(slot_bytes<R>(P));
     const size_t o_pc = o_q + align256((size_t)cap * sizeof(WalkReq<R>));
     const size_t o_em = o_pc + align256(sizeof(GroupCtl));
     const size_t o_ed = o_em + align256(7 * a0.count * sizeof(R));
-    const size_t need = o_ed + align256(a0.count * sizeof(uint32_t));
+    const size_t o_eh = o_ed + align256(a0.count * sizeof(uint32_t));
+    const size_t need = o_eh + align256(a0.count * sizeof(int32_t));
     SG_REQUIRE(need <= kStaticScratchBytes, "sg_sim_run_static: the run needs " + std::to_string(need) +
                                                 " bytes of work memory, more than the static array holds");
     unsigned char* base = static_cast<unsigned char*>(g_scratch[g_device]);
@@ -1856,8 +1879,6 @@ static void run_static(sg_sim* s, const typename W::View& v, const McArgs& a0, i
     pg.q[0].req = reinterpret_cast<WalkReq<R>*>(base + o_q);
     pg.q[0].cap = cap;
     McArgs a = a0;
-    a.emitted = base + o_em;
-    a.emit_draw = reinterpret_cast<uint32_t*>(base + o_ed);
     a.next_packet = s->next.as<unsigned long long>();
     // cleared by kernels: slot states (PS_FRESH) and counts, progress, the packet claims, counters, error flag
     fill_u32(sl.u + (size_t)SU_STATE * P, P * (SU_NU - SU_STATE), st);
@@ -1874,12 +1895,8 @@ static void run_static(sg_sim* s, const typename W::View& v, const McArgs& a0, i
     pg.ebs = 256;
     while (pg.ebs > 64 && staged_bytes<R>(pg.ebs, a.ni) > 64 * 1024) pg.ebs /= 2;
     pg.eshm = staged_bytes<R>(pg.ebs, a.ni);
-    if (a.count > 0) {
-        const int emb = (int)std::min<uint64_t>((a.count + 255) / 256, (uint64_t)g_cus * 16);
-        hipLaunchKernelGGL(k_emit<R>, dim3(emb), dim3(256), 0, st, a, static_cast<R*>(const_cast<void*>(a.emitted)),
-                           const_cast<uint32_t*>(a.emit_draw));
-        SG_HIP(hipGetLastError());
-    }
+    if (a.count > 0)
+        launch_emit<W>(v, a, base + o_em, reinterpret_cast<uint32_t*>(base + o_ed), reinterpret_cast<int32_t*>(base + o_eh), st);
     run_passes<W, ABS>(v, a, pg);
     hipLaunchKernelGGL(k_slot_counts, dim3(std::min<int64_t>((P + 255) / 256, 1024)), dim3(256), 0, st, sl.u, P, a.counters);
     SG_HIP(hipGetLastError());
@@ -1904,8 +1921,8 @@ static void dispatch_static(sg_sim* s, const McArgs& a, int precision, int& bloc
         else if (rope_walk(g)) run_static<TreeW32, ABS>(s, g->tree, a, SG_LDS_NODES, blocks);
         else run_static<TreeW32TopDown, ABS>(s, g->tree, a, SG_LDS_NODES, blocks);
     } else {
-        if (mixed) run_static<VoroW<float>, ABS>(s, g->voro, a, 0, blocks);
-        else run_static<VoroW<double>, ABS>(s, g->voro, a, 0, blocks);
+        if (mixed) run_static<VoroWalk<float>, ABS>(s, g->voro, a, 0, blocks);
+        else run_static<VoroWalk<double>, ABS>(s, g->voro, a, 0, blocks);
     }
 }
 

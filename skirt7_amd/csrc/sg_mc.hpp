@@ -14,10 +14,11 @@
 namespace sg {
 
 // Each walking stage is followed by its finished stage (a walk ends by stepping its stage by one).
+// ST_LOC (walk kernel only): the walk has become the location of the interaction point.
 enum Stage : int { ST_NEWPKT = 0, ST_PEEL, ST_PEELW, ST_PEELW_DONE, ST_OWN_START, ST_OWN, ST_OWN_DONE, ST_PROP,
-                   ST_PROP_DONE, ST_SCATTER, ST_DEAD };
-static_assert(ST_PEELW_DONE == ST_PEELW + 1 && ST_OWN_DONE == ST_OWN + 1 && ST_PROP_DONE == ST_PROP + 1,
-              "a finished stage follows its walking stage");
+                   ST_PROP_DONE, ST_SCATTER, ST_LOC, ST_LOC_DONE, ST_DEAD };
+static_assert(ST_PEELW_DONE == ST_PEELW + 1 && ST_OWN_DONE == ST_OWN + 1 && ST_PROP_DONE == ST_PROP + 1 &&
+              ST_LOC_DONE == ST_LOC + 1, "a finished stage follows its walking stage");
 
 // ------------------------------------------------------------------------- emission (FP64)
 
@@ -180,6 +181,18 @@ __global__ void __launch_bounds__(256) k_emit(const McArgs a, R* out, uint32_t* 
         emit_one<R>(a, out, draws, i);
 }
 
+// The same for the event/walk passes of a walker that takes start cells: hint[i] receives the cell of packet i's
+// position, found once here at full width instead of at the start of each of the packet's first walks.
+template <class W>
+__global__ void __launch_bounds__(256) k_emit_located(const typename W::View g, const McArgs a, typename W::Real* out,
+                                                      uint32_t* draws, int32_t* hint)
+{
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.count; i += (size_t)gridDim.x * blockDim.x) {
+        emit_one<typename W::Real>(a, out, draws, i);
+        hint[i] = W::locate_start(g, (double)out[i], (double)out[a.count + i], (double)out[2 * (size_t)a.count + i]);
+    }
+}
+
 // Emission for a table of packet ranges laid end to end (range k owns positions
 // [roff[k], roff[k+1])); each range writes where its own `emitted` and `emit_draw` point.
 template <typename R>
@@ -319,6 +332,22 @@ __device__ __forceinline__ double exponcutoff(PacketRng& rng, double xmax)
     else if (xmax < 1e-10) return rng.ud() * xmax;
     double x = -log(1.0 - rng.ud() * (1.0 - exp(-xmax)));
     while (x > xmax) x = -log(1.0 - rng.ud() * (1.0 - exp(-xmax)));
+    return x;
+}
+// Random::exponcutoff with its first deviate u (of rng's stream) already drawn, for xmax > 0.
+__device__ __forceinline__ double exponcutoff_from(PacketRng& rng, double u, double xmax)
+{
+    if (xmax < 1e-10) return u * xmax;
+    double x = -log(1.0 - u * (1.0 - exp(-xmax)));
+    while (x > xmax) x = -log(1.0 - rng.ud() * (1.0 - exp(-xmax)));
+    return x;
+}
+__device__ __forceinline__ float exponcutoff_from(PacketRng& rng, float u, float xmax)
+{
+    if (xmax < 1e-10f) return u * xmax;
+    const float em = -expm1f(-xmax);
+    float x = -log1pf(-u * em);
+    while (x > xmax) x = -log1pf(-rng.uf() * em);
     return x;
 }
 // FP32 form: -log1p(-U * (-expm1(-xmax))) keeps full relative accuracy at small optical depth.
@@ -594,6 +623,9 @@ __device__ __noinline__ void service_call(uint32_t* park, int nl, int lane, Cold
     lds_store(q, park, nl, lane);
 }
 
+// The lane of a walk's lanes that makes its tallies (walkers of one lane: every lane).
+template <class W> __device__ __forceinline__ bool leads() { return (threadIdx.x & (W::kLanes - 1)) == 0; }
+
 // One step of the current walk; marks the walk finished (its stage steps to the finished one) when
 // the path ends, or when the optical depth passes the walk's limit (the propagation target, or the
 // peel-off cut). Returns whether the walk goes on. Crossings are counted per walk when it ends
@@ -632,7 +664,7 @@ __device__ __forceinline__ bool crossing(Hot<W>& h, const typename W::View& g, c
         R expfactorm = -rexpm1<R>(-dtau);
         R Lintm = h.L0 * rexp<R>(-h.tau) * expfactorm;
         R Labsm = ((R)1.0 - (R)a.albedo) * Lintm;
-        unsafeAtomicAdd(a.labs + (size_t)a.ell * a.ncells + W::cell_of(g, m), (double)Labsm);
+        if (leads<W>()) unsafeAtomicAdd(a.labs + (size_t)a.ell * a.ncells + W::cell_of(g, m), (double)Labsm);
     }
     // running sums, kept for every walk kind without branching (only the propagation re-walk reads
     // the path length and the previous segment's sums): cumulative s and tau per segment
@@ -641,10 +673,10 @@ __device__ __forceinline__ bool crossing(Hot<W>& h, const typename W::View& g, c
     h.s += dsv;
     h.tau += dtau;
     h.nseg += seg ? 1 : 0;
-    // the walk ends at the end of the path, for a peel-off beyond the optical-depth cut, and for the
-    // propagation re-walk at the first segment past the target optical depth (prop_length then
-    // interpolates the interaction point)
-    const bool end = !got || h.tau > h.limit;
+    // the walk ends at the end of the path (known with its last segment: no further step finds that out),
+    // for a peel-off beyond the optical-depth cut, and for the propagation re-walk at the first segment past
+    // the target optical depth (prop_length then interpolates the interaction point)
+    const bool end = !got || (h.w.done & (h.w.entries() == 0)) || h.tau > h.limit;
     h.stage += end ? 1 : 0;
     return !end;
 }
@@ -659,17 +691,17 @@ template <class W> __device__ __forceinline__ void count_walk(const Hot<W>& h, u
     n_re += h.stage == ST_PROP_DONE ? c : 0u;
 }
 
-// ST_PEELW, ST_OWN or ST_PROP, as a bit test (a chain of comparisons compiles to branches)
+// ST_PEELW, ST_OWN, ST_PROP or ST_LOC, as a bit test (a chain of comparisons compiles to branches)
 __device__ __forceinline__ bool walking_stage(int st)
 {
-    static_assert(ST_PEELW < 32 && ST_OWN < 32 && ST_PROP < 32, "stage bits");
-    return ((1u << ST_PEELW | 1u << ST_OWN | 1u << ST_PROP) >> (uint32_t)st) & 1u;
+    static_assert(ST_DEAD < 32, "stage bits");
+    return ((1u << ST_PEELW | 1u << ST_OWN | 1u << ST_PROP | 1u << ST_LOC) >> (uint32_t)st) & 1u;
 }
 
-// ST_PEELW_DONE, ST_OWN_DONE or ST_PROP_DONE
+// ST_PEELW_DONE, ST_OWN_DONE, ST_PROP_DONE or ST_LOC_DONE
 __device__ __forceinline__ bool finished_stage(int st)
 {
-    return ((1u << ST_PEELW_DONE | 1u << ST_OWN_DONE | 1u << ST_PROP_DONE) >> (uint32_t)st) & 1u;
+    return ((1u << ST_PEELW_DONE | 1u << ST_OWN_DONE | 1u << ST_PROP_DONE | 1u << ST_LOC_DONE) >> (uint32_t)st) & 1u;
 }
 
 __device__ __forceinline__ void add_wave(unsigned long long* dst, unsigned long long x)

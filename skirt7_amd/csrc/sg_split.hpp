@@ -348,7 +348,7 @@ __global__ void __launch_bounds__(256) k_events(const McArgs a, Slots<R> sl, Wal
                     philox10(rng.w0, rng.w1, rng.w2, rng.w3, rng.k0, rng.k1);
                 }
                 nscatt = 0;
-                hint = -1;   // a new position: the leaf is not known yet
+                hint = a.emit_hint ? a.emit_hint[p] : -1;
                 uint32_t np = peel_offs<R>(a, s_instr, sq, false, rx, ry, rz, kx, ky, kz, L, hint);
                 c_npeel += np;
                 if (!a.has_dust) continue;
@@ -580,8 +580,21 @@ template <> struct WalkWaves<TreeW32> { static constexpr int value = SG_W32_WAVE
 #define SG_W64_WAVES 3
 #endif
 template <> struct WalkWaves<TreeW64> { static constexpr int value = SG_W64_WAVES; };
-template <> struct WalkWaves<VoroW<double>> { static constexpr int value = 3; };   // 4 would spill
-template <> struct WalkWaves<VoroW<float>> { static constexpr int value = 3; };
+// Lanes per Voronoi walk and entries per lane and step: 8 x 3 = 24 entries a step, which most lists (19 on average
+// along the walks) fit, at three waves per SIMD, where nothing spills in the walk. On 1e5 sites with 3 x 1e5 packets:
+// 33 ms a run; four lanes x 6 42 ms, 8 x 2 50 ms and 8 x 3 51 ms at four waves (spills), 16 x 2 50 ms; one lane x 16
+// entries (VoroW, as the lane pipeline walks) spilled and took 106 ms.
+#ifndef SG_VORO_LANES
+#define SG_VORO_LANES 8
+#endif
+#ifndef SG_VORO_EACH
+#define SG_VORO_EACH 3
+#endif
+#ifndef SG_VORO_WAVES
+#define SG_VORO_WAVES 3
+#endif
+template <typename R> using VoroWalk = VoroC<R, SG_VORO_LANES, SG_VORO_EACH>;
+template <typename R> struct WalkWaves<VoroWalk<R>> { static constexpr int value = SG_VORO_WAVES; };
 
 // The end of an own path (lane's walk of slot idx, request w): DustSystem::fillOpticalDepth's check
 // (DustSystem.cpp:952-955), simulateescapeandabsorption (MonteCarloSimulation.cpp:432-461), the stop test
@@ -620,11 +633,16 @@ __device__ __forceinline__ void own_path_end(Hot<W>& h, const typename W::View& 
     rng.k0 = a.seed; rng.k1 = a.member; rng.ell = (uint32_t)a.ell;
     rng.plo = sl.fu(SU_PLO, idx); rng.phi = sl.fu(SU_PHI, idx); rng.draw = sl.fu(SU_DRAW, idx);
     rng.w0 = sl.fu(SU_W0, idx); rng.w1 = sl.fu(SU_W1, idx); rng.w2 = sl.fu(SU_W2, idx); rng.w3 = sl.fu(SU_W3, idx);
-    R tt;
-    if (a.xi == 0.0) tt = exponcutoff(rng, taupath);
-    else {
-        const R X = uni<R>(rng);
-        tt = (X < (R)a.xi) ? uni<R>(rng) * taupath : exponcutoff(rng, taupath);
+    // one deviate, or (biased) one for the choice of distribution and one for the depth
+    R tt, u = 0;
+    bool uniform = false;
+    for (int k = a.xi == 0.0 ? 1 : 0; k < 2; k++) {
+        uniform = k == 1 && a.xi != 0.0 && u < (R)a.xi;
+        u = uni<R>(rng);
+    }
+    if (uniform) tt = u * taupath;
+    else tt = exponcutoff_from(rng, u, taupath);
+    if (a.xi != 0.0) {
         const R pp = -rexp<R>(-tt) / rexpm1<R>(-taupath);
         const R qq = ((R)1.0 - (R)a.xi) * pp + (R)a.xi / taupath;
         L = L * (pp / qq);
@@ -647,12 +665,24 @@ __device__ __forceinline__ void walk_end(Hot<W>& h, const typename W::View& g, c
 {
     if (h.stage == ST_PEELW_DONE) {
         const InstrDev& in = instr[inst];
-        unsafeAtomicAdd(in.frame + (size_t)a.ell * in.Nx * in.Ny + idx, (double)(h.L0 * rexp<typename W::Real>(-h.tau)));
+        if (leads<W>())
+            unsafeAtomicAdd(in.frame + (size_t)a.ell * in.Nx * in.Ny + idx, (double)(h.L0 * rexp<typename W::Real>(-h.tau)));
         h.stage = ST_NEWPKT;
     } else if (h.stage == ST_PROP_DONE) {
-        sl.fr(SR_RES, idx) = prop_length(h);
-        // the leaf holding the interaction point: where the packet's next walks start
-        if constexpr (W::kHint) sl.fu(SU_HINT, idx) = (uint32_t)h.w.hint();
+        using R = typename W::Real;
+        const R d = prop_length(h);
+        sl.fr(SR_RES, idx) = d;
+        h.stage = ST_NEWPKT;
+        // the leaf holding the interaction point, where the packet's next walks start: the last segment's, or
+        // (a walker whose start cells are exact) looked for by this lane, once for all of those walks, at the
+        // point that the event kernel computes by the same formula
+        if constexpr (W::kLocates) {
+            h.w.locate_next(g, (double)(w->o[0] + d * w->d[0]), (double)(w->o[1] + d * w->d[1]),
+                            (double)(w->o[2] + d * w->d[2]));
+            h.start_walk(ST_LOC, (R)0);
+        } else if constexpr (W::kHint) sl.fu(SU_HINT, idx) = (uint32_t)h.w.hint();
+    } else if (h.stage == ST_LOC_DONE) {
+        if constexpr (W::kLocates) sl.fu(SU_HINT, idx) = (uint32_t)h.w.hint();
         h.stage = ST_NEWPKT;
     } else if (h.stage == ST_OWN_DONE) own_path_end(h, g, lds, nlds, a, sl, idx, w);
 }
@@ -703,13 +733,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WalkWa
     const int thr = a.compact;
     for (;;) {
         if (finished_stage(h.stage)) {
-            count_walk(h, n_own, n_peel, n_re);
+            if (leads<W>()) count_walk(h, n_own, n_peel, n_re);
             walk_end(h, g, s_nodes, nlds, a, sl, s_instr, inst, idx, reqs + req);
         }
         const bool want = h.stage == ST_NEWPKT;
         uint64_t r = 0;
-        const bool got = xcd_segments ? seg_claim(pc->seg, nq, want, seg, tried, ccur, cend, r, exhausted)
-                                      : chunk_claim(&pc->claim, nq, nwaves, want, ccur, cend, clast, r);
+        // a walk's lanes (neighbours, all in the same stage) share the request that their first lane claims
+        const bool asks = want && leads<W>();
+        bool got = xcd_segments ? seg_claim(pc->seg, nq, asks, seg, tried, ccur, cend, r, exhausted)
+                                : chunk_claim(&pc->claim, nq, nwaves, asks, ccur, cend, clast, r);
+        if constexpr (W::kLanes > 1) {
+            const uint32_t first = __lane_id() & ~(uint32_t)(W::kLanes - 1);
+            got = __shfl((int)got, first) != 0;
+            r = __shfl((uint32_t)r, first);   // requests number fewer than 2^32
+        }
         if (want && !got && xcd_segments && !exhausted) {
             // not served by this claim: the lane stays idle and claims again
         } else if (want) {
@@ -758,8 +795,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WalkWa
     add_wave(a.counters + 1, n_own);
     add_wave(a.counters + 2, n_peel);
     add_wave(a.counters + 8, n_re);
-    add_wave(a.counters + 5, h.w.nstuck);
-    add_wave(a.counters + 9, h.w.nrecompute);
+    add_wave(a.counters + 5, leads<W>() ? h.w.nstuck : 0u);
+    add_wave(a.counters + 9, leads<W>() ? h.w.nrecompute : 0u);
     if (__lane_id() == 0) atomicMax(&pc->t1, (unsigned long long)wall_clock64());
 }
 

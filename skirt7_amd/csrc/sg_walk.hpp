@@ -82,6 +82,8 @@ struct CartW64 {
     static constexpr int kParkWords = 25;
     __device__ __forceinline__ static int cell_of(const View&, int n) { return n; }
     static constexpr bool kHint = false;
+    static constexpr int kLanes = 1;
+    static constexpr bool kLocates = false;
     __device__ __forceinline__ int entries() const { return ne; }
     static constexpr bool kStep = false;   // next() only
     template <class P> __device__ __forceinline__ void park(P& p)
@@ -233,6 +235,8 @@ struct CartW32 {
     static constexpr int kParkWords = 19;
     __device__ __forceinline__ static int cell_of(const View&, int n) { return n; }
     static constexpr bool kHint = false;
+    static constexpr int kLanes = 1;
+    static constexpr bool kLocates = false;
     __device__ __forceinline__ int entries() const { return ne; }
     static constexpr bool kStep = false;   // next() only
     template <class P> __device__ __forceinline__ void park(P& p)
@@ -379,6 +383,12 @@ __device__ __forceinline__ int descend64(const TreeView& t, const int32_t* lds, 
     return -w - 1;
 }
 
+// Inside the box and on none of its walls: moveInside leaves such a point as it is.
+__device__ __forceinline__ bool strictly_inside(const double* b, double x, double y, double z)
+{
+    return x > b[0] && x < b[3] && y > b[1] && y < b[4] && z > b[2] && z < b[5];
+}
+
 // DustGridPath::moveInside (DustGridPath.cpp:57-150). Returns false for the OUTSIDE result.
 struct Entry {
     int ne;
@@ -440,20 +450,22 @@ struct TreeW64 {
     double x, y, z, kx, ky, kz;
     double lo[3], hi[3];
     double rho;
-    int m;
+    int m, lm;               // current cell, cell of the last segment returned
     Entry en;
     bool done;
     uint32_t steps, nrecompute, nstuck;
-    static constexpr int kParkWords = 38;
+    static constexpr int kParkWords = 39;
     __device__ __forceinline__ static int cell_of(const View&, int n) { return n; }
-    static constexpr bool kHint = false;
+    static constexpr bool kHint = true;
+    static constexpr int kLanes = 1;
+    static constexpr bool kLocates = false;
     __device__ __forceinline__ int entries() const { return en.ne; }
     static constexpr bool kStep = false;   // next() only
     template <class P> __device__ __forceinline__ void park(P& p)
     {
         p.io(x); p.io(y); p.io(z); p.io(kx); p.io(ky); p.io(kz);
         p.io(lo[0]); p.io(lo[1]); p.io(lo[2]); p.io(hi[0]); p.io(hi[1]); p.io(hi[2]);
-        p.io(rho); p.io(m); p.io(en.ne); p.io(en.e0); p.io(en.e1); p.io(en.e2);
+        p.io(rho); p.io(m); p.io(lm); p.io(en.ne); p.io(en.e0); p.io(en.e1); p.io(en.e2);
         p.io(done); p.io(steps); p.io(nrecompute); p.io(nstuck);
     }
 
@@ -480,13 +492,42 @@ struct TreeW64 {
                          double dy, double dz)
     {
         kx = dx; ky = dy; kz = dz;
-        steps = 0; done = false;
+        steps = 0; done = false; lm = -1;
         if (!en.move_inside(t.ext, t.eps, rx, ry, rz, kx, ky, kz)) {
             // OUTSIDE sentinel: no node contains it, path cleared
             en.ne = 0; done = true; return;
         }
         x = rx; y = ry; z = rz;
         if (!descend(t, lds, nlds)) { en.ne = 0; done = true; }
+    }
+    // The cell of the last segment returned (-1 before the first one): after a walk that stopped inside a
+    // segment, the cell holding the stopping point.
+    __device__ __forceinline__ int hint() const { return lm; }
+    // The cell of a walk's start point strictly inside the grid (which move_inside leaves as it is), else -1.
+    __device__ __forceinline__ static int locate_start(const View& t, double x, double y, double z)
+    {
+        if (!strictly_inside(t.ext, x, y, z)) return -1;
+        double l[3], h[3];
+        return descend64(t, t.node, 0, x, y, z, l, h);
+    }
+    // init for a start point strictly inside the grid with a candidate cell hn: the cell is taken when it
+    // contains the point in the half-open sense lo <= p < hi, by the planes that the descent from the root
+    // compares with, so it is the cell that the descent selects; otherwise init. (Eight levels of descent cost a
+    // third of an average FP64 walk.)
+    __device__ __forceinline__ void init_hinted(const View& t, const int32_t* lds, int nlds, double rx, double ry,
+                                                double rz, double dx, double dy, double dz, int hn)
+    {
+        if (strictly_inside(t.ext, rx, ry, rz) && hn >= 0 && hn < t.ncells) {
+            const TreeRec64& r = t.rec64[hn];
+            if (rx >= r.lo[0] && rx < r.hi[0] && ry >= r.lo[1] && ry < r.hi[1] && rz >= r.lo[2] && rz < r.hi[2]) {
+                kx = dx; ky = dy; kz = dz;
+                x = rx; y = ry; z = rz;
+                steps = 0; done = false; lm = -1; en.ne = 0;
+                load_cell(t, hn);
+                return;
+            }
+        }
+        init(t, lds, nlds, rx, ry, rz, dx, dy, dz);
     }
     __device__ __forceinline__ bool next(const View& t, const int32_t* lds, int nlds, int& mo, double& ds,
                                          double& rh)
@@ -533,7 +574,7 @@ struct TreeW64 {
                 else if (m == oldm) done = true;
             }
             if (++steps > SG_MAX_STEPS) done = true;
-            if (d > 0) { mo = segm; ds = d; rh = segrho; return true; }
+            if (d > 0) { mo = segm; ds = d; rh = segrho; lm = segm; return true; }
         }
         return false;
     }
@@ -558,6 +599,8 @@ struct TreeW64Book {
     // segments carry cell numbers
     __device__ __forceinline__ static int cell_of(const View&, int n) { return n; }
     static constexpr bool kHint = false;
+    static constexpr int kLanes = 1;
+    static constexpr bool kLocates = false;
     __device__ __forceinline__ int entries() const { return en.ne; }
     static constexpr bool kStep = false;   // next() only
     template <class P> __device__ __forceinline__ void park(P& p)
@@ -698,6 +741,8 @@ struct TreeW32 {
     uint32_t steps, nrecompute, nstuck;
     static constexpr int kParkWords = 34;
     static constexpr bool kHint = true;
+    static constexpr int kLanes = 1;
+    static constexpr bool kLocates = false;
     template <class P> __device__ __forceinline__ void park(P& p)
     {
         p.io(x); p.io(y); p.io(z); p.io(kx); p.io(ky); p.io(kz); p.io(ix); p.io(iy); p.io(iz);
@@ -876,6 +921,16 @@ struct TreeW32 {
         if (n < 0) { ne = 0; done = true; return; }
         descend_from(t, n, i, j, k);
     }
+    // The leaf of a walk's start point strictly inside the grid, as init finds it, else -1.
+    __device__ __forceinline__ static int locate_start(const View& t, double rx_, double ry_, double rz_)
+    {
+        if (!strictly_inside(t.ext, rx_, ry_, rz_)) return -1;
+        TreeW32 w;
+        w.x = (float)rx_; w.y = (float)ry_; w.z = (float)rz_;
+        w.kx = 0; w.ky = 0; w.kz = 0;
+        int32_t i, j, k;
+        return w.descend_root(t, nullptr, 0, -1, 0, i, j, k);
+    }
     // The leaf of the last segment returned (-1 before the first one): after a walk that stopped
     // inside a segment, the leaf holding the stopping point.
     __device__ __forceinline__ int hint() const { return lm; }
@@ -885,9 +940,7 @@ struct TreeW32 {
     __device__ __forceinline__ void init_hinted(const View& t, const int32_t* lds, int nlds, double rx_, double ry_,
                                                 double rz_, double dx, double dy, double dz, int hn)
     {
-        const double* e = t.ext;
-        const bool inside = rx_ > e[0] && rx_ < e[3] && ry_ > e[1] && ry_ < e[4] && rz_ > e[2] && rz_ < e[5];
-        if (!(inside && hn >= 0 && hn < t.nnodes)) { init(t, lds, nlds, rx_, ry_, rz_, dx, dy, dz); return; }
+        if (!(strictly_inside(t.ext, rx_, ry_, rz_) && hn >= 0 && hn < t.nnodes)) { init(t, lds, nlds, rx_, ry_, rz_, dx, dy, dz); return; }
         steps = 0; done = false; m = -1; lm = -1; ne = 0;
         x = (float)rx_; y = (float)ry_; z = (float)rz_;
         set_direction(dx, dy, dz);
@@ -1050,7 +1103,7 @@ struct TreeW32TopDown : TreeW32 {
 
 // VoronoiMesh::cellIndex (VoronoiMesh.cpp:541-570): the nearest site, ties to the lower index,
 // found over a uniform bucket grid by growing shells until no closer site can remain.
-__device__ int voro_nearest(const VoroView& g, double x, double y, double z)
+__device__ __noinline__ int voro_nearest(const VoroView& g, double x, double y, double z)
 {
     if (!box_contains(g.ext, x, y, z)) return -1;
     int n = g.nbk;
@@ -1161,6 +1214,29 @@ __device__ __forceinline__ double voro_wall_si(const VoroView& g, double x, doub
     }
 }
 
+// The same two distances as fractions a / b with the sign of b made positive (the quotient's bits stay): a plane
+// that does not lie ahead has b <= 0 or a NaN, as a wall the ray runs along.
+__device__ __forceinline__ void voro_site_fraction(double x, double y, double z, double kx, double ky, double kz,
+                                                   double px, double py, double pz, double qx, double qy, double qz,
+                                                   double& a, double& b)
+{
+    const double nx = qx - px, ny = qy - py, nz = qz - pz;
+    b = nx * kx + ny * ky + nz * kz;
+    const double mx = 0.5 * (qx + px), my = 0.5 * (qy + py), mz = 0.5 * (qz + pz);
+    a = nx * (mx - x) + ny * (my - y) + nz * (mz - z);
+}
+__device__ __forceinline__ void voro_wall_fraction(const VoroView& g, double x, double y, double z, double kx, double ky,
+                                                   double kz, int mi, double& a, double& b)
+{
+    const int w = -1 - mi;   // 0..5: -x +x -y +y -z +z
+    const bool fy = (w >> 1) == 1, fz = (w >> 1) == 2;
+    const double lo = pick3(fy, fz, g.ext[0], g.ext[1], g.ext[2]), hi = pick3(fy, fz, g.ext[3], g.ext[4], g.ext[5]);
+    const double e = (w & 1) ? hi : lo, p = pick3(fy, fz, x, y, z), k = pick3(fy, fz, kx, ky, kz);
+    const bool neg = k < 0;
+    a = neg ? p - e : e - p;
+    b = neg ? -k : k;
+}
+
 #ifndef SG_VORO_GROUP
 #define SG_VORO_GROUP 16
 #endif
@@ -1185,6 +1261,8 @@ template <typename R> struct VoroW {
     static constexpr int kParkWords = 31;
     __device__ __forceinline__ static int cell_of(const View&, int n) { return n; }
     static constexpr bool kHint = true;
+    static constexpr int kLanes = 1;
+    static constexpr bool kLocates = false;
     __device__ __forceinline__ int entries() const { return en.ne; }
     static constexpr bool kStep = true;
     template <class P> __device__ __forceinline__ void park(P& p)
@@ -1284,6 +1362,300 @@ template <typename R> struct VoroW {
         while (step(g, lds, nlds, mo, ds, rh))
             if (segout) return true;
         return false;
+    }
+};
+
+// ---------------------------------------------------------------- Voronoi walks of several lanes
+
+// Value of the lane whose place in the group of L lanes differs from this lane's in one bit (the steps over 4
+// and 8 mirror eight and sixteen lanes, which serves once the quads, and the eights, are uniform).
+template <int BIT> __device__ __forceinline__ uint32_t group_xor(uint32_t v)
+{
+    // quad_perm 1 0 3 2, quad_perm 2 3 0 1, row_half_mirror, row_mirror
+    constexpr int ctrl = BIT == 1 ? 0xB1 : BIT == 2 ? 0x4E : BIT == 4 ? 0x141 : 0x140;
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xf, 0xf, true);
+}
+template <int BIT> __device__ __forceinline__ double group_xor(double v)
+{
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    const uint32_t lo = group_xor<BIT>((uint32_t)b), hi = group_xor<BIT>((uint32_t)(b >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+// The smallest (v, k) over the group's lanes (v first, then k), with k's payload if there is one.
+template <int BIT> __device__ __forceinline__ void group_min_step(double& v, int& k, uint32_t* u)
+{
+    const double ov = group_xor<BIT>(v);
+    const int ok = (int)group_xor<BIT>((uint32_t)k);
+    const bool take = (ov < v) | ((ov == v) & (ok < k));
+    if (u) {
+        const uint32_t ou = group_xor<BIT>(*u);
+        *u = take ? ou : *u;
+    }
+    v = take ? ov : v;
+    k = take ? ok : k;
+}
+template <int L> __device__ __forceinline__ void group_min(double& v, int& k, uint32_t* u = nullptr)
+{
+    if constexpr (L >= 2) group_min_step<1>(v, k, u);
+    if constexpr (L >= 4) group_min_step<2>(v, k, u);
+    if constexpr (L >= 8) group_min_step<4>(v, k, u);
+    if constexpr (L >= 16) group_min_step<8>(v, k, u);
+}
+template <int L> __device__ __forceinline__ uint32_t group_or(uint32_t v)
+{
+    if constexpr (L >= 2) v |= group_xor<1>(v);
+    if constexpr (L >= 4) v |= group_xor<2>(v);
+    if constexpr (L >= 8) v |= group_xor<4>(v);
+    if constexpr (L >= 16) v |= group_xor<8>(v);
+    return v;
+}
+
+// VoroW's walk taken by a group of L neighbouring lanes: every lane of the group holds the same walk, the
+// entries of a cell's list are dealt out to the lanes, and the nearest plane ahead is the group's smallest
+// (distance, place in the list), which is the reference's strict "<" in list order, bit for bit. One lane per
+// walk leaves the wave waiting for its longest lists (a third of the lanes active) with every load touching
+// 64 cache lines, and the sixteen entries it holds cost 256 registers; four lanes per walk load a whole
+// 128-byte line at once and hold G entries each. The location of a walk's start (voro_locate's greedy search)
+// runs in the same steps: a step tests the next L * G entries of the current cell's list, for the nearest site
+// while the walk is locating its start and for the nearest plane afterwards, so that there is one place that
+// loads entries and a lane that starts a walk does not hold up its wave.
+template <typename R, int L, int G> struct VoroC {
+    using Real = R;
+    using View = VoroView;
+    static constexpr int NO_INDEX = -99;
+    double x, y, z, kx, ky, kz;
+    double sqc;              // the best entry of the current cell's list so far: its plane's distance along the
+    int mqc;                 // ray (its squared distance from the position while locating), its id and its list
+    uint32_t lqc;
+    int mr, lm;
+    int hb, tcur, tend;      // the current cell's header record, next entry to test, end of its entries
+    Entry en;
+    bool done, segout, loc, thin;
+    bool located;            // the walk only locates its position, and ends there
+    uint32_t steps, nrecompute, nstuck;
+    __device__ __forceinline__ static int cell_of(const View&, int n) { return n; }
+    static constexpr bool kHint = true;
+    static constexpr int kLanes = L;
+    static constexpr bool kLocates = true;
+    static constexpr bool kStep = true;
+    __device__ __forceinline__ int entries() const { return en.ne; }
+    __device__ __forceinline__ static int place() { return (int)(threadIdx.x & (L - 1)); }
+    __device__ __forceinline__ int hint() const { return lm; }
+    // Enters cell mr, whose list is at `list` (0: looked up).
+    __device__ __forceinline__ void enter(const View& g, uint32_t list)
+    {
+        int n = (int)(list & kVoroMaxCount);
+        hb = (int)(list >> 7) * kVoroLine;
+        if (list == 0) {
+            const int2 be = g.off[mr];
+            hb = be.x; n = be.y;
+        }
+        tcur = hb + 1; tend = hb + 1 + n;
+        sqc = DBL_MAX; mqc = NO_INDEX; lqc = 0;
+        thin = false;
+    }
+    // Starts locating the position from cell `start`, or (-1) from the start site of the position's bucket;
+    // false when it lies outside the box.
+    __device__ __forceinline__ bool start_locating(const View& g, int start)
+    {
+        if (!box_contains(g.ext, x, y, z)) return false;
+        if (start < 0 || start >= g.nsites) {
+            const int n = g.nbk;
+            const int ci = min(n - 1, max(0, (int)(n * (x - g.ext[0]) / (g.ext[3] - g.ext[0]))));
+            const int cj = min(n - 1, max(0, (int)(n * (y - g.ext[1]) / (g.ext[4] - g.ext[1]))));
+            const int ck = min(n - 1, max(0, (int)(n * (z - g.ext[2]) / (g.ext[5] - g.ext[2]))));
+            start = g.brep[(ci * n + cj) * n + ck];
+        }
+        mr = start;
+        loc = true;
+        enter(g, 0);
+        return true;
+    }
+    // hn >= 0: the cell of the start point as locate_start or locate_next found it (it is not looked for again)
+    __device__ __forceinline__ void init_hinted(const View& g, const int32_t*, int, double rx, double ry, double rz,
+                                                double dx, double dy, double dz, int hn)
+    {
+        kx = dx; ky = dy; kz = dz;
+        steps = 0; done = false; lm = -1; located = false;
+        if (hn >= 0 && hn < g.nsites && strictly_inside(g.ext, rx, ry, rz)) {
+            x = rx; y = ry; z = rz;
+            en.ne = 0;
+            mr = hn;
+            loc = false;
+            enter(g, 0);
+            return;
+        }
+        if (!en.move_inside(g.ext, g.eps, rx, ry, rz, kx, ky, kz)) { en.ne = 0; done = true; return; }
+        x = rx; y = ry; z = rz;
+        if (!start_locating(g, -1)) { en.ne = 0; done = true; }
+    }
+    // The cell of a walk's start point strictly inside the grid (which move_inside leaves as it is), else -1. One
+    // lane per point.
+    __device__ __forceinline__ static int locate_start(const View& g, double x, double y, double z)
+    {
+        return strictly_inside(g.ext, x, y, z) ? voro_locate(g, x, y, z, -1) : -1;
+    }
+    // Turns the walk into the location of a point, whose cell hint() is at the end (-1 unless strictly inside
+    // the grid); the search starts at the cell of the walk's last segment.
+    __device__ __forceinline__ void locate_next(const View& g, double rx, double ry, double rz)
+    {
+        x = rx; y = ry; z = rz;
+        const int start = lm;
+        lm = -1;
+        en.ne = 0;
+        done = !strictly_inside(g.ext, rx, ry, rz) || !start_locating(g, start);
+        located = true;
+    }
+    // One step: an entry segment; or L * G more entries of the cell's list (no segment, segout false); or, when
+    // they end the list, the cell's segment (the position moves onto the next cell), or the next cell of the
+    // location. False at the end of the path. Every lane of the group takes the same decisions. What few walks
+    // need at a time (entries, walls, near-ties, locating) is skipped by a test over the wave, and the rest is
+    // straight-line code: a wave with few walks left is bound by the instructions of a step, branches above all.
+    __device__ __forceinline__ bool step(const View& g, const int32_t*, int, int& mo, R& ds, R& rh)
+    {
+        segout = true;
+        if (en.ne) { ds = (R)en.pop(); mo = -1; rh = (R)0; return true; }
+        if (done) return false;
+        const VoroSite pr = load_header(g.nbr + hb);
+        const VoroNbr* p = g.nbr + (tcur + place());
+        const int left = tend - tcur - place();   // the lane's i-th entry is in the list when i * L < left
+        VoroNbr q[G];
+#pragma unroll
+        for (int i = 0; i < G; i++)
+            if (i * L < left) q[i] = load_nbr(p + i * L);
+        // the lane's nearest plane as a fraction num / den (den > 0), without a division per entry: fractions whose
+        // cross products differ by more than 1e-12 are in that order after the division too; if two are closer,
+        // every entry is divided
+        double num = DBL_MAX, den = 0;
+        int best = 0;
+        bool near = false;
+#pragma unroll
+        for (int i = 0; i < G; i++) {
+            double a, b;
+            voro_site_fraction(x, y, z, kx, ky, kz, pr.x, pr.y, pr.z, q[i].x, q[i].y, q[i].z, a, b);
+            if (i == 0 || !g.walls_lead) {
+                const bool wall = (i * L < left) & (q[i].id < 0);
+                if (__any(wall)) {
+                    double wa, wb;
+                    voro_wall_fraction(g, x, y, z, kx, ky, kz, q[i].id, wa, wb);
+                    a = wall ? wa : a;
+                    b = wall ? wb : b;
+                }
+            }
+            const bool ahead = (i * L < left) & (a > 0) & (b > 0);
+            const double ab = a * den, ba = num * b;   // the first plane ahead meets DBL_MAX / 0
+            if (i > 0) near = near | (ahead & (den > 0) & (fabs(ab - ba) <= 1e-12 * ba));
+            const bool take = ahead & (ab < ba);
+            num = take ? a : num;
+            den = take ? b : den;
+            best = take ? i : best;
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        double v = num / den;   // infinite where no plane lies ahead
+        if (__any(near)) {
+            if (near) {
+                v = DBL_MAX;
+#pragma unroll 1
+                for (int i = 0; i < G; i++) {
+                    if (i * L >= left) break;
+                    const VoroNbr e = load_nbr(p + i * L);
+                    const double si = e.id >= 0 ? voro_site_si(x, y, z, kx, ky, kz, pr.x, pr.y, pr.z, e.x, e.y, e.z)
+                                                : voro_wall_si(g, x, y, z, kx, ky, kz, e.id);
+                    if (si > 0 && si < v) { v = si; best = i; }
+                }
+            }
+        }
+        // the lane's entry, then the group's nearest plane: the smallest place in the list among equal ones
+        int id = q[0].id;
+        uint32_t list = q[0].list;
+#pragma unroll
+        for (int i = 1; i < G; i++) {
+            id = best == i ? q[i].id : id;
+            list = best == i ? q[i].list : list;
+        }
+        int at = v < DBL_MAX ? best * L + place() : INT32_MAX;
+        v = v < DBL_MAX ? v : DBL_MAX;
+        group_min<L>(v, at);
+        const int src = (int)(__lane_id() & ~(uint32_t)(L - 1)) | (at & (L - 1));
+        id = __shfl(id, src);
+        list = __shfl(list, src);
+        if (__any(loc)) {
+            if (loc) locate_entries(pr, q, left, v, id, list);
+        }
+        // the entries tested before come first in the list; among sites the lower index wins a tie
+        const bool better = (v < sqc) | (loc & (v == sqc) & (id < mqc));
+        sqc = better ? v : sqc;
+        mqc = better ? id : mqc;
+        lqc = better ? list : lqc;
+        tcur += L * G;
+        const bool ends = tcur >= tend;
+        const int segm = mr;
+        const double d = sqc;
+        bool moves = ends & !loc & (mqc != NO_INDEX);
+        steps += moves ? 1 : 0;
+        if (__any(ends & !moves)) {
+            if (ends & !moves) {
+                segout = false; mo = -1; ds = (R)0; rh = (R)0;
+                return list_end(g);
+            }
+        }
+        const double dm = d + g.eps;
+        x = moves ? x + dm * kx : x;
+        y = moves ? y + dm * ky : y;
+        z = moves ? z + dm * kz : z;
+        mr = moves ? mqc : mr;
+        lm = moves ? segm : lm;
+        done = done | (moves & ((mr < 0) | (steps > SG_MAX_STEPS)));
+        if (moves & (mr >= 0)) enter(g, lqc);
+        segout = moves;
+        mo = moves ? segm : -1; ds = moves ? (R)d : (R)0; rh = (R)pr.rho;
+        return true;
+    }
+    // The location's part of a step: the nearest site among the group's entries (ties to the lower index).
+    __device__ __forceinline__ void locate_entries(const VoroSite& pr, const VoroNbr* q, int left, double& v, int& id,
+                                                   uint32_t& list)
+    {
+        const double dc = (x - pr.x) * (x - pr.x) + (y - pr.y) * (y - pr.y) + (z - pr.z) * (z - pr.z);
+        if (tcur == hb + 1) { sqc = dc; mqc = mr; }
+        v = DBL_MAX; id = INT32_MAX; list = 0;
+#pragma unroll
+        for (int i = 0; i < G; i++) {
+            const int mi = q[i].id;
+            const double d = (x - q[i].x) * (x - q[i].x) + (y - q[i].y) * (y - q[i].y) + (z - q[i].z) * (z - q[i].z);
+            const bool site = (i * L < left) & (mi >= 0);
+            thin = thin | (site & (d - dc <= 1e-9 * d));
+            const bool take = site & ((d < v) | ((d == v) & (mi < id)));
+            v = take ? d : v;
+            id = take ? mi : id;
+            list = take ? q[i].list : list;
+        }
+        group_min<L>(v, id, &list);
+    }
+    // The end of a list that gives no segment: the location moves on to the nearer site or is finished (exactly,
+    // where a neighbour is as near), or no plane lies ahead and the walk moves on by eps and locates the point
+    // again. False when the walk ends here.
+    __device__ __forceinline__ bool list_end(const View& g)
+    {
+        if (loc) {
+            if (mqc != mr) {
+                mr = mqc;
+                enter(g, lqc);
+                return true;
+            }
+            loc = false;
+            const bool exact = group_or<L>(thin ? 1u : 0u) != 0;
+            if (exact) mr = voro_nearest(g, x, y, z);
+            if (located) {
+                lm = mr;
+                done = true;
+            } else enter(g, 0);
+            return true;
+        }
+        if (++steps > SG_MAX_STEPS) { done = true; return false; }
+        nstuck++;
+        x += kx * g.eps; y += ky * g.eps; z += kz * g.eps;
+        if (!start_locating(g, mr)) { done = true; return false; }
+        return true;
     }
 };
 
