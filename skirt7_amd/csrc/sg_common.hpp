@@ -35,6 +35,7 @@ struct CartView {
     int Nx, Ny, Nz;
     double xmin, ymin, zmin, xmax, ymax, zmax;
     float wminf;                     // smallest cell width over the three axes
+    double binsx, binsy, binsz;      // mean number of cells per length along each axis
 };
 
 // Mixed-precision walk record, one per tree NODE (device id), 32 bytes, read as two 16-byte loads:

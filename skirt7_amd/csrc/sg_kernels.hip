@@ -40,6 +40,15 @@ static uint64_t g_emit_batch = 0;   // packets emitted at once (0: each pipeline
 // descents were asked for a TopDown tree.
 static bool rope_walk(const sg_grid* g) { return g->tree.search == SG_NEIGHBOR || !g_topdown_descent; }
 
+// LDS words in which a walker stages a grid's view: a tree's top nodes, or a Cartesian grid's borders where they fit
+// the same room (grids of up to about 1360 cells per axis in FP32, half of that in FP64; larger ones are read from
+// global memory).
+template <typename R> static int cart_words(const sg_grid* g)
+{
+    const int64_t n = border_words(g->cart, sizeof(R));
+    return n <= SG_LDS_NODES ? (int)n : 0;
+}
+
 static void ensure_init()
 {
     if (g_device >= 0) return;
@@ -53,9 +62,9 @@ template <class W>
 __global__ void __launch_bounds__(256) k_paths(const typename W::View g, int64_t n, const double* rk, int maxseg,
                                                 int32_t* counts, int32_t* mo, double* dso)
 {
-    __shared__ int32_t s_nodes[SG_LDS_NODES];
+    __shared__ __align__(16) int32_t s_nodes[SG_LDS_NODES];
     int nlds;
-    stage_tree_nodes(g, s_nodes, nlds);
+    stage_view<W>(g, s_nodes, SG_LDS_NODES, threadIdx.x, blockDim.x, nlds);
     __syncthreads();
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -78,9 +87,9 @@ __global__ void __launch_bounds__(256) k_tau(const typename W::View g, int64_t n
                                               const double* taus, int mode, double* out)
 {
     using R = typename W::Real;
-    __shared__ int32_t s_nodes[SG_LDS_NODES];
+    __shared__ __align__(16) int32_t s_nodes[SG_LDS_NODES];
     int nlds;
-    stage_tree_nodes(g, s_nodes, nlds);
+    stage_view<W>(g, s_nodes, SG_LDS_NODES, threadIdx.x, blockDim.x, nlds);
     __syncthreads();
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -317,6 +326,7 @@ int sg_grid_create_cartesian(const double ext[6], const double* xv, int nxv, con
     for (int i = 0; i + 1 < nyv; i++) wmin = std::min(wmin, yv[i + 1] - yv[i]);
     for (int i = 0; i + 1 < nzv; i++) wmin = std::min(wmin, zv[i + 1] - zv[i]);
     c.wminf = (float)wmin;
+    c.binsx = c.Nx / (c.xmax - c.xmin); c.binsy = c.Ny / (c.ymax - c.ymin); c.binsz = c.Nz / (c.zmax - c.zmin);
     *out = g;
     SG_CATCH
 }
@@ -1283,8 +1293,8 @@ template <bool ABS, bool MULTI = false> static void dispatch_mc(sg_sim* s, const
         return;
     }
     if (g->kind == GK_CART) {
-        if (mixed) launch_mc<CartW32, ABS, MULTI>(g->cart, a, blocks, s->cold, s->args);
-        else launch_mc<CartW64, ABS, MULTI>(g->cart, a, blocks, s->cold, s->args);
+        if (mixed) launch_mc<CartW32, ABS, MULTI>(g->cart, a, blocks, s->cold, s->args, cart_words<float>(g));
+        else launch_mc<CartW64, ABS, MULTI>(g->cart, a, blocks, s->cold, s->args, cart_words<double>(g));
     } else if (g->kind == GK_TREE) {
         if (!mixed && g->tree.search == SG_BOOKKEEPING)
             launch_mc<TreeW64Book, ABS, MULTI>(g->tree, a, blocks, s->cold, s->args, 0);
@@ -1588,8 +1598,8 @@ static void dispatch_split(sg_sim* s, const McArgs& a, int precision, uint64_t f
         return;
     }
     if (g->kind == GK_CART) {
-        if (mixed) run_split<CartW32, ABS>(s, g->cart, a, first, count, 0, lt, blocks);
-        else run_split<CartW64, ABS>(s, g->cart, a, first, count, 0, lt, blocks);
+        if (mixed) run_split<CartW32, ABS>(s, g->cart, a, first, count, cart_words<float>(g), lt, blocks);
+        else run_split<CartW64, ABS>(s, g->cart, a, first, count, cart_words<double>(g), lt, blocks);
     } else if (g->kind == GK_TREE) {
         if (!mixed && g->tree.search == SG_BOOKKEEPING) run_split<TreeW64Book, ABS>(s, g->tree, a, first, count, 0, lt, blocks);
         else if (!mixed) run_split<TreeW64, ABS>(s, g->tree, a, first, count, SG_LDS_NODES, lt, blocks);
@@ -1913,8 +1923,8 @@ static void dispatch_static(sg_sim* s, const McArgs& a, int precision, int& bloc
         if (mixed) run_static<CartW32, false>(s, v, a, 0, blocks);
         else run_static<CartW64, false>(s, v, a, 0, blocks);
     } else if (g->kind == GK_CART) {
-        if (mixed) run_static<CartW32, ABS>(s, g->cart, a, 0, blocks);
-        else run_static<CartW64, ABS>(s, g->cart, a, 0, blocks);
+        if (mixed) run_static<CartW32, ABS>(s, g->cart, a, cart_words<float>(g), blocks);
+        else run_static<CartW64, ABS>(s, g->cart, a, cart_words<double>(g), blocks);
     } else if (g->kind == GK_TREE) {
         if (!mixed && g->tree.search == SG_BOOKKEEPING) run_static<TreeW64Book, ABS>(s, g->tree, a, 0, blocks);
         else if (!mixed) run_static<TreeW64, ABS>(s, g->tree, a, SG_LDS_NODES, blocks);
@@ -2132,7 +2142,12 @@ static void launch_batch(sg_sim* s0, const std::vector<McArgs>& rg, const std::v
     SG_HIP(hipGetLastError());
 
     int bs = g_tune_block;
-    size_t shm = SG_PARK ? hot_words<W>() * 4 * (size_t)bs : 0;
+    // each wave stages its range's Cartesian borders in LDS, up to 4 KB per wave
+    int64_t words = 0;
+    if constexpr (std::is_same<V, CartView>::value)
+        for (const V& v : views) words = std::max<int64_t>(words, (border_words(v, sizeof(R)) + 3) / 4 * 4);
+    const int nlds = (int)std::min<int64_t>(words, 1024);
+    size_t shm = (SG_PARK ? hot_words<W>() * 4 * (size_t)bs : 0) + (size_t)(bs / 64) * nlds * sizeof(int32_t);
     int per = 0;
     SG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_mc_batch<W, ABS>, bs, shm));
     if (per < 1) per = 1;
@@ -2144,7 +2159,7 @@ static void launch_batch(sg_sim* s0, const std::vector<McArgs>& rg, const std::v
     R* cr = s0->cold.as<R>();
     uint32_t* cu = reinterpret_cast<uint32_t*>(s0->cold.as<unsigned char>() + (size_t)nslots * CR_NR * sizeof(R));
     lt.start();
-    hipLaunchKernelGGL((k_mc_batch<W, ABS>), dim3(blocks), dim3(bs), shm, 0, vtab, atab, (int)nr, cr, cu, nslots);
+    hipLaunchKernelGGL((k_mc_batch<W, ABS>), dim3(blocks), dim3(bs), shm, 0, vtab, atab, (int)nr, cr, cu, nslots, nlds);
     SG_HIP(hipGetLastError());
     lt.stop();
 }

@@ -802,10 +802,7 @@ k_mc(const typename W::View g, const McArgs a, int nlds_req, typename W::Real* c
     uint32_t* park = reinterpret_cast<uint32_t*>(smem);
     int32_t* s_nodes = reinterpret_cast<int32_t*>(smem + (SG_PARK ? hot_words<W>() * 4 * nl : 0));
     int nlds = 0;
-    if (nlds_req > 0) {
-        stage_tree_nodes(g, s_nodes, nlds);
-        nlds = min(nlds, nlds_req);
-    }
+    if (nlds_req > 0) stage_view<W>(g, s_nodes, nlds_req, threadIdx.x, blockDim.x, nlds);
     if (threadIdx.x < SG_MAX_INSTR) s_instr[threadIdx.x] = a.scene->instr[threadIdx.x];
     ColdSlot<typename W::Real> c;
     c.r = cold_r; c.u = cold_u; c.nl = nslots;
@@ -823,11 +820,14 @@ k_mc(const typename W::View g, const McArgs a, int nlds_req, typename W::Real* c
 template <class W, bool ABS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(McWaves<W>::value, 8)))
 k_mc_batch(const typename W::View* gtab, const McArgs* atab, int nranges, typename W::Real* cold_r,
-           uint32_t* cold_u, int nslots)
+           uint32_t* cold_u, int nslots, int nlds_req)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ InstrDev s_instr[4 * SG_MAX_INSTR];   // one instrument table per wave of the block
     uint32_t* park = reinterpret_cast<uint32_t*>(smem);
+    // the wave's part of its range's grid view (nlds_req words per wave)
+    int32_t* my_nodes = reinterpret_cast<int32_t*>(smem + (SG_PARK ? hot_words<W>() * 4 * blockDim.x : 0)) +
+                        (threadIdx.x >> 6) * nlds_req;
     InstrDev* my_instr = s_instr + (threadIdx.x >> 6) * SG_MAX_INSTR;
     ColdSlot<typename W::Real> c;
     c.r = cold_r; c.u = cold_u; c.nl = nslots;
@@ -846,10 +846,12 @@ k_mc_batch(const typename W::View* gtab, const McArgs* atab, int nranges, typena
         }
         __builtin_amdgcn_wave_barrier();
         if (__lane_id() < SG_MAX_INSTR) my_instr[__lane_id()] = ap->scene->instr[__lane_id()];
+        int nlds = 0;
+        if (nlds_req > 0) stage_view<W>(gtab[r], my_nodes, nlds_req, (int)__lane_id(), 64, nlds);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        drain<W, ABS>(gtab[r], *ap, park, nullptr, 0, c, my_instr, gtab + r, ap);
+        drain<W, ABS>(gtab[r], *ap, park, my_nodes, nlds, c, my_instr, gtab + r, ap);
         scanned = 0;
     }
 }

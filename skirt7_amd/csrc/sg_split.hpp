@@ -580,6 +580,8 @@ template <> struct WalkWaves<TreeW32> { static constexpr int value = SG_W32_WAVE
 #define SG_W64_WAVES 3
 #endif
 template <> struct WalkWaves<TreeW64> { static constexpr int value = SG_W64_WAVES; };
+// the exact Cartesian walk spills nothing at three (1e6 packets on 50^3 cells: 9.2 ms; 9.4 at four, 11.1 at five)
+template <> struct WalkWaves<CartW64> { static constexpr int value = 3; };
 // Lanes per Voronoi walk and entries per lane and step: 8 x 3 = 24 entries a step, which most lists (19 on average
 // along the walks) fit, at three waves per SIMD, where nothing spills in the walk. On 1e5 sites with 3 x 1e5 packets:
 // 33 ms a run; four lanes x 6 42 ms, 8 x 2 50 ms and 8 x 3 51 ms at four waves (spills), 16 x 2 50 ms; one lane x 16
@@ -713,10 +715,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WalkWa
     if ((uint64_t)blockIdx.x * (blockDim.x >> 6) * kClaimMin >= nq) return;
     int32_t* s_nodes = reinterpret_cast<int32_t*>(smem);
     int nlds = 0;
-    if (nlds_req > 0) {
-        stage_tree_nodes(g, s_nodes, nlds);
-        nlds = min(nlds, nlds_req);
-    }
+    if (nlds_req > 0) stage_view<W>(g, s_nodes, nlds_req, threadIdx.x, blockDim.x, nlds);
     if (threadIdx.x < SG_MAX_INSTR) s_instr[threadIdx.x] = a.scene->instr[threadIdx.x];
     __syncthreads();
     const WalkReq<R>* reqs = q.sorted ? q.sorted : q.req;

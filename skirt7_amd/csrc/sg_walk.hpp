@@ -58,38 +58,123 @@ template <bool LOAD> struct Park {
     }
 };
 
-// Stages the first breadth-first tree node words (the top levels) in LDS.
-__device__ __forceinline__ void stage_tree_nodes(const TreeView& t, int32_t* lds, int& n)
+// The part of a grid view that a walker reads from LDS, staged by the lanes first, first + step, ...: the top
+// levels' node words of a tree, the cell borders of a Cartesian grid (in the walker's real type); at most `room`
+// words, n receives the number staged (0: the walker reads global memory).
+template <class W>
+__device__ __forceinline__ void stage_view(const TreeView& t, int32_t* lds, int room, int first, int step, int& n)
 {
-    n = min((int)t.nnodes, SG_LDS_NODES);
-    for (int i = threadIdx.x; i < n; i += blockDim.x) lds[i] = t.node[i];
+    n = min((int)t.nnodes, min(room, SG_LDS_NODES));
+    for (int i = first; i < n; i += step) lds[i] = t.node[i];
 }
-__device__ __forceinline__ void stage_tree_nodes(const CartView&, int32_t*, int& n) { n = 0; }
-__device__ __forceinline__ void stage_tree_nodes(const VoroView&, int32_t*, int& n) { n = 0; }
+__host__ __device__ inline int64_t border_words(const CartView& g, size_t real)
+{
+    return ((int64_t)g.Nx + g.Ny + g.Nz + 3) * (int64_t)(real / sizeof(int32_t));
+}
+template <class W>
+__device__ __forceinline__ void stage_view(const CartView& g, int32_t* lds, int room, int first, int step, int& n)
+{
+    using R = typename W::Real;
+    n = 0;
+    if (border_words(g, sizeof(R)) > room) return;
+    n = (int)border_words(g, sizeof(R));
+    R* b = reinterpret_cast<R*>(lds);
+    for (int i = first; i <= g.Nx; i += step) b[i] = W::border(g, 0, i);
+    b += g.Nx + 1;
+    for (int i = first; i <= g.Ny; i += step) b[i] = W::border(g, 1, i);
+    b += g.Ny + 1;
+    for (int i = first; i <= g.Nz; i += step) b[i] = W::border(g, 2, i);
+}
+template <class W>
+__device__ __forceinline__ void stage_view(const VoroView&, int32_t*, int, int, int, int& n) { n = 0; }
 
 // ====================================================================== Cartesian
 
-// CartesianDustGrid.cpp:136-283, exact FP64.
+// One of three per-axis values by flags (fy: y, fz: z, neither: x). The values pass through an empty
+// register constraint first: a select between two loads of one structure is otherwise folded into a
+// load through a selected address, which keeps the whole walker in private (scratch) memory.
+template <typename T> __device__ __forceinline__ T pick3(bool fy, bool fz, T vx, T vy, T vz)
+{
+    asm("" : "+v"(vx), "+v"(vy), "+v"(vz));
+    return fz ? vz : fy ? vy : vx;
+}
+
+// x / k for y = 1 / k correctly rounded (a walk's reciprocal direction): two Newton steps on the quotient, each with
+// its remainder from one fused multiply-add. The first leaves a quotient within one unit in the last place, the
+// second rounds it correctly (P. Markstein, Computation of elementary functions on the IBM RISC System/6000, IBM J.
+// Res. Dev. 34, 1990: with y = RN(1/k) and a faithful q, RN(q + y RN(x - k q)) = RN(x / k)), barring overflow and
+// underflow, which lengths over direction components above 1e-15 stay far from. 5 operations instead of about 12.
+__device__ __forceinline__ double quotient(double x, double k, double y)
+{
+    double q = x * y;
+    q = fma(fma(-k, q, x), y, q);
+    return fma(fma(-k, q, x), y, q);
+}
+
+// The borders of a Cartesian grid as a walker reads them: from LDS when they are staged there.
+template <typename R> struct Borders {
+    bool staged;
+    const R* lds;            // x, y and z borders one after another (when staged)
+    const R *xv, *yv, *zv;
+    int oy, oz;              // places of the y and z borders in lds
+    // border `at` of the axis given by the flags fy, fz (neither: x)
+    __device__ __forceinline__ R get(bool fy, bool fz, int at) const
+    {
+        if (staged) return lds[at + pick3(fy, fz, 0, oy, oz)];
+        return pick3(fy, fz, xv, yv, zv)[at];
+    }
+    // NR::locate_clip over the axis's n + 1 borders: the bin guessed from an even spacing (scale bins per length) is
+    // taken when it holds x, the only one that does; else a binary search finds it
+    __device__ __forceinline__ int locate(bool fy, bool fz, int n, R x, R lo, R scale) const
+    {
+        const int i = max(0, min(n - 1, (int)((x - lo) * scale)));
+        if (get(fy, fz, i) <= x && (i == n - 1 || x < get(fy, fz, i + 1))) return i;
+        if (x < get(fy, fz, 0)) return 0;
+        int jl = -1, ju = n;
+        while (ju - jl > 1) {
+            const int jm = (ju + jl) >> 1;
+            if (x < get(fy, fz, jm)) ju = jm;
+            else jl = jm;
+        }
+        return jl;
+    }
+};
+
+// CartesianDustGrid.cpp:136-283, exact FP64. A step is bound by its chain of dependent operations: the exit walls
+// of the current cell are kept, so that a step reads one border (from LDS), the distances are quotients by the
+// walk's reciprocal direction (the same bits as a division), and the next cell's density is loaded one step ahead.
 struct CartW64 {
     using Real = double;
     using View = CartView;
-    double x, y, z, kx, ky, kz;
-    int i, j, k;
+    double x, y, z, kx, ky, kz, ix, iy, iz;
+    double xE, yE, zE;       // exit walls of the current cell
+    double rho;              // its density
+    int i, j, k, m;          // its indices and number
     int ne;
     double e0, e1, e2;
     bool done;
     uint32_t nrecompute, nstuck;
-    static constexpr int kParkWords = 25;
+    static constexpr int kParkWords = 38;
     __device__ __forceinline__ static int cell_of(const View&, int n) { return n; }
     static constexpr bool kHint = false;
     static constexpr int kLanes = 1;
     static constexpr bool kLocates = false;
     __device__ __forceinline__ int entries() const { return ne; }
-    static constexpr bool kStep = false;   // next() only
+    static constexpr bool kStep = true;
+    __device__ __forceinline__ static double border(const View& g, int axis, int i)
+    {
+        return (axis == 0 ? g.xv : axis == 1 ? g.yv : g.zv)[i];
+    }
+    __device__ __forceinline__ static Borders<double> borders(const View& g, const int32_t* lds, int nlds)
+    {
+        return Borders<double>{nlds > 0, reinterpret_cast<const double*>(lds), g.xv, g.yv, g.zv, g.Nx + 1,
+                               g.Nx + g.Ny + 2};
+    }
     template <class P> __device__ __forceinline__ void park(P& p)
     {
-        p.io(x); p.io(y); p.io(z); p.io(kx); p.io(ky); p.io(kz);
-        p.io(i); p.io(j); p.io(k); p.io(ne); p.io(e0); p.io(e1); p.io(e2);
+        p.io(x); p.io(y); p.io(z); p.io(kx); p.io(ky); p.io(kz); p.io(ix); p.io(iy); p.io(iz);
+        p.io(xE); p.io(yE); p.io(zE); p.io(rho);
+        p.io(i); p.io(j); p.io(k); p.io(m); p.io(ne); p.io(e0); p.io(e1); p.io(e2);
         p.io(done); p.io(nrecompute); p.io(nstuck);
     }
 
@@ -103,8 +188,8 @@ struct CartW64 {
             ne++;
         }
     }
-    __device__ __forceinline__ void init(const View& g, const int32_t*, int, double rx, double ry, double rz, double dx, double dy,
-                         double dz)
+    __device__ __forceinline__ void init(const View& g, const int32_t* lds, int nlds, double rx, double ry, double rz, double dx,
+                                         double dy, double dz)
     {
         x = rx; y = ry; z = rz; kx = dx; ky = dy; kz = dz;
         ne = 0; done = false;
@@ -139,44 +224,67 @@ struct CartW64 {
         if (x < g.xmin || x > g.xmax || y < g.ymin || y > g.ymax || z < g.zmin || z > g.zmax) {
             ne = 0; done = true; return;
         }
-        i = locate_clip(g.xv, g.Nx + 1, x);
-        j = locate_clip(g.yv, g.Ny + 1, y);
-        k = locate_clip(g.zv, g.Nz + 1, z);
+        const Borders<double> b = borders(g, lds, nlds);
+        i = b.locate(false, false, g.Nx, x, g.xmin, g.binsx);
+        j = b.locate(true, false, g.Ny, y, g.ymin, g.binsy);
+        k = b.locate(false, true, g.Nz, z, g.zmin, g.binsz);
+        ix = fabs(kx) > 1e-15 ? 1.0 / kx : 0.0;
+        iy = fabs(ky) > 1e-15 ? 1.0 / ky : 0.0;
+        iz = fabs(kz) > 1e-15 ? 1.0 / kz : 0.0;
+        xE = b.get(false, false, kx < 0.0 ? i : i + 1);
+        yE = b.get(true, false, ky < 0.0 ? j : j + 1);
+        zE = b.get(false, true, kz < 0.0 ? k : k + 1);
+        m = k + g.Nz * j + g.Nz * g.Ny * i;
+        rho = g.rho[m];
     }
-    __device__ __forceinline__ bool next(const View& g, const int32_t*, int, int& m, double& ds, double& rho)
+    // One wall step: an entry segment, or the segment to the next wall (of length zero on an edge or corner); false
+    // at the end of the path.
+    __device__ __forceinline__ bool step(const View& g, const int32_t* lds, int nlds, int& mo, double& ds, double& rh)
     {
         if (ne) {
-            ds = e0; e0 = e1; e1 = e2; ne--; m = -1; rho = 0.0;
+            ds = e0; e0 = e1; e1 = e2; ne--; mo = -1; rh = 0.0;
             return true;
         }
-        while (!done) {
-            int mm = k + g.Nz * j + g.Nz * g.Ny * i;
-            double xE = (kx < 0.0) ? g.xv[i] : g.xv[i + 1];
-            double yE = (ky < 0.0) ? g.yv[j] : g.yv[j + 1];
-            double zE = (kz < 0.0) ? g.zv[k] : g.zv[k + 1];
-            double dsx = (fabs(kx) > 1e-15) ? (xE - x) / kx : DBL_MAX;
-            double dsy = (fabs(ky) > 1e-15) ? (yE - y) / ky : DBL_MAX;
-            double dsz = (fabs(kz) > 1e-15) ? (zE - z) / kz : DBL_MAX;
-            double d;
-            if (dsx <= dsy && dsx <= dsz) {
-                d = dsx; i += (kx < 0.0) ? -1 : 1;
-                if (i >= g.Nx || i < 0) done = true;
-                else { x = xE; y += ky * d; z += kz * d; }
-            } else if (dsy < dsx && dsy <= dsz) {
-                d = dsy; j += (ky < 0.0) ? -1 : 1;
-                if (j >= g.Ny || j < 0) done = true;
-                else { x += kx * d; y = yE; z += kz * d; }
-            } else if (dsz < dsx && dsz < dsy) {
-                d = dsz; k += (kz < 0.0) ? -1 : 1;
-                if (k >= g.Nz || k < 0) done = true;
-                else { x += kx * d; y += ky * d; z = zE; }
-            } else {
-                // only reachable with NaN input; the reference would not terminate
-                done = true;
-                return false;
-            }
-            if (d > 0) { m = mm; ds = d; rho = g.rho[mm]; return true; }
+        if (done) return false;
+        const double dsx = ix != 0.0 ? quotient(xE - x, kx, ix) : DBL_MAX;
+        const double dsy = iy != 0.0 ? quotient(yE - y, ky, iy) : DBL_MAX;
+        const double dsz = iz != 0.0 ? quotient(zE - z, kz, iz) : DBL_MAX;
+        const bool fx = (dsx <= dsy) & (dsx <= dsz);
+        const bool fy = !fx & (dsy < dsx) & (dsy <= dsz);
+        const bool fz = !fx & !fy & (dsz < dsx) & (dsz < dsy);
+        if (!(fx | fy | fz)) {
+            // only reachable with NaN input; the reference would not terminate
+            done = true;
+            return false;
         }
+        const double d = fx ? dsx : fy ? dsy : dsz;
+        mo = m; ds = d; rh = rho;
+        const int s = pick3(fy, fz, kx, ky, kz) < 0.0 ? -1 : 1;
+        const int at = pick3(fy, fz, i, j, k) + s;   // the new index along the exit axis
+        i = fx ? at : i;
+        j = fy ? at : j;
+        k = fz ? at : k;
+        if ((at < 0) | (at >= pick3(fy, fz, g.Nx, g.Ny, g.Nz))) {
+            done = true;
+            return true;
+        }
+        m += s * pick3(fy, fz, g.Nz * g.Ny, g.Nz, 1);
+        rho = g.rho[m];
+        const double xn = x + kx * d, yn = y + ky * d, zn = z + kz * d;
+        x = fx ? xE : xn;
+        y = fy ? yE : yn;
+        z = fz ? zE : zn;
+        const double e = borders(g, lds, nlds).get(fy, fz, at + (s > 0 ? 1 : 0));
+        xE = fx ? e : xE;
+        yE = fy ? e : yE;
+        zE = fz ? e : zE;
+        return true;
+    }
+    // The next segment of positive length.
+    __device__ __forceinline__ bool next(const View& g, const int32_t* lds, int nlds, int& mo, double& ds, double& rh)
+    {
+        while (step(g, lds, nlds, mo, ds, rh))
+            if (ds > 0) return true;
         return false;
     }
 };
@@ -184,12 +292,6 @@ struct CartW64 {
 // Chooses the exit wall among three distances with the reference tie rules
 // (CartesianDustGrid.cpp:243-269: x on <=, y on < x and <= z, z strictly smallest).
 __device__ __forceinline__ int choose_axis_cart(double dx, double dy, double dz)
-{
-    if (dx <= dy && dx <= dz) return 0;
-    if (dy < dx && dy <= dz) return 1;
-    return 2;
-}
-__device__ __forceinline__ int choose_axis_cart(float dx, float dy, float dz)
 {
     if (dx <= dy && dx <= dz) return 0;
     if (dy < dx && dy <= dz) return 1;
@@ -203,46 +305,43 @@ template <typename T> __device__ __forceinline__ int choose_axis_tree(T dx, T dy
     return 2;
 }
 
-// One of three per-axis values by flags (fy: y, fz: z, neither: x). The values pass through an empty
-// register constraint first: a select between two loads of one structure is otherwise folded into a
-// load through a selected address, which keeps the whole walker in private (scratch) memory.
-template <typename T> __device__ __forceinline__ T pick3(bool fy, bool fz, T vx, T vy, T vz)
-{
-    asm("" : "+v"(vx), "+v"(vy), "+v"(vz));
-    return fz ? vz : fy ? vy : vx;
-}
-
-// True when the FP32 exit decision is ambiguous: the two smallest wall distances agree to 1e-5
-// relative (a corner or edge crossing), or the chosen distance d is within 1e-5 of zero relative
-// to the cell, measured along the exit axis (ka: direction component, wa: cell width on that axis).
-// Distances of directions parallel to a wall are FLT_MAX and never count as ambiguous.
-__device__ __forceinline__ bool ambiguous(float dx, float dy, float dz, float d, float ka, float wa)
-{
-    float mid = fmaxf(fminf(dx, dy), fminf(fmaxf(dx, dy), dz));
-    return ((mid < FLT_MAX) & ((mid - d) <= 1e-5f * mid)) | (d * fabsf(ka) <= 1e-5f * wa);
-}
-
-// Mixed-precision Cartesian walk.
+// Mixed-precision Cartesian walk, in the manner of CartW64: kept exit walls, one border per step, the density one
+// step ahead. The FP32 exit decision is ambiguous, and taken in FP64, when the two smallest wall distances agree to
+// 1e-5 relative (a corner or edge crossing), or the chosen distance is within 1e-5 of zero relative to the smallest
+// cell width, measured along the exit axis. Distances of directions parallel to a wall are FLT_MAX and never count
+// as ambiguous.
 struct CartW32 {
     using Real = float;
     using View = CartView;
     float x, y, z, kx, ky, kz, ix, iy, iz;
-    int i, j, k;
+    float xE, yE, zE;        // exit walls of the current cell
+    float rho;               // its density
+    int i, j, k, m;          // its indices and number
     int ne;
     float e0, e1, e2;
     bool done;
     uint32_t nrecompute, nstuck;
-    static constexpr int kParkWords = 19;
+    static constexpr int kParkWords = 24;
     __device__ __forceinline__ static int cell_of(const View&, int n) { return n; }
     static constexpr bool kHint = false;
     static constexpr int kLanes = 1;
     static constexpr bool kLocates = false;
     __device__ __forceinline__ int entries() const { return ne; }
-    static constexpr bool kStep = false;   // next() only
+    static constexpr bool kStep = true;
+    __device__ __forceinline__ static float border(const View& g, int axis, int i)
+    {
+        return (axis == 0 ? g.xvf : axis == 1 ? g.yvf : g.zvf)[i];
+    }
+    __device__ __forceinline__ static Borders<float> borders(const View& g, const int32_t* lds, int nlds)
+    {
+        return Borders<float>{nlds > 0, reinterpret_cast<const float*>(lds), g.xvf, g.yvf, g.zvf, g.Nx + 1,
+                              g.Nx + g.Ny + 2};
+    }
     template <class P> __device__ __forceinline__ void park(P& p)
     {
         p.io(x); p.io(y); p.io(z); p.io(kx); p.io(ky); p.io(kz); p.io(ix); p.io(iy); p.io(iz);
-        p.io(i); p.io(j); p.io(k); p.io(ne); p.io(e0); p.io(e1); p.io(e2);
+        p.io(xE); p.io(yE); p.io(zE); p.io(rho);
+        p.io(i); p.io(j); p.io(k); p.io(m); p.io(ne); p.io(e0); p.io(e1); p.io(e2);
         p.io(done); p.io(nrecompute); p.io(nstuck);
     }
 
@@ -256,8 +355,8 @@ struct CartW32 {
             ne++;
         }
     }
-    __device__ __forceinline__ void init(const View& g, const int32_t*, int, double rxd, double ryd, double rzd, double dxd,
-                         double dyd, double dzd)
+    __device__ __forceinline__ void init(const View& g, const int32_t* lds, int nlds, double rxd, double ryd, double rzd, double dxd,
+                                         double dyd, double dzd)
     {
         // entry in FP64, state in FP32
         double x0 = rxd, y0 = ryd, z0 = rzd;
@@ -292,49 +391,71 @@ struct CartW32 {
         ix = fabsf(kx) > 1e-15f ? 1.0f / kx : 0.0f;
         iy = fabsf(ky) > 1e-15f ? 1.0f / ky : 0.0f;
         iz = fabsf(kz) > 1e-15f ? 1.0f / kz : 0.0f;
-        i = locate_clip(g.xvf, g.Nx + 1, x);
-        j = locate_clip(g.yvf, g.Ny + 1, y);
-        k = locate_clip(g.zvf, g.Nz + 1, z);
+        const Borders<float> b = borders(g, lds, nlds);
+        i = b.locate(false, false, g.Nx, x, (float)g.xmin, (float)g.binsx);
+        j = b.locate(true, false, g.Ny, y, (float)g.ymin, (float)g.binsy);
+        k = b.locate(false, true, g.Nz, z, (float)g.zmin, (float)g.binsz);
+        xE = b.get(false, false, kx < 0.0f ? i : i + 1);
+        yE = b.get(true, false, ky < 0.0f ? j : j + 1);
+        zE = b.get(false, true, kz < 0.0f ? k : k + 1);
+        m = k + g.Nz * j + g.Nz * g.Ny * i;
+        rho = g.rhof[m];
     }
-    __device__ __forceinline__ bool next(const View& g, const int32_t*, int, int& m, float& ds, float& rho)
+    // One wall step, as CartW64's.
+    __device__ __forceinline__ bool step(const View& g, const int32_t* lds, int nlds, int& mo, float& ds, float& rh)
     {
         if (ne) {
-            ds = e0; e0 = e1; e1 = e2; ne--; m = -1; rho = 0.0f;
+            ds = e0; e0 = e1; e1 = e2; ne--; mo = -1; rh = 0.0f;
             return true;
         }
-        while (!done) {
-            int mm = k + g.Nz * j + g.Nz * g.Ny * i;
-            int ie = (kx < 0.0f) ? i : i + 1, je = (ky < 0.0f) ? j : j + 1, ke = (kz < 0.0f) ? k : k + 1;
-            float xE = g.xvf[ie], yE = g.yvf[je], zE = g.zvf[ke];
-            float dsx = ix != 0.0f ? (xE - x) * ix : FLT_MAX;
-            float dsy = iy != 0.0f ? (yE - y) * iy : FLT_MAX;
-            float dsz = iz != 0.0f ? (zE - z) * iz : FLT_MAX;
-            int a = choose_axis_cart(dsx, dsy, dsz);
-            float d = a == 0 ? dsx : a == 1 ? dsy : dsz;
-            if (ambiguous(dsx, dsy, dsz, d, a == 0 ? kx : a == 1 ? ky : kz, g.wminf)) {
-                nrecompute++;
-                double X = x, Y = y, Z = z;
-                double ddx = ix != 0.0f ? (g.xv[ie] - X) / (double)kx : DBL_MAX;
-                double ddy = iy != 0.0f ? (g.yv[je] - Y) / (double)ky : DBL_MAX;
-                double ddz = iz != 0.0f ? (g.zv[ke] - Z) / (double)kz : DBL_MAX;
-                a = choose_axis_cart(ddx, ddy, ddz);
-                d = (float)(a == 0 ? ddx : a == 1 ? ddy : ddz);
-            }
-            if (a == 0) {
-                i += (kx < 0.0f) ? -1 : 1;
-                if (i >= g.Nx || i < 0) done = true;
-                else { x = xE; y = fmaf(ky, d, y); z = fmaf(kz, d, z); }
-            } else if (a == 1) {
-                j += (ky < 0.0f) ? -1 : 1;
-                if (j >= g.Ny || j < 0) done = true;
-                else { x = fmaf(kx, d, x); y = yE; z = fmaf(kz, d, z); }
-            } else {
-                k += (kz < 0.0f) ? -1 : 1;
-                if (k >= g.Nz || k < 0) done = true;
-                else { x = fmaf(kx, d, x); y = fmaf(ky, d, y); z = zE; }
-            }
-            if (d > 0) { m = mm; ds = d; rho = g.rhof[mm]; return true; }
+        if (done) return false;
+        const float dsx = ix != 0.0f ? (xE - x) * ix : FLT_MAX;
+        const float dsy = iy != 0.0f ? (yE - y) * iy : FLT_MAX;
+        const float dsz = iz != 0.0f ? (zE - z) * iz : FLT_MAX;
+        bool fx = (dsx <= dsy) & (dsx <= dsz);
+        bool fy = !fx & (dsy < dsx) & (dsy <= dsz);
+        float d = fx ? dsx : fy ? dsy : dsz;
+        float ka = pick3(fy, !fx & !fy, kx, ky, kz);
+        const float mid = fmaxf(fminf(dsx, dsy), fminf(fmaxf(dsx, dsy), dsz));
+        if (((mid < FLT_MAX) & ((mid - d) <= 1e-5f * mid)) | (d * fabsf(ka) <= 1e-5f * g.wminf)) {
+            nrecompute++;
+            const double X = x, Y = y, Z = z;
+            const double ddx = ix != 0.0f ? (g.xv[kx < 0.0f ? i : i + 1] - X) / (double)kx : DBL_MAX;
+            const double ddy = iy != 0.0f ? (g.yv[ky < 0.0f ? j : j + 1] - Y) / (double)ky : DBL_MAX;
+            const double ddz = iz != 0.0f ? (g.zv[kz < 0.0f ? k : k + 1] - Z) / (double)kz : DBL_MAX;
+            const int a = choose_axis_cart(ddx, ddy, ddz);
+            fx = a == 0;
+            fy = a == 1;
+            d = (float)(fx ? ddx : fy ? ddy : ddz);
+            ka = pick3(fy, !fx & !fy, kx, ky, kz);
         }
+        const bool fz = !fx & !fy;
+        mo = m; ds = d; rh = rho;
+        const int s = ka < 0.0f ? -1 : 1;
+        const int at = pick3(fy, fz, i, j, k) + s;   // the new index along the exit axis
+        i = fx ? at : i;
+        j = fy ? at : j;
+        k = fz ? at : k;
+        if ((at < 0) | (at >= pick3(fy, fz, g.Nx, g.Ny, g.Nz))) {
+            done = true;
+            return true;
+        }
+        m += s * pick3(fy, fz, g.Nz * g.Ny, g.Nz, 1);
+        rho = g.rhof[m];
+        x = fx ? xE : fmaf(kx, d, x);
+        y = fy ? yE : fmaf(ky, d, y);
+        z = fz ? zE : fmaf(kz, d, z);
+        const float e = borders(g, lds, nlds).get(fy, fz, at + (s > 0 ? 1 : 0));
+        xE = fx ? e : xE;
+        yE = fy ? e : yE;
+        zE = fz ? e : zE;
+        return true;
+    }
+    // The next segment of positive length.
+    __device__ __forceinline__ bool next(const View& g, const int32_t* lds, int nlds, int& mo, float& ds, float& rh)
+    {
+        while (step(g, lds, nlds, mo, ds, rh))
+            if (ds > 0) return true;
         return false;
     }
 };
@@ -447,14 +568,14 @@ struct Entry {
 struct TreeW64 {
     using Real = double;
     using View = TreeView;
-    double x, y, z, kx, ky, kz;
+    double x, y, z, kx, ky, kz, ix, iy, iz;
     double lo[3], hi[3];
     double rho;
     int m, lm;               // current cell, cell of the last segment returned
     Entry en;
     bool done;
     uint32_t steps, nrecompute, nstuck;
-    static constexpr int kParkWords = 39;
+    static constexpr int kParkWords = 45;
     __device__ __forceinline__ static int cell_of(const View&, int n) { return n; }
     static constexpr bool kHint = true;
     static constexpr int kLanes = 1;
@@ -463,7 +584,7 @@ struct TreeW64 {
     static constexpr bool kStep = false;   // next() only
     template <class P> __device__ __forceinline__ void park(P& p)
     {
-        p.io(x); p.io(y); p.io(z); p.io(kx); p.io(ky); p.io(kz);
+        p.io(x); p.io(y); p.io(z); p.io(kx); p.io(ky); p.io(kz); p.io(ix); p.io(iy); p.io(iz);
         p.io(lo[0]); p.io(lo[1]); p.io(lo[2]); p.io(hi[0]); p.io(hi[1]); p.io(hi[2]);
         p.io(rho); p.io(m); p.io(lm); p.io(en.ne); p.io(en.e0); p.io(en.e1); p.io(en.e2);
         p.io(done); p.io(steps); p.io(nrecompute); p.io(nstuck);
@@ -488,10 +609,17 @@ struct TreeW64 {
         rho = t.rec64[c].rho;
         return true;
     }
+    __device__ __forceinline__ void set_direction(double dx, double dy, double dz)
+    {
+        kx = dx; ky = dy; kz = dz;
+        ix = fabs(kx) > 1e-15 ? 1.0 / kx : 0.0;
+        iy = fabs(ky) > 1e-15 ? 1.0 / ky : 0.0;
+        iz = fabs(kz) > 1e-15 ? 1.0 / kz : 0.0;
+    }
     __device__ __forceinline__ void init(const View& t, const int32_t* lds, int nlds, double rx, double ry, double rz, double dx,
                          double dy, double dz)
     {
-        kx = dx; ky = dy; kz = dz;
+        set_direction(dx, dy, dz);
         steps = 0; done = false; lm = -1;
         if (!en.move_inside(t.ext, t.eps, rx, ry, rz, kx, ky, kz)) {
             // OUTSIDE sentinel: no node contains it, path cleared
@@ -520,7 +648,7 @@ struct TreeW64 {
         if (strictly_inside(t.ext, rx, ry, rz) && hn >= 0 && hn < t.ncells) {
             const TreeRec64& r = t.rec64[hn];
             if (rx >= r.lo[0] && rx < r.hi[0] && ry >= r.lo[1] && ry < r.hi[1] && rz >= r.lo[2] && rz < r.hi[2]) {
-                kx = dx; ky = dy; kz = dz;
+                set_direction(dx, dy, dz);
                 x = rx; y = ry; z = rz;
                 steps = 0; done = false; lm = -1; en.ne = 0;
                 load_cell(t, hn);
@@ -537,9 +665,9 @@ struct TreeW64 {
             double xnext = (kx < 0.0) ? lo[0] : hi[0];
             double ynext = (ky < 0.0) ? lo[1] : hi[1];
             double znext = (kz < 0.0) ? lo[2] : hi[2];
-            double dsx = (fabs(kx) > 1e-15) ? (xnext - x) / kx : DBL_MAX;
-            double dsy = (fabs(ky) > 1e-15) ? (ynext - y) / ky : DBL_MAX;
-            double dsz = (fabs(kz) > 1e-15) ? (znext - z) / kz : DBL_MAX;
+            double dsx = ix != 0.0 ? quotient(xnext - x, kx, ix) : DBL_MAX;
+            double dsy = iy != 0.0 ? quotient(ynext - y, ky, iy) : DBL_MAX;
+            double dsz = iz != 0.0 ? quotient(znext - z, kz, iz) : DBL_MAX;
             int a = choose_axis_tree(dsx, dsy, dsz);
             double d = a == 0 ? dsx : a == 1 ? dsy : dsz;
             int wall = 2 * a + ((a == 0 ? kx : a == 1 ? ky : kz) < 0.0 ? 0 : 1);
@@ -1414,8 +1542,8 @@ template <int L> __device__ __forceinline__ uint32_t group_or(uint32_t v)
 // entries of a cell's list are dealt out to the lanes, and the nearest plane ahead is the group's smallest
 // (distance, place in the list), which is the reference's strict "<" in list order, bit for bit. One lane per
 // walk leaves the wave waiting for its longest lists (a third of the lanes active) with every load touching
-// 64 cache lines, and the sixteen entries it holds cost 256 registers; four lanes per walk load a whole
-// 128-byte line at once and hold G entries each. The location of a walk's start (voro_locate's greedy search)
+// 64 cache lines, and the sixteen entries it holds cost 256 registers; eight lanes per walk load two whole
+// 128-byte lines at once and hold G entries each. The location of a walk's start (voro_locate's greedy search)
 // runs in the same steps: a step tests the next L * G entries of the current cell's list, for the nearest site
 // while the walk is locating its start and for the nearest plane afterwards, so that there is one place that
 // loads entries and a lane that starts a walk does not hold up its wave.

@@ -42,3 +42,41 @@ def test_passes_equal_the_lane_pipeline(disc, count, groups, batch, precision):
         S.set_emit_batch(0)
     assert c == cref
     np.testing.assert_allclose(out, ref, rtol=1e-10, atol=0)
+
+
+@pytest.mark.parametrize("lists", ["as built", "shuffled", "superset"])
+def test_voronoi_walks_of_several_lanes(lists):
+    """The walk kernel's Voronoi walk (a group of lanes per walk) against the lane pipeline's (one lane): lists with
+    their walls first, lists in any order, and lists longer than an entry's count holds (more than 127)."""
+    rng = np.random.default_rng(3)
+    ext = np.array([-20.0, -20.0, -20.0, 20.0, 20.0, 20.0])
+    sites = ext[:3] + rng.random((400, 3)) * 40.0
+    off, ids = S.voronoi_neighbors(ext, sites)
+    per = [ids[off[i]:off[i + 1]] for i in range(len(sites))]
+    if lists == "shuffled":
+        per = [rng.permutation(p) for p in per]
+    elif lists == "superset":
+        # more sites than neighbours: planes beyond the cell's faces are never the nearest ahead
+        extra = [np.setdiff1d(rng.choice(len(sites), 150, replace=False), np.append(p, i)) for i, p in enumerate(per)]
+        per = [np.concatenate([p, e]).astype(np.int32) for p, e in zip(per, extra)]
+        assert max(len(p) for p in per) > 127
+    off = np.concatenate([[0], np.cumsum([len(p) for p in per])])
+    grid = S.VoronoiDustGrid(ext, sites, off, np.concatenate(per))
+    w = workloads.disc_cartesian(grid_n=4, pixels=20, packages=100)
+    stars, mix = w["stars"], w["mix"]
+    out = []
+    for mode in (0, 1):
+        dust = S.DustSystem(grid, np.full(len(sites), 0.05), mix, writeMeanIntensity=True)
+        w["instr"].clear()
+        sim = S.OligoMonteCarloSimulation(dust, stars, w["instr"], packages=3000, seed=11)
+        try:
+            S.set_pipeline(mode)
+            c = sim.run_packets(0, 0, 3000, 3000, SG_FP64)
+        finally:
+            S.set_pipeline(1)
+        out.append((np.concatenate([w["instr"].frame(i).ravel() for i in range(3)]), dust.Labs(), c["own_crossings"],
+                    c["peel_crossings"], c["rewalk_crossings"], c["scatterings"]))
+    assert out[0][2:] == out[1][2:]
+    # sums of at most some ten thousand positive FP64 terms in another order
+    np.testing.assert_allclose(out[1][0], out[0][0], rtol=1e-11, atol=0)
+    np.testing.assert_allclose(out[1][1], out[0][1], rtol=1e-11, atol=0)
