@@ -86,8 +86,9 @@ int sg_dust_destroy(sg_dust* d);
  * see KappaRho, the sum over components of kappaext(h) rho(m, h) (DustSystem.cpp:459-485); escape and
  * absorption use each cell's own albedo (MonteCarloSimulation.cpp:463-508); scattering peel-offs weight the
  * components' phase functions by kappasca(h) rho(m, h) (:318-343) and scattering draws the component with
- * those weights (DustSystem::randomMixForPosition, DustSystem.cpp:855-869). Such systems run in the lane
- * pipeline (sg_sim_run and batched runs; sg_sim_run_static refuses them). ncomp == 1 is sg_dust_create. */
+ * those weights (DustSystem::randomMixForPosition, DustSystem.cpp:855-869). sg_sim_run takes such systems in
+ * either pipeline, a batched run one member at a time in the lane pipeline; sg_sim_run_static refuses them.
+ * ncomp == 1 is sg_dust_create. */
 int sg_dust_create_multi(sg_grid* g, int ncomp, const double* rho, int64_t ncells, int nlambda, const double* kappaext,
                          const double* kappasca, const double* albedo, const double* asymmpar, int store_absorption,
                          sg_dust** out);

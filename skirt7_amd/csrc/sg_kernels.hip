@@ -1320,6 +1320,13 @@ static void dispatch_mc_any(sg_sim* s, const McArgs& a, int precision, int& bloc
 }
 // ---------------------------------------------------------------- split pipeline
 
+__global__ void k_set_u64(unsigned long long* p, unsigned long long v) { *p = v; }
+static void launch_set(unsigned long long* p, unsigned long long v, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(1), 0, st, p, v);
+    SG_HIP(hipGetLastError());
+}
+
 __global__ void k_revive(uint32_t* state, int64_t n)
 {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1343,7 +1350,7 @@ static double g_clock_khz = 100000.0;                   // of the device's wall 
 // (runs are synchronous and driven by one host thread): slot groups, walk queues, progress counters,
 // launch states. Allocated on first use, grown as needed, kept until the process ends.
 struct SplitPool {
-    DevBuf slots[2], queue[2], prog[2], emitted, emitdraw, emithint;
+    DevBuf slots[2], queue[2], prog[2], events[2], waves[2], emitted, emitdraw, emithint;
     DevBuf bins[2];   // per group: bin counts (zero between passes: cleared once, then by each pass's scan), offsets
 };
 static SplitPool* g_pool = nullptr;
@@ -1390,15 +1397,17 @@ template <typename R> struct PassGroups {
     Slots<R> sl[2];
     WalkQueue<R> q[2];
     GroupCtl* ctl[2];
+    GroupTally tally[2];
     int pass[2];                // passes enqueued so far (the place in the progress rings)
-    int blocks, bs, ebs, nlds, order;
-    size_t shm, eshm;
+    int blocks, bs, nlds, order;
+    size_t shm;
 };
+static int64_t event_blocks(int64_t slots) { return (slots + kEventBlock - 1) / kEventBlock; }
 
 // Event and walk passes of every group until all packets of ab have been claimed and the groups' walk queues stay
 // empty. Each group keeps kSplitAhead passes enqueued beyond the one whose progress is awaited. Returns the
 // walk launches that had requests.
-template <class W, bool ABS>
+template <class W, bool ABS, bool MULTI>
 static int run_passes(const typename W::View& v, const McArgs& ab, PassGroups<typename W::Real>& pg)
 {
     using R = typename W::Real;
@@ -1406,6 +1415,7 @@ static int run_passes(const typename W::View& v, const McArgs& ab, PassGroups<ty
     int seen[2] = {pg.pass[0], pg.pass[1]};
     bool done[2] = {false, pg.n < 2};
     int launches = 0;
+    const int pass0[2] = {pg.pass[0], pg.pass[1]};
     auto enqueue = [&](int g) {
         const int p = pg.pass[g]++;
         const int w = g * kProgressRing + p % kProgressRing;
@@ -1414,16 +1424,16 @@ static int run_passes(const typename W::View& v, const McArgs& ab, PassGroups<ty
         WalkQueue<R> q = pg.q[g];
         q.tail = &pc->tail;
         const int64_t P = pg.sl[g].n;
-        hipLaunchKernelGGL(k_events<R>, dim3((P + pg.ebs - 1) / pg.ebs), dim3(pg.ebs), pg.eshm, st[g], ab, pg.sl[g], q,
-                           pg.ctl[g], p);
+        hipLaunchKernelGGL((k_events<R, MULTI>), dim3(event_blocks(P) + 1), dim3(kEventBlock), 0, st[g], ab, pg.sl[g], q,
+                           pg.ctl[g], p, p == pass0[g] ? 1 : 0, pg.tally[g]);
         SG_HIP(hipGetLastError());
         if (q.sorted) {
             hipLaunchKernelGGL(k_key_scan, dim3(1), dim3(1024), 0, st[g], q.hist, q.off);
             hipLaunchKernelGGL(k_key_scatter<R>, dim3(g_cus * 8), dim3(256), 0, st[g], q, ab.error);
             SG_HIP(hipGetLastError());
         }
-        hipLaunchKernelGGL((k_walks<W, ABS>), dim3(pg.blocks), dim3(pg.bs), pg.shm, st[g], v, ab, q, pg.sl[g], pc,
-                           g_split_host_dev + w, pg.nlds, pg.order == 2 ? kXcdSegs : 0);
+        hipLaunchKernelGGL((k_walks<W, ABS, MULTI>), dim3(pg.blocks), dim3(pg.bs), pg.shm, st[g], v, ab, q, pg.sl[g], pc,
+                           g_split_host_dev + w, pg.tally[g], pg.nlds, pg.order == 2 ? kXcdSegs : 0);
         SG_HIP(hipGetLastError());
     };
     while (!done[0] || !done[1]) {
@@ -1459,6 +1469,12 @@ static void launch_emit(const typename W::View& v, McArgs& a, void* emitted, uin
     SG_HIP(hipGetLastError());
 }
 
+static void launch_counts(const GroupTally& ta, unsigned long long* counters, hipStream_t st)
+{
+    const int64_t n = std::max<int64_t>(ta.nevents, ta.nwaves);
+    hipLaunchKernelGGL(k_run_counts, dim3(std::min<int64_t>((n + 255) / 256, 16)), dim3(256), 0, st, ta, counters);
+}
+
 // Duration of the groups' walk kernels (the passes have ended).
 static double walk_ms(GroupCtl* const* ctl, int n)
 {
@@ -1474,7 +1490,7 @@ static double walk_ms(GroupCtl* const* ctl, int n)
 // Packets [first, first+count) through event and walk passes over two slot groups that alternate on two
 // streams, so that one group's event pass and the drain of its walk pass overlap the other group's
 // walks. Up to 2^25 packets are emitted at once.
-template <class W, bool ABS>
+template <class W, bool ABS, bool MULTI = false>
 static void run_split(sg_sim* s, const typename W::View& v, const McArgs& a, uint64_t first, uint64_t count, int nlds,
                       LaunchTimer& lt, int& blocks)
 {
@@ -1486,6 +1502,13 @@ static void run_split(sg_sim* s, const typename W::View& v, const McArgs& a, uin
     PassGroups<R> pg{};
     const int G = pg.n = (P >= 2 && g_slot_groups == 2) ? 2 : 1;
     const int64_t Pg[2] = {G == 2 ? (P + 1) / 2 : P, G == 2 ? P / 2 : 0};
+    const int bs = pg.bs = g_tune_block;
+    pg.nlds = nlds;
+    pg.order = g_walk_order;
+    pg.shm = (size_t)nlds * sizeof(int32_t);
+    int per = 0;
+    SG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_walks<W, ABS, MULTI>, bs, pg.shm));
+    pg.blocks = blocks = std::max(1, per) * g_cus;
     for (int g = 0; g < G; g++) {
         const int64_t cap = Pg[g] * (a.ni + 1);
         SplitPool& pl = pool();
@@ -1515,22 +1538,21 @@ static void run_split(sg_sim* s, const typename W::View& v, const McArgs& a, uin
             q.hist = pl.bins[g].as<uint32_t>();
             q.off = q.hist + kKeyBins;
         }
-        // progress records; slot states PS_FRESH and slot counts zero (adjacent arrays)
+        // progress and count records zero; slot states PS_FRESH
+        GroupTally& ta = pg.tally[g];
+        ta.nevents = event_blocks(Pg[g]);
+        ta.nwaves = pg.blocks * (pg.bs / 64);
+        ta.slot0 = g ? Pg[0] : 0;
+        const size_t ebytes = (size_t)ta.nevents * 4 * sizeof(unsigned long long), wbytes = (size_t)ta.nwaves * sizeof(WaveRec);
+        if (pl.events[g].bytes < ebytes) pl.events[g].alloc(ebytes);
+        if (pl.waves[g].bytes < wbytes) pl.waves[g].alloc(wbytes);
+        ta.events = pl.events[g].as<unsigned long long>();
+        ta.waves = pl.waves[g].as<WaveRec>();
         SG_HIP(hipMemsetAsync(pg.ctl[g], 0, sizeof(GroupCtl), st[g]));
-        SG_HIP(hipMemsetAsync(sl.u + (size_t)SU_STATE * Pg[g], 0, (size_t)Pg[g] * (SU_NU - SU_STATE) * sizeof(uint32_t),
-                              st[g]));
+        SG_HIP(hipMemsetAsync(ta.events, 0, ebytes, st[g]));
+        SG_HIP(hipMemsetAsync(ta.waves, 0, wbytes, st[g]));
+        SG_HIP(hipMemsetAsync(sl.u + (size_t)SU_STATE * Pg[g], 0, (size_t)Pg[g] * sizeof(uint32_t), st[g]));
     }
-    const int bs = pg.bs = g_tune_block;
-    pg.nlds = nlds;
-    pg.order = g_walk_order;
-    pg.shm = (size_t)nlds * sizeof(int32_t);
-    int per = 0;
-    SG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_walks<W, ABS>, bs, pg.shm));
-    pg.blocks = blocks = std::max(1, per) * g_cus;
-    // event workgroups stage up to blockDim * (ni + 1) requests in LDS
-    pg.ebs = 256;
-    while (pg.ebs > 64 && staged_bytes<R>(pg.ebs, a.ni) > 64 * 1024) pg.ebs /= 2;
-    pg.eshm = staged_bytes<R>(pg.ebs, a.ni);
     const uint64_t batch = std::min<uint64_t>(count, g_emit_batch ? g_emit_batch : kSplitEmit);
     const size_t rsz = sizeof(R);
     DevBuf& emitted = pool().emitted;
@@ -1555,7 +1577,8 @@ static void run_split(sg_sim* s, const typename W::View& v, const McArgs& a, uin
             SG_HIP(hipEventRecord(ev_join, st[1]));
             SG_HIP(hipStreamWaitEvent(st[0], ev_join, 0));
         }
-        SG_HIP(hipMemsetAsync(claims, 0, sizeof(unsigned long long), st[0]));
+        // the slots take the batch's first packets by their numbers, the others are claimed
+        launch_set(claims, (unsigned long long)P, st[0]);
         launch_emit<W>(v, ab, emitted.p, emitdraw.as<uint32_t>(), emithint.as<int32_t>(), st[0]);
         for (int g = 0; g < G && b > 0; g++)
             hipLaunchKernelGGL(k_revive, dim3((Pg[g] + 255) / 256), dim3(256), 0, st[0],
@@ -1565,12 +1588,11 @@ static void run_split(sg_sim* s, const typename W::View& v, const McArgs& a, uin
             SG_HIP(hipEventRecord(ev_join, st[0]));
             SG_HIP(hipStreamWaitEvent(st[1], ev_join, 0));
         }
-        walk_launches += run_passes<W, ABS>(v, ab, pg);
+        walk_launches += run_passes<W, ABS, MULTI>(v, ab, pg);
     }
     // each group's counts on its own stream, behind its last passes
     for (int g = 0; g < G; g++) {
-        hipLaunchKernelGGL(k_slot_counts, dim3(std::min<int64_t>((Pg[g] + 255) / 256, 1024)), dim3(256), 0, st[g],
-                           pg.sl[g].u, Pg[g], a.counters);
+        launch_counts(pg.tally[g], a.counters, st[g]);
         SG_HIP(hipGetLastError());
         SG_HIP(hipEventRecord(ev_end[g], st[g]));
     }
@@ -1585,7 +1607,7 @@ static void run_split(sg_sim* s, const typename W::View& v, const McArgs& a, uin
     for (int g = 0; g < 2; g++) (void)hipEventDestroy(ev_end[g]);
 }
 
-template <bool ABS>
+template <bool ABS, bool MULTI>
 static void dispatch_split(sg_sim* s, const McArgs& a, int precision, uint64_t first, uint64_t count, LaunchTimer& lt,
                            int& blocks)
 {
@@ -1598,16 +1620,29 @@ static void dispatch_split(sg_sim* s, const McArgs& a, int precision, uint64_t f
         return;
     }
     if (g->kind == GK_CART) {
-        if (mixed) run_split<CartW32, ABS>(s, g->cart, a, first, count, cart_words<float>(g), lt, blocks);
-        else run_split<CartW64, ABS>(s, g->cart, a, first, count, cart_words<double>(g), lt, blocks);
+        if (mixed) run_split<CartW32, ABS, MULTI>(s, g->cart, a, first, count, cart_words<float>(g), lt, blocks);
+        else run_split<CartW64, ABS, MULTI>(s, g->cart, a, first, count, cart_words<double>(g), lt, blocks);
     } else if (g->kind == GK_TREE) {
-        if (!mixed && g->tree.search == SG_BOOKKEEPING) run_split<TreeW64Book, ABS>(s, g->tree, a, first, count, 0, lt, blocks);
-        else if (!mixed) run_split<TreeW64, ABS>(s, g->tree, a, first, count, SG_LDS_NODES, lt, blocks);
-        else if (rope_walk(g)) run_split<TreeW32, ABS>(s, g->tree, a, first, count, SG_LDS_NODES, lt, blocks);
-        else run_split<TreeW32TopDown, ABS>(s, g->tree, a, first, count, SG_LDS_NODES, lt, blocks);
+        if (!mixed && g->tree.search == SG_BOOKKEEPING) run_split<TreeW64Book, ABS, MULTI>(s, g->tree, a, first, count, 0, lt, blocks);
+        else if (!mixed) run_split<TreeW64, ABS, MULTI>(s, g->tree, a, first, count, SG_LDS_NODES, lt, blocks);
+        else if (rope_walk(g)) run_split<TreeW32, ABS, MULTI>(s, g->tree, a, first, count, SG_LDS_NODES, lt, blocks);
+        else run_split<TreeW32TopDown, ABS, MULTI>(s, g->tree, a, first, count, SG_LDS_NODES, lt, blocks);
     } else {
-        if (mixed) run_split<VoroWalk<float>, ABS>(s, g->voro, a, first, count, 0, lt, blocks);
-        else run_split<VoroWalk<double>, ABS>(s, g->voro, a, first, count, 0, lt, blocks);
+        if (mixed) run_split<VoroWalk<float>, ABS, MULTI>(s, g->voro, a, first, count, 0, lt, blocks);
+        else run_split<VoroWalk<double>, ABS, MULTI>(s, g->voro, a, first, count, 0, lt, blocks);
+    }
+}
+
+// The event/walk pipeline for a run's arguments: absorption stored or not, one or several dust components.
+static void dispatch_split_any(sg_sim* s, const McArgs& a, int precision, uint64_t first, uint64_t count, LaunchTimer& lt,
+                               int& blocks)
+{
+    if (a.ncomp > 1) {
+        if (a.store_abs) dispatch_split<true, true>(s, a, precision, first, count, lt, blocks);
+        else dispatch_split<false, true>(s, a, precision, first, count, lt, blocks);
+    } else {
+        if (a.store_abs) dispatch_split<true, false>(s, a, precision, first, count, lt, blocks);
+        else dispatch_split<false, false>(s, a, precision, first, count, lt, blocks);
     }
 }
 
@@ -1625,9 +1660,7 @@ int sg_sim_run(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64_t npp,
     const bool mixed = precision == SG_MIXED;
     const size_t rsz = mixed ? sizeof(float) : sizeof(double);
     const uint64_t batch = std::min<uint64_t>(count, g_emit_batch ? g_emit_batch : (uint64_t)1 << 22);
-    // several dust components run in the lane pipeline
-    const int pipeline = a.ncomp > 1 ? 0 : g_pipeline;
-    if (pipeline != g_pipeline && g_tune_compact <= 0) a.compact = 32;
+    const int pipeline = g_pipeline;
     if (pipeline == 0) {
         if (s->emitted.bytes < 7 * batch * rsz) s->emitted.alloc(7 * batch * rsz);
         if (s->emitdraw.bytes < batch * sizeof(uint32_t)) s->emitdraw.alloc(batch * sizeof(uint32_t));
@@ -1638,10 +1671,7 @@ int sg_sim_run(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64_t npp,
     SG_HIP(hipEventRecord(e0, 0));
     int blocks = 0;
     LaunchTimer lt;
-    if (pipeline == 1 && count > 0) {
-        if (a.store_abs) dispatch_split<true>(s, a, precision, first, count, lt, blocks);
-        else dispatch_split<false>(s, a, precision, first, count, lt, blocks);
-    }
+    if (pipeline == 1 && count > 0) dispatch_split_any(s, a, precision, first, count, lt, blocks);
     // the lane pipeline runs in batches: emission kernel, then the persistent transport kernel
     for (uint64_t b = 0; pipeline == 0 && b < count; b += batch) {
         McArgs ab = a;
@@ -1870,10 +1900,23 @@ static void run_static(sg_sim* s, const typename W::View& v, const McArgs& a0, i
     hipStream_t st = g_split_stream[0];
     const int64_t P = (int64_t)std::max<uint64_t>(1, std::min<uint64_t>(a0.count, (uint64_t)kStaticSlots));
     const int64_t cap = P * (a0.ni + 1);
-    // layout of the static array: slots, walk requests, progress records, launch states, draw counts, start cells
+    // layout of the static array: slots, walk requests, progress records, counts, launch states, draw counts, start cells
     const size_t o_q = align256(slot_bytes<R>(P));
     const size_t o_pc = o_q + align256((size_t)cap * sizeof(WalkReq<R>));
-    const size_t o_em = o_pc + align256(sizeof(GroupCtl));
+    PassGroups<R> pg{};
+    pg.bs = g_tune_block;
+    pg.nlds = nlds;
+    pg.shm = (size_t)nlds * sizeof(int32_t);
+    int per = 0;
+    SG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_walks<W, ABS, false>, pg.bs, pg.shm));
+    pg.blocks = blocks = std::max(1, per) * g_cus;
+    GroupTally& ta = pg.tally[0];
+    ta.nevents = event_blocks(P);
+    ta.nwaves = pg.blocks * (pg.bs / 64);
+    const size_t ebytes = (size_t)ta.nevents * 4 * sizeof(unsigned long long), wbytes = (size_t)ta.nwaves * sizeof(WaveRec);
+    const size_t o_ev = o_pc + align256(sizeof(GroupCtl));
+    const size_t o_wv = o_ev + align256(ebytes);
+    const size_t o_em = o_wv + align256(wbytes);
     const size_t o_ed = o_em + align256(7 * a0.count * sizeof(R));
     const size_t o_eh = o_ed + align256(a0.count * sizeof(uint32_t));
     const size_t need = o_eh + align256(a0.count * sizeof(int32_t));
@@ -1881,34 +1924,28 @@ static void run_static(sg_sim* s, const typename W::View& v, const McArgs& a0, i
                                                 " bytes of work memory, more than the static array holds");
     unsigned char* base = static_cast<unsigned char*>(g_scratch[g_device]);
     SG_REQUIRE(base != nullptr, "sg_sim_run_static: the static work array of this device is not set up");
-    PassGroups<R> pg{};
     pg.n = 1;
     Slots<R>& sl = pg.sl[0];
     sl = Slots<R>{reinterpret_cast<R*>(base), reinterpret_cast<uint32_t*>(base + (size_t)P * SR_NR * sizeof(R)), P};
     pg.ctl[0] = reinterpret_cast<GroupCtl*>(base + o_pc);
+    ta.events = reinterpret_cast<unsigned long long*>(base + o_ev);
+    ta.waves = reinterpret_cast<WaveRec*>(base + o_wv);
     pg.q[0].req = reinterpret_cast<WalkReq<R>*>(base + o_q);
     pg.q[0].cap = cap;
     McArgs a = a0;
     a.next_packet = s->next.as<unsigned long long>();
-    // cleared by kernels: slot states (PS_FRESH) and counts, progress, the packet claims, counters, error flag
-    fill_u32(sl.u + (size_t)SU_STATE * P, P * (SU_NU - SU_STATE), st);
+    // cleared by kernels: slot states (PS_FRESH), counts, progress, the packet claims, counters, error flag
+    fill_u32(sl.u + (size_t)SU_STATE * P, P, st);
+    fill_u32(ta.events, (int64_t)(ebytes / sizeof(uint32_t)), st);
+    fill_u32(ta.waves, (int64_t)(wbytes / sizeof(uint32_t)), st);
     fill_u32(pg.ctl[0], sizeof(GroupCtl) / sizeof(uint32_t), st);
-    fill_u32(s->next.p, 2, st);
+    launch_set(s->next.as<unsigned long long>(), (unsigned long long)P, st);
     fill_u32(s->counters.p, 2 * SG_NCOUNTERS, st);
     fill_u32(s->err.p, 1, st);
-    pg.bs = g_tune_block;
-    pg.nlds = nlds;
-    pg.shm = (size_t)nlds * sizeof(int32_t);
-    int per = 0;
-    SG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_walks<W, ABS>, pg.bs, pg.shm));
-    pg.blocks = blocks = std::max(1, per) * g_cus;
-    pg.ebs = 256;
-    while (pg.ebs > 64 && staged_bytes<R>(pg.ebs, a.ni) > 64 * 1024) pg.ebs /= 2;
-    pg.eshm = staged_bytes<R>(pg.ebs, a.ni);
     if (a.count > 0)
         launch_emit<W>(v, a, base + o_em, reinterpret_cast<uint32_t*>(base + o_ed), reinterpret_cast<int32_t*>(base + o_eh), st);
-    run_passes<W, ABS>(v, a, pg);
-    hipLaunchKernelGGL(k_slot_counts, dim3(std::min<int64_t>((P + 255) / 256, 1024)), dim3(256), 0, st, sl.u, P, a.counters);
+    run_passes<W, ABS, false>(v, a, pg);
+    launch_counts(ta, a.counters, st);
     SG_HIP(hipGetLastError());
     SG_HIP(hipStreamSynchronize(st));
 }
@@ -1989,11 +2026,6 @@ int sg_autotune(sg_sim* s, int ell, uint64_t first, uint64_t sample, int precisi
     SG_TRY
     ensure_init();
     SG_REQUIRE(s != nullptr && sample > 0, "autotune needs a simulation and a positive sample");
-    if (s->dust && s->dust->ncomp > 1) {
-        // several dust components always run in the lane pipeline: tune that
-        choose_pipeline = 0;
-        g_pipeline = 0;
-    }
     std::vector<std::pair<DevBuf*, void*>> keep;
     auto save = [&](void* p, size_t bytes) {
         auto* c = new DevBuf();
@@ -2255,8 +2287,7 @@ int sg_sim_run_batch(int nmembers, sg_sim* const* sims, const int* ells, const u
     for (int i = 0; g_pipeline == 1 && g_batch_alone > 0 && i < nmembers; i++) {
         if (done[i] == counts[i]) continue;
         if (counts[i] < g_batch_alone) continue;
-        if (base[i].store_abs) dispatch_split<true>(sims[i], base[i], precision, 0, counts[i], lt, blocks);
-        else dispatch_split<false>(sims[i], base[i], precision, 0, counts[i], lt, blocks);
+        dispatch_split_any(sims[i], base[i], precision, 0, counts[i], lt, blocks);
         done[i] = counts[i];
     }
     int j = 0;

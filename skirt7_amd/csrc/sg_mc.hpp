@@ -655,7 +655,7 @@ __device__ __forceinline__ bool crossing(Hot<W>& h, const typename W::View& g, c
                 R Lintm = h.L0 * rexp<R>(-h.tau) * expfactorm;
                 R alb = (R)a.albm[cell];
                 h.lsca += alb * Lintm;
-                if (ABS) unsafeAtomicAdd(a.labs + (size_t)a.ell * a.ncells + cell, (double)(((R)1.0 - alb) * Lintm));
+                if (ABS && leads<W>()) unsafeAtomicAdd(a.labs + (size_t)a.ell * a.ncells + cell, (double)(((R)1.0 - alb) * Lintm));
             }
             h.mcell = (int)cell;
         }
@@ -704,12 +704,18 @@ __device__ __forceinline__ bool finished_stage(int st)
     return ((1u << ST_PEELW_DONE | 1u << ST_OWN_DONE | 1u << ST_PROP_DONE | 1u << ST_LOC_DONE) >> (uint32_t)st) & 1u;
 }
 
-__device__ __forceinline__ void add_wave(unsigned long long* dst, unsigned long long x)
+// The sum over the wave's lanes, in lane 0.
+__device__ __forceinline__ unsigned long long wave_sum(unsigned long long x)
 {
     for (int off = 32; off > 0; off >>= 1) {
         uint32_t lo = __shfl_down((uint32_t)x, off), hi = __shfl_down((uint32_t)(x >> 32), off);
         x += ((unsigned long long)hi << 32) | lo;
     }
+    return x;
+}
+__device__ __forceinline__ void add_wave(unsigned long long* dst, unsigned long long x)
+{
+    x = wave_sum(x);
     if (__lane_id() == 0 && x) atomicAdd(dst, x);
 }
 
@@ -739,11 +745,12 @@ template <> struct McWaves<TreeW32> { static constexpr int value = SG_MC_TREE32_
 
 // The lane pipeline of one wave over the packet range of `a`: lanes claim packets until the range
 // is exhausted and every packet the wave claimed has finished; then the wave's event counts go
-// to a.counters.
+// to counters (the workgroup's in LDS, or a.counters).
 template <class W, bool ABS, bool MULTI = false>
 __device__ __forceinline__ void drain(const typename W::View& g, const McArgs& a, uint32_t* park,
                                       const int32_t* s_nodes, int nlds, const ColdSlot<typename W::Real>& c,
-                                      const InstrDev* s_instr, const typename W::View* gdev, const McArgs* adev)
+                                      const InstrDev* s_instr, const typename W::View* gdev, const McArgs* adev,
+                                      unsigned long long* counters)
 {
     const int nl = blockDim.x, lane = threadIdx.x;
     (void)park; (void)nl; (void)lane; (void)gdev; (void)adev;
@@ -778,15 +785,15 @@ __device__ __forceinline__ void drain(const typename W::View& g, const McArgs& a
             if (__popcll(alive & ~wm) >= need_n || !wm) break;
         }
     }
-    add_wave(a.counters + 1, n_own);
-    add_wave(a.counters + 2, n_peel);
-    add_wave(a.counters + 8, n_re);
-    add_wave(a.counters + 0, c.fu(CU_PK));
-    add_wave(a.counters + 3, c.fu(CU_SCAT));
-    add_wave(a.counters + 4, c.fu(CU_NPEEL));
-    add_wave(a.counters + 5, h.w.nstuck);
-    add_wave(a.counters + 7, c.fu(CU_WALKS));
-    add_wave(a.counters + 9, h.w.nrecompute);
+    add_wave(counters + 1, n_own);
+    add_wave(counters + 2, n_peel);
+    add_wave(counters + 8, n_re);
+    add_wave(counters + 0, c.fu(CU_PK));
+    add_wave(counters + 3, c.fu(CU_SCAT));
+    add_wave(counters + 4, c.fu(CU_NPEEL));
+    add_wave(counters + 5, h.w.nstuck);
+    add_wave(counters + 7, c.fu(CU_WALKS));
+    add_wave(counters + 9, h.w.nrecompute);
 }
 
 // Persistent transport kernel. Dynamic LDS: the hot-state parking area (hot_words<W>() per lane),
@@ -807,8 +814,14 @@ k_mc(const typename W::View g, const McArgs a, int nlds_req, typename W::Real* c
     ColdSlot<typename W::Real> c;
     c.r = cold_r; c.u = cold_u; c.nl = nslots;
     c.lane = blockIdx.x * blockDim.x + threadIdx.x;
+    // the workgroup's counts: one addition per workgroup to the run's counters (their cache line takes about 10 ns
+    // each, so nine per wave would cost a short launch 180 us)
+    __shared__ unsigned long long s_counters[10];
+    if (threadIdx.x < 10) s_counters[threadIdx.x] = 0;
     __syncthreads();
-    drain<W, ABS, MULTI>(g, a, park, s_nodes, nlds, c, s_instr, gdev, adev);
+    drain<W, ABS, MULTI>(g, a, park, s_nodes, nlds, c, s_instr, gdev, adev, s_counters);
+    __syncthreads();
+    if (threadIdx.x < 10 && s_counters[threadIdx.x]) atomicAdd(a.counters + threadIdx.x, s_counters[threadIdx.x]);
 }
 
 // Batched transport over many packet ranges, each with its own grid view and run arguments (one
@@ -851,7 +864,7 @@ k_mc_batch(const typename W::View* gtab, const McArgs* atab, int nranges, typena
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        drain<W, ABS>(gtab[r], *ap, park, my_nodes, nlds, c, my_instr, gtab + r, ap);
+        drain<W, ABS>(gtab[r], *ap, park, my_nodes, nlds, c, my_instr, gtab + r, ap, ap->counters);
         scanned = 0;
     }
 }

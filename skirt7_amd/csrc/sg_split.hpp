@@ -21,12 +21,11 @@
 namespace sg {
 
 enum SlotR { SR_RX = 0, SR_RY, SR_RZ, SR_KX, SR_KY, SR_KZ, SR_L, SR_RES, SR_NR };
-// The last four slot words count the slot's packets, scatterings, detected peel-offs and started
-// walks over a run; they are summed once at the end (no per-pass atomics).
+// SU_MCELL: several dust components: the cell of the interaction point (-1: none).
 // SU_HINT: the leaf (tree node, or Voronoi cell) the packet's position lies in, as the last
 // propagation walk left it (-1: unknown), handed to the walks that start there.
 enum SlotU { SU_PLO = 0, SU_PHI, SU_DRAW, SU_W0, SU_W1, SU_W2, SU_W3, SU_NSCATT, SU_HINT,
-             SU_STATE, SU_CPK, SU_CSCAT, SU_CPEEL, SU_CWALK, SU_NU };
+             SU_MCELL, SU_STATE, SU_NU };
 // PS_OWN: the packet's own path is in the walk queue; the walk kernel leaves it at its interaction point
 // (PS_PROP) or finished (PS_FRESH: the slot takes a new packet).
 enum PacketState : uint32_t { PS_FRESH = 0, PS_OWN, PS_PROP, PS_DEAD };
@@ -46,12 +45,10 @@ template <typename R> __host__ __device__ constexpr size_t slot_bytes(int64_t n)
 }
 
 // Walk requests: origin (3), direction (3, unused for peel-offs: the instrument's direction is
-// taken from its record) and a value (peel-off or own-path luminosity) in the run's real type; a tag (kind | instrument << 2), an index (packet
-// slot, or pixel for a peel-off) and the start leaf hint of the walker. In the LDS staging area
-// they are structure-of-arrays (QR_*, QU_* fields); in the queues one record per request, so that
-// a request moved to its sorted place, or read by a lane, is one contiguous block.
-enum QueueR { QR_OX = 0, QR_OY, QR_OZ, QR_DX, QR_DY, QR_DZ, QR_VAL, QR_NR };
-enum QueueU { QU_TAG = 0, QU_IDX, QU_HINT, QU_NU };
+// taken from its record) and a value (peel-off or own-path luminosity) in the run's real type; a tag
+// (kind | instrument << 2), an index (packet slot, or pixel for a peel-off) and the start cell hint of the
+// walker. One record per request, so that a request moved to its sorted place, or read by a lane, is one
+// contiguous block.
 template <typename R> struct alignas(16) WalkReq {
     R o[3], d[3], val;
     uint32_t tag, idx, hint;
@@ -65,12 +62,26 @@ struct PassCtl {
     unsigned long long tail;            // requests appended by the event kernel
     unsigned long long claim;           // requests taken by the walk kernel
     unsigned long long seg[kXcdSegs];   // the same per XCD segment
-    unsigned long long t0inv, t1;       // walk kernel: complement of its first wave's start, last wave's end (clock ticks)
+    unsigned long long t0;              // walk kernel: its start (clock ticks; 0: it had no requests)
 };
 constexpr int kPassRing = 4;
 struct GroupCtl {
     PassCtl pass[kPassRing];
     unsigned long long ticks;           // walk kernels' durations, summed over the finished passes
+};
+// What each wave of the walk kernel keeps from pass to pass in a record of its own: the end of its last pass
+// (clock ticks) and its counts. (Added up with atomics at the end of every pass, on one cache line at about 10 ns
+// each, they took 100 us of it.)
+struct WaveRec {
+    unsigned long long t1, own, peel, re, stuck, recompute;
+};
+// A group's count records, added up at the end of a run.
+struct GroupTally {
+    WaveRec* waves;                     // per wave of the walk kernel
+    int nwaves;
+    unsigned long long* events;         // per workgroup of the event kernel: packets, scatterings, peel-offs, walks
+    int64_t nevents;
+    int64_t slot0;                      // the group's first slot among all groups' (its first packet in a batch)
 };
 
 // Walk order. The walks of a pass are sorted by a coherence key before the walk kernel takes them:
@@ -139,120 +150,36 @@ __device__ __forceinline__ uint32_t walk_key(const McArgs& a, const InstrDev* in
     return (8u << 12) | spread3(qx) | (spread3(qy) << 1) | (spread3(qz) << 2);
 }
 
-// Appends one request per active lane (one atomic per wave); returns this lane's queue position.
-__device__ __forceinline__ uint64_t wave_append(unsigned long long* tail)
-{
-    uint64_t mask = __ballot(1);
-    int lane = __lane_id();
-    int leader = __ffsll((unsigned long long)mask) - 1;
-    unsigned long long base = 0;
-    if (lane == leader) base = atomicAdd(tail, (unsigned long long)__popcll(mask));
-    uint32_t lo = __shfl((uint32_t)base, leader), hi = __shfl((uint32_t)(base >> 32), leader);
-    base = ((uint64_t)hi << 32) | lo;
-    uint64_t below = lane ? (mask & ((~0ull) >> (64 - lane))) : 0ull;
-    return base + (uint64_t)__popcll(below);
-}
-
-// Walk requests of one workgroup staged in LDS (structure of arrays) in two parts: peel-offs (origin,
-// value, tag, index, hint: a peel-off walks toward its instrument, so it carries no direction) in capp
-// entries, and the own paths (with their direction) in capw entries, each part with
-// its own count. A lane stages at most ni peel-offs and one own path per pass, so capp = ni and capw = 1
-// entries per lane suffice, 28 + 40 / ni bytes per request slot in FP32 instead of 40, which leaves room
-// for more workgroups per CU. The workgroup appends them to the walk queue as one block with a single
-// global atomic.
-enum StagedPeelR { QP_OX = 0, QP_OY, QP_OZ, QP_VAL, QP_NR };
-template <typename R> struct StagedQueue {
-    R* pr;                      // peel-offs: QP_NR reals and QU_NU words per entry
-    uint32_t* pu;
-    int capp;
-    unsigned* cntp;
-    R* wr;                      // other walks: QR_NR reals and QU_NU words per entry
-    uint32_t* wu;
-    int capw;
-    unsigned* cntw;
-    __device__ __forceinline__ void push(uint32_t kind, uint32_t inst, uint32_t idx, R ox, R oy, R oz, R dx, R dy,
-                                         R dz, R val, int32_t hint) const
-    {
-        const bool peel = kind == WK_PEEL;   // the same for every lane of a call
-        uint64_t mask = __ballot(1);
-        int lane = __lane_id();
-        int leader = __ffsll((unsigned long long)mask) - 1;
-        unsigned base = 0;
-        if (lane == leader) base = atomicAdd(peel ? cntp : cntw, (unsigned)__popcll(mask));
-        base = __shfl(base, leader);
-        uint64_t below = lane ? (mask & ((~0ull) >> (64 - lane))) : 0ull;
-        const int i = (int)(base + (unsigned)__popcll(below));
-        if (peel) {
-            pr[QP_OX * capp + i] = ox; pr[QP_OY * capp + i] = oy; pr[QP_OZ * capp + i] = oz;
-            pr[QP_VAL * capp + i] = val;
-            pu[QU_TAG * capp + i] = kind | (inst << 2);
-            pu[QU_IDX * capp + i] = idx;
-            pu[QU_HINT * capp + i] = (uint32_t)hint;
-        } else {
-            wr[QR_OX * capw + i] = ox; wr[QR_OY * capw + i] = oy; wr[QR_OZ * capw + i] = oz;
-            wr[QR_DX * capw + i] = dx; wr[QR_DY * capw + i] = dy; wr[QR_DZ * capw + i] = dz;
-            wr[QR_VAL * capw + i] = val;
-            wu[QU_TAG * capw + i] = kind | (inst << 2);
-            wu[QU_IDX * capw + i] = idx;
-            wu[QU_HINT * capw + i] = (uint32_t)hint;
-        }
-    }
-    // Request j of the workgroup's block: the peel-offs first, then the other walks.
-    __device__ __forceinline__ WalkReq<R> get(unsigned j, unsigned np) const
-    {
-        WalkReq<R> w;
-        if (j < np) {
-            w.o[0] = pr[QP_OX * capp + j]; w.o[1] = pr[QP_OY * capp + j]; w.o[2] = pr[QP_OZ * capp + j];
-            w.d[0] = (R)0; w.d[1] = (R)0; w.d[2] = (R)0;
-            w.val = pr[QP_VAL * capp + j];
-            w.tag = pu[QU_TAG * capp + j]; w.idx = pu[QU_IDX * capp + j]; w.hint = pu[QU_HINT * capp + j];
-        } else {
-            const unsigned k = j - np;
-            w.o[0] = wr[QR_OX * capw + k]; w.o[1] = wr[QR_OY * capw + k]; w.o[2] = wr[QR_OZ * capw + k];
-            w.d[0] = wr[QR_DX * capw + k]; w.d[1] = wr[QR_DY * capw + k]; w.d[2] = wr[QR_DZ * capw + k];
-            w.val = wr[QR_VAL * capw + k];
-            w.tag = wu[QU_TAG * capw + k]; w.idx = wu[QU_IDX * capw + k]; w.hint = wu[QU_HINT * capw + k];
-        }
-        return w;
-    }
+// An instrument as the event kernel uses it, in the run's real type: pixel_on_detector's products of two angle
+// functions taken once.
+template <typename R> struct EventInstr {
+    R sinphi, cosphi, c1, c2, sintheta, cospa, sinpa, xpmin, xpsiz, ypmin, ypsiz, k[3];
+    int Nx, Ny;
+    double* frame;
 };
-// LDS of a workgroup's staging area for block lanes and ni instruments (the peel-off part first; its
-// size is a multiple of 8 bytes, so that the FP64 reals of the other part stay aligned)
-template <typename R> __host__ __device__ constexpr size_t staged_peel_bytes(int block, int ni)
+template <typename R> __device__ __forceinline__ EventInstr<R> event_instr(const InstrDev& in)
 {
-    return (((size_t)block * ni * (QP_NR * sizeof(R) + QU_NU * sizeof(uint32_t))) + 7) / 8 * 8;
+    EventInstr<R> e;
+    e.sinphi = (R)in.sinphi; e.cosphi = (R)in.cosphi;
+    e.c1 = -(R)in.cosphi * (R)in.costheta; e.c2 = (R)in.sinphi * (R)in.costheta; e.sintheta = (R)in.sintheta;
+    e.cospa = (R)in.cospa; e.sinpa = (R)in.sinpa;
+    e.xpmin = (R)in.xpmin; e.xpsiz = (R)in.xpsiz; e.ypmin = (R)in.ypmin; e.ypsiz = (R)in.ypsiz;
+    for (int a = 0; a < 3; a++) e.k[a] = (R)in.kobs[a];
+    e.Nx = in.Nx; e.Ny = in.Ny; e.frame = in.frame;
+    return e;
 }
-template <typename R> __host__ __device__ constexpr size_t staged_bytes(int block, int ni)
+// SingleFrameInstrument::pixelondetector (SingleFrameInstrument.cpp:130-147), operation for operation as
+// pixel_on_detector
+template <typename R> __device__ __forceinline__ int event_pixel(const EventInstr<R>& in, R x, R y, R z)
 {
-    return staged_peel_bytes<R>(block, ni) + (size_t)block * (QR_NR * sizeof(R) + QU_NU * sizeof(uint32_t));
-}
-
-// Peel-offs toward every instrument (MonteCarloSimulation::peeloffemission/peeloffscattering,
-// MonteCarloSimulation.cpp:299-357): pixel, phase-function weight (scattering only), and either the
-// walk request or, without a dust system, the detection itself.
-template <typename R, class Q>
-__device__ __forceinline__ uint32_t peel_offs(const McArgs& a, const InstrDev* instr, const Q& q,
-                                              bool scattering, R rx, R ry, R rz, R kx, R ky, R kz, R L,
-                                              int32_t hint)
-{
-    const R gg = (R)a.g;
-    uint32_t n = 0;
-    for (int i = 0; i < a.ni; i++) {
-        const InstrDev& in = instr[i];
-        int pix = pixel_on_detector<R>(in, rx, ry, rz);
-        if (pix < 0) continue;
-        R Lp = L;
-        if (scattering) {
-            // DustMix::phaseFunctionValue, Henyey-Greenstein (DustMix.cpp:648-653)
-            R cosalpha = kx * (R)in.kobs[0] + ky * (R)in.kobs[1] + kz * (R)in.kobs[2];
-            R t = (R)1.0 + gg * gg - (R)2 * gg * cosalpha;
-            Lp = L * (((R)1.0 - gg) * ((R)1.0 + gg) / sqrt(t * t * t));
-        }
-        n++;
-        if (!a.has_dust) unsafeAtomicAdd(in.frame + (size_t)a.ell * in.Nx * in.Ny + pix, (double)Lp);
-        else q.push(WK_PEEL, (uint32_t)i, (uint32_t)pix, rx, ry, rz, (R)0, (R)0, (R)0, Lp, hint);
-    }
-    return n;
+    const R xpp = -in.sinphi * x + in.cosphi * y;
+    const R ypp = in.c1 * x - in.c2 * y + in.sintheta * z;
+    const R xp = in.cospa * xpp - in.sinpa * ypp;
+    const R yp = in.sinpa * xpp + in.cospa * ypp;
+    const R fi = floor((xp - in.xpmin) / in.xpsiz);
+    const R fj = floor((yp - in.ypmin) / in.ypsiz);
+    if (!(fi >= (R)0 && fi < (R)in.Nx && fj >= (R)0 && fj < (R)in.Ny)) return -1;
+    return (int)fi + in.Nx * (int)fj;
 }
 
 // Henyey-Greenstein scattering direction (DustMix.cpp:596-601) and Random::direction(k, cos)
@@ -283,121 +210,215 @@ __device__ __forceinline__ void hg_scatter(PacketRng& rng, R gg, R& kx, R& ky, R
     kx = nkx; ky = nky; kz = nkz;
 }
 
-// Event pass: every slot advances its packet to its next own path (or takes a new packet). Dynamic LDS:
-// the workgroup's staged requests, blockDim.x * a.ni peel-offs and blockDim.x own paths (the most one
-// pass can append: a lane's pass ends with the own path it requests, after at most one set of peel-offs).
-// gc/pass: the group's progress ring; this pass's record is q.tail's.
+// A launched packet's state and random stream, which continues where the emission left it; false when every
+// packet has been claimed (*p then not set), or for a packet without luminosity.
 template <typename R>
-__global__ void __launch_bounds__(256) k_events(const McArgs a, Slots<R> sl, WalkQueue<R> q, GroupCtl* gc, int pass)
+__device__ __forceinline__ bool take_packet(const McArgs& a, uint64_t p, PacketRng& rng, R& rx, R& ry, R& rz, R& kx, R& ky,
+                                            R& kz, R& L, int32_t& hint)
 {
-    __shared__ InstrDev s_instr[SG_MAX_INSTR];
-    __shared__ unsigned s_cntp, s_cntw;
+    const R* e = reinterpret_cast<const R*>(a.emitted);
+    const size_t n = a.count;
+    L = e[6 * n + p];
+    if (!(L > (R)0)) return false;
+    rx = e[p]; ry = e[n + p]; rz = e[2 * n + p];
+    kx = e[3 * n + p]; ky = e[4 * n + p]; kz = e[5 * n + p];
+    rng.start(a.seed, a.member, a.first + p, a.ell);
+    rng.draw = a.emit_draw[p];
+    if (rng.draw & 3u) {
+        rng.w0 = rng.plo; rng.w1 = rng.phi; rng.w2 = rng.draw >> 2; rng.w3 = rng.ell;
+        philox10(rng.w0, rng.w1, rng.w2, rng.w3, rng.k0, rng.k1);
+    }
+    hint = a.emit_hint ? a.emit_hint[p] : -1;
+    return true;
+}
+
+// Event pass: every slot advances its packet to its next own path (or takes a new packet): peel-offs toward every
+// instrument (MonteCarloSimulation::peeloffemission/peeloffscattering, MonteCarloSimulation.cpp:299-357), the
+// scattered direction, and the requests for their walks. The requests are counted first (one ballot per kind and
+// wave), the workgroup takes its part of the queue with one atomic, and each lane writes its own requests, so
+// that only the counts pass through LDS: staged whole there (51 KB a workgroup in FP64) they left three workgroups
+// on a CU. Within the workgroup's part the requests lie instrument by instrument, own paths last: neighbours in
+// the queue walk in the same direction. gc/pass: the group's progress ring; this pass's record is q.tail's.
+// The device adds to one address about once in 10 ns, so atomics are few: one per workgroup for its part of the
+// queue, and one per wave that needs packets while there are unclaimed ones, none in a batch's first pass (`first`:
+// every slot is free and takes the packet of its own number, slot0 + i).
+constexpr int kEventBlock = 512;
+template <typename R, bool MULTI>
+__global__ void __launch_bounds__(kEventBlock) k_events(const McArgs a, Slots<R> sl, WalkQueue<R> q, GroupCtl* gc, int pass,
+                                                        int first, const GroupTally ta)
+{
+    constexpr int kKinds = SG_MAX_INSTR + 1, nw = kEventBlock / 64;
+    __shared__ EventInstr<R> s_instr[SG_MAX_INSTR];
+    __shared__ uint32_t s_n[kKinds * nw];                 // requests per kind and wave, then their places in the part
+    __shared__ uint32_t s_stat[4 * nw];
     __shared__ unsigned long long s_base;
-    extern __shared__ __align__(16) unsigned char smem[];
-    const int capp = (int)blockDim.x * a.ni, capw = (int)blockDim.x;
-    unsigned char* wbase = smem + staged_peel_bytes<R>((int)blockDim.x, a.ni);
-    StagedQueue<R> sq{reinterpret_cast<R*>(smem), reinterpret_cast<uint32_t*>(smem + (size_t)capp * QP_NR * sizeof(R)),
-                      capp, &s_cntp, reinterpret_cast<R*>(wbase),
-                      reinterpret_cast<uint32_t*>(wbase + (size_t)capw * QR_NR * sizeof(R)), capw, &s_cntw};
-    if (threadIdx.x < SG_MAX_INSTR) s_instr[threadIdx.x] = a.scene->instr[threadIdx.x];
-    if (threadIdx.x == 0) { s_cntp = 0; s_cntw = 0; }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        // the previous pass's walk kernel has ended: its duration; the next pass's record, last used three
-        // passes ago, is cleared
+    const int wave = (int)threadIdx.x >> 6, lane = __lane_id();
+    if ((int)threadIdx.x < a.ni) s_instr[threadIdx.x] = event_instr<R>(a.scene->instr[threadIdx.x]);
+    if (blockIdx.x == gridDim.x - 1) {
+        // a workgroup of its own for the bookkeeping. The previous pass's walk kernel has ended: its duration, from
+        // its start to its last wave's end; the next pass's record, last used three passes ago, is cleared
         const PassCtl& pv = gc->pass[(pass + kPassRing - 1) % kPassRing];
-        if (pv.t1 > ~pv.t0inv) gc->ticks += pv.t1 - ~pv.t0inv;
-        PassCtl& nx = gc->pass[(pass + 1) % kPassRing];
-        nx.tail = 0; nx.claim = 0; nx.t0inv = 0; nx.t1 = 0;
-        for (int k = 0; k < kXcdSegs; k++) nx.seg[k] = 0;
+        if (threadIdx.x == 0) {
+            s_base = 0;
+            PassCtl& nx = gc->pass[(pass + 1) % kPassRing];
+            nx.tail = 0; nx.claim = 0; nx.t0 = 0;
+            for (int k = 0; k < kXcdSegs; k++) nx.seg[k] = 0;
+        }
+        __syncthreads();
+        unsigned long long t1 = 0;
+        for (int w = (int)threadIdx.x; w < ta.nwaves; w += kEventBlock) t1 = max(t1, ta.waves[w].t1);
+        atomicMax(&s_base, t1);
+        __syncthreads();
+        if (threadIdx.x == 0 && pv.t0 && s_base > pv.t0) gc->ticks += s_base - pv.t0;
+        return;
     }
     __syncthreads();
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    // every lane stays to the end: the counts below are summed over the whole wave
-    uint32_t state = i < sl.n ? sl.fu(SU_STATE, i) : (uint32_t)PS_DEAD;
-    uint32_t c_pk = 0, c_scat = 0, c_npeel = 0, c_walks = 0;
-    if (state != PS_DEAD) {
-        const R gg = (R)a.g;
-        R rx = sl.fr(SR_RX, i), ry = sl.fr(SR_RY, i), rz = sl.fr(SR_RZ, i);
-        R kx = sl.fr(SR_KX, i), ky = sl.fr(SR_KY, i), kz = sl.fr(SR_KZ, i);
-        R L = sl.fr(SR_L, i);
-        PacketRng rng;
-        rng.k0 = a.seed; rng.k1 = a.member; rng.ell = (uint32_t)a.ell;
+    const uint32_t state0 = i < sl.n ? sl.fu(SU_STATE, i) : (uint32_t)PS_DEAD;
+    uint32_t state = state0;
+    R rx = 0, ry = 0, rz = 0, kx = 0, ky = 0, kz = 0, L = 0;
+    int32_t hint = -1;
+    PacketRng rng;
+    rng.k0 = a.seed; rng.k1 = a.member; rng.ell = (uint32_t)a.ell;
+    rng.plo = 0; rng.phi = 0; rng.draw = 0; rng.w0 = 0; rng.w1 = 0; rng.w2 = 0; rng.w3 = 0;
+    uint32_t c_pk = 0, c_peel = 0;   // wave totals
+    bool acts = false;               // the lane makes peel-offs and requests an own path
+    const bool scatters = state0 == PS_PROP;
+    int mcell = -1;
+    if (scatters) {
+        // PhotonPackage::propagate (PhotonPackage.cpp:93-96) by pathlength(tau)
+        const R d = sl.fr(SR_RES, i);
+        kx = sl.fr(SR_KX, i); ky = sl.fr(SR_KY, i); kz = sl.fr(SR_KZ, i);
+        rx = sl.fr(SR_RX, i) + d * kx; ry = sl.fr(SR_RY, i) + d * ky; rz = sl.fr(SR_RZ, i) + d * kz;
+        L = sl.fr(SR_L, i);
         rng.plo = sl.fu(SU_PLO, i); rng.phi = sl.fu(SU_PHI, i); rng.draw = sl.fu(SU_DRAW, i);
         rng.w0 = sl.fu(SU_W0, i); rng.w1 = sl.fu(SU_W1, i); rng.w2 = sl.fu(SU_W2, i); rng.w3 = sl.fu(SU_W3, i);
-        int nscatt = (int)sl.fu(SU_NSCATT, i);
-        int32_t hint = (int32_t)sl.fu(SU_HINT, i);
-        // at most a few transitions per pass: a finished packet is replaced by a new one at once; a slot
-        // without a dust system detects its peel-offs directly and takes up to four packets per pass
-        for (int step = 0; step < 4; step++) {
-            if (state == PS_FRESH) {
-                uint64_t p;
-                if (!wave_claim(a.next_packet, a.count, p)) { state = PS_DEAD; break; }
-                // launch state from the emission kernel; continue the packet's random stream
-                const R* e = reinterpret_cast<const R*>(a.emitted);
-                const size_t n = a.count;
-                c_pk++;
-                R Le = e[6 * n + p];
-                if (!(Le > (R)0)) continue;
-                rx = e[p]; ry = e[n + p]; rz = e[2 * n + p];
-                kx = e[3 * n + p]; ky = e[4 * n + p]; kz = e[5 * n + p];
-                L = Le;
-                rng.start(a.seed, a.member, a.first + p, a.ell);
-                rng.draw = a.emit_draw[p];
-                if (rng.draw & 3u) {
-                    rng.w0 = rng.plo; rng.w1 = rng.phi; rng.w2 = rng.draw >> 2; rng.w3 = rng.ell;
-                    philox10(rng.w0, rng.w1, rng.w2, rng.w3, rng.k0, rng.k1);
-                }
-                nscatt = 0;
-                hint = a.emit_hint ? a.emit_hint[p] : -1;
-                uint32_t np = peel_offs<R>(a, s_instr, sq, false, rx, ry, rz, kx, ky, kz, L, hint);
-                c_npeel += np;
-                if (!a.has_dust) continue;
-                c_walks += np + 1;
-                sq.push(WK_OWN, 0, (uint32_t)i, rx, ry, rz, kx, ky, kz, L, hint);
-                state = PS_OWN;
-                break;
-            }
-            if (state == PS_PROP) {
-                // PhotonPackage::propagate (PhotonPackage.cpp:93-96) by pathlength(tau)
-                R d = sl.fr(SR_RES, i);
-                rx = rx + d * kx; ry = ry + d * ky; rz = rz + d * kz;
-                uint32_t np = peel_offs<R>(a, s_instr, sq, true, rx, ry, rz, kx, ky, kz, L, hint);
-                c_npeel += np;
-                hg_scatter<R>(rng, gg, kx, ky, kz);
-                nscatt++;
-                c_scat++;
-                c_walks += np + 1;
-                sq.push(WK_OWN, 0, (uint32_t)i, rx, ry, rz, kx, ky, kz, L, hint);
-                state = PS_OWN;
-            }
-            break;   // PS_OWN here: a request that was refused; the slot stays idle
+        hint = (int32_t)sl.fu(SU_HINT, i);
+        if (MULTI) mcell = (int)sl.fu(SU_MCELL, i);
+        acts = true;
+    }
+    // without a dust system the peel-offs are detected here, and a slot takes up to four packets per pass
+    for (int turn = 0; turn < (a.has_dust ? 1 : 4); turn++) {
+        uint64_t p = 0;
+        bool got = false;
+        if (state == PS_FRESH) {
+            if (first && turn == 0) {
+                p = (uint64_t)(ta.slot0 + i);
+                got = p < a.count;
+            } else if (__hip_atomic_load(a.next_packet, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < a.count)
+                got = wave_claim(a.next_packet, a.count, p);
+            if (!got) state = PS_DEAD;
         }
+        c_pk += (uint32_t)__popcll(__ballot(got));
+        const bool lit = got && take_packet<R>(a, p, rng, rx, ry, rz, kx, ky, kz, L, hint);
+        if (a.has_dust) {
+            acts = acts | lit;
+            break;
+        }
+        for (int k = 0; k < a.ni; k++) {
+            const int pix = lit ? event_pixel<R>(s_instr[k], rx, ry, rz) : -1;
+            if (pix >= 0) unsafeAtomicAdd(s_instr[k].frame + (size_t)a.ell * s_instr[k].Nx * s_instr[k].Ny + pix, (double)L);
+            c_peel += (uint32_t)__popcll(__ballot(pix >= 0));
+        }
+    }
+    // peel-off pixels and luminosities (the phase-function weight of a scattering)
+    int pix[SG_MAX_INSTR];
+    R Lp[SG_MAX_INSTR];
+    const R gg = (R)a.g;
+    // peeloffscattering aborts when the scattering point has no scattering dust (MonteCarloSimulation.cpp:321-327)
+    const bool peels = acts && !(MULTI && scatters && !peel_weights_ok<R>(a, mcell));
+#pragma unroll
+    for (int k = 0; k < SG_MAX_INSTR; k++) {
+        pix[k] = -1;
+        Lp[k] = L;
+        if (k >= a.ni) continue;   // the same for every lane
+        if (peels) {
+            const EventInstr<R>& in = s_instr[k];
+            pix[k] = event_pixel<R>(in, rx, ry, rz);
+            if (scatters) {
+                // DustMix::phaseFunctionValue, Henyey-Greenstein (DustMix.cpp:648-653)
+                const R cosalpha = kx * in.k[0] + ky * in.k[1] + kz * in.k[2];
+                if (MULTI) Lp[k] = L * mixed_phase<R>(a, mcell, cosalpha);
+                else {
+                    const R t = (R)1.0 + gg * gg - (R)2 * gg * cosalpha;
+                    Lp[k] = L * (((R)1.0 - gg) * ((R)1.0 + gg) / sqrt(t * t * t));
+                }
+            }
+        }
+        const uint32_t n = (uint32_t)__popcll(__ballot(pix[k] >= 0));
+        c_peel += n;
+        if (lane == 0) s_n[k * nw + wave] = n;
+    }
+    const uint64_t own = __ballot(acts), scattered = __ballot(scatters);
+    if (lane == 0) {
+        s_n[a.ni * nw + wave] = (uint32_t)__popcll(own);
+        s_stat[wave] = c_pk;
+        s_stat[nw + wave] = (uint32_t)__popcll(scattered);
+        s_stat[2 * nw + wave] = c_peel;
+        s_stat[3 * nw + wave] = a.has_dust ? c_peel + (uint32_t)__popcll(own) : 0u;
+    }
+    __syncthreads();
+    // places of the (kind, wave) runs in the workgroup's part of the queue, kind by kind
+    const int runs = (a.ni + 1) * nw;
+    static_assert(kKinds * nw <= 128, "two runs per lane");
+    if (wave == 0) {
+        const bool dust = a.has_dust != 0;
+        const uint32_t n0 = dust && 2 * lane < runs ? s_n[2 * lane] : 0u;
+        const uint32_t n1 = dust && 2 * lane + 1 < runs ? s_n[2 * lane + 1] : 0u;
+        uint32_t x = n0 + n1;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(x, o);
+            if (lane >= o) x += y;
+        }
+        if (2 * lane < runs) s_n[2 * lane] = x - n0 - n1;
+        if (2 * lane + 1 < runs) s_n[2 * lane + 1] = x - n1;
+        if (lane == 63) s_base = x ? atomicAdd(q.tail, (unsigned long long)x) : 0ull;
+    }
+    if (threadIdx.x >= 64 && threadIdx.x < 68) {
+        const int k = (int)threadIdx.x & 3;
+        unsigned long long t = 0;
+        for (int w = 0; w < nw; w++) t += s_stat[k * nw + w];
+        if (t) ta.events[4 * (size_t)blockIdx.x + k] += t;
+    }
+    // the scattered direction meanwhile (several components: the mix drawn first, DustSystem.cpp:855-869)
+    R nx = kx, ny = ky, nz = kz;
+    int nscatt = 0;
+    if (scatters) {
+        const R gs = MULTI ? (R)a.scene->gc[random_mix(a, mcell, rng)] : gg;
+        hg_scatter<R>(rng, gs, nx, ny, nz);
+        nscatt = (int)sl.fu(SU_NSCATT, i) + 1;
+    }
+    if (acts) {
+        state = PS_OWN;
         sl.fr(SR_RX, i) = rx; sl.fr(SR_RY, i) = ry; sl.fr(SR_RZ, i) = rz;
-        sl.fr(SR_KX, i) = kx; sl.fr(SR_KY, i) = ky; sl.fr(SR_KZ, i) = kz;
-        sl.fr(SR_L, i) = L;
+        sl.fr(SR_KX, i) = nx; sl.fr(SR_KY, i) = ny; sl.fr(SR_KZ, i) = nz;
         sl.fu(SU_PLO, i) = rng.plo; sl.fu(SU_PHI, i) = rng.phi; sl.fu(SU_DRAW, i) = rng.draw;
         sl.fu(SU_W0, i) = rng.w0; sl.fu(SU_W1, i) = rng.w1; sl.fu(SU_W2, i) = rng.w2; sl.fu(SU_W3, i) = rng.w3;
         sl.fu(SU_NSCATT, i) = (uint32_t)nscatt;
         sl.fu(SU_HINT, i) = (uint32_t)hint;
-        sl.fu(SU_CPK, i) += c_pk; sl.fu(SU_CSCAT, i) += c_scat; sl.fu(SU_CPEEL, i) += c_npeel;
-        sl.fu(SU_CWALK, i) += c_walks;
     }
-    if (i < sl.n) sl.fu(SU_STATE, i) = state;
-    // append the workgroup's requests to the walk queue
+    if (state != state0) sl.fu(SU_STATE, i) = state;
     __syncthreads();
-    const unsigned np = s_cntp, n = s_cntp + s_cntw;
-    if (threadIdx.x == 0) s_base = n ? atomicAdd(q.tail, (unsigned long long)n) : 0ull;
-    __syncthreads();
-    const uint64_t base = s_base;
-    for (unsigned j = threadIdx.x; j < n; j += blockDim.x) {
-        const WalkReq<R> w = sq.get(j, np);
-        q.req[base + j] = w;
+    const uint64_t below = lane ? (~0ull >> (64 - lane)) : 0ull;
+    auto put = [&](bool has, int k, const WalkReq<R>& w) {
+        const uint64_t mask = __ballot(has);
+        if (!has) return;
+        const uint64_t at = s_base + s_n[k * nw + wave] + (uint64_t)__popcll(mask & below);
+        q.req[at] = w;
         if (q.sorted) {
-            const uint32_t k = walk_key<R>(a, s_instr, w.tag, w.idx, w.o[0], w.o[1], w.o[2]);
-            q.key[base + j] = k;
-            q.rank[base + j] = atomicAdd(q.hist + k, 1u);
+            const uint32_t key = walk_key<R>(a, a.scene->instr, w.tag, w.idx, w.o[0], w.o[1], w.o[2]);
+            q.key[at] = key;
+            q.rank[at] = atomicAdd(q.hist + key, 1u);
         }
+    };
+#pragma unroll
+    for (int k = 0; k < SG_MAX_INSTR; k++) {
+        if (k >= a.ni) continue;
+        put(pix[k] >= 0, k, WalkReq<R>{{rx, ry, rz}, {(R)0, (R)0, (R)0}, Lp[k], (uint32_t)WK_PEEL | (uint32_t)k << 2,
+                                       (uint32_t)pix[k], (uint32_t)hint});
     }
+    put(acts, a.ni, WalkReq<R>{{rx, ry, rz}, {nx, ny, nz}, L, (uint32_t)WK_OWN, (uint32_t)i, (uint32_t)hint});
 }
 
 // Bin offsets of the walk order: exclusive prefix sum of the bin counts, which are cleared for the
@@ -455,32 +476,19 @@ __global__ void __launch_bounds__(256) k_key_scatter(WalkQueue<R> q, int* error)
     }
 }
 
-// End of a run: the slots' packet, scattering, peel-off and walk counts into the run counters.
-__global__ void __launch_bounds__(256) k_slot_counts(const uint32_t* u, int64_t n, unsigned long long* counters)
+// End of a run: the event workgroups' and the walk waves' counts into the run counters.
+__global__ void __launch_bounds__(256) k_run_counts(const GroupTally ta, unsigned long long* counters)
 {
-    __shared__ unsigned long long part[4][4];
-    unsigned long long v[4] = {0, 0, 0, 0};
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        v[0] += u[SU_CPK * n + i]; v[1] += u[SU_CSCAT * n + i]; v[2] += u[SU_CPEEL * n + i];
-        v[3] += u[SU_CWALK * n + i];
+    unsigned long long v[9] = {};
+    for (int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; b < ta.nevents; b += (int64_t)gridDim.x * blockDim.x)
+        for (int k = 0; k < 4; k++) v[k] += ta.events[4 * b + k];
+    for (int w = (int)(blockIdx.x * blockDim.x + threadIdx.x); w < ta.nwaves; w += (int)(gridDim.x * blockDim.x)) {
+        const WaveRec& r = ta.waves[w];
+        v[4] += r.own; v[5] += r.peel; v[6] += r.re; v[7] += r.stuck; v[8] += r.recompute;
     }
-    for (int k = 0; k < 4; k++)
-        for (int off = 32; off > 0; off >>= 1) {
-            uint32_t lo = __shfl_down((uint32_t)v[k], off), hi = __shfl_down((uint32_t)(v[k] >> 32), off);
-            v[k] += ((unsigned long long)hi << 32) | lo;
-        }
-    const int w = threadIdx.x >> 6;
-    if (__lane_id() == 0)
-        for (int k = 0; k < 4; k++) part[k][w] = v[k];
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const int dst[4] = {0, 3, 4, 7};
-        for (int k = 0; k < 4; k++) {
-            unsigned long long t = 0;
-            for (int j = 0; j < (int)(blockDim.x >> 6); j++) t += part[k][j];
-            if (t) atomicAdd(counters + dst[k], t);
-        }
-    }
+    const int dst[9] = {0, 3, 4, 7, 1, 2, 8, 5, 9};
+#pragma unroll
+    for (int k = 0; k < 9; k++) add_wave(counters + dst[k], v[k]);
 }
 
 // Request claims of one wave: chunks of requests by one global atomic each, handed out in order to the lanes
@@ -599,13 +607,13 @@ template <typename R> using VoroWalk = VoroC<R, SG_VORO_LANES, SG_VORO_EACH>;
 template <typename R> struct WalkWaves<VoroWalk<R>> { static constexpr int value = SG_VORO_WAVES; };
 
 // The end of an own path (lane's walk of slot idx, request w): DustSystem::fillOpticalDepth's check
-// (DustSystem.cpp:952-955), simulateescapeandabsorption (MonteCarloSimulation.cpp:432-461), the stop test
+// (DustSystem.cpp:952-955), simulateescapeandabsorption (MonteCarloSimulation.cpp:432-508), the stop test
 // and simulatepropagation (:513-531). Either the packet is finished or scatters where it is, which the slot's
 // state tells the next event pass, or the lane goes on with the walk to the interaction point (ST_PROP).
 // Done here rather than in the event kernel, the re-walk shares this pass with the long walks: as a pass of
 // its own it took a fifth of the walk time for 3% of the crossings, and each scattering took two event
 // passes.
-template <class W>
+template <class W, bool MULTI>
 __device__ __forceinline__ void own_path_end(Hot<W>& h, const typename W::View& g, const int32_t* lds, int nlds,
                                              const McArgs& a, const Slots<typename W::Real>& sl, uint32_t idx,
                                              const WalkReq<typename W::Real>* w)
@@ -618,8 +626,13 @@ __device__ __forceinline__ void own_path_end(Hot<W>& h, const typename W::View& 
         sl.fu(SU_STATE, idx) = PS_FRESH;
         return;
     }
-    const R expfactor = -rexpm1<R>(-taupath);
-    R L = h.L0 * (R)a.albedo * expfactor;
+    // one component, or the sum of each cell's albedo times its interacting luminosity, gathered along the walk
+    R L;
+    if (MULTI) L = h.lsca;
+    else {
+        const R expfactor = -rexpm1<R>(-taupath);
+        L = h.L0 * (R)a.albedo * expfactor;
+    }
     if (L <= (R)0 || (L <= (R)a.Lthreshold && (int)sl.fu(SU_NSCATT, idx) >= a.minfs)) {
         sl.fu(SU_STATE, idx) = PS_FRESH;
         return;
@@ -629,6 +642,7 @@ __device__ __forceinline__ void own_path_end(Hot<W>& h, const typename W::View& 
         // zero optical depth along the path: scattering in place
         sl.fr(SR_L, idx) = L;
         sl.fr(SR_RES, idx) = (R)0;
+        if (MULTI) sl.fu(SU_MCELL, idx) = (uint32_t)-1;
         return;
     }
     PacketRng rng;
@@ -660,7 +674,7 @@ __device__ __forceinline__ void own_path_end(Hot<W>& h, const typename W::View& 
 // A finished walk's result: a peel-off's detection (FrameInstrument::detect, FrameInstrument.cpp:33-47), an own
 // path's end, or the interaction point's distance and leaf for the packet slot. Afterwards the lane is idle, or
 // walks on to the interaction point.
-template <class W>
+template <class W, bool MULTI>
 __device__ __forceinline__ void walk_end(Hot<W>& h, const typename W::View& g, const int32_t* lds, int nlds,
                                          const McArgs& a, const Slots<typename W::Real>& sl, const InstrDev* instr,
                                          uint32_t inst, uint32_t idx, const WalkReq<typename W::Real>* w)
@@ -674,6 +688,7 @@ __device__ __forceinline__ void walk_end(Hot<W>& h, const typename W::View& g, c
         using R = typename W::Real;
         const R d = prop_length(h);
         sl.fr(SR_RES, idx) = d;
+        if (MULTI) sl.fu(SU_MCELL, idx) = (uint32_t)h.mcell;
         h.stage = ST_NEWPKT;
         // the leaf holding the interaction point, where the packet's next walks start: the last segment's, or
         // (a walker whose start cells are exact) looked for by this lane, once for all of those walks, at the
@@ -686,7 +701,7 @@ __device__ __forceinline__ void walk_end(Hot<W>& h, const typename W::View& g, c
     } else if (h.stage == ST_LOC_DONE) {
         if constexpr (W::kLocates) sl.fu(SU_HINT, idx) = (uint32_t)h.w.hint();
         h.stage = ST_NEWPKT;
-    } else if (h.stage == ST_OWN_DONE) own_path_end(h, g, lds, nlds, a, sl, idx, w);
+    } else if (h.stage == ST_OWN_DONE) own_path_end<W, MULTI>(h, g, lds, nlds, a, sl, idx, w);
 }
 
 // Walk kernel bookkeeping of a pass: its first wave's start and, by block 0, the host's progress word (bit 63:
@@ -695,17 +710,17 @@ __device__ __forceinline__ void pass_begin(PassCtl* pc, const McArgs& a, uint64_
 {
     if (blockIdx.x != 0 || threadIdx.x != 0) return;
     const bool claimed = *a.next_packet >= a.count;
-    pc->t0inv = ~(unsigned long long)wall_clock64();
+    pc->t0 = nq ? (unsigned long long)wall_clock64() : 0ull;
     __hip_atomic_store(progress, (1ull << 63) | (claimed ? 1ull << 62 : 0ull) | (unsigned long long)nq, __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Walk pass: persistent lanes over the requests [0, *q.tail). A queue with fewer requests than the launch
 // has chunks needs only the first workgroups.
-template <class W, bool ABS>
+template <class W, bool ABS, bool MULTI>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WalkWaves<W>::value, 8))) k_walks(const typename W::View g, const McArgs a, WalkQueue<typename W::Real> q,
                                               Slots<typename W::Real> sl, PassCtl* pc, unsigned long long* progress,
-                                              int nlds_req, int xcd_segments)
+                                              const GroupTally ta, int nlds_req, int xcd_segments)
 {
     using R = typename W::Real;
     __shared__ InstrDev s_instr[SG_MAX_INSTR];
@@ -733,7 +748,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WalkWa
     for (;;) {
         if (finished_stage(h.stage)) {
             if (leads<W>()) count_walk(h, n_own, n_peel, n_re);
-            walk_end(h, g, s_nodes, nlds, a, sl, s_instr, inst, idx, reqs + req);
+            walk_end<W, MULTI>(h, g, s_nodes, nlds, a, sl, s_instr, inst, idx, reqs + req);
         }
         const bool want = h.stage == ST_NEWPKT;
         uint64_t r = 0;
@@ -775,6 +790,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WalkWa
                 else
                     h.w.init(g, s_nodes, nlds, ox, oy, oz, dx, dy, dz);
                 h.L0 = w.val;
+                h.lsca = (R)0;
                 if (kind == WK_PEEL) h.start_walk(ST_PEELW, (R)a.tau_cut);
                 else h.start_walk(ST_OWN, (R)0);
             }
@@ -785,18 +801,21 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WalkWa
         const int need_n = __builtin_amdgcn_readfirstlane(max(1, min(thr, __popcll(alive) >> 1)));
         bool walk = walking_stage(h.stage);
         for (;;) {
-            if (walk) walk = crossing<W, ABS>(h, g, s_nodes, nlds, a);
+            if (walk) walk = crossing<W, ABS, MULTI>(h, g, s_nodes, nlds, a);
             // lanes alive and not walking are idle (alive is fixed while the wave walks)
             const uint64_t wm = __ballot(walk);
             if (__popcll(alive & ~wm) >= need_n || !wm) break;
         }
     }
-    add_wave(a.counters + 1, n_own);
-    add_wave(a.counters + 2, n_peel);
-    add_wave(a.counters + 8, n_re);
-    add_wave(a.counters + 5, leads<W>() ? h.w.nstuck : 0u);
-    add_wave(a.counters + 9, leads<W>() ? h.w.nrecompute : 0u);
-    if (__lane_id() == 0) atomicMax(&pc->t1, (unsigned long long)wall_clock64());
+    // the wave's record: only this wave writes it
+    WaveRec& rec = ta.waves[blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)];
+    const unsigned long long own = wave_sum(n_own), peel = wave_sum(n_peel), re = wave_sum(n_re);
+    const unsigned long long stuck = wave_sum(leads<W>() ? h.w.nstuck : 0u);
+    const unsigned long long recompute = wave_sum(leads<W>() ? h.w.nrecompute : 0u);
+    if (__lane_id() == 0) {
+        rec.own += own; rec.peel += peel; rec.re += re; rec.stuck += stuck; rec.recompute += recompute;
+        rec.t1 = (unsigned long long)wall_clock64();
+    }
 }
 
 } // namespace sg

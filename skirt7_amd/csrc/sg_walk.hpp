@@ -118,10 +118,12 @@ template <typename R> struct Borders {
     const R *xv, *yv, *zv;
     int oy, oz;              // places of the y and z borders in lds
     // border `at` of the axis given by the flags fy, fz (neither: x)
+    // (Through pointers of their own address spaces: merged into one flat load, a border from LDS waits for the
+    // density's load from memory as well, 0.3 us a step.)
     __device__ __forceinline__ R get(bool fy, bool fz, int at) const
     {
-        if (staged) return lds[at + pick3(fy, fz, 0, oy, oz)];
-        return pick3(fy, fz, xv, yv, zv)[at];
+        if (staged) return ((const __attribute__((address_space(3))) R*)lds)[at + pick3(fy, fz, 0, oy, oz)];
+        return ((const __attribute__((address_space(1))) R*)pick3(fy, fz, xv, yv, zv))[at];
     }
     // NR::locate_clip over the axis's n + 1 borders: the bin guessed from an even spacing (scale bins per length) is
     // taken when it holds x, the only one that does; else a binary search finds it

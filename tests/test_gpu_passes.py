@@ -80,3 +80,31 @@ def test_voronoi_walks_of_several_lanes(lists):
     # sums of at most some ten thousand positive FP64 terms in another order
     np.testing.assert_allclose(out[1][0], out[0][0], rtol=1e-11, atol=0)
     np.testing.assert_allclose(out[1][1], out[0][1], rtol=1e-11, atol=0)
+
+
+@pytest.mark.parametrize("kind", ["cartesian", "octree", "voronoi"])
+@pytest.mark.parametrize("precision", [SG_FP64, SG_MIXED])
+@pytest.mark.parametrize("count,batch", [(1, 0), (511, 0), (513, 128), (3001, 0)])
+def test_passes_of_several_dust_components(kind, precision, count, batch):
+    """Two dust components in the passes against the lane pipeline, at packet counts around the event kernel's
+    workgroup (512 slots): the same histories, absorption and counts."""
+    w = workloads.two_dust_disc(kind, grid_n=12, maxlevel=4, nsites=600, pixels=20, packages=4000)
+    out = []
+    for mode in (0, 1):
+        w["instr"].clear()
+        w["dust"].clear()
+        try:
+            S.set_pipeline(mode)
+            S.set_emit_batch(batch)
+            c = w["sim"].run_packets(1, 5, count, count, precision)
+        finally:
+            S.set_pipeline(1)
+            S.set_emit_batch(0)
+        n = len(w["instr"].instruments)
+        out.append((np.concatenate([w["instr"].frame(i).ravel() for i in range(n)]), w["dust"].Labs(),
+                    {k: c[k] for k in ("packets", "own_crossings", "peel_crossings", "rewalk_crossings", "scatterings",
+                                       "peeloffs", "walks")}))
+    assert out[0][2] == out[1][2]
+    # sums of at most some ten thousand positive FP64 terms in another order
+    np.testing.assert_allclose(out[1][0], out[0][0], rtol=1e-11, atol=0)
+    np.testing.assert_allclose(out[1][1], out[0][1], rtol=1e-11, atol=0)
