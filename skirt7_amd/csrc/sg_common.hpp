@@ -65,6 +65,10 @@ struct alignas(16) TreeRec64 {       // 64 bytes
     int32_t pad;
 };
 
+// What lies across a leaf's wall for the FP64 walk: a cell number, the complement of an internal node's device id,
+// or on the grid's boundary this.
+constexpr int32_t kNoRope = INT32_MIN;
+
 struct TreeView {
     const int32_t* node;             // breadth-first node words
     const TreeRec64* rec64;
@@ -77,6 +81,7 @@ struct TreeView {
     const int32_t* bkchild0;
     const int32_t* bkfather;
     const int32_t* bkcell;
+    const int32_t* rope64;           // per cell 8 words: what lies across walls -x +x -y +y -z +z
     const int32_t* nboff;            // CSR offsets, index cell*6 + wall
     const int32_t* nbids;            // neighbour cell numbers
     int32_t nnodes, ncells;

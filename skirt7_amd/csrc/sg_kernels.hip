@@ -33,7 +33,7 @@ static uint64_t g_batch_alone = (uint64_t)1 << 21;   // batched members this lar
 static int g_topdown_descent = 0;   // 1: mixed walks of TopDown trees descend from the root at every step
 static int g_walk_order = 0;        // 1: the walk kernel takes each pass's walks in coherence-key order; 2: so,
                                     // claimed by XCD segment
-static int g_slot_groups = 2;       // slot groups of the event/walk pipeline (2: alternating on two streams)
+static int g_slot_groups = 0;       // slot groups of the event/walk pipeline (2: alternating on two streams; 0: slot_groups)
 static uint64_t g_emit_batch = 0;   // packets emitted at once (0: each pipeline's default)
 
 // Mixed-precision tree walks follow the ropes (the same cells as any search method) unless TopDown
@@ -414,6 +414,12 @@ int sg_grid_create_tree(int arity, const double ext[6], const uint8_t* subdivide
     std::vector<uint64_t> kpack(ndev, 0);
     std::vector<int32_t> ropes;
     h.build_ropes(ropes);
+    std::vector<int32_t> rope64(8 * (size_t)nc, kNoRope);
+    for (int64_t c = 0; c < nc; c++)
+        for (int w = 0; w < 6; w++) {
+            const int32_t r = ropes[6 * (size_t)h.idv[c] + w];
+            if (r >= 0) rope64[8 * (size_t)c + w] = h.child0[r] < 0 ? h.cellnumber[r] : ~nid[r];
+        }
     std::vector<uint32_t> nsub(nn, 0);   // nx | ny << 5 | nz << 10
     for (int64_t l = 0; l < nn; l++) {
         const int32_t c0 = h.child0[l];
@@ -486,6 +492,7 @@ int sg_grid_create_tree(int arity, const double ext[6], const uint8_t* subdivide
     }
     g->cellof.upload(cellof);
     g->kpack.upload(kpack);
+    g->rope64.upload(rope64);
     off[nc * 6] = (int32_t)ids.size();
     SG_REQUIRE(ids.size() < ((size_t)1 << 31), "neighbour lists too long");
     g->nboff.upload(off);
@@ -499,6 +506,7 @@ int sg_grid_create_tree(int arity, const double ext[6], const uint8_t* subdivide
     t.node32 = g->node32.as<TreeNode32>();
     t.cellof = g->cellof.as<int32_t>();
     t.kpack = g->kpack.as<uint64_t>();
+    t.rope64 = g->rope64.as<int32_t>();
     t.nboff = g->nboff.as<int32_t>();
     t.nbids = g->nbids.as<int32_t>();
     t.nnodes = (int32_t)ndev; t.ncells = (int32_t)nc;
@@ -1487,7 +1495,18 @@ static double walk_ms(GroupCtl* const* ctl, int n)
     return ms;
 }
 
-// Packets [first, first+count) through event and walk passes over two slot groups that alternate on two
+// Slot groups of a run of P slots. A second group hides the drain of the first one's passes, whose last walks
+// leave most of the device idle, but doubles the launches and halves the queues. It pays where walks are long (large
+// trees, Voronoi grids, whose steps cost most) and, in a tree, queues hold enough of them. One and two groups, ms:
+// Voronoi 1e5 sites, 3e4 packets 20.1, 18.9 and 3e5 36.5, 33.4; kd-tree of 5e5 particles, 2.5e5 packets 13.2, 12.7 and
+// 5e5 19.8, 19.4; octree of 7e5 leaves, 4e6 packets 52.7, 52.2 and 4e5 12.1, 12.3; a smaller octree, 2e5 packets 2.75,
+// 3.67 and 3e6 12.9, 13.2; Cartesian 50^3, 3e5 packets 4.1, 4.6, 1e6 8.4, 8.8 and 4e6 26.6, 26.4.
+template <class W> static int slot_groups(int64_t ncells, int64_t P)
+{
+    return W::kLanes > 1 || (W::kHint && ncells >= (int64_t)1 << 19 && P >= (int64_t)1 << 17) ? 2 : 1;
+}
+
+// Packets [first, first+count) through event and walk passes over one slot group, or two that alternate on two
 // streams, so that one group's event pass and the drain of its walk pass overlap the other group's
 // walks. Up to 2^25 packets are emitted at once.
 template <class W, bool ABS, bool MULTI = false>
@@ -1500,7 +1519,7 @@ static void run_split(sg_sim* s, const typename W::View& v, const McArgs& a, uin
     const int64_t slots = g_tune_slots > 0 ? g_tune_slots : kSplitSlots;
     const int64_t P = (int64_t)std::max<uint64_t>(1, std::min<uint64_t>(count, (uint64_t)slots));
     PassGroups<R> pg{};
-    const int G = pg.n = (P >= 2 && g_slot_groups == 2) ? 2 : 1;
+    const int G = pg.n = P >= 2 ? (g_slot_groups ? g_slot_groups : slot_groups<W>(a.ncells, P)) : 1;
     const int64_t Pg[2] = {G == 2 ? (P + 1) / 2 : P, G == 2 ? P / 2 : 0};
     const int bs = pg.bs = g_tune_block;
     pg.nlds = nlds;

@@ -567,17 +567,27 @@ struct Entry {
 };
 
 // TreeDustGrid::path, TopDown (:393-437) and Neighbor (:441-502) methods, exact FP64.
+//
+// Both methods move the point just across the exit wall and look for the leaf that holds it: in the wall's list of
+// neighbours (closed boxes), or from the root. A point strictly inside a leaf lies in no other leaf's closed box and
+// on no plane of the descent, so that leaf is what either search returns, and the walk may find it as it likes. It
+// tries the node across the wall first (`rope64`: a leaf's cell number, or an internal node that is descended by the
+// FP32 split planes of the mixed records), and takes the leaf it reaches if its FP64 box strictly holds the point;
+// points on a wall, and the few that an edge or the FP32 planes send elsewhere, go through the searches themselves.
+// Bound by the latency of dependent loads: the searches took three of them per crossing (list bounds, list, boxes) and
+// about seven cache lines, a leaf of the same size or a larger one now takes one.
 struct TreeW64 {
     using Real = double;
     using View = TreeView;
     double x, y, z, kx, ky, kz, ix, iy, iz;
-    double lo[3], hi[3];
+    double ex, ey, ez;       // the current cell's walls ahead
+    int qx, qy, qz;          // what lies across them (rope64)
     double rho;
     int m, lm;               // current cell, cell of the last segment returned
     Entry en;
     bool done;
     uint32_t steps, nrecompute, nstuck;
-    static constexpr int kParkWords = 45;
+    static constexpr int kParkWords = 42;
     __device__ __forceinline__ static int cell_of(const View&, int n) { return n; }
     static constexpr bool kHint = true;
     static constexpr int kLanes = 1;
@@ -587,28 +597,59 @@ struct TreeW64 {
     template <class P> __device__ __forceinline__ void park(P& p)
     {
         p.io(x); p.io(y); p.io(z); p.io(kx); p.io(ky); p.io(kz); p.io(ix); p.io(iy); p.io(iz);
-        p.io(lo[0]); p.io(lo[1]); p.io(lo[2]); p.io(hi[0]); p.io(hi[1]); p.io(hi[2]);
+        p.io(ex); p.io(ey); p.io(ez); p.io(qx); p.io(qy); p.io(qz);
         p.io(rho); p.io(m); p.io(lm); p.io(en.ne); p.io(en.e0); p.io(en.e1); p.io(en.e2);
         p.io(done); p.io(steps); p.io(nrecompute); p.io(nstuck);
     }
 
+    // Makes c, with the box lo, hi, the current cell.
+    __device__ __forceinline__ void enter(const View& t, int c, double lx, double ly, double lz, double hx, double hy,
+                                          double hz, double density)
+    {
+        const int4* q = reinterpret_cast<const int4*>(t.rope64) + 2 * (size_t)c;
+        const int4 qa = q[0], qb = q[1];
+        const bool bx = kx < 0.0, by = ky < 0.0, bz = kz < 0.0;
+        ex = bx ? lx : hx; ey = by ? ly : hy; ez = bz ? lz : hz;
+        qx = bx ? qa.x : qa.y; qy = by ? qa.z : qa.w; qz = bz ? qb.x : qb.y;
+        rho = density;
+        m = c;
+    }
     __device__ __forceinline__ void load_cell(const View& t, int c)
     {
         const TreeRec64& r = t.rec64[c];
-        lo[0] = r.lo[0]; lo[1] = r.lo[1]; lo[2] = r.lo[2];
-        hi[0] = r.hi[0]; hi[1] = r.hi[1]; hi[2] = r.hi[2];
-        rho = r.rho;
-        m = c;
+        const double lx = r.lo[0], ly = r.lo[1], lz = r.lo[2], hx = r.hi[0], hy = r.hi[1], hz = r.hi[2];
+        enter(t, c, lx, ly, lz, hx, hy, hz, r.rho);
+    }
+    // The leaf strictly holding the point among those below `q`, what lies across the wall just crossed.
+    __device__ __forceinline__ bool follow(const View& t, int q)
+    {
+        if (q == kNoRope) return false;
+        while (q < 0) {
+            const TreeNode32& n = t.node32[~q];
+            const float fx = (float)x, fy = (float)y, fz = (float)z;
+            const float p0 = __int_as_float(n.rope[0]);
+            int k;
+            if (t.arity == 8)
+                k = (fx < p0 ? 0 : 1) + (fy < __int_as_float(n.rope[1]) ? 0 : 2) + (fz < __int_as_float(n.rope[2]) ? 0 : 4);
+            else {
+                const int a = (n.code >> 16) & 3;
+                k = pick3(a == 1, a == 2, fx, fy, fz) < p0 ? 0 : 1;
+            }
+            const int child = (int)n.val + k, c = t.cellof[child];
+            q = c >= 0 ? c : ~child;
+        }
+        const TreeRec64& r = t.rec64[q];
+        const double lx = r.lo[0], ly = r.lo[1], lz = r.lo[2], hx = r.hi[0], hy = r.hi[1], hz = r.hi[2];
+        if (!(x > lx && x < hx && y > ly && y < hy && z > lz && z < hz)) return false;
+        enter(t, q, lx, ly, lz, hx, hy, hz, r.rho);
+        return true;
     }
     __device__ __forceinline__ bool descend(const View& t, const int32_t* lds, int nlds)
     {
         double l[3], h[3];
         int c = descend64(t, lds, nlds, x, y, z, l, h);
         if (c < 0) return false;
-        lo[0] = l[0]; lo[1] = l[1]; lo[2] = l[2];
-        hi[0] = h[0]; hi[1] = h[1]; hi[2] = h[2];
-        m = c;
-        rho = t.rec64[c].rho;
+        enter(t, c, l[0], l[1], l[2], h[0], h[1], h[2], t.rec64[c].rho);
         return true;
     }
     __device__ __forceinline__ void set_direction(double dx, double dy, double dz)
@@ -664,23 +705,20 @@ struct TreeW64 {
     {
         if (en.ne) { ds = en.pop(); mo = -1; rh = 0.0; return true; }
         while (!done) {
-            double xnext = (kx < 0.0) ? lo[0] : hi[0];
-            double ynext = (ky < 0.0) ? lo[1] : hi[1];
-            double znext = (kz < 0.0) ? lo[2] : hi[2];
-            double dsx = ix != 0.0 ? quotient(xnext - x, kx, ix) : DBL_MAX;
-            double dsy = iy != 0.0 ? quotient(ynext - y, ky, iy) : DBL_MAX;
-            double dsz = iz != 0.0 ? quotient(znext - z, kz, iz) : DBL_MAX;
+            double dsx = ix != 0.0 ? quotient(ex - x, kx, ix) : DBL_MAX;
+            double dsy = iy != 0.0 ? quotient(ey - y, ky, iy) : DBL_MAX;
+            double dsz = iz != 0.0 ? quotient(ez - z, kz, iz) : DBL_MAX;
             int a = choose_axis_tree(dsx, dsy, dsz);
-            double d = a == 0 ? dsx : a == 1 ? dsy : dsz;
-            int wall = 2 * a + ((a == 0 ? kx : a == 1 ? ky : kz) < 0.0 ? 0 : 1);
+            double d = pick3(a == 1, a == 2, dsx, dsy, dsz);
+            int wall = 2 * a + (pick3(a == 1, a == 2, kx, ky, kz) < 0.0 ? 0 : 1);
             int segm = m;
             double segrho = rho;
             x += (d + t.eps) * kx;
             y += (d + t.eps) * ky;
             z += (d + t.eps) * kz;
             int oldm = m;
-            bool found = false;
-            if (t.search == 1) {
+            bool found = follow(t, pick3(a == 1, a == 2, qx, qy, qz));
+            if (!found && t.search == 1) {
                 int i0 = t.nboff[oldm * 6 + wall], i1 = t.nboff[oldm * 6 + wall + 1];
                 for (int q = i0; q < i1; q++) {
                     int c = t.nbids[q];

@@ -816,8 +816,8 @@ def set_emit_batch(packets=0):
 
 
 def set_slot_groups(groups=2):
-    """Event/walk pipeline: 2 (default) slot groups alternating on two streams; 1 runs every pass on one stream,
-    one kernel at a time."""
+    """Event/walk pipeline: 2 slot groups alternating on two streams; 1 runs every pass on one stream, one kernel at a
+    time. Until it is set, a run takes two where its grid's walks are long and one elsewhere."""
     check(lib().sg_set_slot_groups(int(groups)))
 
 
