@@ -1175,10 +1175,10 @@ struct LaunchTimer {
     }
 };
 
-static void fill_args(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64_t npp, McArgs& a)
+// A run's arguments, and its scene in host memory for the caller to copy to a.scene.
+static void fill_args(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64_t npp, McArgs& a, SceneDev& sd)
 {
     std::memset(&a, 0, sizeof a);
-    SceneDev sd;
     std::memset(&sd, 0, sizeof sd);
     sg_stars* st = s->stars;
     int ns = (int)(st->params.size() / SG_STAR_NPARAM);
@@ -1257,8 +1257,13 @@ static void fill_args(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64
     a.next_packet = s->next.as<unsigned long long>();
     a.error = s->err.as<int>();
     a.compact = g_tune_compact > 0 ? g_tune_compact : (g_pipeline == 1 ? 24 : 32);
-    SG_HIP(hipMemcpy(s->scene.p, &sd, sizeof sd, hipMemcpyHostToDevice));
     a.scene = s->scene.as<SceneDev>();
+}
+static void fill_args(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64_t npp, McArgs& a)
+{
+    SceneDev sd;
+    fill_args(s, ell, first, count, npp, a, sd);
+    SG_HIP(hipMemcpy(s->scene.p, &sd, sizeof sd, hipMemcpyHostToDevice));
 }
 
 template <class W, bool ABS, bool MULTI = false>
@@ -1354,11 +1359,22 @@ static hipStream_t g_split_stream[2] = {nullptr, nullptr};
 static unsigned long long* g_split_host = nullptr;
 static unsigned long long* g_split_host_dev = nullptr;
 static double g_clock_khz = 100000.0;                   // of the device's wall clock
+// A run's scene on its way to the device and its result on the way back, in pinned host memory, and the event that
+// joins the two streams.
+struct RunHost {
+    SceneDev scene;
+    RunResult result;
+};
+static RunHost* g_run_host = nullptr;
+static RunHost* g_run_host_dev = nullptr;
+static hipEvent_t g_split_join = nullptr;
 // Work buffers of the split pipeline and of the emission, shared by every simulation of the process
 // (runs are synchronous and driven by one host thread): slot groups, walk queues, progress counters,
 // launch states. Allocated on first use, grown as needed, kept until the process ends.
 struct SplitPool {
     DevBuf slots[2], queue[2], prog[2], events[2], waves[2], emitted, emitdraw, emithint;
+    DevBuf run;       // a run's start on the device clock and its end's ticket
+    DevBuf cells;     // dust emission: cumulative and own luminosities of the cells
     DevBuf bins[2];   // per group: bin counts (zero between passes: cleared once, then by each pass's scan), offsets
 };
 static SplitPool* g_pool = nullptr;
@@ -1375,6 +1391,9 @@ static void split_resources()
     SG_HIP(hipHostMalloc(reinterpret_cast<void**>(&g_split_host), 2 * kProgressRing * sizeof(unsigned long long),
                          hipHostMallocMapped | hipHostMallocCoherent));
     SG_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&g_split_host_dev), g_split_host, 0));
+    SG_HIP(hipHostMalloc(reinterpret_cast<void**>(&g_run_host), sizeof(RunHost), hipHostMallocMapped | hipHostMallocCoherent));
+    SG_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&g_run_host_dev), g_run_host, 0));
+    SG_HIP(hipEventCreateWithFlags(&g_split_join, hipEventDisableTiming));
     int khz = 0;
     if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, g_device) == hipSuccess && khz > 0) g_clock_khz = khz;
 }
@@ -1477,22 +1496,30 @@ static void launch_emit(const typename W::View& v, McArgs& a, void* emitted, uin
     SG_HIP(hipGetLastError());
 }
 
-static void launch_counts(const GroupTally& ta, unsigned long long* counters, hipStream_t st)
+// Emission of a's packets by the dust cells.
+template <typename R>
+static void launch_emit_dust(const DustLaunch& dl, McArgs& a, void* emitted, uint32_t* draws, hipStream_t st)
 {
-    const int64_t n = std::max<int64_t>(ta.nevents, ta.nwaves);
-    hipLaunchKernelGGL(k_run_counts, dim3(std::min<int64_t>((n + 255) / 256, 16)), dim3(256), 0, st, ta, counters);
+    a.emitted = emitted;
+    a.emit_draw = draws;
+    const int blocks = (int)std::min<uint64_t>((a.count + 255) / 256, (uint64_t)g_cus * 16);
+    hipLaunchKernelGGL(k_emit_dust<R>, dim3(blocks), dim3(256), 0, st, a, dl, static_cast<R*>(emitted), draws);
+    SG_HIP(hipGetLastError());
 }
 
-// Duration of the groups' walk kernels (the passes have ended).
-static double walk_ms(GroupCtl* const* ctl, int n)
+// The run's start and end words on the device: clock ticks, ticket.
+static unsigned long long* run_words()
 {
-    double ms = 0;
-    for (int g = 0; g < n; g++) {
-        unsigned long long t = 0;
-        SG_HIP(hipMemcpy(&t, &ctl[g]->ticks, sizeof t, hipMemcpyDeviceToHost));
-        ms += (double)t / g_clock_khz;
-    }
-    return ms;
+    DevBuf& b = pool().run;
+    if (!b.bytes) b.alloc(2 * sizeof(unsigned long long));
+    return b.as<unsigned long long>();
+}
+static void launch_end(const RunEnd& e, hipStream_t st)
+{
+    int64_t n = 1;
+    for (int g = 0; g < e.n; g++) n = std::max({n, e.tally[g].nevents, (int64_t)e.tally[g].nwaves});
+    hipLaunchKernelGGL(k_run_end, dim3(std::min<int64_t>((n + 255) / 256, 16)), dim3(256), 0, st, e);
+    SG_HIP(hipGetLastError());
 }
 
 // Slot groups of a run of P slots. A second group hides the drain of the first one's passes, whose last walks
@@ -1506,12 +1533,19 @@ template <class W> static int slot_groups(int64_t ncells, int64_t P)
     return W::kLanes > 1 || (W::kHint && ncells >= (int64_t)1 << 19 && P >= (int64_t)1 << 17) ? 2 : 1;
 }
 
+// What a run of the event/walk pipeline is given and returns beyond its result in g_run_host: dust emission instead of
+// the stars', whether the scene is to be taken from there, and the walk launches that had requests.
+struct SplitRun {
+    const DustLaunch* dust = nullptr;
+    bool scene = true;
+    int launches = 0;
+};
 // Packets [first, first+count) through event and walk passes over one slot group, or two that alternate on two
 // streams, so that one group's event pass and the drain of its walk pass overlap the other group's
 // walks. Up to 2^25 packets are emitted at once.
 template <class W, bool ABS, bool MULTI = false>
 static void run_split(sg_sim* s, const typename W::View& v, const McArgs& a, uint64_t first, uint64_t count, int nlds,
-                      LaunchTimer& lt, int& blocks)
+                      SplitRun& run, int& blocks)
 {
     using R = typename W::Real;
     split_resources();
@@ -1528,6 +1562,8 @@ static void run_split(sg_sim* s, const typename W::View& v, const McArgs& a, uin
     int per = 0;
     SG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_walks<W, ABS, MULTI>, bs, pg.shm));
     pg.blocks = blocks = std::max(1, per) * g_cus;
+    RunBegin rb{};
+    auto zero = [&](void* p, size_t bytes) { rb.zero[rb.nzero++] = {static_cast<uint32_t*>(p), (int64_t)(bytes / 4)}; };
     for (int g = 0; g < G; g++) {
         const int64_t cap = Pg[g] * (a.ni + 1);
         SplitPool& pl = pool();
@@ -1557,7 +1593,6 @@ static void run_split(sg_sim* s, const typename W::View& v, const McArgs& a, uin
             q.hist = pl.bins[g].as<uint32_t>();
             q.off = q.hist + kKeyBins;
         }
-        // progress and count records zero; slot states PS_FRESH
         GroupTally& ta = pg.tally[g];
         ta.nevents = event_blocks(Pg[g]);
         ta.nwaves = pg.blocks * (pg.bs / 64);
@@ -1567,10 +1602,11 @@ static void run_split(sg_sim* s, const typename W::View& v, const McArgs& a, uin
         if (pl.waves[g].bytes < wbytes) pl.waves[g].alloc(wbytes);
         ta.events = pl.events[g].as<unsigned long long>();
         ta.waves = pl.waves[g].as<WaveRec>();
-        SG_HIP(hipMemsetAsync(pg.ctl[g], 0, sizeof(GroupCtl), st[g]));
-        SG_HIP(hipMemsetAsync(ta.events, 0, ebytes, st[g]));
-        SG_HIP(hipMemsetAsync(ta.waves, 0, wbytes, st[g]));
-        SG_HIP(hipMemsetAsync(sl.u + (size_t)SU_STATE * Pg[g], 0, (size_t)Pg[g] * sizeof(uint32_t), st[g]));
+        // progress and count records zero; slot states PS_FRESH
+        zero(pg.ctl[g], sizeof(GroupCtl));
+        zero(ta.events, ebytes);
+        zero(ta.waves, wbytes);
+        zero(sl.u + (size_t)SU_STATE * Pg[g], (size_t)Pg[g] * sizeof(uint32_t));
     }
     const uint64_t batch = std::min<uint64_t>(count, g_emit_batch ? g_emit_batch : kSplitEmit);
     const size_t rsz = sizeof(R);
@@ -1581,87 +1617,92 @@ static void run_split(sg_sim* s, const typename W::View& v, const McArgs& a, uin
     DevBuf& emithint = pool().emithint;
     if (W::kHint && emithint.bytes < batch * sizeof(int32_t)) emithint.alloc(batch * sizeof(int32_t));
     unsigned long long* claims = s->next.as<unsigned long long>();
-    hipEvent_t ev_start, ev_join, ev_end[2];
-    SG_HIP(hipEventCreateWithFlags(&ev_join, hipEventDisableTiming));
-    SG_HIP(hipEventCreate(&ev_start));
-    for (int g = 0; g < 2; g++) SG_HIP(hipEventCreate(&ev_end[g]));
-    int walk_launches = 0;
+    unsigned long long* words = run_words();
+    zero(a.counters, SG_NCOUNTERS * sizeof(unsigned long long));
+    zero(a.error, sizeof(int));
+    zero(words + 1, sizeof(unsigned long long));
+    rb.scene_host = run.scene ? reinterpret_cast<const uint32_t*>(&g_run_host_dev->scene) : nullptr;
+    rb.scene = s->scene.as<uint32_t>();
+    rb.next = claims;
+    // the slots take a batch's first packets by their numbers, the others are claimed
+    rb.first_claim = (unsigned long long)P;
+    rb.begin = words;
+    int64_t most = 1;
+    for (int k = 0; k < rb.nzero; k++) most = std::max(most, rb.zero[k].words);
+    hipLaunchKernelGGL(k_run_begin, dim3((unsigned)std::min<int64_t>((most + 1023) / 1024, (int64_t)g_cus * 4)), dim3(256), 0,
+                       st[0], rb);
+    SG_HIP(hipGetLastError());
+    auto join = [](hipStream_t from, hipStream_t to) {
+        SG_HIP(hipEventRecord(g_split_join, from));
+        SG_HIP(hipStreamWaitEvent(to, g_split_join, 0));
+    };
     for (uint64_t b = 0; b < count; b += batch) {
         McArgs ab = a;
         ab.first = first + b;
         ab.count = std::min(batch, count - b);
         ab.next_packet = claims;
         // the previous batch is finished on both streams: emit on stream 0, then both groups start
-        if (G == 2) {
-            SG_HIP(hipEventRecord(ev_join, st[1]));
-            SG_HIP(hipStreamWaitEvent(st[0], ev_join, 0));
+        if (b > 0) {
+            if (G == 2) join(st[1], st[0]);
+            launch_set(claims, (unsigned long long)P, st[0]);
         }
-        // the slots take the batch's first packets by their numbers, the others are claimed
-        launch_set(claims, (unsigned long long)P, st[0]);
-        launch_emit<W>(v, ab, emitted.p, emitdraw.as<uint32_t>(), emithint.as<int32_t>(), st[0]);
+        if (run.dust) launch_emit_dust<R>(*run.dust, ab, emitted.p, emitdraw.as<uint32_t>(), st[0]);
+        else launch_emit<W>(v, ab, emitted.p, emitdraw.as<uint32_t>(), emithint.as<int32_t>(), st[0]);
         for (int g = 0; g < G && b > 0; g++)
             hipLaunchKernelGGL(k_revive, dim3((Pg[g] + 255) / 256), dim3(256), 0, st[0],
                                pg.sl[g].u + (size_t)SU_STATE * Pg[g], Pg[g]);
-        if (b == 0) SG_HIP(hipEventRecord(ev_start, st[0]));
-        if (G == 2) {
-            SG_HIP(hipEventRecord(ev_join, st[0]));
-            SG_HIP(hipStreamWaitEvent(st[1], ev_join, 0));
-        }
-        walk_launches += run_passes<W, ABS, MULTI>(v, ab, pg);
+        if (G == 2) join(st[0], st[1]);
+        run.launches += run_passes<W, ABS, MULTI>(v, ab, pg);
     }
-    // each group's counts on its own stream, behind its last passes
-    for (int g = 0; g < G; g++) {
-        launch_counts(pg.tally[g], a.counters, st[g]);
-        SG_HIP(hipGetLastError());
-        SG_HIP(hipEventRecord(ev_end[g], st[g]));
-    }
+    if (G == 2) join(st[1], st[0]);
+    RunEnd re{};
+    re.n = G;
+    for (int g = 0; g < G; g++) { re.tally[g] = pg.tally[g]; re.ctl[g] = pg.ctl[g]; }
+    re.counters = a.counters;
+    re.err = a.error;
+    re.begin = words;
+    re.ticket = reinterpret_cast<unsigned int*>(words + 1);
+    re.out = &g_run_host_dev->result;
+    launch_end(re, st[0]);
     SG_HIP(hipStreamSynchronize(st[0]));
-    if (G == 2) SG_HIP(hipStreamSynchronize(st[1]));
-    float ms = 0, ms1 = 0;
-    SG_HIP(hipEventElapsedTime(&ms, ev_start, ev_end[0]));
-    if (G == 2) SG_HIP(hipEventElapsedTime(&ms1, ev_start, ev_end[1]));
-    lt.add(std::max(ms, ms1), walk_launches, walk_ms(pg.ctl, G));
-    (void)hipEventDestroy(ev_start);
-    (void)hipEventDestroy(ev_join);
-    for (int g = 0; g < 2; g++) (void)hipEventDestroy(ev_end[g]);
 }
 
 template <bool ABS, bool MULTI>
-static void dispatch_split(sg_sim* s, const McArgs& a, int precision, uint64_t first, uint64_t count, LaunchTimer& lt,
+static void dispatch_split(sg_sim* s, const McArgs& a, int precision, uint64_t first, uint64_t count, SplitRun& run,
                            int& blocks)
 {
     const bool mixed = precision == SG_MIXED;
     sg_grid* g = s->dust ? s->dust->grid : nullptr;
     if (!g) {
         CartView v{};
-        if (mixed) run_split<CartW32, false>(s, v, a, first, count, 0, lt, blocks);
-        else run_split<CartW64, false>(s, v, a, first, count, 0, lt, blocks);
+        if (mixed) run_split<CartW32, false>(s, v, a, first, count, 0, run, blocks);
+        else run_split<CartW64, false>(s, v, a, first, count, 0, run, blocks);
         return;
     }
     if (g->kind == GK_CART) {
-        if (mixed) run_split<CartW32, ABS, MULTI>(s, g->cart, a, first, count, cart_words<float>(g), lt, blocks);
-        else run_split<CartW64, ABS, MULTI>(s, g->cart, a, first, count, cart_words<double>(g), lt, blocks);
+        if (mixed) run_split<CartW32, ABS, MULTI>(s, g->cart, a, first, count, cart_words<float>(g), run, blocks);
+        else run_split<CartW64, ABS, MULTI>(s, g->cart, a, first, count, cart_words<double>(g), run, blocks);
     } else if (g->kind == GK_TREE) {
-        if (!mixed && g->tree.search == SG_BOOKKEEPING) run_split<TreeW64Book, ABS, MULTI>(s, g->tree, a, first, count, 0, lt, blocks);
-        else if (!mixed) run_split<TreeW64, ABS, MULTI>(s, g->tree, a, first, count, SG_LDS_NODES, lt, blocks);
-        else if (rope_walk(g)) run_split<TreeW32, ABS, MULTI>(s, g->tree, a, first, count, SG_LDS_NODES, lt, blocks);
-        else run_split<TreeW32TopDown, ABS, MULTI>(s, g->tree, a, first, count, SG_LDS_NODES, lt, blocks);
+        if (!mixed && g->tree.search == SG_BOOKKEEPING) run_split<TreeW64Book, ABS, MULTI>(s, g->tree, a, first, count, 0, run, blocks);
+        else if (!mixed) run_split<TreeW64, ABS, MULTI>(s, g->tree, a, first, count, SG_LDS_NODES, run, blocks);
+        else if (rope_walk(g)) run_split<TreeW32, ABS, MULTI>(s, g->tree, a, first, count, SG_LDS_NODES, run, blocks);
+        else run_split<TreeW32TopDown, ABS, MULTI>(s, g->tree, a, first, count, SG_LDS_NODES, run, blocks);
     } else {
-        if (mixed) run_split<VoroWalk<float>, ABS, MULTI>(s, g->voro, a, first, count, 0, lt, blocks);
-        else run_split<VoroWalk<double>, ABS, MULTI>(s, g->voro, a, first, count, 0, lt, blocks);
+        if (mixed) run_split<VoroWalk<float>, ABS, MULTI>(s, g->voro, a, first, count, 0, run, blocks);
+        else run_split<VoroWalk<double>, ABS, MULTI>(s, g->voro, a, first, count, 0, run, blocks);
     }
 }
 
 // The event/walk pipeline for a run's arguments: absorption stored or not, one or several dust components.
-static void dispatch_split_any(sg_sim* s, const McArgs& a, int precision, uint64_t first, uint64_t count, LaunchTimer& lt,
+static void dispatch_split_any(sg_sim* s, const McArgs& a, int precision, uint64_t first, uint64_t count, SplitRun& run,
                                int& blocks)
 {
     if (a.ncomp > 1) {
-        if (a.store_abs) dispatch_split<true, true>(s, a, precision, first, count, lt, blocks);
-        else dispatch_split<false, true>(s, a, precision, first, count, lt, blocks);
+        if (a.store_abs) dispatch_split<true, true>(s, a, precision, first, count, run, blocks);
+        else dispatch_split<false, true>(s, a, precision, first, count, run, blocks);
     } else {
-        if (a.store_abs) dispatch_split<true, false>(s, a, precision, first, count, lt, blocks);
-        else dispatch_split<false, false>(s, a, precision, first, count, lt, blocks);
+        if (a.store_abs) dispatch_split<true, false>(s, a, precision, first, count, run, blocks);
+        else dispatch_split<false, false>(s, a, precision, first, count, run, blocks);
     }
 }
 
@@ -1673,58 +1714,71 @@ int sg_sim_run(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64_t npp,
     ensure_init();
     SG_REQUIRE(npp > 0, "npp must be positive");
     McArgs a;
-    fill_args(s, ell, first, count, npp, a);
-    s->counters.zero();
-    s->err.zero();
-    const bool mixed = precision == SG_MIXED;
-    const size_t rsz = mixed ? sizeof(float) : sizeof(double);
-    const uint64_t batch = std::min<uint64_t>(count, g_emit_batch ? g_emit_batch : (uint64_t)1 << 22);
-    const int pipeline = g_pipeline;
-    if (pipeline == 0) {
+    int err = 0, blocks = 0;
+    if (g_pipeline == 1 && count > 0) {
+        split_resources();
+        fill_args(s, ell, first, count, npp, a, g_run_host->scene);
+        SplitRun run;
+        dispatch_split_any(s, a, precision, first, count, run, blocks);
+        const RunResult& r = g_run_host->result;
+        err = (int)r.err;
+        if (counters) {
+            for (int i = 0; i < SG_NCOUNTERS; i++) counters[i] = r.counters[i];
+            counters[6] = npp;
+            counters[10] = (uint64_t)(r.span * 1000.0 / g_clock_khz);
+            counters[11] = blocks;
+            counters[12] = (uint64_t)(r.transport * 1000.0 / g_clock_khz);
+            counters[13] = run.launches;
+            counters[14] = (uint64_t)(r.walk * 1000.0 / g_clock_khz);
+        }
+    } else {
+        fill_args(s, ell, first, count, npp, a);
+        s->counters.zero();
+        s->err.zero();
+        const bool mixed = precision == SG_MIXED;
+        const size_t rsz = mixed ? sizeof(float) : sizeof(double);
+        const uint64_t batch = std::min<uint64_t>(count, g_emit_batch ? g_emit_batch : (uint64_t)1 << 22);
         if (s->emitted.bytes < 7 * batch * rsz) s->emitted.alloc(7 * batch * rsz);
         if (s->emitdraw.bytes < batch * sizeof(uint32_t)) s->emitdraw.alloc(batch * sizeof(uint32_t));
-    }
-    hipEvent_t e0, e1;
-    SG_HIP(hipEventCreate(&e0));
-    SG_HIP(hipEventCreate(&e1));
-    SG_HIP(hipEventRecord(e0, 0));
-    int blocks = 0;
-    LaunchTimer lt;
-    if (pipeline == 1 && count > 0) dispatch_split_any(s, a, precision, first, count, lt, blocks);
-    // the lane pipeline runs in batches: emission kernel, then the persistent transport kernel
-    for (uint64_t b = 0; pipeline == 0 && b < count; b += batch) {
-        McArgs ab = a;
-        ab.first = first + b;
-        ab.count = std::min(batch, count - b);
-        ab.emitted = s->emitted.p;
-        ab.emit_draw = s->emitdraw.as<uint32_t>();
-        s->next.zero();
-        int eb = (int)std::min<uint64_t>((ab.count + 255) / 256, (uint64_t)g_cus * 16);
-        if (mixed) hipLaunchKernelGGL(k_emit<float>, dim3(eb), dim3(256), 0, 0, ab, s->emitted.as<float>(), s->emitdraw.as<uint32_t>());
-        else hipLaunchKernelGGL(k_emit<double>, dim3(eb), dim3(256), 0, 0, ab, s->emitted.as<double>(), s->emitdraw.as<uint32_t>());
-        SG_HIP(hipGetLastError());
-        lt.start();
-        dispatch_mc_any(s, ab, precision, blocks);
-        lt.stop();
-    }
-    SG_HIP(hipEventRecord(e1, 0));
-    SG_HIP(hipEventSynchronize(e1));
-    float ms = 0;
-    SG_HIP(hipEventElapsedTime(&ms, e0, e1));
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    unsigned long long c[SG_NCOUNTERS];
-    SG_HIP(hipMemcpy(c, s->counters.p, sizeof c, hipMemcpyDeviceToHost));
-    int err = 0;
-    SG_HIP(hipMemcpy(&err, s->err.p, sizeof err, hipMemcpyDeviceToHost));
-    if (counters) {
-        for (int i = 0; i < SG_NCOUNTERS; i++) counters[i] = c[i];
-        counters[6] = npp;
-        counters[10] = (uint64_t)(ms * 1000.0);
-        counters[11] = blocks;
-        counters[12] = (uint64_t)(lt.total_ms() * 1000.0);
-        counters[13] = lt.launches();
-        counters[14] = (uint64_t)(lt.kernel_ms() * 1000.0);
+        hipEvent_t e0, e1;
+        SG_HIP(hipEventCreate(&e0));
+        SG_HIP(hipEventCreate(&e1));
+        SG_HIP(hipEventRecord(e0, 0));
+        LaunchTimer lt;
+        // the lane pipeline runs in batches: emission kernel, then the persistent transport kernel
+        for (uint64_t b = 0; b < count; b += batch) {
+            McArgs ab = a;
+            ab.first = first + b;
+            ab.count = std::min(batch, count - b);
+            ab.emitted = s->emitted.p;
+            ab.emit_draw = s->emitdraw.as<uint32_t>();
+            s->next.zero();
+            int eb = (int)std::min<uint64_t>((ab.count + 255) / 256, (uint64_t)g_cus * 16);
+            if (mixed) hipLaunchKernelGGL(k_emit<float>, dim3(eb), dim3(256), 0, 0, ab, s->emitted.as<float>(), s->emitdraw.as<uint32_t>());
+            else hipLaunchKernelGGL(k_emit<double>, dim3(eb), dim3(256), 0, 0, ab, s->emitted.as<double>(), s->emitdraw.as<uint32_t>());
+            SG_HIP(hipGetLastError());
+            lt.start();
+            dispatch_mc_any(s, ab, precision, blocks);
+            lt.stop();
+        }
+        SG_HIP(hipEventRecord(e1, 0));
+        SG_HIP(hipEventSynchronize(e1));
+        float ms = 0;
+        SG_HIP(hipEventElapsedTime(&ms, e0, e1));
+        (void)hipEventDestroy(e0);
+        (void)hipEventDestroy(e1);
+        unsigned long long c[SG_NCOUNTERS];
+        SG_HIP(hipMemcpy(c, s->counters.p, sizeof c, hipMemcpyDeviceToHost));
+        SG_HIP(hipMemcpy(&err, s->err.p, sizeof err, hipMemcpyDeviceToHost));
+        if (counters) {
+            for (int i = 0; i < SG_NCOUNTERS; i++) counters[i] = c[i];
+            counters[6] = npp;
+            counters[10] = (uint64_t)(ms * 1000.0);
+            counters[11] = blocks;
+            counters[12] = (uint64_t)(lt.total_ms() * 1000.0);
+            counters[13] = lt.launches();
+            counters[14] = (uint64_t)(lt.total_ms() * 1000.0);
+        }
     }
     SG_REQUIRE(!(err & 2), "walk order: a request's sorted place lies beyond the pass's requests");
     SG_REQUIRE(!(err & 4), "walk queue: a request names no instrument pixel or packet slot");
@@ -1820,22 +1874,41 @@ int sg_sim_run_dust(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64_t
     if (!(Ltot > 0) || count == 0) return 0;
     const double norm = cum[nc];
     for (int64_t m = 0; m <= nc; m++) cum[m] /= norm;
+    const bool passes = g_pipeline == 1;
     McArgs a;
-    fill_args(s, ell, first, count, npp, a);
+    if (passes) {
+        split_resources();
+        fill_args(s, ell, first, count, npp, a, g_run_host->scene);
+    } else fill_args(s, ell, first, count, npp, a);
     a.member = a.member ^ (stream * 0x9E3779B9u);
     a.Lpkt = Ltot / (double)npp;
     a.Lthreshold = a.Lpkt / s->mc[1];
     a.store_abs = store_absorption && s->dust->store_abs;
     if (!a.store_abs) a.labs = nullptr;
     if (!peeloffs) a.ni = 0;
-    if (g_tune_compact <= 0) a.compact = 32;
-    DevBuf b_cum, b_lv;
-    b_cum.upload(cum);
-    b_lv.upload(Lv, nc);
+    // the cumulative luminosities, then the cells' own
+    cum.insert(cum.end(), Lv, Lv + nc);
+    DevBuf& cells = pool().cells;
+    if (cells.bytes < cum.size() * sizeof(double)) cells.alloc(cum.size() * sizeof(double));
+    SG_HIP(hipMemcpy(cells.p, cum.data(), cum.size() * sizeof(double), hipMemcpyHostToDevice));
     DustLaunch dl{};
-    dl.cum = b_cum.as<double>(); dl.Lv = b_lv.as<double>(); dl.ncells = nc;
+    dl.cum = cells.as<double>(); dl.Lv = dl.cum + nc + 1; dl.ncells = nc;
     dl.xi = bias; dl.Lmean = Ltot / nc; dl.Lem = Ltot / (double)npp;
     dl.cb = cell_boxes(g);
+    int blocks = 0;
+    if (passes) {
+        SplitRun run;
+        run.dust = &dl;
+        dispatch_split_any(s, a, precision, first, count, run, blocks);
+        const RunResult& r = g_run_host->result;
+        if (counters) {
+            for (int i = 0; i < SG_NCOUNTERS; i++) counters[i] = r.counters[i];
+            counters[6] = npp;
+            counters[11] = blocks;
+        }
+        SG_REQUIRE(r.err == 0, "The optical depth along the path is not a positive number");
+        return 0;
+    }
     s->counters.zero();
     s->err.zero();
     const bool mixed = precision == SG_MIXED;
@@ -1843,7 +1916,6 @@ int sg_sim_run_dust(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64_t
     const uint64_t batch = std::min<uint64_t>(count, g_emit_batch ? g_emit_batch : (uint64_t)1 << 22);
     if (s->emitted.bytes < 7 * batch * rsz) s->emitted.alloc(7 * batch * rsz);
     if (s->emitdraw.bytes < batch * sizeof(uint32_t)) s->emitdraw.alloc(batch * sizeof(uint32_t));
-    int blocks = 0;
     for (uint64_t b = 0; b < count; b += batch) {
         McArgs ab = a;
         ab.first = first + b;
@@ -1964,8 +2036,11 @@ static void run_static(sg_sim* s, const typename W::View& v, const McArgs& a0, i
     if (a.count > 0)
         launch_emit<W>(v, a, base + o_em, reinterpret_cast<uint32_t*>(base + o_ed), reinterpret_cast<int32_t*>(base + o_eh), st);
     run_passes<W, ABS, false>(v, a, pg);
-    launch_counts(ta, a.counters, st);
-    SG_HIP(hipGetLastError());
+    RunEnd re{};
+    re.n = 1;
+    re.tally[0] = ta;
+    re.counters = a.counters;
+    launch_end(re, st);
     SG_HIP(hipStreamSynchronize(st));
 }
 
@@ -2306,7 +2381,11 @@ int sg_sim_run_batch(int nmembers, sg_sim* const* sims, const int* ells, const u
     for (int i = 0; g_pipeline == 1 && g_batch_alone > 0 && i < nmembers; i++) {
         if (done[i] == counts[i]) continue;
         if (counts[i] < g_batch_alone) continue;
-        dispatch_split_any(sims[i], base[i], precision, 0, counts[i], lt, blocks);
+        SplitRun run;
+        run.scene = false;
+        dispatch_split_any(sims[i], base[i], precision, 0, counts[i], run, blocks);
+        const RunResult& r = g_run_host->result;
+        lt.add(r.transport / g_clock_khz, run.launches, r.walk / g_clock_khz);
         done[i] = counts[i];
     }
     int j = 0;

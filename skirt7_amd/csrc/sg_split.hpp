@@ -68,6 +68,7 @@ constexpr int kPassRing = 4;
 struct GroupCtl {
     PassCtl pass[kPassRing];
     unsigned long long ticks;           // walk kernels' durations, summed over the finished passes
+    unsigned long long start;           // the first pass's start (clock ticks)
 };
 // What each wave of the walk kernel keeps from pass to pass in a record of its own: the end of its last pass
 // (clock ticks) and its counts. (Added up with atomics at the end of every pass, on one cache line at about 10 ns
@@ -260,6 +261,7 @@ __global__ void __launch_bounds__(kEventBlock) k_events(const McArgs a, Slots<R>
         const PassCtl& pv = gc->pass[(pass + kPassRing - 1) % kPassRing];
         if (threadIdx.x == 0) {
             s_base = 0;
+            if (pass == 0) gc->start = wall_clock64();
             PassCtl& nx = gc->pass[(pass + 1) % kPassRing];
             nx.tail = 0; nx.claim = 0; nx.t0 = 0;
             for (int k = 0; k < kXcdSegs; k++) nx.seg[k] = 0;
@@ -476,19 +478,94 @@ __global__ void __launch_bounds__(256) k_key_scatter(WalkQueue<R> q, int* error)
     }
 }
 
-// End of a run: the event workgroups' and the walk waves' counts into the run counters.
-__global__ void __launch_bounds__(256) k_run_counts(const GroupTally ta, unsigned long long* counters)
+// Start of a run: what its kernels expect to be zero, the packet claims, the scene, the clock.
+struct RunBegin {
+    struct Fill { uint32_t* p; int64_t words; } zero[11];
+    int nzero;
+    const uint32_t* scene_host;         // pinned host memory, or null: the scene is there already
+    uint32_t* scene;
+    unsigned long long* next;
+    unsigned long long first_claim;
+    unsigned long long* begin;          // clock ticks
+};
+// One launch: the scene's blocking copy, eleven fills and the event records took about 250 us of a run between them
+// (a run of 5e3 packets on 24^3 cells: 1.08 ms with them).
+__global__ void __launch_bounds__(256) k_run_begin(const RunBegin b)
 {
-    unsigned long long v[9] = {};
-    for (int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; b < ta.nevents; b += (int64_t)gridDim.x * blockDim.x)
-        for (int k = 0; k < 4; k++) v[k] += ta.events[4 * b + k];
-    for (int w = (int)(blockIdx.x * blockDim.x + threadIdx.x); w < ta.nwaves; w += (int)(gridDim.x * blockDim.x)) {
-        const WaveRec& r = ta.waves[w];
-        v[4] += r.own; v[5] += r.peel; v[6] += r.re; v[7] += r.stuck; v[8] += r.recompute;
+    const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, n = (int64_t)gridDim.x * blockDim.x;
+    if (blockIdx.x == 0) {
+        for (int i = (int)threadIdx.x; b.scene_host && i < (int)(sizeof(SceneDev) / 4); i += (int)blockDim.x) b.scene[i] = b.scene_host[i];
+        if (threadIdx.x == 0) {
+            *b.next = b.first_claim;
+            *b.begin = wall_clock64();
+        }
     }
+    for (int k = 0; k < b.nzero; k++)
+        for (int64_t i = i0; i < b.zero[k].words; i += n) b.zero[k].p[i] = 0;
+}
+
+// What a run leaves in pinned host memory: its counters, error bits, and on the device clock its walk kernels'
+// duration and its span from the start and from the first pass on.
+struct RunResult {
+    unsigned long long counters[SG_NCOUNTERS];
+    unsigned long long err, walk, span, transport;
+};
+struct RunEnd {
+    GroupTally tally[2];
+    GroupCtl* ctl[2];
+    int n;
+    unsigned long long* counters;
+    const int* err;
+    const unsigned long long* begin;
+    unsigned int* ticket;               // zero at the run's start
+    RunResult* out;                     // or null: the counters alone
+};
+// End of a run: the event workgroups' and the walk waves' counts into the run counters, by the last workgroup to
+// finish written to the host with the rest of the result.
+__global__ void __launch_bounds__(256) k_run_end(const RunEnd e)
+{
+    __shared__ unsigned long long s_sum[9];
+    __shared__ bool s_last;
+    if (threadIdx.x < 9) s_sum[threadIdx.x] = 0;
+    __syncthreads();
+    unsigned long long v[9] = {};
+    const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, n = (int64_t)gridDim.x * blockDim.x;
+    for (int g = 0; g < e.n; g++) {
+        for (int64_t b = i0; b < e.tally[g].nevents; b += n)
+            for (int k = 0; k < 4; k++) v[k] += e.tally[g].events[4 * b + k];
+        for (int64_t w = i0; w < e.tally[g].nwaves; w += n) {
+            const WaveRec& r = e.tally[g].waves[w];
+            v[4] += r.own; v[5] += r.peel; v[6] += r.re; v[7] += r.stuck; v[8] += r.recompute;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 9; k++) add_wave(&s_sum[k], v[k]);
+    __syncthreads();
     const int dst[9] = {0, 3, 4, 7, 1, 2, 8, 5, 9};
 #pragma unroll
-    for (int k = 0; k < 9; k++) add_wave(counters + dst[k], v[k]);
+    for (int k = 0; k < 9; k++)
+        if ((int)threadIdx.x == k && s_sum[k]) atomicAdd(e.counters + dst[k], s_sum[k]);
+    if (!e.out) return;
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0) s_last = atomicAdd(e.ticket, 1u) == gridDim.x - 1;
+    __syncthreads();
+    if (!s_last) return;
+    __threadfence();
+    if (threadIdx.x < SG_NCOUNTERS)
+        e.out->counters[threadIdx.x] = __hip_atomic_load(e.counters + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == SG_NCOUNTERS) {
+        unsigned long long walk = 0, start = ~0ull;
+        for (int g = 0; g < e.n; g++) {
+            walk += e.ctl[g]->ticks;
+            start = min(start, e.ctl[g]->start);
+        }
+        const unsigned long long now = wall_clock64();
+        e.out->err = (unsigned long long)*e.err;
+        e.out->walk = walk;
+        e.out->span = now - *e.begin;
+        e.out->transport = now > start ? now - start : 0;
+    }
 }
 
 // Request claims of one wave: chunks of requests by one global atomic each, handed out in order to the lanes
