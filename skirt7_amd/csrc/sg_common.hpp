@@ -65,14 +65,22 @@ struct alignas(16) TreeRec64 {       // 64 bytes
     int32_t pad;
 };
 
-// What lies across a leaf's wall for the FP64 walk: a cell number, the complement of an internal node's device id,
-// or on the grid's boundary this.
-constexpr int32_t kNoRope = INT32_MIN;
+// FP64 walk record, one per tree node (device id), one 128-byte line: a leaf's box, density, the nodes across its walls
+// -x +x -y +y -z +z (as TreeNode32's ropes) and its cell number; an internal node's split planes (the mixed record's, in
+// lo), first child and -1 - split axis.
+struct alignas(128) TreeNode64 {
+    double lo[3], hi[3];
+    double rho;
+    int32_t rope[6];
+    int32_t cell, child;
+};
+static_assert(sizeof(TreeNode64) == 128, "one line");
 
 struct TreeView {
     const int32_t* node;             // breadth-first node words
     const TreeRec64* rec64;
     const TreeNode32* node32;        // mixed-precision walk records
+    const TreeNode64* node64;        // FP64 walk records
     const int32_t* cellof;           // cell number per node (-1 for internal nodes)
     const uint64_t* kpack;           // integer indices per node, i | j << 21 | k << 42
     // Bookkeeping search (octrees): per node in the reference's breadth-first order, its box (6 doubles),
@@ -81,7 +89,6 @@ struct TreeView {
     const int32_t* bkchild0;
     const int32_t* bkfather;
     const int32_t* bkcell;
-    const int32_t* rope64;           // per cell 8 words: what lies across walls -x +x -y +y -z +z
     const int32_t* nboff;            // CSR offsets, index cell*6 + wall
     const int32_t* nbids;            // neighbour cell numbers
     int32_t nnodes, ncells;

@@ -92,9 +92,8 @@ struct sg_grid {
     sg::CartView cart{};
     // tree
     sg::HostTree ht;
-    sg::DevBuf node, rec64, node32, cellof, kpack, rope64, nboff, nbids, bkb, bkchild0, bkfather, bkcell;
+    sg::DevBuf node, rec64, node32, cellof, kpack, node64, nboff, nbids, bkb, bkchild0, bkfather, bkcell;
     std::vector<sg::TreeRec64> hrec64;
-    std::vector<sg::TreeNode32> hnode32;
     sg::TreeView tree{};
     // Voronoi
     sg::DevBuf site, voff, vnb, boff, bids, brep;

@@ -150,6 +150,42 @@ __global__ void k_resample_cart(const double* xv, const double* yv, const double
     rhof[m] = (float)r;
 }
 
+// FP64 walk records from a tree's mixed records, boxes and cell numbers.
+__global__ void __launch_bounds__(256) k_tree_nodes64(const TreeNode32* node32, const TreeRec64* rec, const int32_t* cellof,
+                                                      int32_t nnodes, int arity, TreeNode64* out)
+{
+    const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (n >= nnodes) return;
+    const TreeNode32 f = node32[n];
+    TreeNode64 r{};
+    if (f.code & kTreeLeaf) {
+        const int32_t c = cellof[n];
+        for (int a = 0; a < 3; a++) { r.lo[a] = rec[c].lo[a]; r.hi[a] = rec[c].hi[a]; }
+        r.rho = rec[c].rho;
+        for (int w = 0; w < 6; w++) r.rope[w] = f.rope[w];
+        r.cell = c;
+        r.child = -1;
+    } else {
+        for (int a = 0; a < 3; a++) r.lo[a] = (double)__int_as_float(f.rope[a]);
+        r.cell = -1 - (arity == 8 ? 0 : (int)((f.code >> 16) & 3u));
+        r.child = (int32_t)f.val;
+    }
+    out[n] = r;
+}
+
+// The cells' densities into a tree's records. (The host rewrote and sent all records, 96 bytes per cell and more: for
+// a system of several dust components at every change of wavelength.)
+__global__ void __launch_bounds__(256) k_tree_rho(const double* rho, int64_t ncells, TreeRec64* rec, TreeNode32* node32,
+                                                  TreeNode64* node64)
+{
+    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= ncells) return;
+    const int32_t n = rec[c].node;
+    rec[c].rho = rho[c];
+    node32[n].val = __float_as_uint((float)rho[c]);
+    node64[n].rho = rho[c];
+}
+
 __global__ void k_whichcell_cart(const CartView g, int64_t n, const double* r, int32_t* out)
 {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -395,7 +431,7 @@ int sg_grid_create_tree(int arity, const double ext[6], const uint8_t* subdivide
     for (int64_t l = 0; l < nn; l++) words[nid[l]] = h.child0[l] >= 0 ? nid[h.child0[l]] : -(h.cellnumber[l] + 1);
     g->node.upload(words);
     g->hrec64.assign(nc, TreeRec64{});
-    g->hnode32.assign(ndev, TreeNode32{});
+    std::vector<TreeNode32> hnode32(ndev, TreeNode32{});
     std::vector<int32_t> off(nc * 6 + 1, 0), ids;
     for (int64_t c = 0; c < nc; c++) {
         int l = h.idv[c];
@@ -414,12 +450,6 @@ int sg_grid_create_tree(int arity, const double ext[6], const uint8_t* subdivide
     std::vector<uint64_t> kpack(ndev, 0);
     std::vector<int32_t> ropes;
     h.build_ropes(ropes);
-    std::vector<int32_t> rope64(8 * (size_t)nc, kNoRope);
-    for (int64_t c = 0; c < nc; c++)
-        for (int w = 0; w < 6; w++) {
-            const int32_t r = ropes[6 * (size_t)h.idv[c] + w];
-            if (r >= 0) rope64[8 * (size_t)c + w] = h.child0[r] < 0 ? h.cellnumber[r] : ~nid[r];
-        }
     std::vector<uint32_t> nsub(nn, 0);   // nx | ny << 5 | nz << 10
     for (int64_t l = 0; l < nn; l++) {
         const int32_t c0 = h.child0[l];
@@ -454,7 +484,7 @@ int sg_grid_create_tree(int arity, const double ext[6], const uint8_t* subdivide
         uint32_t nx = nsub[l] & 31u, ny = (nsub[l] >> 5) & 31u, nz = (nsub[l] >> 10) & 31u;
         SG_REQUIRE(nx <= 21 && ny <= 21 && nz <= 21,
                    "tree too deep for the mixed-precision records (21 subdivisions per axis)");
-        TreeNode32& f = g->hnode32[nid[l]];
+        TreeNode32& f = hnode32[nid[l]];
         const bool leaf = h.child0[l] < 0;
         f.code = nsub[l] | (leaf ? kTreeLeaf : 0u) | ((uint32_t)(leaf ? 0 : h.dir[l]) << 16);
         f.val = leaf ? 0u : (uint32_t)nid[h.child0[l]];
@@ -492,21 +522,25 @@ int sg_grid_create_tree(int arity, const double ext[6], const uint8_t* subdivide
     }
     g->cellof.upload(cellof);
     g->kpack.upload(kpack);
-    g->rope64.upload(rope64);
     off[nc * 6] = (int32_t)ids.size();
     SG_REQUIRE(ids.size() < ((size_t)1 << 31), "neighbour lists too long");
     g->nboff.upload(off);
     if (ids.empty()) ids.push_back(-1);
     g->nbids.upload(ids);
     g->rec64.upload(g->hrec64);
-    g->node32.upload(g->hnode32);
+    g->node32.upload(hnode32);
     TreeView& t = g->tree;
     t.node = g->node.as<int32_t>();
     t.rec64 = g->rec64.as<TreeRec64>();
     t.node32 = g->node32.as<TreeNode32>();
+    g->node64.alloc((size_t)ndev * sizeof(TreeNode64));
+    t.node64 = g->node64.as<TreeNode64>();
+    hipLaunchKernelGGL(k_tree_nodes64, dim3((unsigned)((ndev + 255) / 256)), dim3(256), 0, 0, t.node32, t.rec64,
+                       g->cellof.as<int32_t>(), (int32_t)ndev, arity, g->node64.as<TreeNode64>());
+    SG_HIP(hipGetLastError());
+    SG_HIP(hipStreamSynchronize(0));   // the walks run on streams that do not wait for this one
     t.cellof = g->cellof.as<int32_t>();
     t.kpack = g->kpack.as<uint64_t>();
-    t.rope64 = g->rope64.as<int32_t>();
     t.nboff = g->nboff.as<int32_t>();
     t.nbids = g->nbids.as<int32_t>();
     t.nnodes = (int32_t)ndev; t.ncells = (int32_t)nc;
@@ -679,13 +713,12 @@ void sg_grid::set_rho(const double* r)
         std::vector<float> f(r, r + ncells);
         SG_HIP(hipMemcpy(rhof.p, f.data(), ncells * sizeof(float), hipMemcpyHostToDevice));
     } else if (kind == GK_TREE) {
-        for (int64_t c = 0; c < ncells; c++) {
-            hrec64[c].rho = r[c];
-            float f = (float)r[c];
-            std::memcpy(&hnode32[hrec64[c].node].val, &f, sizeof f);
-        }
-        SG_HIP(hipMemcpy(rec64.p, hrec64.data(), ncells * sizeof(TreeRec64), hipMemcpyHostToDevice));
-        SG_HIP(hipMemcpy(node32.p, hnode32.data(), hnode32.size() * sizeof(TreeNode32), hipMemcpyHostToDevice));
+        if (rho.bytes < ncells * sizeof(double)) rho.alloc(ncells * sizeof(double));
+        SG_HIP(hipMemcpy(rho.p, r, ncells * sizeof(double), hipMemcpyHostToDevice));
+        hipLaunchKernelGGL(k_tree_rho, dim3((unsigned)((ncells + 255) / 256)), dim3(256), 0, 0, rho.as<double>(), ncells,
+                           rec64.as<TreeRec64>(), node32.as<TreeNode32>(), node64.as<TreeNode64>());
+        SG_HIP(hipGetLastError());
+        SG_HIP(hipStreamSynchronize(0));
     } else {
         for (int64_t c = 0; c < ncells; c++) hsite[c].rho = r[c];
         SG_HIP(hipMemcpy(site.p, hsite.data(), ncells * sizeof(VoroSite), hipMemcpyHostToDevice));

@@ -571,85 +571,62 @@ struct Entry {
 // Both methods move the point just across the exit wall and look for the leaf that holds it: in the wall's list of
 // neighbours (closed boxes), or from the root. A point strictly inside a leaf lies in no other leaf's closed box and
 // on no plane of the descent, so that leaf is what either search returns, and the walk may find it as it likes. It
-// tries the node across the wall first (`rope64`: a leaf's cell number, or an internal node that is descended by the
-// FP32 split planes of the mixed records), and takes the leaf it reaches if its FP64 box strictly holds the point;
-// points on a wall, and the few that an edge or the FP32 planes send elsewhere, go through the searches themselves.
-// Bound by the latency of dependent loads: the searches took three of them per crossing (list bounds, list, boxes) and
-// about seven cache lines, a leaf of the same size or a larger one now takes one.
+// goes to the node across the wall (its rope) and down from there, one node record per step, so that every lane of a
+// wave loads one record per iteration, and takes the leaf it reaches if the leaf's box strictly holds the point;
+// points on a wall, and the few that an edge or the records' FP32 split planes send elsewhere, go through the searches
+// themselves. Bound by the latency of dependent loads: the searches took three of them per crossing (list bounds, list,
+// boxes) and about seven cache lines, a record is one line (3e5 packets, optical depth 5: 22.7 ms by the searches,
+// 14.9 ms with boxes and ropes in two lines and the descent as a loop inside the step, 13.0 ms now).
 struct TreeW64 {
     using Real = double;
     using View = TreeView;
     double x, y, z, kx, ky, kz, ix, iy, iz;
     double ex, ey, ez;       // the current cell's walls ahead
-    int qx, qy, qz;          // what lies across them (rope64)
+    int qx, qy, qz;          // the nodes across them
+    int down, wall;          // the node a descent has come to or -1, the wall that it started from
     double rho;
     int m, lm;               // current cell, cell of the last segment returned
     Entry en;
     bool done;
     uint32_t steps, nrecompute, nstuck;
-    static constexpr int kParkWords = 42;
+    static constexpr int kParkWords = 44;
     __device__ __forceinline__ static int cell_of(const View&, int n) { return n; }
     static constexpr bool kHint = true;
     static constexpr int kLanes = 1;
     static constexpr bool kLocates = false;
     __device__ __forceinline__ int entries() const { return en.ne; }
-    static constexpr bool kStep = false;   // next() only
     template <class P> __device__ __forceinline__ void park(P& p)
     {
         p.io(x); p.io(y); p.io(z); p.io(kx); p.io(ky); p.io(kz); p.io(ix); p.io(iy); p.io(iz);
-        p.io(ex); p.io(ey); p.io(ez); p.io(qx); p.io(qy); p.io(qz);
+        p.io(ex); p.io(ey); p.io(ez); p.io(qx); p.io(qy); p.io(qz); p.io(down); p.io(wall);
         p.io(rho); p.io(m); p.io(lm); p.io(en.ne); p.io(en.e0); p.io(en.e1); p.io(en.e2);
         p.io(done); p.io(steps); p.io(nrecompute); p.io(nstuck);
     }
 
-    // Makes c, with the box lo, hi, the current cell.
-    __device__ __forceinline__ void enter(const View& t, int c, double lx, double ly, double lz, double hx, double hy,
-                                          double hz, double density)
+    // Makes c the current cell: its walls ahead and the nodes across them.
+    __device__ __forceinline__ void enter(int c, double lx, double ly, double lz, double hx, double hy, double hz,
+                                          double density, int4 ra, int2 rb)
     {
-        const int4* q = reinterpret_cast<const int4*>(t.rope64) + 2 * (size_t)c;
-        const int4 qa = q[0], qb = q[1];
         const bool bx = kx < 0.0, by = ky < 0.0, bz = kz < 0.0;
         ex = bx ? lx : hx; ey = by ? ly : hy; ez = bz ? lz : hz;
-        qx = bx ? qa.x : qa.y; qy = by ? qa.z : qa.w; qz = bz ? qb.x : qb.y;
+        qx = bx ? ra.x : ra.y; qy = by ? ra.z : ra.w; qz = bz ? rb.x : rb.y;
         rho = density;
         m = c;
+        down = -1;
     }
     __device__ __forceinline__ void load_cell(const View& t, int c)
     {
-        const TreeRec64& r = t.rec64[c];
+        const TreeNode64& r = t.node64[t.rec64[c].node];
         const double lx = r.lo[0], ly = r.lo[1], lz = r.lo[2], hx = r.hi[0], hy = r.hi[1], hz = r.hi[2];
-        enter(t, c, lx, ly, lz, hx, hy, hz, r.rho);
-    }
-    // The leaf strictly holding the point among those below `q`, what lies across the wall just crossed.
-    __device__ __forceinline__ bool follow(const View& t, int q)
-    {
-        if (q == kNoRope) return false;
-        while (q < 0) {
-            const TreeNode32& n = t.node32[~q];
-            const float fx = (float)x, fy = (float)y, fz = (float)z;
-            const float p0 = __int_as_float(n.rope[0]);
-            int k;
-            if (t.arity == 8)
-                k = (fx < p0 ? 0 : 1) + (fy < __int_as_float(n.rope[1]) ? 0 : 2) + (fz < __int_as_float(n.rope[2]) ? 0 : 4);
-            else {
-                const int a = (n.code >> 16) & 3;
-                k = pick3(a == 1, a == 2, fx, fy, fz) < p0 ? 0 : 1;
-            }
-            const int child = (int)n.val + k, c = t.cellof[child];
-            q = c >= 0 ? c : ~child;
-        }
-        const TreeRec64& r = t.rec64[q];
-        const double lx = r.lo[0], ly = r.lo[1], lz = r.lo[2], hx = r.hi[0], hy = r.hi[1], hz = r.hi[2];
-        if (!(x > lx && x < hx && y > ly && y < hy && z > lz && z < hz)) return false;
-        enter(t, q, lx, ly, lz, hx, hy, hz, r.rho);
-        return true;
+        enter(c, lx, ly, lz, hx, hy, hz, r.rho, make_int4(r.rope[0], r.rope[1], r.rope[2], r.rope[3]),
+              make_int2(r.rope[4], r.rope[5]));
     }
     __device__ __forceinline__ bool descend(const View& t, const int32_t* lds, int nlds)
     {
         double l[3], h[3];
         int c = descend64(t, lds, nlds, x, y, z, l, h);
         if (c < 0) return false;
-        enter(t, c, l[0], l[1], l[2], h[0], h[1], h[2], t.rec64[c].rho);
+        load_cell(t, c);
         return true;
     }
     __device__ __forceinline__ void set_direction(double dx, double dy, double dz)
@@ -700,50 +677,87 @@ struct TreeW64 {
         }
         init(t, lds, nlds, rx, ry, rz, dx, dy, dz);
     }
-    __device__ __forceinline__ bool next(const View& t, const int32_t* lds, int nlds, int& mo, double& ds,
-                                         double& rh)
+    // The searches themselves for the cell across `wall` of cell m, and the walk's end where there is none.
+    __device__ __forceinline__ void search(const View& t, const int32_t* lds, int nlds)
+    {
+        const int oldm = m;
+        down = -1;
+        bool found = false;
+        if (t.search == 1) {
+            int i0 = t.nboff[oldm * 6 + wall], i1 = t.nboff[oldm * 6 + wall + 1];
+            for (int q = i0; q < i1; q++) {
+                int c = t.nbids[q];
+                const TreeRec64& r = t.rec64[c];
+                if (x >= r.lo[0] && x <= r.hi[0] && y >= r.lo[1] && y <= r.hi[1] && z >= r.lo[2] && z <= r.hi[2]) {
+                    load_cell(t, c);
+                    found = true;
+                    break;
+                }
+            }
+        }
+        if (!found) found = descend(t, lds, nlds);
+        if (!found) done = true;
+        else if (m == oldm) {
+            nstuck++;
+            x = nextafter(x, (kx < 0.0) ? -DBL_MAX : DBL_MAX);
+            y = nextafter(y, (ky < 0.0) ? -DBL_MAX : DBL_MAX);
+            z = nextafter(z, (kz < 0.0) ? -DBL_MAX : DBL_MAX);
+            if (!descend(t, lds, nlds)) done = true;
+            else if (m == oldm) done = true;
+        }
+    }
+    // One wall step, whose segment may have no length, or one level of the descent to the leaf behind that wall (length
+    // zero); false at the end of the path.
+    static constexpr bool kStep = true;
+    __device__ __forceinline__ bool step(const View& t, const int32_t* lds, int nlds, int& mo, double& ds, double& rh)
     {
         if (en.ne) { ds = en.pop(); mo = -1; rh = 0.0; return true; }
-        while (!done) {
+        if (done) return false;
+        mo = m; rh = rho; ds = 0.0;
+        int n = down;
+        if (n < 0) {
             double dsx = ix != 0.0 ? quotient(ex - x, kx, ix) : DBL_MAX;
             double dsy = iy != 0.0 ? quotient(ey - y, ky, iy) : DBL_MAX;
             double dsz = iz != 0.0 ? quotient(ez - z, kz, iz) : DBL_MAX;
-            int a = choose_axis_tree(dsx, dsy, dsz);
-            double d = pick3(a == 1, a == 2, dsx, dsy, dsz);
-            int wall = 2 * a + (pick3(a == 1, a == 2, kx, ky, kz) < 0.0 ? 0 : 1);
-            int segm = m;
-            double segrho = rho;
-            x += (d + t.eps) * kx;
-            y += (d + t.eps) * ky;
-            z += (d + t.eps) * kz;
-            int oldm = m;
-            bool found = follow(t, pick3(a == 1, a == 2, qx, qy, qz));
-            if (!found && t.search == 1) {
-                int i0 = t.nboff[oldm * 6 + wall], i1 = t.nboff[oldm * 6 + wall + 1];
-                for (int q = i0; q < i1; q++) {
-                    int c = t.nbids[q];
-                    const TreeRec64& r = t.rec64[c];
-                    if (x >= r.lo[0] && x <= r.hi[0] && y >= r.lo[1] && y <= r.hi[1] && z >= r.lo[2] &&
-                        z <= r.hi[2]) {
-                        load_cell(t, c);
-                        found = true;
-                        break;
-                    }
-                }
-            }
-            if (!found) found = descend(t, lds, nlds);
-            if (!found) done = true;
-            else if (m == oldm) {
-                nstuck++;
-                x = nextafter(x, (kx < 0.0) ? -DBL_MAX : DBL_MAX);
-                y = nextafter(y, (ky < 0.0) ? -DBL_MAX : DBL_MAX);
-                z = nextafter(z, (kz < 0.0) ? -DBL_MAX : DBL_MAX);
-                if (!descend(t, lds, nlds)) done = true;
-                else if (m == oldm) done = true;
-            }
-            if (++steps > SG_MAX_STEPS) done = true;
-            if (d > 0) { mo = segm; ds = d; rh = segrho; lm = segm; return true; }
+            const int a = choose_axis_tree(dsx, dsy, dsz);
+            ds = pick3(a == 1, a == 2, dsx, dsy, dsz);
+            wall = 2 * a + (pick3(a == 1, a == 2, kx, ky, kz) < 0.0 ? 0 : 1);
+            n = pick3(a == 1, a == 2, qx, qy, qz);
+            x += (ds + t.eps) * kx;
+            y += (ds + t.eps) * ky;
+            z += (ds + t.eps) * kz;
+            lm = ds > 0 ? m : lm;
+            steps++;
         }
+        bool found = false;
+        if (n >= 0) {
+            const TreeNode64& r = t.node64[n];
+            const double lx = r.lo[0], ly = r.lo[1], lz = r.lo[2], hx = r.hi[0], hy = r.hi[1], hz = r.hi[2], density = r.rho;
+            const int4 ra = make_int4(r.rope[0], r.rope[1], r.rope[2], r.rope[3]);
+            const int2 rb = make_int2(r.rope[4], r.rope[5]);
+            const int c = r.cell, c0 = r.child;
+            if (c >= 0) {
+                if ((x > lx) & (x < hx) & (y > ly) & (y < hy) & (z > lz) & (z < hz)) {
+                    enter(c, lx, ly, lz, hx, hy, hz, density, ra, rb);
+                    found = true;
+                }
+            } else {
+                // an internal node: split planes for its box, the split axis of a binary one in its cell number; children
+                // have higher ids than their parent, so a descent ends
+                if (t.arity == 8) down = c0 + (x < lx ? 0 : 1) + (y < ly ? 0 : 2) + (z < lz ? 0 : 4);
+                else down = c0 + (pick3(c == -2, c == -3, x, y, z) < lx ? 0 : 1);
+                found = down > n;
+            }
+        }
+        if (!found) search(t, lds, nlds);
+        if (steps > SG_MAX_STEPS) done = true;
+        return true;
+    }
+    // The next segment of positive length.
+    __device__ __forceinline__ bool next(const View& t, const int32_t* lds, int nlds, int& mo, double& ds, double& rh)
+    {
+        while (step(t, lds, nlds, mo, ds, rh))
+            if (ds > 0) return true;
         return false;
     }
 };
