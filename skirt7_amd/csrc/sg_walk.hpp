@@ -954,9 +954,16 @@ struct TreeW32 {
     {
         const bool nx = kx < 0.0f, ny = ky < 0.0f, nz = kz < 0.0f;
         const uint32_t ns = a.x & 0x7fffu;
-        const float wx = ldexpf(t.widthf[0], -(int)(ns & 31u));
-        const float wy = ldexpf(t.widthf[1], -(int)((ns >> 5) & 31u));
-        const float wz = ldexpf(t.widthf[2], -(int)((ns >> 10) & 31u));
+        float wx, wy, wz;
+        if (t.arity == 8) {
+            // one count for the three axes: 2^-n by its exponent bits (n is at most 21)
+            const float s = __uint_as_float((127u - (ns & 31u)) << 23);
+            wx = t.widthf[0] * s; wy = t.widthf[1] * s; wz = t.widthf[2] * s;
+        } else {
+            wx = ldexpf(t.widthf[0], -(int)(ns & 31u));
+            wy = ldexpf(t.widthf[1], -(int)((ns >> 5) & 31u));
+            wz = ldexpf(t.widthf[2], -(int)((ns >> 10) & 31u));
+        }
         px = fmaf((float)(nx ? i : i + 1), wx, t.extf[0]);
         py = fmaf((float)(ny ? j : j + 1), wy, t.extf[1]);
         pz = fmaf((float)(nz ? k : k + 1), wz, t.extf[2]);
@@ -979,9 +986,8 @@ struct TreeW32 {
     {
         // upper child: beyond the plane, or on it while heading up (bitwise forms stay in mask registers)
         const bool ux = !(kx < 0.0f), uy = !(ky < 0.0f), uz = !(kz < 0.0f);
-        int level = 0;
+        // ends: children are deeper than their parent, and no node is deeper than 63 levels
         while (!(a.x & kTreeLeaf)) {
-            if (++level > 128) { done = true; return; }   // no tree the records describe is this deep
             const int c0 = (int)a.y;
             if (t.arity == 8) {
                 // split planes ext + (2k + 1) * width / 2^(n + 1), held by the internal node's record
@@ -1176,7 +1182,7 @@ struct TreeW32 {
             fy = !fx && ddy <= ddz;
             d = (float)(fx ? ddx : fy ? ddy : ddz);
         }
-        const float dd = d > 0.0f ? d : 0.0f;   // a select: fmaxf would first canonicalize d
+        const float dd = __builtin_amdgcn_fmed3f(d, 0.0f, FLT_MAX);   // d > 0 ? d : 0 in one instruction
         const bool fz = !fx && !fy;
         x = fx ? px : fmaf(kx, dd, x);
         y = fy ? py : fmaf(ky, dd, y);
@@ -1219,7 +1225,7 @@ struct TreeW32 {
             const int32_t i = (ci + (fx ? (kx < 0.0f ? -1 : 1) : 0)) >> (dn & 31u);
             const int32_t j = (cj + (fy ? (ky < 0.0f ? -1 : 1) : 0)) >> ((dn >> 5) & 31u);
             const int32_t k = (ck + (fz ? (kz < 0.0f ? -1 : 1) : 0)) >> ((dn >> 10) & 31u);
-            if (on >= 0.0f) descend_loaded(t, a, b, r, i, j, k);
+            if (on >= 0.0f) descend_loaded(t, a, b, r, i, j, k);   // never the leaf itself, which lies before the wall
             else {
                 const int xa = fx ? 0 : fy ? 1 : 2;
                 const float ka = fx ? kx : fy ? ky : kz;
@@ -1227,8 +1233,8 @@ struct TreeW32 {
                 const int n = descend_root(t, lds, nlds, xa, ka < 0.0f ? -1 : 1, i2, j2, k2);
                 if (n < 0) done = true;
                 else descend_from(t, n, i2, j2, k2);
+                if (!done && m == segm) { nstuck++; done = true; }
             }
-            if (!done && m == segm) { nstuck++; done = true; }
         }
         if (++steps > SG_MAX_STEPS) done = true;
         mo = segm; ds = d; rh = segrho;
