@@ -170,8 +170,9 @@ int sg_sim_run_static(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64
                       uint64_t* counters);
 /* Batched population (one persistent launch over many members, each its own simulation on a
  * grid of the same kind): member i runs packets [0, counts[i]) at wavelength ells[i]. With the
- * event/walk pipeline selected, members of at least sg_set_batch_alone packets run one at a time
- * through it and the rest share the persistent launches; each member's result is its single run. */
+ * event/walk pipeline selected, members of at least sg_set_batch_alone packets run through it, a few at
+ * a time on streams of their own, and the rest share the persistent launches; each member's result is its
+ * single run. */
 int sg_sim_run_batch(int nmembers, sg_sim* const* sims, const int* ells, const uint64_t* counts, int precision,
                      uint64_t* counters);
 /* ---- PanMonteCarloSimulation: dust emission (PanMonteCarloSimulation.cpp:106-340) ------------------- */
@@ -270,8 +271,8 @@ int sg_set_slots(int64_t slots);
  * removed again (frames and absorption as before). */
 int sg_autotune(sg_sim* s, int ell, uint64_t first, uint64_t sample, int precision, int choose_pipeline,
                 int64_t* best, double* rate);
-/* Smallest member (packets) that sg_sim_run_batch runs alone through the event/walk pipeline
- * instead of in the shared persistent launch (0 = never; default 2^21). */
+/* Smallest member (packets) that sg_sim_run_batch runs by passes of its own through the event/walk
+ * pipeline instead of in the shared persistent launch (0 = never; default 3 * 2^16). */
 int sg_set_batch_alone(uint64_t min_packets);
 /* Mixed-precision walks of trees built with the TopDown search method: 0 (default) follow the ropes
  * between leaves, as for Neighbor trees (the same cells: the search method only decides how the next

@@ -29,7 +29,10 @@ static int g_cus = 256;
 static int g_tune_block = 256, g_tune_waves = 0, g_tune_compact = 0;
 static int64_t g_tune_slots = 0;   // in-flight packet slots of the event/walk pipeline (0: its default)
 static int g_pipeline = 1;   // 0: persistent lane pipeline (k_mc); 1: event and walk kernels (k_events/k_walks)
-static uint64_t g_batch_alone = (uint64_t)1 << 21;   // batched members this large run alone (0: never)
+// Batched members this large take their own passes (0: never), four at a time. 24 galaxies of 1e5 to 1e6 packets on 96^3
+// cells, by threshold, ms: 2^21 (none) 82.6, 2^16 65.8, 3 * 2^16 60.6, 2^18 61.1, 2^19 65.5; 24 of 2e4 to 2e5: none
+// 21.7, 2^16 24.8, 3 * 2^16 21.5.
+static uint64_t g_batch_alone = (uint64_t)3 << 16;
 static int g_topdown_descent = 0;   // 1: mixed walks of TopDown trees descend from the root at every step
 static int g_walk_order = 0;        // 1: the walk kernel takes each pass's walks in coherence-key order; 2: so,
                                     // claimed by XCD segment
@@ -1386,17 +1389,18 @@ static const uint64_t kSplitEmit = (uint64_t)1 << 25;   // packets emitted at on
 static const int kSplitAhead = 3;
 static const int kProgressRing = 8;                     // progress words per group (more than are in flight)
 
-// Two non-blocking streams of default priority, one per slot group, and their progress words, which the walk
-// kernels write into coherent host memory.
-static hipStream_t g_split_stream[2] = {nullptr, nullptr};
+// Non-blocking streams of default priority, one per slot group of a run or per member of a batched run, and their
+// progress words, which the walk kernels write into coherent host memory.
+static const int kStreams = 4;
+static hipStream_t g_split_stream[kStreams] = {};
 static unsigned long long* g_split_host = nullptr;
 static unsigned long long* g_split_host_dev = nullptr;
 static double g_clock_khz = 100000.0;                   // of the device's wall clock
-// A run's scene on its way to the device and its result on the way back, in pinned host memory, and the event that
-// joins the two streams.
+// Per stream: a run's scene on its way to the device and its result on the way back, in pinned host memory; and the
+// event that joins the two streams.
 struct RunHost {
-    SceneDev scene;
-    RunResult result;
+    SceneDev scene[kStreams];
+    RunResult result[kStreams];
 };
 static RunHost* g_run_host = nullptr;
 static RunHost* g_run_host_dev = nullptr;
@@ -1405,10 +1409,11 @@ static hipEvent_t g_split_join = nullptr;
 // (runs are synchronous and driven by one host thread): slot groups, walk queues, progress counters,
 // launch states. Allocated on first use, grown as needed, kept until the process ends.
 struct SplitPool {
-    DevBuf slots[2], queue[2], prog[2], events[2], waves[2], emitted, emitdraw, emithint;
-    DevBuf run;       // a run's start on the device clock and its end's ticket
+    DevBuf slots[kStreams], queue[kStreams], prog[kStreams], events[kStreams], waves[kStreams];
+    DevBuf emitted[kStreams], emitdraw[kStreams], emithint[kStreams];
+    DevBuf run;       // per group: a run's start on the device clock and its end's ticket
     DevBuf cells;     // dust emission: cumulative and own luminosities of the cells
-    DevBuf bins[2];   // per group: bin counts (zero between passes: cleared once, then by each pass's scan), offsets
+    DevBuf bins[kStreams];   // per group: bin counts (zero between passes: cleared once, then by each pass's scan), offsets
 };
 static SplitPool* g_pool = nullptr;
 static SplitPool& pool()
@@ -1420,8 +1425,8 @@ static SplitPool& pool()
 static void split_resources()
 {
     if (g_split_stream[0]) return;
-    for (int g = 0; g < 2; g++) SG_HIP(hipStreamCreateWithFlags(&g_split_stream[g], hipStreamNonBlocking));
-    SG_HIP(hipHostMalloc(reinterpret_cast<void**>(&g_split_host), 2 * kProgressRing * sizeof(unsigned long long),
+    for (int g = 0; g < kStreams; g++) SG_HIP(hipStreamCreateWithFlags(&g_split_stream[g], hipStreamNonBlocking));
+    SG_HIP(hipHostMalloc(reinterpret_cast<void**>(&g_split_host), kStreams * kProgressRing * sizeof(unsigned long long),
                          hipHostMallocMapped | hipHostMallocCoherent));
     SG_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&g_split_host_dev), g_split_host, 0));
     SG_HIP(hipHostMalloc(reinterpret_cast<void**>(&g_run_host), sizeof(RunHost), hipHostMallocMapped | hipHostMallocCoherent));
@@ -1454,15 +1459,41 @@ static unsigned long long wait_progress(const unsigned long long* word, hipStrea
 // The slot groups of a run of the event/walk pipeline, and the launch shapes of its kernels.
 template <typename R> struct PassGroups {
     int n;
-    Slots<R> sl[2];
-    WalkQueue<R> q[2];
-    GroupCtl* ctl[2];
-    GroupTally tally[2];
-    int pass[2];                // passes enqueued so far (the place in the progress rings)
+    Slots<R> sl[kStreams];
+    WalkQueue<R> q[kStreams];
+    GroupCtl* ctl[kStreams];
+    GroupTally tally[kStreams];
+    int pass[kStreams];         // passes enqueued so far (the place in the progress rings)
     int blocks, bs, nlds, order;
     size_t shm;
 };
 static int64_t event_blocks(int64_t slots) { return (slots + kEventBlock - 1) / kEventBlock; }
+
+// Enqueues group g's next event and walk pass on its stream; `first`: the slots take their packets by their numbers.
+template <class W, bool ABS, bool MULTI>
+static void enqueue_pass(const typename W::View& v, const McArgs& ab, PassGroups<typename W::Real>& pg, int g, bool first)
+{
+    using R = typename W::Real;
+    const hipStream_t st = g_split_stream[g];
+    const int p = pg.pass[g]++;
+    const int w = g * kProgressRing + p % kProgressRing;
+    __atomic_store_n(g_split_host + w, 0ull, __ATOMIC_RELEASE);
+    PassCtl* pc = &pg.ctl[g]->pass[p % kPassRing];
+    WalkQueue<R> q = pg.q[g];
+    q.tail = &pc->tail;
+    const int64_t P = pg.sl[g].n;
+    hipLaunchKernelGGL((k_events<R, MULTI>), dim3(event_blocks(P) + 1), dim3(kEventBlock), 0, st, ab, pg.sl[g], q,
+                       pg.ctl[g], p, first ? 1 : 0, pg.tally[g]);
+    SG_HIP(hipGetLastError());
+    if (q.sorted) {
+        hipLaunchKernelGGL(k_key_scan, dim3(1), dim3(1024), 0, st, q.hist, q.off);
+        hipLaunchKernelGGL(k_key_scatter<R>, dim3(g_cus * 8), dim3(256), 0, st, q, ab.error);
+        SG_HIP(hipGetLastError());
+    }
+    hipLaunchKernelGGL((k_walks<W, ABS, MULTI>), dim3(pg.blocks), dim3(pg.bs), pg.shm, st, v, ab, q, pg.sl[g], pc,
+                       g_split_host_dev + w, pg.tally[g], pg.nlds, pg.order == 2 ? kXcdSegs : 0);
+    SG_HIP(hipGetLastError());
+}
 
 // Event and walk passes of every group until all packets of ab have been claimed and the groups' walk queues stay
 // empty. Each group keeps kSplitAhead passes enqueued beyond the one whose progress is awaited. Returns the
@@ -1476,26 +1507,7 @@ static int run_passes(const typename W::View& v, const McArgs& ab, PassGroups<ty
     bool done[2] = {false, pg.n < 2};
     int launches = 0;
     const int pass0[2] = {pg.pass[0], pg.pass[1]};
-    auto enqueue = [&](int g) {
-        const int p = pg.pass[g]++;
-        const int w = g * kProgressRing + p % kProgressRing;
-        __atomic_store_n(g_split_host + w, 0ull, __ATOMIC_RELEASE);
-        PassCtl* pc = &pg.ctl[g]->pass[p % kPassRing];
-        WalkQueue<R> q = pg.q[g];
-        q.tail = &pc->tail;
-        const int64_t P = pg.sl[g].n;
-        hipLaunchKernelGGL((k_events<R, MULTI>), dim3(event_blocks(P) + 1), dim3(kEventBlock), 0, st[g], ab, pg.sl[g], q,
-                           pg.ctl[g], p, p == pass0[g] ? 1 : 0, pg.tally[g]);
-        SG_HIP(hipGetLastError());
-        if (q.sorted) {
-            hipLaunchKernelGGL(k_key_scan, dim3(1), dim3(1024), 0, st[g], q.hist, q.off);
-            hipLaunchKernelGGL(k_key_scatter<R>, dim3(g_cus * 8), dim3(256), 0, st[g], q, ab.error);
-            SG_HIP(hipGetLastError());
-        }
-        hipLaunchKernelGGL((k_walks<W, ABS, MULTI>), dim3(pg.blocks), dim3(pg.bs), pg.shm, st[g], v, ab, q, pg.sl[g], pc,
-                           g_split_host_dev + w, pg.tally[g], pg.nlds, pg.order == 2 ? kXcdSegs : 0);
-        SG_HIP(hipGetLastError());
-    };
+    auto enqueue = [&](int g) { enqueue_pass<W, ABS, MULTI>(v, ab, pg, g, pg.pass[g] == pass0[g]); };
     while (!done[0] || !done[1]) {
         for (int i = 0; i < kSplitAhead; i++)
             for (int g = 0; g < pg.n; g++)
@@ -1540,12 +1552,12 @@ static void launch_emit_dust(const DustLaunch& dl, McArgs& a, void* emitted, uin
     SG_HIP(hipGetLastError());
 }
 
-// The run's start and end words on the device: clock ticks, ticket.
-static unsigned long long* run_words()
+// The start and end words of a run led by group g on the device: clock ticks, ticket.
+static unsigned long long* run_words(int g)
 {
     DevBuf& b = pool().run;
-    if (!b.bytes) b.alloc(2 * sizeof(unsigned long long));
-    return b.as<unsigned long long>();
+    if (!b.bytes) b.alloc(2 * kStreams * sizeof(unsigned long long));
+    return b.as<unsigned long long>() + 2 * g;
 }
 static void launch_end(const RunEnd& e, hipStream_t st)
 {
@@ -1566,11 +1578,112 @@ template <class W> static int slot_groups(int64_t ncells, int64_t P)
     return W::kLanes > 1 || (W::kHint && ncells >= (int64_t)1 << 19 && P >= (int64_t)1 << 17) ? 2 : 1;
 }
 
+// The launch shape of a run's walk kernels.
+template <class W, bool ABS, bool MULTI> static void pass_shape(PassGroups<typename W::Real>& pg, int nlds)
+{
+    pg.bs = g_tune_block;
+    pg.nlds = nlds;
+    pg.order = g_walk_order;
+    pg.shm = (size_t)nlds * sizeof(int32_t);
+    int per = 0;
+    SG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_walks<W, ABS, MULTI>, pg.bs, pg.shm));
+    pg.blocks = std::max(1, per) * g_cus;
+}
+static void zero_at_begin(RunBegin& rb, void* p, size_t bytes)
+{
+    rb.zero[rb.nzero++] = {static_cast<uint32_t*>(p), (int64_t)(bytes / 4)};
+}
+// Group g's work buffers for P slots, the first of them slot0, and what the run's start has to clear in them:
+// progress and count records zero, slot states PS_FRESH.
+template <typename R> static void group_buffers(PassGroups<R>& pg, int g, int64_t P, int64_t slot0, int ni, RunBegin& rb)
+{
+    SplitPool& pl = pool();
+    const int64_t cap = P * (ni + 1);
+    const bool sorted = pg.order != 0;
+    if (pl.slots[g].bytes < slot_bytes<R>(P)) pl.slots[g].alloc(slot_bytes<R>(P));
+    if (pl.queue[g].bytes < queue_bytes<R>(cap, sorted)) pl.queue[g].alloc(queue_bytes<R>(cap, sorted));
+    if (sorted && pl.bins[g].bytes == 0) {
+        pl.bins[g].alloc(2 * (size_t)kKeyBins * sizeof(uint32_t));
+        SG_HIP(hipMemsetAsync(pl.bins[g].p, 0, kKeyBins * sizeof(uint32_t), g_split_stream[g]));
+    }
+    if (pl.prog[g].bytes < sizeof(GroupCtl)) pl.prog[g].alloc(sizeof(GroupCtl));
+    pg.ctl[g] = pl.prog[g].as<GroupCtl>();
+    pg.sl[g] = Slots<R>{pl.slots[g].as<R>(),
+                        reinterpret_cast<uint32_t*>(pl.slots[g].as<unsigned char>() + (size_t)P * SR_NR * sizeof(R)), P};
+    // requests, then (sorted order) the sorted requests, keys, ranks, bin counts and offsets
+    unsigned char* qb = pl.queue[g].as<unsigned char>();
+    WalkQueue<R>& q = pg.q[g];
+    q.req = reinterpret_cast<WalkReq<R>*>(qb);
+    q.cap = cap;
+    if (sorted) {
+        unsigned char* p = qb + (size_t)cap * sizeof(WalkReq<R>);
+        q.sorted = reinterpret_cast<WalkReq<R>*>(p);
+        p += (size_t)cap * sizeof(WalkReq<R>);
+        q.key = reinterpret_cast<uint32_t*>(p);
+        q.rank = q.key + cap;
+        q.hist = pl.bins[g].as<uint32_t>();
+        q.off = q.hist + kKeyBins;
+    }
+    GroupTally& ta = pg.tally[g];
+    ta.nevents = event_blocks(P);
+    ta.nwaves = pg.blocks * (pg.bs / 64);
+    ta.slot0 = slot0;
+    const size_t ebytes = (size_t)ta.nevents * 4 * sizeof(unsigned long long), wbytes = (size_t)ta.nwaves * sizeof(WaveRec);
+    if (pl.events[g].bytes < ebytes) pl.events[g].alloc(ebytes);
+    if (pl.waves[g].bytes < wbytes) pl.waves[g].alloc(wbytes);
+    ta.events = pl.events[g].as<unsigned long long>();
+    ta.waves = pl.waves[g].as<WaveRec>();
+    zero_at_begin(rb, pg.ctl[g], sizeof(GroupCtl));
+    zero_at_begin(rb, ta.events, ebytes);
+    zero_at_begin(rb, ta.waves, wbytes);
+    zero_at_begin(rb, pg.sl[g].u + (size_t)SU_STATE * P, (size_t)P * sizeof(uint32_t));
+}
+// The run's start on group g's stream: what it clears, the packet claims, and the scene from pinned memory.
+static void launch_begin(RunBegin& rb, const McArgs& a, sg_sim* s, int g, int64_t P)
+{
+    unsigned long long* words = run_words(g);
+    zero_at_begin(rb, a.counters, SG_NCOUNTERS * sizeof(unsigned long long));
+    zero_at_begin(rb, a.error, sizeof(int));
+    zero_at_begin(rb, words + 1, sizeof(unsigned long long));
+    rb.scene_host = reinterpret_cast<const uint32_t*>(&g_run_host_dev->scene[g]);
+    rb.scene = s->scene.as<uint32_t>();
+    rb.next = s->next.as<unsigned long long>();
+    // the slots take a batch's first packets by their numbers, the others are claimed
+    rb.first_claim = (unsigned long long)P;
+    rb.begin = words;
+    int64_t most = 1;
+    for (int k = 0; k < rb.nzero; k++) most = std::max(most, rb.zero[k].words);
+    hipLaunchKernelGGL(k_run_begin, dim3((unsigned)std::min<int64_t>((most + 1023) / 1024, (int64_t)g_cus * 4)), dim3(256), 0,
+                       g_split_stream[g], rb);
+    SG_HIP(hipGetLastError());
+}
+// The launch states' buffers of group g for `batch` packets.
+template <class W> static void emission_buffers(int g, uint64_t batch)
+{
+    SplitPool& pl = pool();
+    const size_t rsz = sizeof(typename W::Real);
+    if (pl.emitted[g].bytes < 7 * batch * rsz) pl.emitted[g].alloc(7 * batch * rsz);
+    if (pl.emitdraw[g].bytes < batch * sizeof(uint32_t)) pl.emitdraw[g].alloc(batch * sizeof(uint32_t));
+    if (W::kHint && pl.emithint[g].bytes < batch * sizeof(int32_t)) pl.emithint[g].alloc(batch * sizeof(int32_t));
+}
+// The run's end on group g0's stream, the groups g0 and up to g0 + n - 1 having ended.
+template <typename R> static void launch_result(const PassGroups<R>& pg, int g0, int n, const McArgs& a)
+{
+    RunEnd re{};
+    re.n = n;
+    for (int g = 0; g < n; g++) { re.tally[g] = pg.tally[g0 + g]; re.ctl[g] = pg.ctl[g0 + g]; }
+    re.counters = a.counters;
+    re.err = a.error;
+    re.begin = run_words(g0);
+    re.ticket = reinterpret_cast<unsigned int*>(run_words(g0) + 1);
+    re.out = &g_run_host_dev->result[g0];
+    launch_end(re, g_split_stream[g0]);
+}
+
 // What a run of the event/walk pipeline is given and returns beyond its result in g_run_host: dust emission instead of
-// the stars', whether the scene is to be taken from there, and the walk launches that had requests.
+// the stars', and the walk launches that had requests.
 struct SplitRun {
     const DustLaunch* dust = nullptr;
-    bool scene = true;
     int launches = 0;
 };
 // Packets [first, first+count) through event and walk passes over one slot group, or two that alternate on two
@@ -1588,83 +1701,15 @@ static void run_split(sg_sim* s, const typename W::View& v, const McArgs& a, uin
     PassGroups<R> pg{};
     const int G = pg.n = P >= 2 ? (g_slot_groups ? g_slot_groups : slot_groups<W>(a.ncells, P)) : 1;
     const int64_t Pg[2] = {G == 2 ? (P + 1) / 2 : P, G == 2 ? P / 2 : 0};
-    const int bs = pg.bs = g_tune_block;
-    pg.nlds = nlds;
-    pg.order = g_walk_order;
-    pg.shm = (size_t)nlds * sizeof(int32_t);
-    int per = 0;
-    SG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_walks<W, ABS, MULTI>, bs, pg.shm));
-    pg.blocks = blocks = std::max(1, per) * g_cus;
+    pass_shape<W, ABS, MULTI>(pg, nlds);
+    blocks = pg.blocks;
     RunBegin rb{};
-    auto zero = [&](void* p, size_t bytes) { rb.zero[rb.nzero++] = {static_cast<uint32_t*>(p), (int64_t)(bytes / 4)}; };
-    for (int g = 0; g < G; g++) {
-        const int64_t cap = Pg[g] * (a.ni + 1);
-        SplitPool& pl = pool();
-        const bool sorted = g_walk_order != 0;
-        if (pl.slots[g].bytes < slot_bytes<R>(Pg[g])) pl.slots[g].alloc(slot_bytes<R>(Pg[g]));
-        if (pl.queue[g].bytes < queue_bytes<R>(cap, sorted)) pl.queue[g].alloc(queue_bytes<R>(cap, sorted));
-        if (sorted && pl.bins[g].bytes == 0) {
-            pl.bins[g].alloc(2 * (size_t)kKeyBins * sizeof(uint32_t));
-            SG_HIP(hipMemsetAsync(pl.bins[g].p, 0, kKeyBins * sizeof(uint32_t), st[g]));
-        }
-        if (pl.prog[g].bytes < sizeof(GroupCtl)) pl.prog[g].alloc(sizeof(GroupCtl));
-        pg.ctl[g] = pl.prog[g].as<GroupCtl>();
-        Slots<R>& sl = pg.sl[g];
-        sl = Slots<R>{pl.slots[g].as<R>(),
-                      reinterpret_cast<uint32_t*>(pl.slots[g].as<unsigned char>() + (size_t)Pg[g] * SR_NR * sizeof(R)), Pg[g]};
-        // requests, then (sorted order) the sorted requests, keys, ranks, bin counts and offsets
-        unsigned char* qb = pl.queue[g].as<unsigned char>();
-        WalkQueue<R>& q = pg.q[g];
-        q.req = reinterpret_cast<WalkReq<R>*>(qb);
-        q.cap = cap;
-        if (sorted) {
-            unsigned char* p = qb + (size_t)cap * sizeof(WalkReq<R>);
-            q.sorted = reinterpret_cast<WalkReq<R>*>(p);
-            p += (size_t)cap * sizeof(WalkReq<R>);
-            q.key = reinterpret_cast<uint32_t*>(p);
-            q.rank = q.key + cap;
-            q.hist = pl.bins[g].as<uint32_t>();
-            q.off = q.hist + kKeyBins;
-        }
-        GroupTally& ta = pg.tally[g];
-        ta.nevents = event_blocks(Pg[g]);
-        ta.nwaves = pg.blocks * (pg.bs / 64);
-        ta.slot0 = g ? Pg[0] : 0;
-        const size_t ebytes = (size_t)ta.nevents * 4 * sizeof(unsigned long long), wbytes = (size_t)ta.nwaves * sizeof(WaveRec);
-        if (pl.events[g].bytes < ebytes) pl.events[g].alloc(ebytes);
-        if (pl.waves[g].bytes < wbytes) pl.waves[g].alloc(wbytes);
-        ta.events = pl.events[g].as<unsigned long long>();
-        ta.waves = pl.waves[g].as<WaveRec>();
-        // progress and count records zero; slot states PS_FRESH
-        zero(pg.ctl[g], sizeof(GroupCtl));
-        zero(ta.events, ebytes);
-        zero(ta.waves, wbytes);
-        zero(sl.u + (size_t)SU_STATE * Pg[g], (size_t)Pg[g] * sizeof(uint32_t));
-    }
+    for (int g = 0; g < G; g++) group_buffers(pg, g, Pg[g], g ? Pg[0] : 0, a.ni, rb);
     const uint64_t batch = std::min<uint64_t>(count, g_emit_batch ? g_emit_batch : kSplitEmit);
-    const size_t rsz = sizeof(R);
-    DevBuf& emitted = pool().emitted;
-    DevBuf& emitdraw = pool().emitdraw;
-    if (emitted.bytes < 7 * batch * rsz) emitted.alloc(7 * batch * rsz);
-    if (emitdraw.bytes < batch * sizeof(uint32_t)) emitdraw.alloc(batch * sizeof(uint32_t));
-    DevBuf& emithint = pool().emithint;
-    if (W::kHint && emithint.bytes < batch * sizeof(int32_t)) emithint.alloc(batch * sizeof(int32_t));
+    emission_buffers<W>(0, batch);
+    DevBuf &emitted = pool().emitted[0], &emitdraw = pool().emitdraw[0], &emithint = pool().emithint[0];
+    launch_begin(rb, a, s, 0, P);
     unsigned long long* claims = s->next.as<unsigned long long>();
-    unsigned long long* words = run_words();
-    zero(a.counters, SG_NCOUNTERS * sizeof(unsigned long long));
-    zero(a.error, sizeof(int));
-    zero(words + 1, sizeof(unsigned long long));
-    rb.scene_host = run.scene ? reinterpret_cast<const uint32_t*>(&g_run_host_dev->scene) : nullptr;
-    rb.scene = s->scene.as<uint32_t>();
-    rb.next = claims;
-    // the slots take a batch's first packets by their numbers, the others are claimed
-    rb.first_claim = (unsigned long long)P;
-    rb.begin = words;
-    int64_t most = 1;
-    for (int k = 0; k < rb.nzero; k++) most = std::max(most, rb.zero[k].words);
-    hipLaunchKernelGGL(k_run_begin, dim3((unsigned)std::min<int64_t>((most + 1023) / 1024, (int64_t)g_cus * 4)), dim3(256), 0,
-                       st[0], rb);
-    SG_HIP(hipGetLastError());
     auto join = [](hipStream_t from, hipStream_t to) {
         SG_HIP(hipEventRecord(g_split_join, from));
         SG_HIP(hipStreamWaitEvent(to, g_split_join, 0));
@@ -1688,15 +1733,7 @@ static void run_split(sg_sim* s, const typename W::View& v, const McArgs& a, uin
         run.launches += run_passes<W, ABS, MULTI>(v, ab, pg);
     }
     if (G == 2) join(st[1], st[0]);
-    RunEnd re{};
-    re.n = G;
-    for (int g = 0; g < G; g++) { re.tally[g] = pg.tally[g]; re.ctl[g] = pg.ctl[g]; }
-    re.counters = a.counters;
-    re.err = a.error;
-    re.begin = words;
-    re.ticket = reinterpret_cast<unsigned int*>(words + 1);
-    re.out = &g_run_host_dev->result;
-    launch_end(re, st[0]);
+    launch_result(pg, 0, G, a);
     SG_HIP(hipStreamSynchronize(st[0]));
 }
 
@@ -1750,10 +1787,10 @@ int sg_sim_run(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64_t npp,
     int err = 0, blocks = 0;
     if (g_pipeline == 1 && count > 0) {
         split_resources();
-        fill_args(s, ell, first, count, npp, a, g_run_host->scene);
+        fill_args(s, ell, first, count, npp, a, g_run_host->scene[0]);
         SplitRun run;
         dispatch_split_any(s, a, precision, first, count, run, blocks);
-        const RunResult& r = g_run_host->result;
+        const RunResult& r = g_run_host->result[0];
         err = (int)r.err;
         if (counters) {
             for (int i = 0; i < SG_NCOUNTERS; i++) counters[i] = r.counters[i];
@@ -1911,7 +1948,7 @@ int sg_sim_run_dust(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64_t
     McArgs a;
     if (passes) {
         split_resources();
-        fill_args(s, ell, first, count, npp, a, g_run_host->scene);
+        fill_args(s, ell, first, count, npp, a, g_run_host->scene[0]);
     } else fill_args(s, ell, first, count, npp, a);
     a.member = a.member ^ (stream * 0x9E3779B9u);
     a.Lpkt = Ltot / (double)npp;
@@ -1933,7 +1970,7 @@ int sg_sim_run_dust(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64_t
         SplitRun run;
         run.dust = &dl;
         dispatch_split_any(s, a, precision, first, count, run, blocks);
-        const RunResult& r = g_run_host->result;
+        const RunResult& r = g_run_host->result[0];
         if (counters) {
             for (int i = 0; i < SG_NCOUNTERS; i++) counters[i] = r.counters[i];
             counters[6] = npp;
@@ -2344,6 +2381,134 @@ static void dispatch_batch(sg_sim* s0, const std::vector<McArgs>& rg, const std:
     }
 }
 
+// A member of a batched run that takes the event/walk pipeline, and what its run left.
+struct BatchMember {
+    sg_sim* s;
+    int ell;
+    uint64_t count;
+};
+struct BatchSum {
+    unsigned long long counters[SG_NCOUNTERS] = {};
+    int err = 0, launches = 0, blocks = 0;
+    double transport_ms = 0, walk_ms = 0;
+};
+
+// Members through event and walk passes, kStreams at a time, each on a stream of its own with one slot group: a pass of one
+// member fills the device while the others' drain. The host looks at the members' progress in turn, and the next
+// member takes the place of one that has ended. (24 galaxies of 1e5 to 1e6 packets in the shared launch of the lane
+// pipeline: 96 ms.)
+template <class W, bool ABS> static void run_members(const std::vector<BatchMember>& ms, BatchSum& sum)
+{
+    using R = typename W::Real;
+    using V = typename W::View;
+    struct Lane {
+        bool busy = false;
+        V v{};
+        McArgs a;
+        PassGroups<R> pg{};
+        int seen = 0;
+    };
+    Lane lane[kStreams];
+    int busy = 0;
+    size_t next = 0;
+    auto add = [&](const RunResult& r) {
+        for (int k = 0; k < SG_NCOUNTERS; k++) sum.counters[k] += r.counters[k];
+        sum.err |= (int)r.err;
+        sum.transport_ms += r.transport / g_clock_khz;
+        sum.walk_ms += r.walk / g_clock_khz;
+    };
+    auto start = [&](int l) {
+        const BatchMember& m = ms[next++];
+        Lane& ln = lane[l];
+        ln = Lane{};
+        int nlds = 0;
+        if constexpr (std::is_same<V, CartView>::value) {
+            if (m.s->dust) { ln.v = m.s->dust->grid->cart; nlds = cart_words<R>(m.s->dust->grid); }
+        } else if constexpr (std::is_same<V, TreeView>::value) {
+            ln.v = m.s->dust->grid->tree;
+            nlds = std::is_same<W, TreeW64Book>::value ? 0 : SG_LDS_NODES;
+        } else ln.v = m.s->dust->grid->voro;
+        fill_args(m.s, m.ell, 0, m.count, m.count, ln.a, g_run_host->scene[l]);
+        ln.pg.n = 1;
+        pass_shape<W, ABS, false>(ln.pg, nlds);
+        sum.blocks = ln.pg.blocks;
+        const int64_t P = (int64_t)std::min<uint64_t>(m.count, (uint64_t)(g_tune_slots > 0 ? g_tune_slots : kSplitSlots));
+        RunBegin rb{};
+        group_buffers(ln.pg, l, P, 0, ln.a.ni, rb);
+        emission_buffers<W>(l, m.count);
+        launch_begin(rb, ln.a, m.s, l, P);
+        SplitPool& pl = pool();
+        launch_emit<W>(ln.v, ln.a, pl.emitted[l].p, pl.emitdraw[l].as<uint32_t>(), pl.emithint[l].as<int32_t>(),
+                       g_split_stream[l]);
+        for (int k = 0; k < kSplitAhead; k++) enqueue_pass<W, ABS, false>(ln.v, ln.a, ln.pg, l, k == 0);
+        ln.busy = true;
+        busy++;
+    };
+    auto advance = [&](int l, unsigned long long w) {
+        Lane& ln = lane[l];
+        ln.seen++;
+        const unsigned long long nq = w & ((1ull << 62) - 1);
+        SG_REQUIRE(nq <= (unsigned long long)ln.pg.q[l].cap, "walk queue overflow");
+        sum.launches += nq > 0;
+        if (nq > 0 || !((w >> 62) & 1)) {
+            enqueue_pass<W, ABS, false>(ln.v, ln.a, ln.pg, l, false);
+            return;
+        }
+        launch_result(ln.pg, l, 1, ln.a);
+        SG_HIP(hipStreamSynchronize(g_split_stream[l]));
+        add(g_run_host->result[l]);
+        ln.busy = false;
+        busy--;
+    };
+    // a member of several emission batches runs by itself (the largest members come first)
+    const uint64_t limit = g_emit_batch ? g_emit_batch : kSplitEmit;
+    for (; next < ms.size() && ms[next].count > limit; next++) {
+        const BatchMember& m = ms[next];
+        McArgs a;
+        fill_args(m.s, m.ell, 0, m.count, m.count, a, g_run_host->scene[0]);
+        SplitRun run;
+        dispatch_split<ABS, false>(m.s, a, std::is_same<R, float>::value ? SG_MIXED : SG_FP64, 0, m.count, run, sum.blocks);
+        sum.launches += run.launches;
+        add(g_run_host->result[0]);
+    }
+    for (uint64_t spin = 1; next < ms.size() || busy > 0; spin++) {
+        for (int l = 0; l < kStreams; l++) {
+            if (!lane[l].busy) {
+                if (next < ms.size()) start(l);
+                continue;
+            }
+            const unsigned long long* word = g_split_host + l * kProgressRing + lane[l].seen % kProgressRing;
+            unsigned long long w = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+            // now and then the stream's own state, so that one that failed, or drained without writing, ends the wait
+            if (!(w >> 63) && (spin & 0xffff) == 0 && hipStreamQuery(g_split_stream[l]) != hipErrorNotReady)
+                w = wait_progress(word, g_split_stream[l]);
+            if (w >> 63) advance(l, w);
+        }
+        __builtin_ia32_pause();
+    }
+}
+
+template <bool ABS> static void dispatch_members(const std::vector<BatchMember>& ms, int precision, BatchSum& sum)
+{
+    const bool mixed = precision == SG_MIXED;
+    const sg_grid* g = ms[0].s->dust ? ms[0].s->dust->grid : nullptr;
+    if (!g) {
+        if (mixed) run_members<CartW32, false>(ms, sum);
+        else run_members<CartW64, false>(ms, sum);
+    } else if (g->kind == GK_CART) {
+        if (mixed) run_members<CartW32, ABS>(ms, sum);
+        else run_members<CartW64, ABS>(ms, sum);
+    } else if (g->kind == GK_TREE) {
+        if (!mixed && g->tree.search == SG_BOOKKEEPING) run_members<TreeW64Book, ABS>(ms, sum);
+        else if (!mixed) run_members<TreeW64, ABS>(ms, sum);
+        else if (rope_walk(g)) run_members<TreeW32, ABS>(ms, sum);
+        else run_members<TreeW32TopDown, ABS>(ms, sum);
+    } else {
+        if (mixed) run_members<VoroWalk<float>, ABS>(ms, sum);
+        else run_members<VoroWalk<double>, ABS>(ms, sum);
+    }
+}
+
 extern "C" {
 
 int sg_sim_run_batch(int nmembers, sg_sim* const* sims, const int* ells, const uint64_t* counts, int precision,
@@ -2366,18 +2531,28 @@ int sg_sim_run_batch(int nmembers, sg_sim* const* sims, const int* ells, const u
                    "a simulation may appear only once in a batched run");
         seen.push_back(sims[i]);
     }
-    std::vector<McArgs> base(nmembers);
-    uint64_t total = 0;
+    // large members: their own event/walk passes, the largest first; the others share the persistent launches
+    std::vector<BatchMember> passes;
+    std::vector<uint64_t> done(nmembers, 0);
+    std::vector<McArgs> base(nmembers, McArgs{});
+    uint64_t total = 0, shared = 0;
     for (int i = 0; i < nmembers; i++) {
+        total += counts[i];
+        if (g_pipeline == 1 && g_batch_alone > 0 && counts[i] >= g_batch_alone && !(sims[i]->dust && sims[i]->dust->ncomp > 1)) {
+            done[i] = counts[i];
+            if (counts[i] > 0) passes.push_back({sims[i], ells[i], counts[i]});
+            continue;
+        }
         fill_args(sims[i], ells[i], 0, counts[i], std::max<uint64_t>(counts[i], 1), base[i]);
         sims[i]->counters.zero();
         sims[i]->err.zero();
-        total += counts[i];
+        shared += counts[i];
     }
+    std::stable_sort(passes.begin(), passes.end(), [](const BatchMember& a, const BatchMember& b) { return a.count > b.count; });
     const bool mixed = precision == SG_MIXED;
     const size_t rsz = mixed ? sizeof(float) : sizeof(double);
     // packets per round: the emission buffer holds one round's launch states
-    const uint64_t B = std::max<uint64_t>(1, std::min<uint64_t>(total, (uint64_t)1 << 23));
+    const uint64_t B = std::max<uint64_t>(1, std::min<uint64_t>(shared, (uint64_t)1 << 23));
     if (s0->emitted.bytes < 7 * B * rsz) s0->emitted.alloc(7 * B * rsz);
     if (s0->emitdraw.bytes < B * sizeof(uint32_t)) s0->emitdraw.alloc(B * sizeof(uint32_t));
     if (s0->bnext.bytes < (size_t)nmembers * sizeof(unsigned long long))
@@ -2388,10 +2563,9 @@ int sg_sim_run_batch(int nmembers, sg_sim* const* sims, const int* ells, const u
     SG_HIP(hipEventRecord(e0, 0));
     int blocks = 0;
     LaunchTimer lt;
-    std::vector<uint64_t> done(nmembers, 0);
     // members with several dust components: one at a time through the lane pipeline
     for (int i = 0; i < nmembers; i++) {
-        if (base[i].ncomp < 2 || counts[i] == 0) continue;
+        if (base[i].ncomp < 2 || done[i] == counts[i]) continue;
         for (uint64_t b = 0; b < counts[i]; b += B) {
             McArgs ab = base[i];
             ab.first = b;
@@ -2408,17 +2582,6 @@ int sg_sim_run_batch(int nmembers, sg_sim* const* sims, const int* ells, const u
             dispatch_mc_any(sims[i], ab, precision, blocks);
             lt.stop();
         }
-        done[i] = counts[i];
-    }
-    // large members: their own event/walk passes, which keep the walk kernel full on their own
-    for (int i = 0; g_pipeline == 1 && g_batch_alone > 0 && i < nmembers; i++) {
-        if (done[i] == counts[i]) continue;
-        if (counts[i] < g_batch_alone) continue;
-        SplitRun run;
-        run.scene = false;
-        dispatch_split_any(sims[i], base[i], precision, 0, counts[i], run, blocks);
-        const RunResult& r = g_run_host->result;
-        lt.add(r.transport / g_clock_khz, run.launches, r.walk / g_clock_khz);
         done[i] = counts[i];
     }
     int j = 0;
@@ -2448,15 +2611,26 @@ int sg_sim_run_batch(int nmembers, sg_sim* const* sims, const int* ells, const u
         if (abs_of(s0)) dispatch_batch<true>(s0, rg, owner, precision, blocks, lt);
         else dispatch_batch<false>(s0, rg, owner, precision, blocks, lt);
     }
+    // the shared launches are under way on the default stream, which these do not wait for
+    BatchSum own;
+    if (!passes.empty()) {
+        split_resources();
+        if (abs_of(s0)) dispatch_members<true>(passes, precision, own);
+        else dispatch_members<false>(passes, precision, own);
+        lt.add(own.transport_ms, own.launches, own.walk_ms);
+        if (shared == 0) blocks = own.blocks;
+    }
     SG_HIP(hipEventRecord(e1, 0));
     SG_HIP(hipEventSynchronize(e1));
     float ms = 0;
     SG_HIP(hipEventElapsedTime(&ms, e0, e1));
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    unsigned long long sum[SG_NCOUNTERS] = {0};
-    int err = 0;
+    unsigned long long sum[SG_NCOUNTERS];
+    std::copy(own.counters, own.counters + SG_NCOUNTERS, sum);
+    int err = own.err;
     for (int i = 0; i < nmembers; i++) {
+        if (base[i].counters == nullptr) continue;   // ran its own passes
         unsigned long long c[SG_NCOUNTERS];
         SG_HIP(hipMemcpy(c, sims[i]->counters.p, sizeof c, hipMemcpyDeviceToHost));
         for (int k = 0; k < SG_NCOUNTERS; k++) sum[k] += c[k];

@@ -482,7 +482,7 @@ __global__ void __launch_bounds__(256) k_key_scatter(WalkQueue<R> q, int* error)
 struct RunBegin {
     struct Fill { uint32_t* p; int64_t words; } zero[11];
     int nzero;
-    const uint32_t* scene_host;         // pinned host memory, or null: the scene is there already
+    const uint32_t* scene_host;         // pinned host memory
     uint32_t* scene;
     unsigned long long* next;
     unsigned long long first_claim;
@@ -494,7 +494,7 @@ __global__ void __launch_bounds__(256) k_run_begin(const RunBegin b)
 {
     const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, n = (int64_t)gridDim.x * blockDim.x;
     if (blockIdx.x == 0) {
-        for (int i = (int)threadIdx.x; b.scene_host && i < (int)(sizeof(SceneDev) / 4); i += (int)blockDim.x) b.scene[i] = b.scene_host[i];
+        for (int i = (int)threadIdx.x; i < (int)(sizeof(SceneDev) / 4); i += (int)blockDim.x) b.scene[i] = b.scene_host[i];
         if (threadIdx.x == 0) {
             *b.next = b.first_claim;
             *b.begin = wall_clock64();

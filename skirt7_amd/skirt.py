@@ -791,8 +791,8 @@ def set_pipeline(mode):
 
 
 def set_batch_alone(min_packets):
-    """Members of run_batch with at least this many packets run one at a time through the event and walk
-    kernels; the rest share the persistent batched launches (0: every member shares them)."""
+    """Members of run_batch with at least this many packets run through the event and walk kernels, a few at a time;
+    the rest share the persistent batched launches (0: every member shares them)."""
     check(lib().sg_set_batch_alone(int(min_packets)))
 
 
