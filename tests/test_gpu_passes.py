@@ -3,6 +3,7 @@ two slot groups and several emission batches, against the lane pipeline's same p
 import numpy as np
 import pytest
 
+from skirt7_amd import capi
 from skirt7_amd import skirt as S
 from skirt7_amd import workloads
 from skirt7_amd.capi import SG_FP64, SG_MIXED
@@ -106,5 +107,61 @@ def test_passes_of_several_dust_components(kind, precision, count, batch):
                                        "peeloffs", "walks")}))
     assert out[0][2] == out[1][2]
     # sums of at most some ten thousand positive FP64 terms in another order
+    np.testing.assert_allclose(out[1][0], out[0][0], rtol=1e-11, atol=0)
+    np.testing.assert_allclose(out[1][1], out[0][1], rtol=1e-11, atol=0)
+
+
+@pytest.mark.parametrize("precision", [SG_FP64, SG_MIXED])
+@pytest.mark.parametrize("alone,batch", [(1, 0), (1, 1000), (900, 0)])
+def test_batched_members_by_passes(alone, batch, precision):
+    """More members than there are streams, each by passes of its own (from one packet up; with small emission batches
+    the larger ones one at a time), or some of them in the shared launch, against their single runs."""
+    counts = [700, 1, 3000, 64, 1500, 129, 2, 901]
+    pop = workloads.fit_population(members=len(counts), packets=(1.0e3, 3.0e3), grid_n=(6, 14), pixels=(32, 16), nsamples=2)
+    ms = pop["members"]
+    single, walks = [], 0
+    for m, n in zip(ms, counts):
+        m["instr"].clear()
+        walks += m["sim"].run_packets(0, 0, n, n, precision)["walks"]
+        single.append(m["instr"].frame(0)[0].copy())
+        m["instr"].clear()
+    try:
+        S.set_batch_alone(alone)
+        S.set_emit_batch(batch)
+        c = S.run_batch([m["sim"] for m in ms], counts, precision=precision)
+    finally:
+        S.set_batch_alone(3 << 16)
+        S.set_emit_batch(0)
+    assert c["packets"] == sum(counts) and c["walks"] == walks
+    for m, f in zip(ms, single):
+        # sums of at most some thousand positive FP64 terms in another order
+        np.testing.assert_allclose(m["instr"].frame(0)[0], f, rtol=1e-11, atol=0)
+
+
+@pytest.mark.parametrize("kind", ["cartesian", "octree"])
+@pytest.mark.parametrize("count,batch", [(1, 0), (513, 0), (3001, 1024)])
+def test_dust_emission_by_passes(kind, count, batch):
+    """Dust emission in the passes against the lane pipeline: the same histories, with peel-offs and with absorption."""
+    w = workloads.pan_disc(kind=kind, nlambda=12, grid_n=10, maxlevel=3, pixels=16, packages=500)
+    pan = w["pan"]
+    nc = w["grid"].numCells()
+    Lv = np.ascontiguousarray(np.random.default_rng(4).random(nc))
+    out = []
+    for mode in (0, 1):
+        pan.dust.ds.clear()
+        w["instr"].clear()
+        c = np.zeros(capi.SG_NCOUNTERS, np.uint64)
+        try:
+            S.set_pipeline(mode)
+            S.set_emit_batch(batch)
+            for peel in (1, 0):
+                capi.check(capi.lib().sg_sim_run_dust(pan.sim._h, 9, 0, count, count, capi.dptr(Lv), 0.5, peel, 1 - peel, 5,
+                                                      SG_MIXED, c.ctypes.data_as(capi._U64)))
+        finally:
+            S.set_pipeline(1)
+            S.set_emit_batch(0)
+        out.append((np.concatenate([w["instr"].frame(i).ravel() for i in range(len(w["instr"].instruments))]),
+                    pan.dust.ds.Labs(), [int(c[k]) for k in (0, 1, 2, 3, 4, 7, 8)]))
+    assert out[0][2] == out[1][2]
     np.testing.assert_allclose(out[1][0], out[0][0], rtol=1e-11, atol=0)
     np.testing.assert_allclose(out[1][1], out[0][1], rtol=1e-11, atol=0)
