@@ -2150,7 +2150,7 @@ int sg_sim_run_static(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64
                                                " packets per call (the static work array holds their launch states); "
                                                "split the packet range over several calls");
     SG_REQUIRE(!s->dust || s->dust->ncomp == 1,
-               "sg_sim_run_static: a dust system of several components needs sg_sim_run (lane pipeline)");
+               "sg_sim_run_static: a dust system of several components needs sg_sim_run");
     McArgs a;
     fill_args(s, ell, first, count, npp, a);
     int blocks = 0;
