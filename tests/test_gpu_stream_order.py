@@ -1,0 +1,85 @@
+"""GPU: a run begins behind what the calls before it left on the default stream. Densities resampled on the device and
+cleared frames and tables are still being written when those calls return; a run called at once gives the same as one
+called after a wait for the device."""
+import numpy as np
+import pytest
+
+from skirt7_amd import skirt as S
+from skirt7_amd import workloads
+from skirt7_amd.capi import SG_FP64, SG_MIXED
+
+pytestmark = pytest.mark.gpu
+
+COUNTS = ("packets", "own_crossings", "peel_crossings", "rewalk_crossings", "scatterings", "peeloffs", "walks")
+PACKETS = 3000
+
+
+def _galaxy(seed):
+    comps, dgeom, mix, scale = workloads._galaxy()
+    grid = S.CartesianDustGrid.uniform(workloads.EXTENT, 128, 128, 128)
+    dust = S.DustSystem(grid, np.zeros(grid.numCells()), mix, writeMeanIntensity=True)
+    stars = S.StellarSystem(comps)
+    instr = workloads._frames((0.0, 60.0), 40)
+    sim = S.OligoMonteCarloSimulation(dust, stars, instr, packages=PACKETS, seed=seed)
+    return dict(grid=grid, dgeom=dgeom, scale=scale, dust=dust, stars=stars, instr=instr, sim=sim)
+
+
+def _wait(dust):
+    dust.opticaldepths(np.array([[0.0, 0.0, 0.0, 0.0, 0.0, 1.0]]))   # waits for the device
+
+
+def _results(w):
+    return np.concatenate([w["instr"].frame(i).ravel() for i in range(len(w["instr"].instruments))] + [w["dust"].Labs().ravel()])
+
+
+@pytest.fixture(scope="module")
+def galaxies():
+    return [_galaxy(seed) for seed in (3, 4)]
+
+
+@pytest.mark.parametrize("precision", [SG_FP64, SG_MIXED])
+@pytest.mark.parametrize("batched", [False, True])
+def test_run_behind_resampled_density(galaxies, batched, precision):
+    out, counts = [], []
+    for wait in (True, False):
+        # from a density that gives other results: a third of the depth
+        for w in galaxies:
+            S.resample_density(w["grid"], w["dgeom"], w["scale"] / 3.0, 1, 5)
+            _wait(w["dust"])
+        for w in galaxies:
+            w["instr"].clear()
+            w["dust"].clear()
+            S.resample_density(w["grid"], w["dgeom"], w["scale"], 200, 7)
+            if wait:
+                _wait(w["dust"])
+            if not batched:
+                c = w["sim"].run_packets(0, 0, PACKETS, PACKETS, precision)
+                counts.append([c[k] for k in COUNTS])
+        if batched:
+            try:
+                S.set_batch_alone(1)
+                c = S.run_batch([w["sim"] for w in galaxies], [PACKETS] * len(galaxies), precision=precision)
+            finally:
+                S.set_batch_alone(3 << 16)
+            counts.append([c[k] for k in COUNTS])
+        out.append(np.concatenate([_results(w) for w in galaxies]))
+    half = len(counts) // 2
+    assert counts[:half] == counts[half:]
+    # sums of at most some ten thousand positive FP64 terms in another order
+    np.testing.assert_allclose(out[1], out[0], rtol=1e-11, atol=0)
+
+
+@pytest.mark.parametrize("precision", [SG_FP64, SG_MIXED])
+def test_run_without_dust_behind_cleared_frames(galaxies, precision):
+    instr = workloads._frames((0.0, 30.0, 60.0, 88.0), 2048)
+    sim = S.OligoMonteCarloSimulation(None, galaxies[0]["stars"], instr, packages=PACKETS, seed=9)
+    out = []
+    for wait in (True, False):
+        sim.run_packets(0, 0, PACKETS, PACKETS, precision)   # frames that are not empty
+        instr.clear()
+        if wait:
+            _wait(galaxies[0]["dust"])
+        sim.run_packets(0, 0, PACKETS, PACKETS, precision)
+        out.append(np.concatenate([instr.frame(i).ravel() for i in range(4)]))
+    assert out[0].sum() > 0
+    np.testing.assert_allclose(out[1], out[0], rtol=1e-11, atol=0)
