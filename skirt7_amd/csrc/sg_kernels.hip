@@ -2399,11 +2399,13 @@ static void dispatch_batch(sg_sim* s0, const std::vector<McArgs>& rg, const std:
     }
 }
 
-// A member of a batched run that takes the event/walk pipeline, and what its run left.
+// A member of a batched run that takes the event/walk pipeline, with its run's arguments and scene, and what its run
+// left.
 struct BatchMember {
     sg_sim* s;
-    int ell;
     uint64_t count;
+    McArgs a;
+    SceneDev scene;
 };
 struct BatchSum {
     unsigned long long counters[SG_NCOUNTERS] = {};
@@ -2446,7 +2448,8 @@ template <class W, bool ABS> static void run_members(const std::vector<BatchMemb
             ln.v = m.s->dust->grid->tree;
             nlds = std::is_same<W, TreeW64Book>::value ? 0 : SG_LDS_NODES;
         } else ln.v = m.s->dust->grid->voro;
-        fill_args(m.s, m.ell, 0, m.count, m.count, ln.a, g_run_host->scene[l]);
+        ln.a = m.a;
+        g_run_host->scene[l] = m.scene;
         ln.pg.n = 1;
         pass_shape<W, ABS, false>(ln.pg, nlds);
         sum.blocks = ln.pg.blocks;
@@ -2482,10 +2485,9 @@ template <class W, bool ABS> static void run_members(const std::vector<BatchMemb
     const uint64_t limit = g_emit_batch ? g_emit_batch : kSplitEmit;
     for (; next < ms.size() && ms[next].count > limit; next++) {
         const BatchMember& m = ms[next];
-        McArgs a;
-        fill_args(m.s, m.ell, 0, m.count, m.count, a, g_run_host->scene[0]);
+        g_run_host->scene[0] = m.scene;
         SplitRun run;
-        dispatch_split<ABS, false>(m.s, a, std::is_same<R, float>::value ? SG_MIXED : SG_FP64, 0, m.count, run, sum.blocks);
+        dispatch_split<ABS, false>(m.s, m.a, std::is_same<R, float>::value ? SG_MIXED : SG_FP64, 0, m.count, run, sum.blocks);
         sum.launches += run.launches;
         add(g_run_host->result[0]);
     }
@@ -2549,7 +2551,8 @@ int sg_sim_run_batch(int nmembers, sg_sim* const* sims, const int* ells, const u
                    "a simulation may appear only once in a batched run");
         seen.push_back(sims[i]);
     }
-    // large members: their own event/walk passes, the largest first; the others share the persistent launches
+    // large members: their own event/walk passes, the largest first; the others share the persistent launches. Every
+    // member's arguments are looked over before the first launch: a call that is refused leaves no tallies
     std::vector<BatchMember> passes;
     std::vector<uint64_t> done(nmembers, 0);
     std::vector<McArgs> base(nmembers, McArgs{});
@@ -2558,7 +2561,8 @@ int sg_sim_run_batch(int nmembers, sg_sim* const* sims, const int* ells, const u
         total += counts[i];
         if (g_pipeline == 1 && g_batch_alone > 0 && counts[i] >= g_batch_alone && !(sims[i]->dust && sims[i]->dust->ncomp > 1)) {
             done[i] = counts[i];
-            if (counts[i] > 0) passes.push_back({sims[i], ells[i], counts[i]});
+            passes.push_back({sims[i], counts[i], McArgs{}, SceneDev{}});
+            fill_args(sims[i], ells[i], 0, counts[i], counts[i], passes.back().a, passes.back().scene);
             continue;
         }
         fill_args(sims[i], ells[i], 0, counts[i], std::max<uint64_t>(counts[i], 1), base[i]);

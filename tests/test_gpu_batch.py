@@ -100,6 +100,23 @@ def test_batch_rejects_mixed_grid_kinds(pop):
         S.run_batch([pop["members"][0]["sim"], pop["members"][0]["sim"]], [10, 10])
 
 
+@pytest.mark.parametrize("ells", [[0, 0, 1], [0, -1, 0], [7, 0, 0]])
+def test_refused_batch_leaves_no_tallies(pop, ells):
+    """A wavelength out of range, on a member of the shared launch (100 packets) or with passes of its own, is found
+    before anything is launched."""
+    ms = pop["members"][:3]
+    for m in ms:
+        m["instr"].clear()
+    try:
+        S.set_batch_alone(1000)
+        with pytest.raises(S.FatalError, match="wavelength index"):
+            S.run_batch([m["sim"] for m in ms], [100, 1500, 3000], ells=ells)
+    finally:
+        S.set_batch_alone(1 << 21)
+    for m in ms:
+        assert not m["instr"].frame(0).any()
+
+
 def test_fit_matches_oracle(pop):
     ms = pop["members"]
     for m in ms:
