@@ -20,6 +20,7 @@ struct Fail {
     do {                                                                                             \
         hipError_t e_ = (expr);                                                                      \
         if (e_ != hipSuccess) {                                                                      \
+            (void)hipGetLastError();   /* reported here, not by the next launch's check */           \
             sg::set_error(std::string(#expr) + ": " + hipGetErrorString(e_));                        \
             throw sg::Fail{-2};                                                                      \
         }                                                                                            \
@@ -42,9 +43,13 @@ struct DevBuf {
     ~DevBuf() { if (p) (void)hipFree(p); }
     void alloc(size_t n)
     {
+        // a failed allocation leaves an empty buffer, which the next user allocates anew
         if (p) { (void)hipFree(p); p = nullptr; }
+        bytes = 0;
+        void* q = nullptr;
+        if (n) SG_HIP(hipMalloc(&q, n));
+        p = q;
         bytes = n;
-        if (n) SG_HIP(hipMalloc(&p, n));
     }
     template <class T> void upload(const T* h, size_t count)
     {
