@@ -6,6 +6,7 @@
 #include <cmath>
 #include <cstddef>
 #include <cstring>
+#include <exception>
 #include <memory>
 #include <string>
 #include <type_traits>
@@ -1450,6 +1451,20 @@ static void mark_default_stream()
     else SG_HIP(e);
 }
 
+// Held by an entry point that runs kernels on the transport streams: where it leaves by an exception, the streams are
+// waited for first, so that no kernel outlives the call with the pinned words and work buffers that the next one takes.
+struct DrainOnThrow {
+    const int thrown = std::uncaught_exceptions();
+    ~DrainOnThrow()
+    {
+        if (std::uncaught_exceptions() <= thrown) return;
+        for (int g = 0; g < kStreams; g++)
+            if (g_split_stream[g]) (void)hipStreamSynchronize(g_split_stream[g]);
+        (void)hipStreamSynchronize(0);
+        (void)hipGetLastError();
+    }
+};
+
 // Waits until a walk kernel on stream st has written its progress word. The stream's state is looked at now and
 // then, so that a stream that failed, or drained without writing, ends the wait.
 static unsigned long long wait_progress(const unsigned long long* word, hipStream_t st)
@@ -1797,6 +1812,7 @@ extern "C" {
 int sg_sim_run(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64_t npp, int precision, uint64_t* counters)
 {
     SG_TRY
+    DrainOnThrow drain;
     ensure_init();
     SG_REQUIRE(npp > 0, "npp must be positive");
     McArgs a;
@@ -1939,6 +1955,7 @@ int sg_sim_run_dust(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64_t
                     int peeloffs, int store_absorption, uint32_t stream, int precision, uint64_t* counters)
 {
     SG_TRY
+    DrainOnThrow drain;
     ensure_init();
     SG_REQUIRE(s && s->dust && Lv, "dust emission needs a simulation with a dust system and the cells' luminosities");
     SG_REQUIRE(npp > 0, "npp must be positive");
@@ -2161,6 +2178,7 @@ int sg_sim_run_static(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64
                       uint64_t* counters)
 {
     SG_TRY
+    DrainOnThrow drain;
     SG_REQUIRE(g_device >= 0, "sg_sim_run_static: call sg_init first (the static work array is set up there)");
     SG_REQUIRE(npp > 0, "npp must be positive");
     SG_REQUIRE(precision == SG_MIXED || precision == SG_FP64, "precision must be SG_FP64 or SG_MIXED");
@@ -2535,6 +2553,7 @@ int sg_sim_run_batch(int nmembers, sg_sim* const* sims, const int* ells, const u
                      uint64_t* counters)
 {
     SG_TRY
+    DrainOnThrow drain;
     ensure_init();
     SG_REQUIRE(nmembers >= 1 && sims && ells && counts, "a batched run needs at least one member");
     sg_sim* s0 = sims[0];
