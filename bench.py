@@ -72,9 +72,9 @@ def parse():
                     help="target duration of each multi-threaded CPU baseline sample")
     ap.add_argument("--ref-mult", type=int, default=10,
                     help="the equal-image-error reference runs this many times the timed steps' packets in FP64")
-    ap.add_argument("--slot-groups", type=int, default=2, choices=(1, 2),
+    ap.add_argument("--slot-groups", type=int, default=0, choices=(0, 1, 2),
                     help="slot groups of the timed steps (2: alternating on two streams; 1: one stream, as the "
-                         "roofline step)")
+                         "roofline step; 0: as a run chooses by itself)")
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-fp64", action="store_true")
     ap.add_argument("--tau-cut", type=float, default=0.0)

@@ -289,8 +289,8 @@ int sg_set_walk_order(int order);
 /* Slot groups of the event/walk pipeline: 2 alternate on two streams, so that one group's event pass and
  * the drain of its walk pass overlap the other group's walks; 1 runs every pass on one stream, one kernel
  * at a time (each walk launch then has the device to itself, which is how its own duration is measured).
- * Until this is called, a run takes two where its grid's walks are long and one elsewhere. No counterpart
- * in the reference. */
+ * 0 (default): a run takes two where its grid's walks are long and one elsewhere. No counterpart in the
+ * reference. */
 int sg_set_slot_groups(int groups);
 /* Packets whose launch states sg_sim_run emits at once (0: the default, 2^25 for the event/walk pipeline and
  * 2^22 for the lane pipeline; otherwise at least 64): a longer range is transported batch by batch, with the

@@ -307,8 +307,8 @@ int sg_set_emit_batch(uint64_t packets)
 
 int sg_set_slot_groups(int groups)
 {
-    if (groups != 1 && groups != 2) {
-        sg::set_error("slot groups must be 1 or 2");
+    if (groups < 0 || groups > 2) {
+        sg::set_error("slot groups must be 0 (chosen for each run), 1 or 2");
         return -1;
     }
     g_slot_groups = groups;

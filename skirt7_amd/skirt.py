@@ -815,9 +815,9 @@ def set_emit_batch(packets=0):
     check(lib().sg_set_emit_batch(int(packets)))
 
 
-def set_slot_groups(groups=2):
+def set_slot_groups(groups=0):
     """Event/walk pipeline: 2 slot groups alternating on two streams; 1 runs every pass on one stream, one kernel at a
-    time. Until it is set, a run takes two where its grid's walks are long and one elsewhere."""
+    time; 0 (default) takes two where a run's grid has long walks and one elsewhere."""
     check(lib().sg_set_slot_groups(int(groups)))
 
 

@@ -62,7 +62,7 @@ def test_batch_splits_members_across_rounds(pop):
     try:
         S.run_batch([m["sim"] for m in ms], counts, precision=SG_MIXED)
     finally:
-        S.set_batch_alone(1 << 21)
+        S.set_batch_alone(3 << 16)
     g = m0["instr"].frame(0)[0].copy()
     m0["instr"].clear()
     m0["sim"].run_packets(0, 0, counts[0], counts[0], SG_MIXED)
@@ -85,7 +85,7 @@ def test_batch_runs_large_members_alone(pop, precision):
     try:
         cb = S.run_batch([m["sim"] for m in ms], [m["packages"] for m in ms], precision=precision)
     finally:
-        S.set_batch_alone(1 << 21)
+        S.set_batch_alone(3 << 16)
     for k in EXACT:
         assert cb[k] == tot[k], k
     for m, f in zip(ms, single):
@@ -112,7 +112,7 @@ def test_refused_batch_leaves_no_tallies(pop, ells):
         with pytest.raises(S.FatalError, match="wavelength index"):
             S.run_batch([m["sim"] for m in ms], [100, 1500, 3000], ells=ells)
     finally:
-        S.set_batch_alone(1 << 21)
+        S.set_batch_alone(3 << 16)
     for m in ms:
         assert not m["instr"].frame(0).any()
 

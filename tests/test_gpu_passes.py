@@ -26,7 +26,8 @@ def disc():
 
 @pytest.mark.parametrize("precision", [SG_FP64, SG_MIXED])
 @pytest.mark.parametrize("count,groups,batch", [(1, 2, 0), (2, 2, 0), (3, 1, 0), (4, 2, 0), (16, 1, 0), (17, 2, 0),
-                                                (63, 1, 0), (129, 2, 64), (700, 2, 0), (701, 1, 100), (5001, 2, 1024)])
+                                                (63, 1, 0), (129, 2, 64), (700, 2, 0), (701, 1, 100), (5001, 2, 1024),
+                                                (130, 0, 64), (3000, 0, 0)])
 def test_passes_equal_the_lane_pipeline(disc, count, groups, batch, precision):
     # the histories are the same, only the order of the tally additions differs: the sums of up to a few hundred
     # thousand positive FP64 terms agree to n eps < 1e-10
@@ -39,10 +40,29 @@ def test_passes_equal_the_lane_pipeline(disc, count, groups, batch, precision):
         out, c = _run(disc, count, precision)
     finally:
         S.set_pipeline(1)
-        S.set_slot_groups(2)
+        S.set_slot_groups(0)
         S.set_emit_batch(0)
     assert c == cref
     np.testing.assert_allclose(out, ref, rtol=1e-10, atol=0)
+
+
+@pytest.mark.parametrize("kind,chosen", [("cartesian", 1), ("voronoi", 2)])
+def test_slot_groups_return_to_the_runs_choice(kind, chosen):
+    """Set and set back to 0, a run takes the groups it chooses by itself: one on a Cartesian grid, two on a Voronoi
+    grid, by its walk launches (every pass of every group; all packets start in the first pass, so that the number
+    of passes is the packets' own)."""
+    w = workloads.two_dust_disc(kind, grid_n=12, nsites=600, pixels=20, packages=4000)
+    launches = {}
+    try:
+        for groups in (1, 2, 0):
+            S.set_slot_groups(groups)
+            launches[groups] = w["sim"].run_packets(0, 0, 2000, 2000, SG_FP64)["transport_launches"]
+        for bad in (-1, 3):
+            with pytest.raises(S.FatalError):
+                S.set_slot_groups(bad)
+    finally:
+        S.set_slot_groups(0)
+    assert launches[1] < launches[2] and launches[0] == launches[chosen]
 
 
 @pytest.mark.parametrize("lists", ["as built", "shuffled", "superset"])
