@@ -245,7 +245,7 @@ template <class W> struct Hot {
     // last segment (for a propagation re-walk, the cell of the interaction point)
     R lsca;
     int mcell;
-    template <class P> __device__ __forceinline__ void park(P& p)
+    template <class P> __host__ __device__ __forceinline__ constexpr void park(P& p)
     {
         w.park(p);
         p.io(tau); p.io(s); p.io(tprev); p.io(sprev); p.io(limit); p.io(L0);
@@ -278,7 +278,10 @@ template <class W> __device__ __forceinline__ typename W::Real prop_length(const
 
 template <class W> __host__ __device__ constexpr int hot_words()
 {
-    return W::kParkWords + (int)(7 * sizeof(typename W::Real) / 4) + 4;
+    Hot<W> h{};
+    ParkCount n;
+    h.park(n);
+    return n.words;
 }
 
 // Hot state is parked in LDS (structure-of-arrays, one slot per lane) while a wave re-arms lanes,

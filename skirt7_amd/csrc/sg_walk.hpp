@@ -57,6 +57,11 @@ template <bool LOAD> struct Park {
         v = __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
     }
 };
+// The 32-bit words that Park moves for a state's fields.
+struct ParkCount {
+    int words = 0;
+    template <typename T> __host__ __device__ constexpr void io(T&) { words += sizeof(T) == 8 ? 2 : 1; }
+};
 
 // The part of a grid view that a walker reads from LDS, staged by the lanes first, first + step, ...: the top
 // levels' node words of a tree, the cell borders of a Cartesian grid (in the walker's real type); at most `room`
@@ -156,7 +161,6 @@ struct CartW64 {
     double e0, e1, e2;
     bool done;
     uint32_t nrecompute, nstuck;
-    static constexpr int kParkWords = 38;
     __device__ __forceinline__ static int cell_of(const View&, int n) { return n; }
     static constexpr bool kHint = false;
     static constexpr int kLanes = 1;
@@ -172,7 +176,7 @@ struct CartW64 {
         return Borders<double>{nlds > 0, reinterpret_cast<const double*>(lds), g.xv, g.yv, g.zv, g.Nx + 1,
                                g.Nx + g.Ny + 2};
     }
-    template <class P> __device__ __forceinline__ void park(P& p)
+    template <class P> __host__ __device__ __forceinline__ constexpr void park(P& p)
     {
         p.io(x); p.io(y); p.io(z); p.io(kx); p.io(ky); p.io(kz); p.io(ix); p.io(iy); p.io(iz);
         p.io(xE); p.io(yE); p.io(zE); p.io(rho);
@@ -323,7 +327,6 @@ struct CartW32 {
     float e0, e1, e2;
     bool done;
     uint32_t nrecompute, nstuck;
-    static constexpr int kParkWords = 24;
     __device__ __forceinline__ static int cell_of(const View&, int n) { return n; }
     static constexpr bool kHint = false;
     static constexpr int kLanes = 1;
@@ -339,7 +342,7 @@ struct CartW32 {
         return Borders<float>{nlds > 0, reinterpret_cast<const float*>(lds), g.xvf, g.yvf, g.zvf, g.Nx + 1,
                               g.Nx + g.Ny + 2};
     }
-    template <class P> __device__ __forceinline__ void park(P& p)
+    template <class P> __host__ __device__ __forceinline__ constexpr void park(P& p)
     {
         p.io(x); p.io(y); p.io(z); p.io(kx); p.io(ky); p.io(kz); p.io(ix); p.io(iy); p.io(iz);
         p.io(xE); p.io(yE); p.io(zE); p.io(rho);
@@ -589,13 +592,12 @@ struct TreeW64 {
     Entry en;
     bool done;
     uint32_t steps, nrecompute, nstuck;
-    static constexpr int kParkWords = 44;
     __device__ __forceinline__ static int cell_of(const View&, int n) { return n; }
     static constexpr bool kHint = true;
     static constexpr int kLanes = 1;
     static constexpr bool kLocates = false;
     __device__ __forceinline__ int entries() const { return en.ne; }
-    template <class P> __device__ __forceinline__ void park(P& p)
+    template <class P> __host__ __device__ __forceinline__ constexpr void park(P& p)
     {
         p.io(x); p.io(y); p.io(z); p.io(kx); p.io(ky); p.io(kz); p.io(ix); p.io(iy); p.io(iz);
         p.io(ex); p.io(ey); p.io(ez); p.io(qx); p.io(qy); p.io(qz); p.io(down); p.io(wall);
@@ -777,7 +779,6 @@ struct TreeW64Book {
     Entry en;
     bool done;
     uint32_t steps, nrecompute, nstuck;
-    static constexpr int kParkWords = 25;
     // segments carry cell numbers
     __device__ __forceinline__ static int cell_of(const View&, int n) { return n; }
     static constexpr bool kHint = false;
@@ -785,7 +786,7 @@ struct TreeW64Book {
     static constexpr bool kLocates = false;
     __device__ __forceinline__ int entries() const { return en.ne; }
     static constexpr bool kStep = false;   // next() only
-    template <class P> __device__ __forceinline__ void park(P& p)
+    template <class P> __host__ __device__ __forceinline__ constexpr void park(P& p)
     {
         p.io(x); p.io(y); p.io(z); p.io(kx); p.io(ky); p.io(kz);
         p.io(l); p.io(en.ne); p.io(en.e0); p.io(en.e1); p.io(en.e2);
@@ -921,11 +922,10 @@ struct TreeW32 {
     float e0, e1, e2;
     bool done;
     uint32_t steps, nrecompute, nstuck;
-    static constexpr int kParkWords = 34;
     static constexpr bool kHint = true;
     static constexpr int kLanes = 1;
     static constexpr bool kLocates = false;
-    template <class P> __device__ __forceinline__ void park(P& p)
+    template <class P> __host__ __device__ __forceinline__ constexpr void park(P& p)
     {
         p.io(x); p.io(y); p.io(z); p.io(kx); p.io(ky); p.io(kz); p.io(ix); p.io(iy); p.io(iz);
         p.io(gx); p.io(gy); p.io(gz); p.io(px); p.io(py); p.io(pz); p.io(ci); p.io(cj); p.io(ck); p.io(nsub);
@@ -1446,14 +1446,13 @@ template <typename R> struct VoroW {
     Entry en;
     bool done, segout;
     uint32_t steps, nrecompute, nstuck;
-    static constexpr int kParkWords = 31;
     __device__ __forceinline__ static int cell_of(const View&, int n) { return n; }
     static constexpr bool kHint = true;
     static constexpr int kLanes = 1;
     static constexpr bool kLocates = false;
     __device__ __forceinline__ int entries() const { return en.ne; }
     static constexpr bool kStep = true;
-    template <class P> __device__ __forceinline__ void park(P& p)
+    template <class P> __host__ __device__ __forceinline__ constexpr void park(P& p)
     {
         p.io(x); p.io(y); p.io(z); p.io(kx); p.io(ky); p.io(kz); p.io(sqc);
         p.io(mr); p.io(lm); p.io(mqc); p.io(hb); p.io(tcur); p.io(tend);

@@ -1,0 +1,36 @@
+"""What the kernel headers promise at compile time, checked by compiling small sources against them (no device)."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "skirt7_amd", "csrc")
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+
+pytestmark = pytest.mark.skipif(shutil.which(HIPCC) is None, reason="needs hipcc")
+
+
+def compiles(tmp_path, body):
+    src = tmp_path / "t.hip"
+    src.write_text('#include <hip/hip_runtime.h>\n#include "../../include/skirt7_amd.h"\n#include "sg_mc.hpp"\n'
+                   '#include "sg_split.hpp"\nusing namespace sg;\n' + body)
+    r = subprocess.run([HIPCC, "--offload-arch=gfx950", "-std=c++17", "-fsyntax-only", "-I" + CSRC, str(src)],
+                       capture_output=True, text=True)
+    return r.returncode == 0, r.stdout + r.stderr
+
+
+def test_parking_area_holds_the_parked_state(tmp_path):
+    """The LDS words set aside per lane are the words that a walk's state moves when it is parked."""
+    ok, text = compiles(tmp_path, """
+struct Words {
+    int n = 0;
+    template <typename T> __host__ __device__ constexpr void io(T&) { n += sizeof(T) == 8 ? 2 : 1; }
+};
+template <class W> constexpr int moved() { Hot<W> h{}; Words w; h.park(w); return w.n; }
+#define SAME(W) static_assert(moved<W>() == hot_words<W>(), "parked words")
+SAME(CartW64); SAME(CartW32); SAME(TreeW64); SAME(TreeW64Book); SAME(TreeW32); SAME(TreeW32TopDown);
+SAME(VoroW<double>); SAME(VoroW<float>);
+static_assert(hot_words<CartW64>() == 2 * (9 + 3 + 1 + 3) + 5 + 3 + 2 * 7 + 4, "exact Cartesian walk");
+""")
+    assert ok, text
