@@ -1627,6 +1627,9 @@ template <typename R, int L, int G> struct VoroC {
     static constexpr bool kStep = true;
     __device__ __forceinline__ int entries() const { return en.ne; }
     __device__ __forceinline__ static int place() { return (int)(threadIdx.x & (L - 1)); }
+    // Whether a lane's i-th entry of a list whose walls are among its first kVoroWalls can be one of them.
+    __host__ __device__ static constexpr bool holds_walls(int i) { return i * L < kVoroWalls; }
+    static_assert(L >= 1 && L <= 16 && (L & (L - 1)) == 0, "the group reductions take 1, 2, 4, 8 or 16 lanes");
     __device__ __forceinline__ int hint() const { return lm; }
     // Enters cell mr, whose list is at `list` (0: looked up).
     __device__ __forceinline__ void enter(const View& g, uint32_t list)
@@ -1720,7 +1723,7 @@ template <typename R, int L, int G> struct VoroC {
         for (int i = 0; i < G; i++) {
             double a, b;
             voro_site_fraction(x, y, z, kx, ky, kz, pr.x, pr.y, pr.z, q[i].x, q[i].y, q[i].z, a, b);
-            if (i == 0 || !g.walls_lead) {
+            if (holds_walls(i) || !g.walls_lead) {
                 const bool wall = (i * L < left) & (q[i].id < 0);
                 if (__any(wall)) {
                     double wa, wb;

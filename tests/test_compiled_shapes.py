@@ -34,3 +34,22 @@ SAME(VoroW<double>); SAME(VoroW<float>);
 static_assert(hot_words<CartW64>() == 2 * (9 + 3 + 1 + 3) + 5 + 3 + 2 * 7 + 4, "exact Cartesian walk");
 """)
     assert ok, text
+
+
+def test_voronoi_groups_look_for_walls_where_they_are(tmp_path):
+    """Of a list whose walls are among its first eight entries, dealt out to L lanes, a step looks for walls in every
+    round of L entries that can hold one; group sizes the reductions cannot take are refused."""
+    ok, text = compiles(tmp_path, """
+template <class W> constexpr bool covers()
+{
+    for (int entry = 0; entry < kVoroWalls; entry++)
+        if (!W::holds_walls(entry / W::kLanes)) return false;
+    return true;
+}
+static_assert(covers<VoroC<float, 2, 12>>() && covers<VoroC<float, 4, 6>>() && covers<VoroC<float, 8, 3>>() &&
+              covers<VoroC<double, 16, 2>>(), "walls beyond the entries looked at");
+static_assert(!VoroC<float, 8, 3>::holds_walls(1), "eight lanes take the walls in one round");
+""")
+    assert ok, text
+    for lanes in (3, 32):
+        assert not compiles(tmp_path, "static_assert(sizeof(VoroC<float, %d, 2>) > 0, \"\");\n" % lanes)[0]
