@@ -33,6 +33,14 @@ struct Fail {
         }                                                                                            \
     } while (0)
 
+// The error that a run's error bits report, the library's own checks (bits 2 and 4) before the packets' (bit 1).
+constexpr const char* run_error(int bits)
+{
+    return bits & 2   ? "walk order: a request's sorted place lies beyond the pass's requests"
+           : bits & 4 ? "walk queue: a request names no instrument pixel or packet slot"
+                      : "The optical depth along the path is not a positive number";
+}
+
 // device buffer owned by a host object
 struct DevBuf {
     void* p = nullptr;

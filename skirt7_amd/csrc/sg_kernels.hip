@@ -24,6 +24,8 @@ namespace sg {
 static thread_local std::string g_err;
 void set_error(const std::string& msg) { g_err = msg; }
 
+static void require_no_error(int bits) { SG_REQUIRE(bits == 0, run_error(bits)); }
+
 static int g_device = -1;
 static int g_cus = 256;
 // compaction threshold 0: each pipeline's own default (32 lanes for the lane pipeline, 24 for the walk kernel)
@@ -1883,9 +1885,7 @@ int sg_sim_run(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64_t npp,
             counters[14] = (uint64_t)(lt.total_ms() * 1000.0);
         }
     }
-    SG_REQUIRE(!(err & 2), "walk order: a request's sorted place lies beyond the pass's requests");
-    SG_REQUIRE(!(err & 4), "walk queue: a request names no instrument pixel or packet slot");
-    SG_REQUIRE(err == 0, "The optical depth along the path is not a positive number");
+    require_no_error(err);
     SG_CATCH
 }
 
@@ -2011,7 +2011,7 @@ int sg_sim_run_dust(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64_t
             counters[6] = npp;
             counters[11] = blocks;
         }
-        SG_REQUIRE(r.err == 0, "The optical depth along the path is not a positive number");
+        require_no_error((int)r.err);
         return 0;
     }
     s->counters.zero();
@@ -2044,7 +2044,7 @@ int sg_sim_run_dust(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64_t
         counters[6] = npp;
         counters[11] = blocks;
     }
-    SG_REQUIRE(err == 0, "The optical depth along the path is not a positive number");
+    require_no_error(err);
     SG_CATCH
 }
 
@@ -2201,8 +2201,7 @@ int sg_sim_run_static(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64
         counters[6] = npp;
         counters[11] = blocks;
     }
-    SG_REQUIRE(!(err & 4), "walk queue: a request names no instrument pixel or packet slot");
-    SG_REQUIRE(err == 0, "The optical depth along the path is not a positive number");
+    require_no_error(err);
     SG_CATCH
 }
 
@@ -2692,9 +2691,7 @@ int sg_sim_run_batch(int nmembers, sg_sim* const* sims, const int* ells, const u
         counters[13] = lt.launches();
         counters[14] = (uint64_t)(lt.kernel_ms() * 1000.0);
     }
-    SG_REQUIRE(!(err & 2), "walk order: a request's sorted place lies beyond the pass's requests");
-    SG_REQUIRE(!(err & 4), "walk queue: a request names no instrument pixel or packet slot");
-    SG_REQUIRE(err == 0, "The optical depth along the path is not a positive number");
+    require_no_error(err);
     SG_CATCH
 }
 

@@ -13,8 +13,8 @@ pytestmark = pytest.mark.skipif(shutil.which(HIPCC) is None, reason="needs hipcc
 
 def compiles(tmp_path, body):
     src = tmp_path / "t.hip"
-    src.write_text('#include <hip/hip_runtime.h>\n#include "../../include/skirt7_amd.h"\n#include "sg_mc.hpp"\n'
-                   '#include "sg_split.hpp"\nusing namespace sg;\n' + body)
+    src.write_text('#include <hip/hip_runtime.h>\n#include "../../include/skirt7_amd.h"\n#include "sg_host.hpp"\n'
+                   '#include "sg_mc.hpp"\n#include "sg_split.hpp"\nusing namespace sg;\n' + body)
     r = subprocess.run([HIPCC, "--offload-arch=gfx950", "-std=c++17", "-fsyntax-only", "-I" + CSRC, str(src)],
                        capture_output=True, text=True)
     return r.returncode == 0, r.stdout + r.stderr
@@ -53,3 +53,19 @@ static_assert(!VoroC<float, 8, 3>::holds_walls(1), "eight lanes take the walls i
     assert ok, text
     for lanes in (3, 32):
         assert not compiles(tmp_path, "static_assert(sizeof(VoroC<float, %d, 2>) > 0, \"\");\n" % lanes)[0]
+
+
+def test_run_errors_name_their_cause(tmp_path):
+    """Every kind of run reports its error bits by the same texts: 1 the optical depth, 2 the walk order, 4 the walk
+    queue, the library's own checks first; no entry point words them by itself."""
+    ok, text = compiles(tmp_path, """
+constexpr bool starts(const char* s, const char* w) { return !*w || (*s == *w && starts(s + 1, w + 1)); }
+static_assert(starts(run_error(1), "The optical depth"), "");
+static_assert(starts(run_error(2), "walk order") && starts(run_error(3), "walk order") && starts(run_error(6), "walk order"), "");
+static_assert(starts(run_error(4), "walk queue") && starts(run_error(5), "walk queue"), "");
+""")
+    assert ok, text
+    with open(os.path.join(CSRC, "sg_kernels.hip")) as f:
+        source = f.read()
+    for words in ("The optical depth along", "walk order: a request", "walk queue: a request"):
+        assert words not in source
