@@ -1399,15 +1399,15 @@ static hipStream_t g_split_stream[kStreams] = {};
 static unsigned long long* g_split_host = nullptr;
 static unsigned long long* g_split_host_dev = nullptr;
 static double g_clock_khz = 100000.0;                   // of the device's wall clock
-// Per stream: a run's scene on its way to the device and its result on the way back, in pinned host memory; the event
-// that joins the two streams; and the event that marks, at a run's start, what was enqueued on the default stream.
+// Per stream: a run's scene on its way to the device and its result on the way back, in pinned host memory; and the
+// event that joins the two streams.
 struct RunHost {
     SceneDev scene[kStreams];
     RunResult result[kStreams];
 };
 static RunHost* g_run_host = nullptr;
 static RunHost* g_run_host_dev = nullptr;
-static hipEvent_t g_split_join = nullptr, g_default_mark = nullptr;
+static hipEvent_t g_split_join = nullptr;
 // Work buffers of the split pipeline and of the emission, shared by every simulation of the process
 // (runs are synchronous and driven by one host thread): slot groups, walk queues, progress counters,
 // launch states. Allocated on first use, grown as needed, kept until the process ends.
@@ -1435,23 +1435,16 @@ static void split_resources()
     SG_HIP(hipHostMalloc(reinterpret_cast<void**>(&g_run_host), sizeof(RunHost), hipHostMallocMapped | hipHostMallocCoherent));
     SG_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&g_run_host_dev), g_run_host, 0));
     SG_HIP(hipEventCreateWithFlags(&g_split_join, hipEventDisableTiming));
-    SG_HIP(hipEventCreateWithFlags(&g_default_mark, hipEventDisableTiming));
     int khz = 0;
     if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, g_device) == hipSuccess && khz > 0) g_clock_khz = khz;
 }
 
-// Marks the work enqueued on the default stream so far. The entry points leave work there that they do not wait for
-// (a resampled density, cleared frames and tables), and the transport streams, being non-blocking, do not wait for it
-// by themselves: launch_begin makes a run's stream wait for the mark, unless that work had ended by then (the event and
-// the wait cost 13 us a run where a program makes many: 60 runs of 2e4 packets 26.9 ms with them, 26.1 ms without).
-static bool g_default_busy = false;
-static void mark_default_stream()
-{
-    const hipError_t e = hipStreamQuery(0);
-    g_default_busy = e == hipErrorNotReady;
-    if (g_default_busy) SG_HIP(hipEventRecord(g_default_mark, 0));
-    else SG_HIP(e);
-}
+// Waits for the work enqueued on the default stream. The entry points leave work there that they do not wait for (a
+// resampled density, cleared frames and tables), and the transport streams, being non-blocking, do not wait for it by
+// themselves. By the host: 8 us behind three cleared frames, too little to measure behind an idle stream. An event that the
+// transport streams wait for took 10 us of the host, and 13 us of a run also where the stream was idle; to look first,
+// 14 us.
+static void wait_default_stream() { SG_HIP(hipStreamSynchronize(0)); }
 
 // Held by an entry point that runs kernels on the transport streams: where it leaves by an exception, the streams are
 // waited for first, so that no kernel outlives the call with the pinned words and work buffers that the next one takes.
@@ -1669,12 +1662,10 @@ template <typename R> static void group_buffers(PassGroups<R>& pg, int g, int64_
     zero_at_begin(rb, ta.waves, wbytes);
     zero_at_begin(rb, pg.sl[g].u + (size_t)SU_STATE * P, (size_t)P * sizeof(uint32_t));
 }
-// The run's start on group g's stream, behind the default stream's work up to the mark: what it clears, the packet
-// claims, and the scene from pinned memory. (The groups beyond the first join the first one's stream.)
+// The run's start on group g's stream: what it clears, the packet claims, and the scene from pinned memory.
 static void launch_begin(RunBegin& rb, const McArgs& a, sg_sim* s, int g, int64_t P)
 {
     unsigned long long* words = run_words(g);
-    if (g_default_busy) SG_HIP(hipStreamWaitEvent(g_split_stream[g], g_default_mark, 0));
     zero_at_begin(rb, a.counters, SG_NCOUNTERS * sizeof(unsigned long long));
     zero_at_begin(rb, a.error, sizeof(int));
     zero_at_begin(rb, words + 1, sizeof(unsigned long long));
@@ -1822,7 +1813,7 @@ int sg_sim_run(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64_t npp,
     if (g_pipeline == 1 && count > 0) {
         split_resources();
         fill_args(s, ell, first, count, npp, a, g_run_host->scene[0]);
-        mark_default_stream();
+        wait_default_stream();
         SplitRun run;
         dispatch_split_any(s, a, precision, first, count, run, blocks);
         const RunResult& r = g_run_host->result[0];
@@ -2001,7 +1992,7 @@ int sg_sim_run_dust(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64_t
     dl.cb = cell_boxes(g);
     int blocks = 0;
     if (passes) {
-        mark_default_stream();
+        wait_default_stream();
         SplitRun run;
         run.dust = &dl;
         dispatch_split_any(s, a, precision, first, count, run, blocks);
@@ -2604,7 +2595,7 @@ int sg_sim_run_batch(int nmembers, sg_sim* const* sims, const int* ells, const u
     if (!passes.empty()) {
         // before the shared launches, which the members with passes of their own do not wait for
         split_resources();
-        mark_default_stream();
+        wait_default_stream();
     }
     int blocks = 0;
     LaunchTimer lt;
@@ -2656,7 +2647,7 @@ int sg_sim_run_batch(int nmembers, sg_sim* const* sims, const int* ells, const u
         if (abs_of(s0)) dispatch_batch<true>(s0, rg, owner, precision, blocks, lt);
         else dispatch_batch<false>(s0, rg, owner, precision, blocks, lt);
     }
-    // the shared launches are under way on the default stream, which these do not wait for beyond the mark
+    // the shared launches are under way on the default stream, which these do not wait for
     BatchSum own;
     if (!passes.empty()) {
         if (abs_of(s0)) dispatch_members<true>(passes, precision, own);
