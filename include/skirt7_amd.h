@@ -172,7 +172,8 @@ int sg_sim_run_static(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64
  * grid of the same kind): member i runs packets [0, counts[i]) at wavelength ells[i]. With the
  * event/walk pipeline selected, members of at least sg_set_batch_alone packets run through it, a few at
  * a time on streams of their own, and the rest share the persistent launches; each member's result is its
- * single run. */
+ * single run. counters as sg_sim_run's, summed over the members: [10] and [12] are spans of the whole call,
+ * [14] adds up launches that overlap. */
 int sg_sim_run_batch(int nmembers, sg_sim* const* sims, const int* ells, const uint64_t* counts, int precision,
                      uint64_t* counters);
 /* ---- PanMonteCarloSimulation: dust emission (PanMonteCarloSimulation.cpp:106-340) ------------------- */

@@ -1172,9 +1172,8 @@ int sg_sim_destroy(sg_sim* s)
 }
 } // extern "C"
 
-// Device time of a run's transport: the span of its passes (start/stop on stream 0, or a span
-// measured elsewhere) and the walk kernel's own duration, summed over its launches (the start/stop spans
-// hold one kernel each; the event/walk passes take the duration on the device, PassCtl).
+// Device time of the lane pipeline's launches: the spans between start and stop on stream 0, one kernel each. (The
+// event/walk passes take their times on the device, PassCtl.)
 struct LaunchTimer {
     std::vector<std::pair<hipEvent_t, hipEvent_t>> ev;
     void start()
@@ -1186,19 +1185,10 @@ struct LaunchTimer {
         SG_HIP(hipEventRecord(a, 0));
     }
     void stop() { SG_HIP(hipEventRecord(ev.back().second, 0)); }
-    // a span measured elsewhere that covered `launches` launches of kernel_ms in all
-    void add(double ms, int launches, double kernel_ms)
-    {
-        extra_ms += ms;
-        extra_launches += launches;
-        extra_kernel_ms += kernel_ms;
-    }
-    double extra_ms = 0, extra_kernel_ms = 0;
-    int extra_launches = 0;
-    int launches() const { return (int)ev.size() + extra_launches; }
+    int launches() const { return (int)ev.size(); }
     double total_ms()
     {
-        double t = extra_ms;
+        double t = 0;
         for (auto& p : ev) {
             float ms = 0;
             SG_HIP(hipEventSynchronize(p.second));
@@ -1207,7 +1197,6 @@ struct LaunchTimer {
         }
         return t;
     }
-    double kernel_ms() { return total_ms() - extra_ms + extra_kernel_ms; }
     ~LaunchTimer()
     {
         for (auto& p : ev) { (void)hipEventDestroy(p.first); (void)hipEventDestroy(p.second); }
@@ -1823,7 +1812,7 @@ int sg_sim_run(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64_t npp,
             counters[6] = npp;
             counters[10] = (uint64_t)(r.span * 1000.0 / g_clock_khz);
             counters[11] = blocks;
-            counters[12] = (uint64_t)(r.transport * 1000.0 / g_clock_khz);
+            counters[12] = (uint64_t)((r.last - r.first) * 1000.0 / g_clock_khz);
             counters[13] = run.launches;
             counters[14] = (uint64_t)(r.walk * 1000.0 / g_clock_khz);
         }
@@ -2418,7 +2407,10 @@ struct BatchMember {
 struct BatchSum {
     unsigned long long counters[SG_NCOUNTERS] = {};
     int err = 0, launches = 0, blocks = 0;
-    double transport_ms = 0, walk_ms = 0;
+    double walk_ms = 0;
+    // device clock: the first pass of any member and the end of the last (the members' spans overlap)
+    unsigned long long first = ~0ull, last = 0;
+    double span_ms() const { return last > first ? (last - first) / g_clock_khz : 0.0; }
 };
 
 // Members through event and walk passes, kStreams at a time, each on a stream of its own with one slot group: a pass of one
@@ -2442,7 +2434,8 @@ template <class W, bool ABS> static void run_members(const std::vector<BatchMemb
     auto add = [&](const RunResult& r) {
         for (int k = 0; k < SG_NCOUNTERS; k++) sum.counters[k] += r.counters[k];
         sum.err |= (int)r.err;
-        sum.transport_ms += r.transport / g_clock_khz;
+        sum.first = std::min(sum.first, r.first);
+        sum.last = std::max(sum.last, r.last);
         sum.walk_ms += r.walk / g_clock_khz;
     };
     auto start = [&](int l) {
@@ -2652,7 +2645,6 @@ int sg_sim_run_batch(int nmembers, sg_sim* const* sims, const int* ells, const u
     if (!passes.empty()) {
         if (abs_of(s0)) dispatch_members<true>(passes, precision, own);
         else dispatch_members<false>(passes, precision, own);
-        lt.add(own.transport_ms, own.launches, own.walk_ms);
         if (shared == 0) blocks = own.blocks;
     }
     SG_HIP(hipEventRecord(e1, 0));
@@ -2678,9 +2670,11 @@ int sg_sim_run_batch(int nmembers, sg_sim* const* sims, const int* ells, const u
         counters[6] = total;
         counters[10] = (uint64_t)(ms * 1000.0);
         counters[11] = blocks;
-        counters[12] = (uint64_t)(lt.total_ms() * 1000.0);
-        counters[13] = lt.launches();
-        counters[14] = (uint64_t)(lt.kernel_ms() * 1000.0);
+        // the members' passes run beside the shared launches
+        const double shared_ms = lt.total_ms();
+        counters[12] = (uint64_t)(std::max(shared_ms, own.span_ms()) * 1000.0);
+        counters[13] = lt.launches() + own.launches;
+        counters[14] = (uint64_t)((shared_ms + own.walk_ms) * 1000.0);
     }
     require_no_error(err);
     SG_CATCH

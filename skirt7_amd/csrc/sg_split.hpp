@@ -505,10 +505,10 @@ __global__ void __launch_bounds__(256) k_run_begin(const RunBegin b)
 }
 
 // What a run leaves in pinned host memory: its counters, error bits, and on the device clock its walk kernels'
-// duration and its span from the start and from the first pass on.
+// duration, its span from the start, and the times of its first pass's start and of its end.
 struct RunResult {
     unsigned long long counters[SG_NCOUNTERS];
-    unsigned long long err, walk, span, transport;
+    unsigned long long err, walk, span, first, last;
 };
 struct RunEnd {
     GroupTally tally[2];
@@ -564,7 +564,8 @@ __global__ void __launch_bounds__(256) k_run_end(const RunEnd e)
         e.out->err = (unsigned long long)*e.err;
         e.out->walk = walk;
         e.out->span = now - *e.begin;
-        e.out->transport = now > start ? now - start : 0;
+        e.out->first = min(start, now);
+        e.out->last = now;
     }
 }
 

@@ -158,6 +158,20 @@ def test_batched_members_by_passes(alone, batch, precision):
         np.testing.assert_allclose(m["instr"].frame(0)[0], f, rtol=1e-11, atol=0)
 
 
+@pytest.mark.parametrize("alone", [1, 100000])
+def test_batched_run_reports_its_span(alone):
+    """Members' passes overlap, beside each other and the shared launches: the transport's span lies within the whole
+    call's."""
+    pop = workloads.fit_population(members=8, packets=(1.0e3, 3.0e3), grid_n=(30, 50), pixels=(32, 16), nsamples=2)
+    try:
+        S.set_batch_alone(alone)
+        for _ in range(2):   # the first call allocates the members' buffers
+            c = S.run_batch([m["sim"] for m in pop["members"]], [60000] * 3 + [250000] * 5, precision=SG_MIXED)
+    finally:
+        S.set_batch_alone(3 << 16)
+    assert 0 < c["transport_us"] <= c["kernel_us"]
+
+
 @pytest.mark.parametrize("kind", ["cartesian", "octree"])
 @pytest.mark.parametrize("count,batch", [(1, 0), (513, 0), (3001, 1024)])
 def test_dust_emission_by_passes(kind, count, batch):
