@@ -408,9 +408,9 @@ def main():
 
     # Three figures for the walk kernel. (1) frac: its algorithmic bytes per launch over its own launch
     # duration, measured on a step run with one slot group on one stream, so that each launch has the device to
-    # itself (HIP events on that stream). (2) overlapped: the same ratio over the timed steps, whose two slot
-    # groups' passes share the device, so a launch's duration includes time shared with the other stream's
-    # kernels. (3) device: the timed steps' algorithmic bytes over their wall time.
+    # itself (its duration taken on the device's clock). (2) overlapped: the same ratio over the timed steps, where
+    # the passes of two slot groups (if the run takes two) share the device, so a launch's duration includes time
+    # shared with the other stream's kernels. (3) device: the timed steps' algorithmic bytes over their wall time.
     bytes_steps = algorithmic_bytes(cm)
     launches = max(1, cm["transport_launches"])
     kwalk = cm["walk_kernel_us"] * 1e-6
@@ -445,7 +445,7 @@ def main():
                        "algorithmic_bytes_per_launch": b1 / l1, "kernel_ms_per_launch": 1e3 * k1 / l1,
                        "launches": l1,
                        "overlapped": {"frac": bytes_steps / kwalk / HBM_PEAK, "kernel_ms_per_launch": 1e3 * kwalk / launches,
-                                      "note": "timed steps, two slot groups on two streams: a launch's duration "
+                                      "note": "timed steps: with two slot groups on two streams a launch's duration "
                                               "includes time shared with the other stream's kernels"},
                        "device": {"frac": bytes_steps / wall / HBM_PEAK, "achieved": bytes_steps / wall / 1e9,
                                   "note": "algorithmic bytes of the timed steps over their wall time"}}

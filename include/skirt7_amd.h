@@ -195,7 +195,7 @@ int sg_dust_emission_spectra(sg_dust* d, const double* rho, const double* labs_s
  * weight: PanMonteCarloSimulation::dodustemissionchunk (PanMonteCarloSimulation.cpp:246-340; the cell drawn
  * uniformly for a fraction `bias` of the packets, PanDustSystem::emissionBias) with emission and scattering
  * peel-offs, or dodustselfabsorptionchunk (:160-204: bias 0, peeloffs 0, store_absorption 1). The packets'
- * transport is the stellar packets' (lane pipeline). Their random streams are keyed by (seed, member ^
+ * transport is the stellar packets', in the pipeline that is set. Their random streams are keyed by (seed, member ^
  * stream * 0x9E3779B9): give each emission phase or self-absorption cycle its own stream. One dust component,
  * Cartesian and tree grids. counters as sg_sim_run without the timings. */
 int sg_sim_run_dust(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64_t npp, const double* Lv, double bias,
@@ -254,7 +254,7 @@ int sg_set_pipeline(int mode);
  * finish their walk before the wave re-arms them; by default 32 for the lane pipeline and 24 for
  * the walk kernel). */
 int sg_set_tuning(int block, int waves_per_cu, int compact_lanes);
-/* In-flight packet slots of the event/walk pipeline, split over its two slot groups (0 = the
+/* In-flight packet slots of the event/walk pipeline, split over its slot groups (0 = the
  * default 2^22; otherwise 1024..2^24). No reference counterpart: SKIRT7's chunk size
  * (MonteCarloSimulation.cpp:68-114) sets the CPU work granularity, this the GPU's. */
 int sg_set_slots(int64_t slots);

@@ -1583,9 +1583,12 @@ static void launch_end(const RunEnd& e, hipStream_t st)
 // Slot groups of a run of P slots. A second group hides the drain of the first one's passes, whose last walks
 // leave most of the device idle, but doubles the launches and halves the queues. It pays where walks are long (large
 // trees, Voronoi grids, whose steps cost most) and, in a tree, queues hold enough of them. One and two groups, ms:
-// Voronoi 1e5 sites, 3e4 packets 20.1, 18.9 and 3e5 36.5, 33.4; kd-tree of 5e5 particles, 2.5e5 packets 13.2, 12.7 and
-// 5e5 19.8, 19.4; octree of 7e5 leaves, 4e6 packets 52.7, 52.2 and 4e5 12.1, 12.3; a smaller octree, 2e5 packets 2.75,
-// 3.67 and 3e6 12.9, 13.2; Cartesian 50^3, 3e5 packets 4.1, 4.6, 1e6 8.4, 8.8 and 4e6 26.6, 26.4.
+// Voronoi 1e5 sites, 3e4 packets 20.1, 18.9 and 3e5 36.5, 33.4; Cartesian 50^3, 3e5 packets 4.1, 4.6, 1e6 8.4, 8.8 and
+// 4e6 26.6, 26.4. Trees, mixed, with 7e4, 1.3e5, 2.6e5 and 1e6 packets: octree of 1.3e5 leaves 4.7, 5.1; 5.1, 5.9; 6.0,
+// 6.8; 11.3, 11.9, of 7.2e5 7.5, 7.9; 8.2, 8.8; 9.6, 9.9; 18.2, 18.1; kd-tree of 3.6e5 leaves 5.9, 6.3; 6.9, 7.1; 9.4,
+// 9.3; 22.4, 22.6, of 8e5 7.7, 7.7; 9.2, 8.9; 12.7, 12.1; 32.6, 32.2. The lines, 2^19 cells and 2^17 packets, keep what
+// the kd-trees gain (up to 5%) at a cost of up to 3% to octrees just beyond them. In FP64 the two differ by up to 4%
+// below the lines and 5% beyond, for two groups.
 template <class W> static int slot_groups(int64_t ncells, int64_t P)
 {
     return W::kLanes > 1 || (W::kHint && ncells >= (int64_t)1 << 19 && P >= (int64_t)1 << 17) ? 2 : 1;

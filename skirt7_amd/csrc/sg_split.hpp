@@ -571,7 +571,7 @@ __global__ void __launch_bounds__(256) k_run_end(const RunEnd e)
 
 // Request claims of one wave: chunks of requests by one global atomic each, handed out in order to the lanes
 // that ask. Called by the whole wave; cur/end is the wave's current chunk and last the place of its latest
-// claim (wave-uniform). The chunk follows what is left of the queue, an eighth of a wave's even share at
+// claim (wave-uniform). The chunk follows what is left of the queue, half of a wave's even share of it and at
 // most kClaimChunk: large while the queue is long (few atomics), small near its end and for short queues, so
 // that the last walks are spread over the waves instead of queueing up in a few. Returns whether this lane
 // got request r; a lane that did not finds the queue exhausted.
@@ -649,11 +649,10 @@ __device__ __forceinline__ bool seg_claim(unsigned long long* ctr, uint64_t nq, 
     return ok && want;
 }
 
-// Occupancy target of the walk kernel (waves per SIMD): four for the mixed tree walk, which then
-// takes 108 registers and spills nothing (five fit in 96 registers with 44 bytes of spills per lane
-// and ran 1-2% slower, six slower still); three for the exact tree walk, whose FP64 state needs about 200 registers (two
-// waves do not spill but hide less of the root descents' latency, four spill more); four for the
-// others.
+// Occupancy target of the walk kernel (waves per SIMD), by measurement; registers and spills as the compiler reports
+// them. Four for the mixed tree walk: 128 registers, 2 to 4 spilled (4e6 packets on 7e5 leaves 51.9 ms; three 55.2,
+// five, which spill more, 54.7). Three for the exact tree walk: 168 registers, 68 to 112 spilled (3e5 packets of optical
+// depth 5: 13.0 ms; two 12.8, four 30.4). Four for the others.
 #ifndef SG_WALK_WAVES_PER_EU
 #define SG_WALK_WAVES_PER_EU 4
 #endif
@@ -666,12 +665,15 @@ template <> struct WalkWaves<TreeW32> { static constexpr int value = SG_W32_WAVE
 #define SG_W64_WAVES 3
 #endif
 template <> struct WalkWaves<TreeW64> { static constexpr int value = SG_W64_WAVES; };
-// the exact Cartesian walk spills nothing at three (1e6 packets on 50^3 cells: 9.2 ms; 9.4 at four, 11.1 at five)
+// the exact Cartesian walk at three: 168 registers, 2 to 4 spilled (1e6 packets on 50^3 cells: 9.2 ms; 9.4 at four, 11.1
+// at five)
 template <> struct WalkWaves<CartW64> { static constexpr int value = 3; };
 // Lanes per Voronoi walk and entries per lane and step: 8 x 3 = 24 entries a step, which most lists (19 on average
-// along the walks) fit, at three waves per SIMD, where nothing spills in the walk. On 1e5 sites with 3 x 1e5 packets:
-// 33 ms a run; four lanes x 6 42 ms, 8 x 2 50 ms and 8 x 3 51 ms at four waves (spills), 16 x 2 50 ms; one lane x 16
-// entries (VoroW, as the lane pipeline walks) spilled and took 106 ms.
+// along the walks) fit, at three waves per SIMD: 168 registers, of which the mixed walk spills 5 to 6. On 1e5 sites with
+// 3 x 1e5 packets: 33 ms a run; four lanes x 6 42 ms, 8 x 2 50 ms and 8 x 3 51 ms at four waves (spills), 16 x 2 50 ms; one lane x 16
+// entries (VoroW, as the lane pipeline walks) spilled and took 106 ms. These are mixed runs; the FP64 walk takes the same
+// shape, where it spills 78 to 91 registers (3e4 packets on 3e4 sites 14.1 ms; VoroW in the passes 61, in the lane
+// pipeline 28).
 #ifndef SG_VORO_LANES
 #define SG_VORO_LANES 8
 #endif

@@ -731,8 +731,9 @@ class OligoMonteCarloSimulation:
 
 def run_batch(simulations, counts, ells=None, precision=SG_FP64):
     """Batched population: simulation i runs packets [0, counts[i]) at wavelength ells[i] (default 0)
-    with normalisation L/counts[i], all members in one persistent launch per round. Each member's result
-    equals its own run_packets(ell, 0, count, count); the returned counters are summed over members."""
+    with normalisation L/counts[i]: large members (set_batch_alone) through the event and walk kernels, a few at a
+    time, the others in shared persistent launches beside them. Each member's result equals its own
+    run_packets(ell, 0, count, count); the returned counters are summed over members."""
     sims = list(simulations)
     n = len(sims)
     if n == 0:

@@ -59,7 +59,8 @@ def test_rope_walk_bitexact(arity, search, tree, shift, unit):
 @pytest.mark.parametrize("arity,search", [(8, SG_TOPDOWN), (8, SG_NEIGHBOR), (2, SG_TOPDOWN), (2, SG_NEIGHBOR)])
 def test_rope_walk_beside_inexact_planes(arity, search):
     """A box at 333 with walls at thirds: FP32 holds its planes to 1.5e-5. The rays start within 3e-5 of a plane and
-    run along it, so that entering finer cells a good part of the descents take the child on the plane's other side."""
+    run along it, about an eighth of them between the plane and its place in FP32, so that a descent into finer cells
+    takes the child on the plane's other side."""
     if arity == 8:
         flags = random_tree_flags(8, 7, 0.3, seed=5, minlevel=2)
     else:
