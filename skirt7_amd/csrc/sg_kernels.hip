@@ -2172,6 +2172,7 @@ int sg_sim_run_static(sg_sim* s, int ell, uint64_t first, uint64_t count, uint64
                "sg_sim_run_static: a dust system of several components needs sg_sim_run");
     McArgs a;
     fill_args(s, ell, first, count, npp, a);
+    wait_default_stream();
     int blocks = 0;
     if (a.store_abs) dispatch_static<true>(s, a, precision, blocks);
     else dispatch_static<false>(s, a, precision, blocks);

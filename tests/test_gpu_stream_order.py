@@ -38,8 +38,9 @@ def galaxies():
 
 
 @pytest.mark.parametrize("precision", [SG_FP64, SG_MIXED])
-@pytest.mark.parametrize("batched", [False, True])
-def test_run_behind_resampled_density(galaxies, batched, precision):
+@pytest.mark.parametrize("kind", ["single", "static", "batched"])
+def test_run_behind_resampled_density(galaxies, kind, precision):
+    batched = kind == "batched"
     out, counts = [], []
     for wait in (True, False):
         # from a density that gives other results: a third of the depth
@@ -53,7 +54,8 @@ def test_run_behind_resampled_density(galaxies, batched, precision):
             if wait:
                 _wait(w["dust"])
             if not batched:
-                c = w["sim"].run_packets(0, 0, PACKETS, PACKETS, precision)
+                run = w["sim"].run_packets_static if kind == "static" else w["sim"].run_packets
+                c = run(0, 0, PACKETS, PACKETS, precision)
                 counts.append([c[k] for k in COUNTS])
         if batched:
             try:
